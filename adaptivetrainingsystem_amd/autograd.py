@@ -206,6 +206,14 @@ FUSE_TRANSPOSED_COPIES = True
 DGRAD_FROM_FORWARD_WEIGHTS = True
 
 
+def _fused_grid(dtype, E, rows, n):
+    """Whether a fused float32 training launch has enough 256 x 256 tiles for half of the CUs.  Below that the two-kernel
+    route is faster, because the plain product then runs on small tiles (8 experts x 512 rows, hidden 512, 1408 columns:
+    a fused dgrad is 96 tiles, 125 us, the two launches 60); the results are the same bits.  bfloat16 experts of any
+    size that trains on this card fill the chip."""
+    return dtype != torch.float32 or E * -(-rows // (256 * E)) * -(-n // 256) >= 128
+
+
 def _ffn_forward(x, wgu, wd, offsets, kept, rows, row_src, k, want_wgrad=False):
     """Expert FFN over the grouped rows, keeping the gate/up pre-activations for the backward pass.
     Returns (gu [rows, 2I], h [rows, I], y [rows, H], hT, wplan): with want_wgrad, wplan = the weight-gradient
@@ -215,8 +223,10 @@ def _ffn_forward(x, wgu, wd, offsets, kept, rows, row_src, k, want_wgrad=False):
     tab_gu, tab_d = ops.weight_pointer_table(wgu), ops.weight_pointer_table(wd)
     wplan = ops.wgrad_plan(kept) if want_wgrad and rows > 0 else None
     hT = None
-    both = ops.grouped_gateup_swiglu_save(x, tab_gu, offsets, kept, rows, rows, H, I, a_rows=row_src, a_row_div=k,
-                                          t_col0=wplan[0] if wplan is not None and FUSE_TRANSPOSED_COPIES else None)
+    both = None
+    if _fused_grid(x.dtype, len(wd), rows, 2 * I):
+        both = ops.grouped_gateup_swiglu_save(x, tab_gu, offsets, kept, rows, rows, H, I, a_rows=row_src, a_row_div=k,
+                                              t_col0=wplan[0] if wplan is not None and FUSE_TRANSPOSED_COPIES else None)
     if both is not None:             # prefill-sized groups: one kernel writes the pre-activations and h
         gu, h, hT = both
     else:
@@ -246,7 +256,9 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
                                             t_col0=t_col0, transposed_weights=False)
     else:
         wdT, tab_dT = ops.transpose_batched(wd)                  # [I, H] per expert; kept alive until return
-        pair = ops.grouped_down_dgrad_dsilu(dy, tab_dT, gu, offsets, kept, rows, H, I, t_col0=t_col0)   # one kernel
+        pair = None
+        if _fused_grid(dtype, E, rows, I):
+            pair = ops.grouped_down_dgrad_dsilu(dy, tab_dT, gu, offsets, kept, rows, H, I, t_col0=t_col0)   # one kernel
     dgu = None
     if pair is not None:
         dgu, dguT = pair

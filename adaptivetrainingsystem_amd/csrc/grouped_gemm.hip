@@ -12,7 +12,7 @@
 // n-tile) so that the 32 workgroups of an XCD share operand panels in that XCD's L2.
 //
 // Kernels, by the rows per expert the host sees (launch_grouped):
-//   grouped_gemm_dma16_kernel     bf16, groups above 192 rows (prefill and fine-grained shapes; also the
+//   grouped_gemm_dma16_kernel     bf16, groups above 192 rows and large launches (prefill and fine-grained shapes; also the
 //                                 training instances that save g/u or apply the SwiGLU gradient).  256 x 256
 //                                 tile, 8 waves of 128 x 64 on v_mfma_f32_16x16x32_bf16, K in 64-element
 //                                 slabs that go from memory straight into LDS (buffer_load ... lds: unpadded
@@ -24,6 +24,8 @@
 //                                 128-row tiles of mid-sized groups, the 32 / 64-row weight-streaming tiles of
 //                                 decode-sized groups (optionally sliced along K), and gather sources whose
 //                                 lane offsets do not fit 32 bits.
+//   grouped_gemm_small_kernel     32 and 64-row tiles for launches whose large tiles would leave most CUs idle, see
+//                                 grouped_gemm_small.hpp.
 //   grouped_gemm_kernel           general fallback for K that is not a multiple of a slab (bounds-checked loads).
 #include <math.h>
 
@@ -96,6 +98,12 @@ __device__ __forceinline__ void mma_step<float>(const u32x4_t& wfrag, const u32x
     c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(wfrag.z), __uint_as_float(afrag.z), c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(wfrag.w), __uint_as_float(afrag.w), c, 0, 0, 0);
 }
+
+}  // namespace ats
+
+#include "grouped_gemm_small.hpp"
+
+namespace ats {
 
 // Views of a wave's accumulators, 32 output rows at a time, as groups of 4 consecutive output columns
 // per lane.  ib: 32-row block of the wave's sub-tile, g: group, half: 0 = gate (or the plain product),
@@ -1485,34 +1493,87 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     return ATS_OK;
 }
 
-// Tile configuration by rows per expert: decode-sized groups stream weights
-// with 32-row tiles, mid-sized groups use 128-row tiles, prefill uses 256x256.
+// Time of a launch on one tile configuration, in microseconds, from the number of tiles that the busiest CU gets:
+// every tile costs per_slab for each 128-byte slab of K (with the CU's other resident tiles running beside it) and
+// per_tile for its set-up and epilogue.  min_tiles: below that many tiles per CU nothing hides the latency of a slab,
+// so fewer tiles are not faster.
+struct TileCost {
+    int rows, cols;
+    float per_slab, per_tile;
+    int min_tiles;
+};
+static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs) {
+    const int64_t avg = (max_rows + E - 1) / E;
+    const int64_t tiles = (int64_t)E * ((avg + c.rows - 1) / c.rows) * ((n_cols + c.cols - 1) / c.cols);
+    const int64_t per_cu = (tiles + 255) / 256;
+    return (float)(per_cu > c.min_tiles ? per_cu : c.min_tiles) * (k_slabs * c.per_slab + c.per_tile);
+}
+
+// Tile configuration by the size of the launch: the one with the least estimated time.  The constants were measured on
+// MI355X, one launch of each configuration over [33 .. 5331] x [1024 .. 6144] x [64 .. 4096] products and over 8 and
+// 64 groups of 40 .. 384 rows.  What the rule decides between, in microseconds:
+//   in-block slices of K, 32 rows | 64 rows | 128 rows, register-staged | 256 rows, direct to LDS
+//   bfloat16  128 x 4096 x 4096    17 |  23 |  48 |  44      float32   512 x  512 x  512     9 |   17 |  62 | 120
+//             300 x 4096 x 4096    37 |  34 |  61 |  71                512 x 2816 x  512    25 |   29 |  67 | 122
+//            1024 x 4096 x 4096    98 |  72 |  68 |  94               1000 x 1000 x 1000    33 |   29 | 157 | 262
+//            2048 x 4096 x 4096   192 | 130 |  69 |  97               2048 x 2048 x 2048   219 |  180 | 246 | 467
+//            5331 x 4096 x 4096   472 | 310 | 197 | 184               4096 x 4096 x 4096  1498 | 1193 | 944 | 937
+//   gate/up, 8 groups of 160, I 14336   942 | 762 | 572 | 408
+//   float32 in 2 x 2 tiles of 32 rows without slices of K: 2048 x 512 x 512 19 (128 rows: 67, 256 rows: 122)
+// Two bounds on the choice keep results independent of the route that a training step takes: bfloat16 groups of more
+// than 192 rows always run on the 16 x 16 x 32 kernel and float32 groups of more than 256 rows are not sliced along K,
+// because the fused training launches and the K-major products, which start at those sizes, accumulate in that order
+// (their results equal those of the separate launches bit for bit).
 template <typename T, typename TO, bool SWIGLU>
 static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s) {
-    const int64_t avg = max_rows / (p.E > 0 ? p.E : 1);
-    // (33-48 rows per group would take two 32-row tiles that each stream the weights: measured 1.6x slower
-    // than the 128-row tiles on the gate/up projection of 8 experts)
+    constexpr bool kBf16 = std::is_same<T, bf16_t>::value;
+    constexpr int BK = 128 / (int)sizeof(T);
+    const int E = p.E > 0 ? p.E : 1;
+    const int64_t avg = max_rows / E;
     if constexpr (!SWIGLU) {
         // K slices with more than 32 rows per group: 64-row tiles, so that up to 64 rows stream the weights once
         if (p.k_splits > 1 && avg > 32) return launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
     }
+    // (with a K per group, p.K is the bound on their sum)
+    const int nk = p.k_count ? (p.K / E + BK - 1) / BK : (p.K + BK - 1) / BK;
     if (avg <= 32 || p.k_splits > 1) {
         // Decode: pure weight streaming, 32-row tiles.  (Measured alternatives: narrower tiles with
         // more blocks per CU, and MFMA fragments loaded straight from global memory without LDS,
         // both stream more slowly - the latter is bound by the address rate of 64-line loads.)
+        // Where those are fewer than half of the CUs the sliced tiles fill the chip instead (8 float32 groups of 16
+        // rows, H 512, I 1408: gate/up 25 -> 18 us).
+        if (p.k_splits <= 1 && (int64_t)E * ((p.N_out + 127) / 128) < 128)
+            return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
         if constexpr (SWIGLU) return launch_cfg<T, TO, 32, 256, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
         else return launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
     }
-    // Up to kMidMaxAvgRows rows per group: 128-row tiles with more resident blocks.  Above that the 256 x 256
-    // direct-to-LDS tile wins even when a group is one and a half tiles high (64 experts x 384 rows: gate/up
-    // 745 vs 657, down 782 vs 747 TFLOP/s), because a wave skips the 64-row halves past its group's end.
-    constexpr int64_t kMidMaxAvgRows = 192;
-    if (avg <= kMidMaxAvgRows) {
+    // (columns: output columns per tile, half of the weight rows with the SwiGLU epilogue)
+    constexpr TileCost kSmall32 = kBf16 ? TileCost{32, 32, SWIGLU ? 0.165f : 0.093f, 1.f, SWIGLU ? 1 : 2}
+                                        : TileCost{32, 32, SWIGLU ? 0.40f : 0.18f, 1.5f, 1};
+    constexpr TileCost kSmall64 = kBf16 ? TileCost{64, SWIGLU ? 32 : 64, 0.245f, 1.5f, 1}
+                                        : TileCost{64, SWIGLU ? 32 : 64, 0.58f, 3.f, 1};
+    constexpr TileCost kMid = kBf16 ? TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 0.58f : 1.05f, 5.f, 1}
+                                    : TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 2.0f : 3.65f, 5.f, 1};
+    const float mid = tile_time(kMid, max_rows, E, p.N_out, nk);
+    const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? 1.45f : 7.3f, 7.f, 1}, max_rows, E, p.N_out, nk);
+    const float least_large = mid < big ? mid : big;
+    if (avg <= (kBf16 ? 192 : 256)) {
+        const float small32 = tile_time(kSmall32, max_rows, E, p.N_out, nk);
+        const float small64 = tile_time(kSmall64, max_rows, E, p.N_out, nk);
+        if (small32 < least_large && small32 <= small64)
+            return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
+        if (small64 < least_large) return launch_small<T, TO, 2, 2, 4, 1, SWIGLU>(p, max_rows, s);
+    } else if constexpr (!kBf16) {
+        constexpr TileCost kSeq = TileCost{64, 64, SWIGLU ? 1.4f : 0.74f, 3.f, 1};
+        if (tile_time(kSeq, max_rows, E, p.N_out, nk) < least_large)
+            return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 1, 2, SWIGLU>(p, max_rows, s);
+    }
+    if (mid < big && !(kBf16 && avg > 192)) {
         if constexpr (SWIGLU) return launch_cfg<T, TO, 128, 128, 2, 2, 4, 8, SWIGLU>(p, max_rows, s);
         else return launch_cfg<T, TO, 128, 256, 2, 4, 4, 8, SWIGLU>(p, max_rows, s);
     }
-    // Prefill: 256 x 256 tile, 8 waves (2 per SIMD: one wave's LDS / memory waits are covered by
-    // the other's MFMAs), 128 accumulator registers per lane.
+    // 256 x 256 tile (128 rows where that leaves fewer CUs idle), 8 waves (2 per SIMD: one wave's LDS / memory waits
+    // are covered by the other's MFMAs), 128 accumulator registers per lane.
     return launch_cfg<T, TO, 256, 256, 2, 4, 4, 8, SWIGLU, true>(p, max_rows, s);
 }
 
