@@ -20,10 +20,10 @@
 //                                 two weight stages in the 160 KiB of LDS, one barrier per slab, fragment
 //                                 reads and loads placed among the MFMAs with sched_group_barrier.
 //   grouped_gemm_dma_kernel       the same data path for float32 operands on v_mfma_f32_32x32x2_f32.
-//   grouped_gemm_pipelined_kernel register-staged, two padded (144-byte pitch) or swizzled stages: the
-//                                 128-row tiles of mid-sized groups, the 32 / 64-row weight-streaming tiles of
-//                                 decode-sized groups (optionally sliced along K), and gather sources whose
-//                                 lane offsets do not fit 32 bits.
+//   grouped_gemm_pipelined_kernel register-staged, two padded stages (144-byte pitch): the 128-row tiles of mid-sized
+//                                 groups, the 32 / 64-row tiles that cut K into slices over workgroups, and gather
+//                                 sources whose lane offsets do not fit 32 bits.
+//   grouped_gemm_stream_kernel    decode-sized groups: a stream of weights, see grouped_gemm_stream.hpp.
 //   grouped_gemm_small_kernel     32 and 64-row tiles for launches whose large tiles would leave most CUs idle, see
 //                                 grouped_gemm_small.hpp.
 //   grouped_gemm_kernel           general fallback for K that is not a multiple of a slab (bounds-checked loads).
@@ -102,6 +102,7 @@ __device__ __forceinline__ void mma_step<float>(const u32x4_t& wfrag, const u32x
 }  // namespace ats
 
 #include "grouped_gemm_small.hpp"
+#include "grouped_gemm_stream.hpp"
 
 namespace ats {
 
@@ -531,11 +532,8 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 //   LDS barrier
 //   k-step 3: MFMAs(buf 1) | read k-step 0 of slab t+1
 // Global loads therefore have a whole slab of MFMA time to land before they are needed.
-// SWZ: staged rows are 128 bytes without padding, and the 16-byte chunk c of row R sits in slot c ^ f(R),
-// f(R) = (R & 7) ^ ((R >> 3) & 1) (the 16 rows a quarter wave reads hit all 64 banks once).  The 32 x 256
-// weight-streaming tile then takes 72 KiB instead of 81, and two of its workgroups share a CU.
 template <typename T, typename TO, int BM, int BN, int WM, int WN, int SM, int SN, bool SWIGLU, bool WARM,
-          bool SLICED = false, bool SWZ = false>
+          bool SLICED = false>
 __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_pipelined_kernel(GroupedArgs p) {
     constexpr int NT = WM * WN * 64;
     constexpr int VEC = 16 / (int)sizeof(T);
@@ -545,10 +543,8 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_pipelined_kernel(Gro
     constexpr int RPP = NT / 8;
     constexpr int PA = BM / RPP;
     constexpr int PB = BN / RPP;
-    constexpr int PITCH = SWZ ? 128 : kRowPitch;
+    constexpr int PITCH = kRowPitch;
     constexpr int STAGE = (BM + BN) * PITCH;
-    constexpr int NOFF = SWZ ? 4 : 1;   // fragment offsets per row: one per k-step when the slots are swizzled
-    static_assert(!SWZ || RPP % 16 == 0, "the loader's passes must keep a row's swizzle");
     constexpr int HALF = BN / 2;
     static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "wave tiling");
     static_assert(BM % RPP == 0 && BN % RPP == 0, "loader tiling");
@@ -648,18 +644,14 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_pipelined_kernel(Gro
 
     const int nk = K / BK;
     u32x4_t ra[PA], rb[PB];
-    const int st_off = lrow * PITCH + (SWZ ? (lchunk ^ (lrow & 7) ^ ((lrow >> 3) & 1)) : lchunk) * 16;
+    const int st_off = lrow * PITCH + lchunk * 16;
 
     const int frow = lane & 31;
     const int fgrp = lane >> 5;
-    // (tile rows of a fragment start at multiples of 32, so a lane's swizzle depends on frow alone)
-    const int fswz = (frow & 7) ^ ((frow >> 3) & 1);
-    int a_row_off[TM][NOFF], b_row_off[TN][NOFF];
+    int a_row_off[TM], b_row_off[TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int q = 0; q < NOFF; ++q)
-            a_row_off[i][q] = (wm * (BM / WM) + i * 32 + frow) * PITCH + (SWZ ? ((2 * q + fgrp) ^ fswz) : fgrp) * 16;
+        a_row_off[i] = (wm * (BM / WM) + i * 32 + frow) * PITCH + fgrp * 16;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         int r;
@@ -669,9 +661,7 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_pipelined_kernel(Gro
         } else {
             r = wn * (BN / WN) + j * 32;
         }
-#pragma unroll
-        for (int q = 0; q < NOFF; ++q)
-            b_row_off[j][q] = BM * PITCH + (r + frow) * PITCH + (SWZ ? ((2 * q + fgrp) ^ fswz) : fgrp) * 16;
+        b_row_off[j] = BM * PITCH + (r + frow) * PITCH + fgrp * 16;
     }
     u32x4_t fa[2][TM], fb[2][TN];
 
@@ -692,11 +682,11 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_pipelined_kernel(Gro
     }
 #define PL_READ(stage_, ks_, buf_)                                                                     \
     {                                                                                                  \
-        const unsigned char* s_ = smem + (stage_) * STAGE + (SWZ ? 0 : (ks_) * 32);                    \
+        const unsigned char* s_ = smem + (stage_) * STAGE + (ks_) * 32;                                \
         _Pragma("unroll") for (int i = 0; i < TM; ++i)                                                 \
-            fa[buf_][i] = *reinterpret_cast<const u32x4_t*>(s_ + a_row_off[i][SWZ ? (ks_) : 0]);         \
+            fa[buf_][i] = *reinterpret_cast<const u32x4_t*>(s_ + a_row_off[i]);                          \
         _Pragma("unroll") for (int j = 0; j < TN; ++j)                                                 \
-            fb[buf_][j] = *reinterpret_cast<const u32x4_t*>(s_ + b_row_off[j][SWZ ? (ks_) : 0]);         \
+            fb[buf_][j] = *reinterpret_cast<const u32x4_t*>(s_ + b_row_off[j]);                          \
     }
 #define PL_MMA(buf_)                                                                                   \
     {                                                                                                  \
@@ -1432,38 +1422,34 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     constexpr size_t smem_staged = 2 * (size_t)(BM + BN) * kRowPitch;
     constexpr size_t smem = DMA && dma_lds_bytes(BM, BN) > smem_staged ? dma_lds_bytes(BM, BN) : smem_staged;
     constexpr int BK = 128 / (int)sizeof(T);
-    auto kern_general = grouped_gemm_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
+    // slices of K: the 32 and 64-row tiles, whose only instance is the sliced one of the register-staged kernel
+    constexpr bool kSliced = !DMA && !SWIGLU && (BM == 32 || BM == 64);
     // the L2 warm-up touches pay where blocks share operand panels; the weight-streaming tiles share nothing
     constexpr bool kWarm = BM > 64;
-    // the gate/up weight-streaming tile: unpadded swizzled rows, so that two workgroups fit a CU
-    constexpr bool kSwz = BM == 32 && BN == 256;
-    constexpr size_t smem_pipe = kSwz ? 2 * (size_t)(BM + BN) * 128 : smem_staged;
-    auto kern_pipe = grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, false, kSwz>;
+    auto kern_pipe = grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, kSliced>;
+    auto kern_general = [] {
+        if constexpr (kSliced) return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, true>;
+        else return grouped_gemm_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
+    }();
     auto kern_dma = [] {
         if constexpr (DMA && std::is_same<T, bf16_t>::value) {
             static_assert(BM == 256 && BN == 256 && WM == 2 && WN == 4, "the 16 x 16 x 32 kernel is the 256 x 256 tile");
             return grouped_gemm_dma16_kernel<TO, SM, SN, SWIGLU>;
         } else if constexpr (DMA) return grouped_gemm_dma_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
-        else return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, false, kSwz>;
+        else return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, kSliced>;
     }();
-    // slices of K: the weight-streaming tiles only, in their own instance of the register-staged kernel
-    constexpr bool kCanSlice = !DMA && !SWIGLU && (BM == 32 || BM == 64);
-    const void* kern_sliced = reinterpret_cast<const void*>(kern_pipe);
-    if constexpr (kCanSlice)
-        kern_sliced = reinterpret_cast<const void*>(
-            grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, true, kSwz>);
     if (smem > 64 * 1024) {
         static LdsReservation reserved;      // one per tile configuration (this function is a template)
         hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern_general),
                                               reinterpret_cast<const void*>(kern_pipe),
-                                              reinterpret_cast<const void*>(kern_dma), kern_sliced}, (int)smem);
+                                              reinterpret_cast<const void*>(kern_dma)}, (int)smem);
         if (e != hipSuccess) {
             set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
             return ATS_ERR_LAUNCH;
         }
     }
     const int splits = p.k_splits > 1 ? p.k_splits : 1;
-    if (splits > 1 && (!kCanSlice || p.k_count || p.K % splits != 0 || (p.K / splits) % BK != 0)) {
+    if ((splits > 1) != kSliced || (kSliced && (p.k_count || p.K % splits != 0 || (p.K / splits) % BK != 0))) {
         set_error("grouped GEMM: %d slices of K=%d are not available for this tile configuration", splits, p.K);
         return ATS_ERR_UNSUPPORTED;
     }
@@ -1478,17 +1464,10 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;
     }
-    if constexpr (kCanSlice) {
-        if (splits > 1) {
-            hipLaunchKernelGGL((grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, true, kSwz>),
-                               dim3((unsigned)blocks), dim3(WM * WN * 64), smem_pipe, s, p);
-            return ATS_OK;
-        }
-    }
     // the direct-to-LDS kernel addresses its operands with 32-bit lane offsets
     const bool dma_ok = DMA && p.K % BK == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0;
     auto kern = dma_ok ? kern_dma : (p.K % BK == 0) ? kern_pipe : kern_general;
-    const size_t smem_launch = (!dma_ok && p.K % BK == 0) ? smem_pipe : smem;
+    const size_t smem_launch = (!dma_ok && p.K % BK == 0) ? smem_staged : smem;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WM * WN * 64), smem_launch, s, p);
     return ATS_OK;
 }
@@ -1531,21 +1510,43 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     const int E = p.E > 0 ? p.E : 1;
     const int64_t avg = max_rows / E;
     if constexpr (!SWIGLU) {
-        // K slices with more than 32 rows per group: 64-row tiles, so that up to 64 rows stream the weights once
-        if (p.k_splits > 1 && avg > 32) return launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+        // K in slices over workgroups: 32-row tiles, 64-row tiles where up to 64 rows can stream the weights once
+        if (p.k_splits > 1) {
+            return avg > 32 ? launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s)
+                            : launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+        }
     }
     // (with a K per group, p.K is the bound on their sum)
     const int nk = p.k_count ? (p.K / E + BK - 1) / BK : (p.K + BK - 1) / BK;
-    if (avg <= 32 || p.k_splits > 1) {
-        // Decode: pure weight streaming, 32-row tiles.  (Measured alternatives: narrower tiles with
-        // more blocks per CU, and MFMA fragments loaded straight from global memory without LDS,
-        // both stream more slowly - the latter is bound by the address rate of 64-line loads.)
-        // Where those are fewer than half of the CUs the sliced tiles fill the chip instead (8 float32 groups of 16
-        // rows, H 512, I 1408: gate/up 25 -> 18 us).
-        if (p.k_splits <= 1 && (int64_t)E * ((p.N_out + 127) / 128) < 128)
-            return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
-        if constexpr (SWIGLU) return launch_cfg<T, TO, 32, 256, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
-        else return launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+    // Few rows per group: a stream of weights (E == 1: the row count is exact; several groups vary around their mean, and
+    // a group beyond 32 rows reads its weights twice).  Measured, microseconds, weights from HBM, against the register-
+    // staged 32-row tiles with two slabs in flight that this kernel replaced:
+    //   8 experts top-2, gate/up [28672, 4096]: 1 token 93 -> 77, 20 tokens 315 -> 271 (6.9 TB/s), 64 tokens 317 -> 289
+    //   64 experts top-6, gate/up [2816, 2048]: 3 tokens 51 -> 39, 20 tokens 134 -> 104, 64 tokens 144 -> 117
+    //   down [4096, 14336]: 1 token 142 -> 43, 20 tokens 178 -> 141, 64 tokens 179 -> 157
+    //   128 tokens (32 rows per expert), gate/up: 430 against 343 with 256-row tiles, hence the bound.
+    const int pieces = (int)(((int64_t)p.K * (int)sizeof(T) + 255) / 256);
+    if (avg <= (E == 1 ? 32 : 20) && p.N_out >= 32 && !p.k_count) {
+        if constexpr (SWIGLU) return launch_stream<T, TO, 2, 2, 4, SWIGLU>(p, max_rows, s);
+        else {
+            // Eight waves split K where there are at least four pieces for each (a panel of 16 rows then reads 2 KB of
+            // every row per step): [4096, 4096] x 16 rows 10.3 us against 11.7 with four waves and 14.5 with four waves
+            // and 32 rows.  With more rows per group the activations, read once per panel, ask for panels of 32 rows
+            // (8 experts x 16 rows, [4096, 14336]: 157 against 167).  A short K keeps four waves (64 experts, [2048, 1408],
+            // 3 tokens: 23 against 37 us).
+            const int64_t groups = max_rows < E ? max_rows : E;
+            if (pieces >= 32 && (pieces >= 64 || groups * p.N_out <= 16 * 1024)) {
+                if (E == 1 || avg <= 8) return launch_stream<T, TO, 1, 2, 8, SWIGLU>(p, max_rows, s);
+                return launch_stream<T, TO, 2, 2, 8, SWIGLU>(p, max_rows, s);
+            }
+            if (groups * p.N_out < 32 * 256) return launch_stream<T, TO, 1, 2, 4, SWIGLU>(p, max_rows, s);
+            return launch_stream<T, TO, 2, 2, 4, SWIGLU>(p, max_rows, s);
+        }
+    }
+    if constexpr (!SWIGLU) {
+        // up to 32 rows per expert against a long K (8 experts x 32 rows, [4096, 14336]: 183 us; two slices of K over
+        // workgroups 196, 256-row tiles 264)
+        if (avg <= 32 && pieces >= 64 && p.N_out >= 32 && !p.k_count) return launch_stream<T, TO, 2, 4, 4, SWIGLU>(p, max_rows, s);
     }
     // (columns: output columns per tile, half of the weight rows with the SwiGLU epilogue)
     constexpr TileCost kSmall32 = kBf16 ? TileCost{32, 32, SWIGLU ? 0.165f : 0.093f, 1.f, SWIGLU ? 1 : 2}
@@ -1557,7 +1558,11 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     const float mid = tile_time(kMid, max_rows, E, p.N_out, nk);
     const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? 1.45f : 7.3f, 7.f, 1}, max_rows, E, p.N_out, nk);
     const float least_large = mid < big ? mid : big;
-    if (avg <= (kBf16 ? 192 : 256)) {
+    // (two full rounds of 256-row tiles: nothing is idle, and groups of unequal size fit them better; 8 experts with 20-45
+    // rows each, gate/up [28672, 4096]: 343 us against 372 in 32-row tiles)
+    const int64_t big_tiles = (int64_t)E * ((avg + 255) / 256) * ((p.N_out + (SWIGLU ? 127 : 255)) / (SWIGLU ? 128 : 256));
+    if (big_tiles >= 512) {
+    } else if (avg <= (kBf16 ? 192 : 256)) {
         const float small32 = tile_time(kSmall32, max_rows, E, p.N_out, nk);
         const float small64 = tile_time(kSmall64, max_rows, E, p.N_out, nk);
         if (small32 < least_large && small32 <= small64)
@@ -1572,8 +1577,8 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
         if constexpr (SWIGLU) return launch_cfg<T, TO, 128, 128, 2, 2, 4, 8, SWIGLU>(p, max_rows, s);
         else return launch_cfg<T, TO, 128, 256, 2, 4, 4, 8, SWIGLU>(p, max_rows, s);
     }
-    // 256 x 256 tile (128 rows where that leaves fewer CUs idle), 8 waves (2 per SIMD: one wave's LDS / memory waits
-    // are covered by the other's MFMAs), 128 accumulator registers per lane.
+    // 256 x 256 tile, 8 waves (2 per SIMD: one wave's LDS / memory waits are covered by the other's MFMAs), 128
+    // accumulator registers per lane.
     return launch_cfg<T, TO, 256, 256, 2, 4, 4, 8, SWIGLU, true>(p, max_rows, s);
 }
 

@@ -209,7 +209,8 @@ inline void pick_supertile(int n_tiles, int* SM, int* SN) {
 inline int64_t grid_blocks(int64_t max_rows, int E, int BM, int n_tiles, int SM, int SN, bool aligned) {
     const int n_groups = (n_tiles + SN - 1) / SN;
     // sum of ceil(count / BM) <= max_rows / BM + E; rounding every group up to a multiple of SM adds < SM each
-    const int64_t mtiles_bound = max_rows / BM + (int64_t)E * (aligned ? SM : 1);
+    int64_t mtiles_bound = max_rows / BM + (int64_t)E * (aligned ? SM : 1);
+    if (!aligned && mtiles_bound > max_rows) mtiles_bound = max_rows;      // a tile has at least one row
     const int64_t supertiles = (mtiles_bound + SM - 1) / SM * n_groups;
     const int64_t blocks = supertiles * kSuperBlocks;
     const int64_t round = (int64_t)kNumXcd * kSuperBlocks;

@@ -80,10 +80,5 @@ class FusedSwiGLU(nn.Module):
         w = self._stacked_up_gate(x2.dtype)
         start = torch.zeros(1, dtype=torch.int32, device=x.device)
         count = torch.full((1,), n, dtype=torch.int32, device=x.device)
-        splits = ops.down_k_splits(1, n, 2 * I, H, x2.dtype) if I % 8 == 0 and n <= 32 else 1
-        if splits > 1:
-            h = ops.swiglu_partials(ops.grouped_down_splitk(x2, ops.weight_pointer_table([w]), start, count, n,
-                                                            2 * I, H, splits), x2.dtype)
-        else:
-            h = ops.grouped_gateup_swiglu(x2, ops.weight_pointer_table([w]), start, count, n, n, H, I)
+        h = ops.grouped_gateup_swiglu(x2, ops.weight_pointer_table([w]), start, count, n, n, H, I)
         return h.view(out_shape)

@@ -1,0 +1,69 @@
+"""Grouped products of a few rows per group (the weight-streaming tiles) against float64: one row up to the last row of a
+tile and beyond it, groups without rows, output columns that do not fill a tile, K from one 16-byte piece over ragged
+256-byte pieces to several pieces per wave, four and eight waves, panels of 16 and 32 weight rows."""
+import pytest
+import torch
+
+from tests.test_gpu_parity import A, BF16_TOL, F32_TOL, gen, ops, rel_err, same_bits  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+#        rows per group            N     K
+CASES = [([1], 32, 8), ([5, 0, 17], 40, 136), ([16, 32, 33, 0, 2], 72, 1000), ([32], 4096, 4160), ([1, 2], 1032, 8200),
+         ([20, 15, 40], 264, 8192), ([3] * 20, 2048, 1408), ([31, 1, 29], 136, 16384), ([9], 3000, 2048)]
+
+
+@pytest.mark.parametrize("counts,N,K", CASES)
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                             (torch.bfloat16, torch.float32)])
+def test_stream_tiles_plain(ops, gpu, counts, N, K, dtype, out_dtype):  # noqa: F811
+    print("case stream tiles", counts, N, K, dtype, out_dtype, flush=True)
+    g = gen(311)
+    E, n = len(counts), sum(counts)
+    w = [(torch.randn(N, K, generator=g) * 0.1).to(dtype).to(gpu) for _ in range(E)]
+    count = torch.tensor(counts, dtype=torch.int32)
+    start = (torch.cumsum(count, 0) - count).to(torch.int32).to(gpu)
+    count = count.to(gpu)
+    a = torch.randn(n + 3, K, generator=g).to(dtype).to(gpu)
+    src = torch.randint(0, 2 * (n + 3), (n,), generator=g).to(torch.int32).to(gpu)
+    tab = ops.weight_pointer_table(w)
+    out = ops.grouped_gemm_nt(tab, K, N, start, count, n + 2, n, N, K, a=a, out_dtype=out_dtype)
+    gathered = ops.grouped_gemm_nt(tab, K, N, start, count, n + 2, n, N, K, a=a, a_rows=src, a_row_div=2, out_dtype=out_dtype)
+    copied = ops.grouped_gemm_nt(tab, K, N, start, count, n + 2, n, N, K, a=a[(src // 2).long()].contiguous(),
+                                 out_dtype=out_dtype)
+    assert same_bits(gathered[:n], copied[:n])
+    off, tol = 0, F32_TOL if dtype == torch.float32 else BF16_TOL
+    for e, c in enumerate(counts):
+        if c:
+            assert rel_err(out[off:off + c], a[off:off + c].cpu().double() @ w[e].cpu().double().T) <= tol
+        off += c
+    # rows outside the groups are not written
+    lib = __import__("adaptivetrainingsystem_amd._lib", fromlist=["load"]).load()
+    buf = torch.full((n + 2, N), 7.0, dtype=out_dtype, device=gpu)
+    tag = lambda t: 0 if t == torch.float32 else 1
+    assert lib.ats_grouped_gemm_nt(a.data_ptr(), None, K, n + 3, None, 1, tab.data_ptr(), K, N, buf.data_ptr(), N,
+                                   start.data_ptr(), count.data_ptr(), None, E, n, N, K, tag(dtype), tag(out_dtype),
+                                   None) == 0
+    torch.cuda.synchronize()
+    assert torch.all(buf[n:] == 7.0) and same_bits(buf[:n], out[:n])
+
+
+@pytest.mark.parametrize("counts,I,H", [([1], 32, 8), ([5, 0, 17], 40, 136), ([16, 32, 0, 20], 72, 1000), ([32], 1032, 4096),
+                                        ([33, 2, 7], 200, 2048)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_stream_tiles_swiglu(ops, gpu, counts, I, H, dtype):  # noqa: F811
+    print("case stream tiles swiglu", counts, I, H, dtype, flush=True)
+    g = gen(312)
+    E, n = len(counts), sum(counts)
+    w = [(torch.randn(2 * I, H, generator=g) * 0.1).to(dtype).to(gpu) for _ in range(E)]
+    count = torch.tensor(counts, dtype=torch.int32)
+    start = (torch.cumsum(count, 0) - count).to(torch.int32).to(gpu)
+    a = torch.randn(n, H, generator=g).to(dtype).to(gpu)
+    h = ops.grouped_gateup_swiglu(a, ops.weight_pointer_table(w), start, count.to(gpu), n, n, H, I)
+    off = 0
+    for e, c in enumerate(counts):
+        if c:
+            r = a[off:off + c].cpu().double() @ w[e].cpu().double().T
+            ref = torch.nn.functional.silu(r[:, :I]) * r[:, I:]
+            assert rel_err(h[off:off + c], ref) <= (F32_TOL if dtype == torch.float32 else BF16_TOL)
+        off += c
