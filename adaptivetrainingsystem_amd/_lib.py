@@ -118,6 +118,8 @@ _SIGNATURES = {
                             c_void_p]),
     "ats_combine_scatter_add": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
                                         c_int, c_void_p]),
+    "ats_moe_forward_layout": (c_int, [c_int64] + [c_int] * 7 + [c_void_p]),
+    "ats_moe_forward": (c_int, [c_void_p] * 11 + [c_int64] + [c_int] * 6 + [c_float, c_int, c_float, c_int, c_void_p]),
     "ats_row_dot": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int, c_int,
                             c_void_p]),
     "ats_row_dot_copy": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int64, c_int,

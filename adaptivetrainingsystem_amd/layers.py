@@ -485,7 +485,7 @@ class MoEFFNLayer(nn.Module):
                                "dropped_tokens": 0}
         self._wcache_key = None
         self._wcache = None
-        self.last_plan = None
+        self._last_plan = None
         self.stage_timer = None            # set to a profiling.StageTimer to time each stage with HIP events
         nn.init.normal_(self.gate.weight, mean=0.0, std=0.01)
 
@@ -497,18 +497,40 @@ class MoEFFNLayer(nn.Module):
         self._wcache_key = None
         self._wcache = None
 
+    def _expert_weights(self):
+        """([gate/up weights], [down weights]) of the experts as they are now.  Read from the modules' own dictionaries:
+        attribute access through nn.Module costs 0.6 us a step, 200 us a pass with 64 experts."""
+        try:
+            mods = [ex._modules for ex in self._modules["experts"]._modules.values()]
+            return ([m["gate_up_proj"]._parameters["weight"] for m in mods],
+                    [m["down_proj"]._parameters["weight"] for m in mods])
+        except (KeyError, AttributeError):       # experts with other innards (a parametrised weight, say)
+            return [ex.gate_up_proj.weight for ex in self.experts], [ex.down_proj.weight for ex in self.experts]
+
     def _weight_tables(self, dtype: torch.dtype, device: torch.device):
-        params = []
-        for ex in self.experts:
-            params.append(ex.gate_up_proj.weight)
-            params.append(ex.down_proj.weight)
-        key = (dtype, device, tuple((p.data_ptr(), p._version if p.dtype != dtype else 0) for p in params))
+        gu, dn = self._expert_weights()
+        params = gu + dn
+        key = (dtype, device, [p.data_ptr() for p in params], [p._version for p in params if p.dtype != dtype])
         if key != self._wcache_key:
-            wgu = [_as_dtype(ex.gate_up_proj.weight, dtype) for ex in self.experts]
-            wd = [_as_dtype(ex.down_proj.weight, dtype) for ex in self.experts]
+            wgu = [_as_dtype(w, dtype) for w in gu]
+            wd = [_as_dtype(w, dtype) for w in dn]
             self._wcache = (ops.weight_pointer_table(wgu), ops.weight_pointer_table(wd), wgu, wd)
             self._wcache_key = key
         return self._wcache
+
+    @property
+    def last_plan(self):
+        """Routing tensors of the last forward pass (None before the first)."""
+        plan = self._last_plan
+        if isinstance(plan, tuple):              # an inference pass: the names are given out when somebody asks
+            handle, aux = plan
+            plan = {"capacity": handle[5], "aux": aux.reshape(1), **ops.moe_plan_views(handle)}
+            self._last_plan = plan
+        return plan
+
+    @last_plan.setter
+    def last_plan(self, plan):
+        self._last_plan = plan
 
     def forward(self, x: torch.Tensor, add_onto: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
                 ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -538,9 +560,11 @@ class MoEFFNLayer(nn.Module):
         else:
             raise AtsError(f"MoEFFNLayer: capacity_mode {self.capacity_mode!r}")
 
-        params = [self.gate.weight] + [ex.gate_up_proj.weight for ex in self.experts] + \
-                 [ex.down_proj.weight for ex in self.experts]
-        if _wants_grad(x, *params):
+        params = None
+        if torch.is_grad_enabled():
+            gu, dn = self._expert_weights()
+            params = [self.gate.weight] + gu + dn
+        if params is not None and _wants_grad(x, *params):
             if add_onto is not None:
                 raise AtsError("MoEFFNLayer: add_onto is an inference option (autograd adds the output itself)")
             stats: Dict[str, Any] = {}
@@ -555,12 +579,26 @@ class MoEFFNLayer(nn.Module):
             return out.view(B, L, H), aux
 
         tm = self.stage_timer
+        variant = {"softmax_topk": ROUTE_SOFTMAX_TOPK, "topk_softmax": ROUTE_TOPK_SOFTMAX}[self.routing]
+        if tm is None and not (self.training and self.noise_std > 0) and T > 0 and C > 0:
+            fused_add = add_onto is not None and self._can_add_onto(add_onto, x_flat, T, H, k)
+            if add_onto is None or fused_add:
+                wgu_ptrs, wd_ptrs, _, _ = self._weight_tables(x.dtype, x.device)
+                target, rows_to = add_onto if fused_add else (None, None)
+                out, aux, handle = ops.moe_forward(x_flat, _as_dtype(self.gate.weight, x.dtype), self.router_logit_bias,
+                                                   wgu_ptrs, wd_ptrs, I, k, C, self.routing_temperature, variant,
+                                                   self.load_balancing_weight, target, rows_to)
+                self._last_plan = (handle, aux)
+                if self.training:
+                    self._update_routing_stats(self.last_plan, T)
+                return (out if fused_add else out.view(B, L, H)), aux
+
+        # the same stages one by one: timed, with noise on the routing logits, or at sizes outside the native call
         with stage(tm, "router_logits"):
             logits = ops.router_logits(x_flat, _as_dtype(self.gate.weight, x.dtype), self.router_logit_bias)
         clean_logits = logits
         if self.training and self.noise_std > 0:
             logits = logits + torch.randn_like(logits) * self.noise_std
-        variant = {"softmax_topk": ROUTE_SOFTMAX_TOPK, "topk_softmax": ROUTE_TOPK_SOFTMAX}[self.routing]
         with stage(tm, "route_topk"):
             route = ops.route_topk(logits, k, self.routing_temperature, variant, self.load_balancing_weight)
             if logits is not clean_logits:      # importance comes from the noise-free logits (model.py:1190-1192)
@@ -586,8 +624,7 @@ class MoEFFNLayer(nn.Module):
             out = None
             if add_onto is not None:
                 target, rows_to = add_onto
-                if target.dim() != 2 or target.shape[1] != H or target.dtype != x.dtype or rows_to.numel() != T:
-                    raise AtsError("MoEFFNLayer: add_onto needs a [rows, hidden] tensor of x's dtype and one row id per token")
+                self._can_add_onto(add_onto, x_flat, T, H, k)
                 if y.dim() == 2 and ops.combine_scatter_add(y, plan["row_of"], route["weights"], T, k, target, rows_to):
                     out = target
             if out is None:
@@ -603,6 +640,16 @@ class MoEFFNLayer(nn.Module):
         if self.training:
             self._update_routing_stats(plan, T)
         return (out if add_onto is not None else out.view(B, L, H)), route["aux"][0]
+
+    @staticmethod
+    def _can_add_onto(add_onto, x, T: int, H: int, k: int) -> bool:
+        """Checks the operands of add_onto; whether the native call serves them (an unsliced down projection, sizes and
+        alignment of the fused combine)."""
+        target, rows_to = add_onto
+        if target.dim() != 2 or target.shape[1] != H or target.dtype != x.dtype or rows_to.numel() != T:
+            raise AtsError("MoEFFNLayer: add_onto needs a [rows, hidden] tensor of x's dtype and one row id per token")
+        return (k <= 8 and H % 8 == 0 and target.is_contiguous() and target.data_ptr() % 16 == 0
+                and rows_to.dtype == torch.int32 and rows_to.is_contiguous() and x.data_ptr() % 16 == 0)
 
     def _update_routing_stats(self, plan, total_tokens: int) -> None:
         hist = plan["hist"].cpu()

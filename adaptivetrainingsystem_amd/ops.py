@@ -7,6 +7,7 @@ GPU; there is no CPU path.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -536,6 +537,80 @@ def combine_partials(parts: torch.Tensor, row_of: torch.Tensor, weights: torch.T
     check(_lib.load().ats_combine_partials(parts.data_ptr(), S, rows * H, row_of.contiguous().data_ptr(),
                                            weights.contiguous().data_ptr(), _ptr(residual), out.data_ptr(),
                                            num_tokens, int(k), H, _tag(out), _stream()), "ats_combine_partials")
+    return out
+
+
+# --------------------------------------------------------------------------- the MoE layer as one call
+_MOE_FIELDS = ("logits", "indices", "weights", "routed", "prob_colsum", "slot", "token_map", "hist", "kept", "offsets",
+               "row_src", "row_of", "status")
+_moe_layouts: dict = {}        # sizes -> ctypes array of byte offsets (numbers only)
+
+
+def _moe_layout(T: int, H: int, I: int, E: int, k: int, C: int, k_splits: int, tag: int):
+    key = (T, H, I, E, k, C, k_splits, tag)
+    layout = _moe_layouts.get(key)
+    if layout is None:
+        layout = (ctypes.c_int64 * 19)()
+        check(_lib.load().ats_moe_forward_layout(*key, layout), "ats_moe_forward_layout")
+        if len(_moe_layouts) >= 256:
+            _moe_layouts.clear()
+        _moe_layouts[key] = layout
+    return layout
+
+
+def moe_forward(x: torch.Tensor, gate: torch.Tensor, gate_bias: Optional[torch.Tensor], w_gu_ptrs: torch.Tensor,
+                w_d_ptrs: torch.Tensor, I: int, k: int, C: int, temperature: float, variant: int,
+                load_balancing_weight: float, target: Optional[torch.Tensor] = None,
+                target_rows: Optional[torch.Tensor] = None):
+    """The layer's inference stages (router .. combine) queued by one native call: x [T, H], gate [E, H] of x's dtype,
+    pointer tables over the expert weights.  Returns (out [T, H], aux float32 scalar, plan); with target / target_rows the
+    result is added onto those rows of target, which is returned as out.  moe_plan_views(plan) names the routing tensors."""
+    _need_gpu(x, gate, gate_bias, w_gu_ptrs, w_d_ptrs, target, target_rows)
+    T, H = x.shape
+    E = gate.shape[0]
+    dev, dtype, tag = x.device, x.dtype, _tag(x)
+    if gate.shape[1] != H or gate.dtype != dtype or w_gu_ptrs.numel() != E or w_d_ptrs.numel() != E:
+        raise AtsError(f"moe_forward: x {tuple(x.shape)}/{dtype}, gate {tuple(gate.shape)}/{gate.dtype}, {w_gu_ptrs.numel()} experts")
+    if not (x.is_contiguous() and gate.is_contiguous()):
+        raise AtsError("moe_forward: x and the gate weight must be contiguous")
+    if gate_bias is not None:
+        if gate_bias.numel() != E:
+            raise AtsError("moe_forward: bias must have one entry per expert")
+        gate_bias = gate_bias.to(torch.float32).contiguous()
+    splits = 1
+    if target is None:
+        if k <= 8 and H % 8 == 0:
+            splits = down_k_splits(E, min(T * k, E * C), H, I, dtype)
+        out = torch.empty(T, H, dtype=dtype, device=dev)
+    else:
+        out = target
+    layout = _moe_layout(T, H, I, E, k, C, splits, tag)
+    plan = torch.empty(layout[15], dtype=torch.uint8, device=dev)
+    scratch = torch.empty(layout[17], dtype=torch.uint8, device=dev)
+    aux = torch.empty((), dtype=torch.float32, device=dev)
+    check(_lib.load().ats_moe_forward(x.data_ptr(), gate.data_ptr(), _ptr(gate_bias), w_gu_ptrs.data_ptr(),
+                                      w_d_ptrs.data_ptr(), out.data_ptr(), _ptr(target_rows), aux.data_ptr(),
+                                      plan.data_ptr(), scratch.data_ptr(), layout, T, H, I, E, k, C, splits,
+                                      float(temperature), variant, float(load_balancing_weight), tag, _stream()),
+          "ats_moe_forward")
+    return out, aux, (plan, layout, T, E, k, C)
+
+
+def moe_plan_views(handle) -> dict:
+    """The routing tensors of a moe_forward call, as route_topk and dispatch_plan return them."""
+    plan, layout, T, E, k, C = handle
+    n = T * k
+    shapes = {"logits": (T, E), "indices": (T, k), "weights": (T, k), "routed": (E,), "prob_colsum": (E,), "slot": (n,),
+              "token_map": (E, C), "hist": (E,), "kept": (E,), "offsets": (E + 1,), "row_src": (min(n, E * C),),
+              "row_of": (n,), "status": (1,)}
+    out = {}
+    for i, name in enumerate(_MOE_FIELDS):
+        count = 1
+        for d in shapes[name]:
+            count *= d
+        dt = torch.float32 if name in ("logits", "weights", "prob_colsum") else torch.int32
+        out[name] = plan[layout[i]:layout[i] + 4 * count].view(dt).view(shapes[name])
+    del out["routed"]          # the same counts as hist
     return out
 
 

@@ -195,13 +195,19 @@ def reset_performance_monitor() -> None:
     _GLOBAL_MONITOR.reset()
 
 
-@contextmanager
-def _null_range():
-    yield
+class _NullRange:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NULL_RANGE = _NullRange()
 
 
 def stage(timer, name: str):
-    return timer.range(name) if timer is not None else _null_range()
+    return timer.range(name) if timer is not None else _NULL_RANGE
 
 
 def calibrate_mfma(shape: str = "16x16x32", random_operands: bool = True, iters: int = 0, reps: int = 4):

@@ -260,6 +260,42 @@ int ats_combine_partials(const float* parts, int n_parts, int64_t part_stride, c
                          const float* w, const void* residual, void* out, int64_t T, int k, int H,
                          int out_dtype, ats_stream_t stream);
 
+/* ---- The whole layer, inference -------------------------------------------
+ * ats_router_logits, ats_route_topk, ats_dispatch_plan, ats_grouped_gateup_swiglu, ats_grouped_down and
+ * ats_combine (with out_rows: ats_combine_scatter_add onto `out`; with k_splits > 1: ats_grouped_down_splitk and
+ * ats_combine_partials) queued by one call, MoEFFNLayer.forward (moe_cuda_wrapper.py:414-470) without gradients.
+ * ats_moe_forward_layout fills `layout` (ATS_MOE_LAYOUT_COUNT values): the byte offsets of the intermediate
+ * integers and floats inside `plan`, its size, the offset of the expert outputs inside `scratch` and its size.
+ * Both buffers 16-byte aligned; scratch is free again when the call's work is done, plan holds the routing
+ * (rows of ats_dispatch_plan and ats_route_topk).  aux: one float. */
+enum {
+    ATS_MOE_LAYOUT_LOGITS = 0,  /* float [T, E] */
+    ATS_MOE_LAYOUT_INDICES,     /* int32 [T, k] */
+    ATS_MOE_LAYOUT_WEIGHTS,     /* float [T, k] */
+    ATS_MOE_LAYOUT_ROUTED,      /* int32 [E], assignments per expert (ats_route_topk's hist) */
+    ATS_MOE_LAYOUT_PROB_COLSUM, /* float [E] */
+    ATS_MOE_LAYOUT_SLOT,        /* int32 [T*k] */
+    ATS_MOE_LAYOUT_TOKEN_MAP,   /* int32 [E, C] */
+    ATS_MOE_LAYOUT_HIST,        /* int32 [E] */
+    ATS_MOE_LAYOUT_KEPT,        /* int32 [E] */
+    ATS_MOE_LAYOUT_OFFSETS,     /* int32 [E+1] */
+    ATS_MOE_LAYOUT_ROW_SRC,     /* int32 [min(T*k, E*C)] */
+    ATS_MOE_LAYOUT_ROW_OF,      /* int32 [T*k] */
+    ATS_MOE_LAYOUT_STATUS,      /* int32 [1] */
+    ATS_MOE_LAYOUT_ROUTE_WS,
+    ATS_MOE_LAYOUT_PLAN_WS,
+    ATS_MOE_LAYOUT_PLAN_BYTES,
+    ATS_MOE_LAYOUT_Y,
+    ATS_MOE_LAYOUT_SCRATCH_BYTES,
+    ATS_MOE_LAYOUT_COUNT
+};
+int ats_moe_forward_layout(int64_t T, int H, int I, int E, int k, int C, int k_splits, int dtype, int64_t* layout);
+int ats_moe_forward(const void* x, const void* gate, const float* gate_bias, const void* const* w_gu,
+                    const void* const* w_d, void* out, const int32_t* out_rows, float* aux, void* plan,
+                    void* scratch, const int64_t* layout, int64_t T, int H, int I, int E, int k, int C,
+                    int k_splits, float temperature, int variant, float load_balancing_weight, int dtype,
+                    ats_stream_t stream);
+
 /* ---- Mixture-of-Depths helpers -------------------------------------------
  * score[t] = x[t,:] . w[:] (+ bias[0]); optionally prob[t] = sigmoid(score/temperature)
  * (MoDRouter.forward, model.py:926-936). */

@@ -67,3 +67,30 @@ def test_stream_tiles_swiglu(ops, gpu, counts, I, H, dtype):  # noqa: F811
             ref = torch.nn.functional.silu(r[:, :I]) * r[:, I:]
             assert rel_err(h[off:off + c], ref) <= (F32_TOL if dtype == torch.float32 else BF16_TOL)
         off += c
+
+
+@pytest.mark.parametrize("T,k,mode,onto", [(1, 2, "none", False), (3, 6, "none", False), (40, 2, "fcfs", False),
+                                           (64, 2, "fcfs", True), (300, 3, "fcfs", True), (700, 2, "none", False)])
+def test_native_layer_call_equals_the_stages(A, gpu, T, k, mode, onto):  # noqa: F811
+    """The inference pass queued by one native call: bits, routing tensors and auxiliary loss of the stages run one by one
+    (which a stage timer selects)."""
+    from adaptivetrainingsystem_amd import profiling
+    from adaptivetrainingsystem_amd import workloads as W
+    print("case native layer", T, k, mode, onto, flush=True)
+    ov = {"batch": 1, "seq": T, "hidden": 256, "num_experts": 8, "top_k": k, "intermediate": 136, "dtype": torch.bfloat16}
+    w = W.make_moe_workload("c1_cpu_reference", device=gpu, overrides=ov)
+    layer = W.build_layer(w, mode)
+    base = torch.randn(2 * T, 256, generator=gen(313)).bfloat16().to(gpu)
+    rows = torch.randperm(2 * T, generator=gen(314))[:T].to(torch.int32).to(gpu)
+    run = lambda: layer(w.x, add_onto=(base.clone(), rows)) if onto else layer(w.x)
+    got, got_aux = run()
+    plan = layer.last_plan
+    layer.stage_timer = profiling.StageTimer()
+    want, want_aux = run()
+    assert same_bits(got, want) and torch.equal(got_aux, want_aux)
+    ref = layer.last_plan
+    assert plan["capacity"] == ref["capacity"] and set(ref) <= set(plan)
+    for name in ("logits", "indices", "weights", "hist", "prob_colsum", "slot", "token_map", "kept", "offsets", "row_of", "aux"):
+        assert torch.equal(plan[name], ref[name].view(plan[name].shape)), name
+    n = int(ref["kept"].sum())
+    assert torch.equal(plan["row_src"][:n], ref["row_src"][:n])
