@@ -19,8 +19,9 @@
 //
 // Two bodies share this layout: attention_q_tile_pipe (whole key range; the prefill / training path) loads
 // K and V straight into LDS and overlaps the score MFMAs of the next key tile with the softmax of the
-// current one inside every wave; attention_q_tile (a key range of a split, for decoding against a long
-// cache) keeps the simpler schedule with loads through registers.
+// current one inside every wave; attention_q_tile (a key range of a split, for short chunks against a long
+// cache) keeps the simpler schedule with loads through registers.  Decoding (up to 16 rows per kv head) has a
+// kernel of its own, attention_decode.hpp.
 #include <math.h>
 
 #include <type_traits>
@@ -887,6 +888,12 @@ __global__ __launch_bounds__(256, 2) void attention_splitkv_kernel(
                                          key_count);
 }
 
+}  // namespace ats
+
+#include "attention_decode.hpp"
+
+namespace ats {
+
 // One wave per query row: out = sum_p 2^(m_p - M) O_p / sum_p 2^(m_p - M) l_p with M = max_p m_p.  Lane p
 // holds the maximum and sum of part p (at most 64 parts), so the weights are ready before the rows of
 // partial outputs are streamed; the sums run over the parts in order.
@@ -927,13 +934,28 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(const float* __res
 // Key ranges for the split: aim at ~1024 workgroups, ranges of whole key tiles and at least two tiles, every
 // range starting at or before the first query's position (so that each row sees a key of each range).
 // Measured (32 query / 8 kv heads, D 128, one new token): 1 sequence x 16384 keys 291 -> 33 us, 8 x 8192
-// 150 -> 50 us, 16 x 2048 41 -> 30 us; from 64 sequences on the single pass is as fast or faster.
-static int attention_split_plan(int B, int Hq, int Hkv, int L, int Lk, int* part_len_out) {
+// 150 -> 50 us, 16 x 2048 41 -> 30 us (rows of more than one position; up to 16 rows see below).
+static int attention_split_plan(int B, int Hq, int Hkv, int L, int Lk, int D, int* part_len_out) {
     const int rep = Hq / Hkv;
     const bool pack = L < att_rows_per_block(256) && Hq > Hkv;
     const int64_t rows = pack ? (int64_t)L * rep : L;
     if (rows > att_rows_per_block(256) || Lk - L < 4 * kAttBN) return 1;
     const int64_t n_base = (int64_t)B * (pack ? Hkv : Hq);
+    if (rows <= kDecRows) {
+        // attention_decode_kernel: about one workgroup per CU (four waves, each with 16 KB in flight).  Measured (32 / 8
+        // heads, D 128, one new token; parts: us): 8 sequences x 2048 keys 1: 26, 2: 18.5, 4: 15.7, 8: 16.7; 1 x 16384
+        // 8: 28, 32: 17.7, 64: 21; 16 x 2048 1: 27.6, 2: 25.8, 4: 26.1; 32 x 2048 1: 43.4, 2: 46.2; 20 x 300 1: 8.0, 2: 9.9.
+        int64_t want = n_base >= 160 ? 1 : 256 / n_base;
+        // between one and two workgroups per CU half of the chip would work twice as long: quarters even it out once the
+        // pass is long enough for the merge (40 x 2048 keys: 63.6 -> 56.1, 33 x 2048: 60.0 -> 50.7; 64 x 2048: 81 against 86)
+        if (n_base > 256 && n_base < 448 && n_base * Lk * (4 * D) >= 200000000) want = 4;
+        if (want > 64) want = 64;
+        int len = (int)(((Lk + want - 1) / want + 127) / 128) * 128;      // whole chunks for the four waves
+        int parts = (Lk + len - 1) / len;
+        while (parts > 1 && (int64_t)(parts - 1) * len > Lk - L) --parts;
+        *part_len_out = len;
+        return parts;
+    }
     if (n_base > 256) return 1;      // one workgroup per (batch, head group) already fills the chip twice over
     int64_t want = 1024 / n_base;
     if (want > 64) want = 64;
@@ -950,7 +972,7 @@ static int attention_split_plan(int B, int Hq, int Hkv, int L, int Lk, int* part
 extern "C" size_t ats_attention_fwd_workspace(int B, int Hq, int Hkv, int L, int Lk, int D) {
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || L <= 0 || Lk < L || (D != 64 && D != 128)) return 0;
     int part_len = 0;
-    const int n_parts = ats::attention_split_plan(B, Hq, Hkv, L, Lk, &part_len);
+    const int n_parts = ats::attention_split_plan(B, Hq, Hkv, L, Lk, D, &part_len);
     return n_parts > 1 ? (size_t)B * Hq * L * n_parts * (D + ats::kPartPad) * sizeof(float) : 0;
 }
 
@@ -1050,9 +1072,27 @@ extern "C" int ats_attention_fwd_ex(const void* q, const void* k, int64_t k_sb, 
         ATS_CHECK_LAUNCH("ats_attention_fwd_ex");
         return ATS_OK;
     }
+    // at most 16 rows per kv head (decoding): waves on their own, see attention_decode.hpp
+    auto launch_decode = [&](int parts_, int len_, float* part_out_) -> int {
+        const int64_t n_groups = (int64_t)B * Hkv;
+        ATS_REQUIRE(n_groups * parts_ <= 0x7fffffff, ATS_ERR_UNSUPPORTED, "ats_attention_fwd: %lld workgroups",
+                    (long long)(n_groups * parts_));
+        auto go = [&](auto kernel, int smem) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(n_groups * parts_)), dim3(kDecWaves * 64), smem, as_stream(stream),
+                               static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k), k_sb, k_sh,
+                               static_cast<const bf16_t*>(v), v_sb, (int)v_sl, v_sh, key_bias, static_cast<bf16_t*>(out), lse,
+                               part_out_, Hq, Hkv, L, Lk, scale_log2, (int)n_groups, parts_, len_);
+        };
+        if (D == 128) key_bias ? go(attention_decode_kernel<128, true>, decode_lds_bytes<128>())
+                               : go(attention_decode_kernel<128, false>, decode_lds_bytes<128>());
+        else key_bias ? go(attention_decode_kernel<64, true>, decode_lds_bytes<64>())
+                      : go(attention_decode_kernel<64, false>, decode_lds_bytes<64>());
+        ATS_CHECK_LAUNCH("ats_attention_fwd(decode)");
+        return ATS_OK;
+    };
     // decoding sizes with a workspace: key ranges in parallel, then a merge
     int part_len = 0;
-    const int n_parts = workspace ? attention_split_plan(B, Hq, Hkv, L, Lk, &part_len) : 1;
+    const int n_parts = workspace ? attention_split_plan(B, Hq, Hkv, L, Lk, D, &part_len) : 1;
     if (n_parts > 1 && workspace_bytes >= (size_t)B * Hq * L * n_parts * (D + kPartPad) * sizeof(float) &&
         aligned16(workspace)) {
         const int pack = (L < att_rows_per_block(256) && Hq > Hkv) ? 1 : 0;
@@ -1073,7 +1113,8 @@ extern "C" int ats_attention_fwd_ex(const void* q, const void* k, int64_t k_sb, 
             return ATS_OK;
         };
         int rc;
-        if (D == 128)
+        if (L * (int64_t)(Hq / Hkv) <= kDecRows) rc = launch_decode(n_parts, part_len, parts);
+        else if (D == 128)
             rc = key_bias ? launch_split(attention_splitkv_kernel<128, true>, reserved_split[0])
                           : launch_split(attention_splitkv_kernel<128, false>, reserved_split[1]);
         else
@@ -1092,6 +1133,7 @@ extern "C" int ats_attention_fwd_ex(const void* q, const void* k, int64_t k_sb, 
         ATS_CHECK_LAUNCH("ats_attention_fwd(merge)");
         return ATS_OK;
     }
+    if (L * (int64_t)(Hq / Hkv) <= kDecRows) return launch_decode(1, 0, nullptr);
     const int nt = L >= 4096 ? 512 : 256;
     const int kAttBM = att_rows_per_block(nt);
     const int pack = (L < kAttBM && Hq > Hkv) ? 1 : 0;
