@@ -1033,8 +1033,22 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // SQ_LDS_IDX_ACTIVE, also over the whole GEMM launch): the lanes that share a cycle are not 16 consecutive ones.
 // LDS was busy 60 % of this kernel's cycles with that conflict; without it the prefill step is 0.45 % faster.
 //
-// A 64-element slab is two 32-element k-steps; the wave's 128 rows are two halves of four 16-row fragments.
-// A slab is four phases of 16 MFMAs, (k-step, row half) = (0,0) (0,1) (1,0) (1,1); fragments live in two
+// MIDROWS: the instance for groups of a few hundred rows.  A group is cut into as few tiles as possible, all of one
+// height (a multiple of 32 rows), and a tile's rows are dealt evenly to the two wave rows, so that every SIMD has the
+// same, smallest number of MFMAs; with 256-row tiles and the rest, a group of 192 rows kept one wave of a SIMD at 128
+// rows beside one at 64.  There the weights also come from HBM instead of from the L2 of an XCD that four or more
+// row tiles share, so the three-stage ring is the weights' and the activations have the two stages (the roles in
+// the phases below trade places).  Rows per group, gate/up [28672, 4096] x 8 | down [4096, 14336] x 8 | gate/up
+// [2816, 2048] x 64, microseconds, before -> now (the second figure: equal heights, but the ring for the activations):
+//   192   569 -> 425 -> 426  |  262 -> 259 -> 261  |  236 -> 187 -> 187
+//   320   601 -> 588 -> 571  |  307 -> 299 -> 283  |  275 -> 276 -> 272
+//   383   642 -> 635 -> 622  |  324 -> 314 -> 306  |  286 -> 295 -> 287
+//   1024 1469 -> 1498 -> 1493 |  815 -> 819 -> 819 |  629 -> 641 -> 639
+//   4096 5473 -> 5520 -> 5556 | 2734 -> 2765 -> 2773 | 2380 -> 2413 -> 2442
+// so launches below kMidRowsMaxAvg rows per group take it.  Sums over K are in the same order in both instances.
+//
+// A 64-element slab is two 32-element k-steps; the wave's rows are up to two halves of up to four 16-row fragments.
+// A slab is four phases of up to 16 MFMAs, (k-step, row half) = (0,0) (0,1) (1,0) (1,1); fragments live in two
 // buffers of four activation fragments and two buffers of four weight fragments:
 //   phase 0 : MFMAs | reads: activations (k0, half 1), weights (k1) 0..1 | loads: activations of slab t+2, 1 of 4
 //   phase 1 : MFMAs | reads: activations (k1, half 0), weights (k1) 2..3 | loads: activations of slab t+2, 1 of 4
@@ -1068,7 +1082,8 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // bits.  The 32-byte chunks of a row are swizzled on the global side, chunk c of stage row r lands in slot
 // c ^ f(r), f(r) = (r % 4) | ((r / 8) % 4) << 2: the 16 row pieces that one read instruction touches fall on 16
 // different slots, i.e. on all banks once.
-template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false>
+template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
+          bool MIDROWS = false>
 __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, unsigned char* smem,
                                                          const int32_t* __restrict__ row_count) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1084,7 +1099,8 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     constexpr int HALF = BN / 2;
     constexpr int A_STAGE = BM * 128;
     constexpr int B_STAGE = BN * 128;
-    constexpr int B_BASE = 3 * A_STAGE;
+    constexpr int B_BASE = (MIDROWS ? 2 : 3) * A_STAGE;
+    static_assert(A_STAGE == B_STAGE, "the two rings share their stage offsets");
 
     typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
@@ -1102,10 +1118,20 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
 
+    // ---- rows of this tile: row_base .. + 2 * wave_share, wave row wm taking the wm-th share
+    int frags = TM;                     // 16-row fragments per wave
+    if constexpr (MIDROWS) {
+        const int m_tiles = (count + BM - 1) / BM;
+        const int f = ((count + m_tiles - 1) / m_tiles + 31) / 32;
+        frags = __builtin_amdgcn_readfirstlane(f > 4 ? f : (f > 2 ? 4 : 2));
+    }
+    const int wave_share = frags * 16;
+    const int tile_row = tc.mt * 2 * wave_share;
+
     // ---- load descriptors and lane offsets: instruction j of this wave covers rows (j*NW + wave)*8 .. +8
     constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
     const bool gather = p.a_rows != nullptr;
-    const T* a_base = gather ? A : A + ((int64_t)arow0 + (int64_t)tc.mt * BM) * p.lda;
+    const T* a_base = gather ? A : A + ((int64_t)arow0 + (int64_t)tile_row) * p.lda;
     const __amdgpu_buffer_rsrc_t rsrc_a =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a_base), 0, (int)p.a_extent_bytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rsrc_b =
@@ -1117,9 +1143,11 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     int a_idx[NIA];
 #pragma unroll
     for (int j = 0; j < NIA; ++j) {
-        int m = tc.mt * BM + (j * NW + wave) * 8 + drow;
+        // stage rows 0 .. 127 belong to wave row 0, the others to wave row 1; rows that nobody has repeat the last one
+        const int r = (j * NW + wave) * 8 + drow;
+        int m = (r & 127) < wave_share ? tile_row + (r >> 7) * wave_share + (r & 127) : count - 1;
         m = m < count ? m : count - 1;
-        a_idx[j] = gather ? p.a_rows[arow0 + m] : m - tc.mt * BM;
+        a_idx[j] = gather ? p.a_rows[arow0 + m] : m - tile_row;
     }
 #pragma unroll
     for (int j = 0; j < NIB; ++j) {
@@ -1195,51 +1223,54 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 #define D16_ISSUE_A1(kt_, aoff_, j_)                                                                   \
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(dma_a + (aoff_) + (j_) * NW * 1024), 16, \
                                              ao[j_], (kt_) * 128, 0, 0)
-#define D16_ISSUE_B(kt_, stage_)                                                                       \
+#define D16_ISSUE_B1(kt_, boff_, j_)                                                                   \
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(dma_b + (boff_) + (j_) * NW * 1024), 16, \
+                                             bo[j_], (kt_) * b_slab, 0, 0)
+#define D16_ISSUE_B(kt_, boff_)                                                                        \
     {                                                                                                  \
         const int soff = (kt_) * b_slab;                                                               \
         _Pragma("unroll") for (int j = 0; j < NIB; ++j)                                                \
             __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                  \
-                rsrc_b, (lds_ptr_t)(dma_b + (stage_) * B_STAGE + j * NW * 1024), 16, bo[j], soff, 0, 0); \
+                rsrc_b, (lds_ptr_t)(dma_b + (boff_) + j * NW * 1024), 16, bo[j], soff, 0, 0); \
     }
 #define D16_B_ROW(j_) (SWIGLU ? ((j_) < TN / 2 ? (j_) * 16 : HALF + ((j_) - TN / 2) * 16) : (j_) * 16)
-#define D16_READ_A(aoff_, ks_, half_, buf_)                                                            \
+#define D16_READ_A(aoff_, ks_, f0_, nf_, buf_)                                                         \
     {                                                                                                  \
-        const unsigned char* fa_ = fa_addr[ks_] + (aoff_) + (half_) * 8192;                            \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i)                                                  \
+        const unsigned char* fa_ = fa_addr[ks_] + (aoff_) + (f0_) * 2048;                              \
+        _Pragma("unroll") for (int i = 0; i < (nf_); ++i)                                              \
             fa[buf_][i] = *reinterpret_cast<const u32x4_t*>(fa_ + i * 2048);                           \
     }
-#define D16_READ_B(stage_, ks_, j_, buf_)                                                              \
+#define D16_READ_B(boff_, ks_, j_, buf_)                                                               \
     if constexpr (BKM) {                                                                               \
         union {                                                                                        \
             tr4_t t[2];                                                                                \
             u32x4_t u;                                                                                 \
         } cv_;                                                                                         \
-        const lds_u8_t pb_ = fb_tr[j_] + (stage_) * B_STAGE + (ks_) * (32 * 512);                      \
+        const lds_u8_t pb_ = fb_tr[j_] + (boff_) + (ks_) * (32 * 512);                      \
         cv_.t[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr_t)(pb_));                       \
         cv_.t[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr_t)(pb_ + 4 * 512));             \
         fb[buf_][j_] = cv_.u;                                                                          \
     } else                                                                                             \
-        fb[buf_][j_] = *reinterpret_cast<const u32x4_t*>(fb_addr[ks_] + (stage_) * B_STAGE + D16_B_ROW(j_) * 128)
-#define D16_MMA(bbuf_, abuf_, half_)                                                                   \
+        fb[buf_][j_] = *reinterpret_cast<const u32x4_t*>(fb_addr[ks_] + (boff_) + D16_B_ROW(j_) * 128)
+#define D16_MMA(bbuf_, abuf_, f0_, nf_)                                                                 \
     {                                                                                                  \
         _Pragma("unroll") for (int j = 0; j < TN; ++j)                                                 \
-            _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                            \
+            _Pragma("unroll") for (int i = 0; i < (nf_); ++i) {                                        \
                 union {                                                                                \
                     u32x4_t u;                                                                         \
                     bf16x8_t v;                                                                        \
                 } w_, a_;                                                                              \
                 w_.u = fb[bbuf_][j];                                                                   \
                 a_.u = fa[abuf_][i];                                                                   \
-                acc[j][(half_) * 4 + i] =                                                              \
-                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_.v, a_.v, acc[j][(half_) * 4 + i], 0, 0, 0); \
+                acc[j][(f0_) + i] =                                                                    \
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_.v, a_.v, acc[j][(f0_) + i], 0, 0, 0);   \
             }                                                                                          \
     }
-// Order inside a phase of 16 MFMAs: its nrd fragment reads go between the first MFMAs, its nvm loads between
+// Order inside a phase of 4 nf MFMAs: its nrd fragment reads go between the first MFMAs, its nvm loads between
 // the MFMAs behind them
-#define D16_MIX(nrd_, nvm_)                                                             \
+#define D16_MIX(nf_, nrd_, nvm_)                                                        \
     _Pragma("unroll") for (int g_ = 0; g_ < (nrd_); ++g_) {                             \
-        __builtin_amdgcn_sched_group_barrier(SG_MFMA, 16 / ((nrd_) + 2), 0);            \
+        __builtin_amdgcn_sched_group_barrier(SG_MFMA, 4 * (nf_) > (nrd_) + 2 ? 4 * (nf_) / ((nrd_) + 2) : 1, 0); \
         __builtin_amdgcn_sched_group_barrier(SG_DS_RD, 1, 0);                           \
     }                                                                                   \
     _Pragma("unroll") for (int g_ = 0; g_ < (nvm_); ++g_) {                             \
@@ -1248,88 +1279,100 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     }
 // phase 3: a fragment read per MFMA over the first half (K-major weights: their four fragments take two read
 // instructions each), a load per two MFMAs over the second
-#define D16_MIX_DMA()                                                                   \
+#define D16_MIX_DMA(nf0_, nf1_)                                                         \
     _Pragma("unroll") for (int g_ = 0; g_ < 4; ++g_) {                                  \
         __builtin_amdgcn_sched_group_barrier(SG_DS_RD, BKM ? 2 : 1, 0);                 \
         __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);                            \
     }                                                                                   \
-    _Pragma("unroll") for (int g_ = 0; g_ < 4; ++g_) {                                  \
+    _Pragma("unroll") for (int g_ = 0; g_ < (nf0_); ++g_) {                             \
         __builtin_amdgcn_sched_group_barrier(SG_DS_RD, 1, 0);                           \
         __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);                            \
     }                                                                                   \
     _Pragma("unroll") for (int g_ = 0; g_ < 4; ++g_) {                                  \
         __builtin_amdgcn_sched_group_barrier(SG_VMEM, 1, 0);                            \
-        __builtin_amdgcn_sched_group_barrier(SG_MFMA, 2, 0);                            \
+        __builtin_amdgcn_sched_group_barrier(SG_MFMA, (nf1_) == 4 ? 2 : 1, 0);          \
     }
-// STG: weight stage of slab kt (compile time); sa_cur / sa_nxt: activation stage offsets of slabs kt, kt+1
+// STG: weight stage of slab kt (compile time); s_cur / s_nxt: offsets in the ring of three of slabs kt, kt+1
 // (the third stage takes slab kt+2).  Slabs past the end are clamped to the last one (their loads land in
 // stages nobody reads again).
-// H0 / H1 (compile time): whether row half 0 / 1 of this wave holds rows of the expert at all; a half made
-// only of rows past the expert's end keeps its loads and barriers but skips its fragment reads and MFMAs.
-#define D16_ITER(kt_, STG, H0, H1)                                                      \
+// N0 / N1 (compile time): fragments in the first and the second part of the wave's rows.  A wave none of whose
+// rows the expert has (0, 0) keeps its loads and barriers but skips its fragment reads and MFMAs.
+#define D16_ISSUE_FAR(j_)                                                               \
     {                                                                                   \
-        const int sa_far = 3 * A_STAGE - sa_cur - sa_nxt;                               \
+        if (MIDROWS) D16_ISSUE_B1(ka_, s_far, j_);                                        \
+        else D16_ISSUE_A1(ka_, s_far, j_);                                              \
+    }
+#define D16_ITER(kt_, STG, N0, N1)                                                      \
+    {                                                                                   \
+        const int s_far = 3 * A_STAGE - s_cur - s_nxt;                                  \
+        const int ca_ = MIDROWS ? STG * A_STAGE : s_cur, na_ = MIDROWS ? (STG ^ 1) * A_STAGE : s_nxt; \
+        const int cb_ = MIDROWS ? s_cur : STG * B_STAGE, nb_ = MIDROWS ? s_nxt : (STG ^ 1) * B_STAGE; \
         __builtin_amdgcn_s_setprio(0);                                                  \
         const int ka_ = min((kt_) + 2, nk - 1);                                         \
-        if (H1) D16_READ_A(sa_cur, 0, 1, 1);                                            \
-        D16_ISSUE_A1(ka_, sa_far, 0);                                                   \
-        if (H0) {                                                                       \
-            D16_READ_B(STG, 1, 0, 1);                                                   \
-            D16_READ_B(STG, 1, 1, 1);                                                   \
-            D16_MMA(0, 0, 0);                                                           \
-            D16_MIX((H1 ? 4 : 0) + RB2, 1);                                             \
+        if (N1) D16_READ_A(ca_, 0, N0, N1, 1);                                       \
+        D16_ISSUE_FAR(0);                                                                 \
+        if (N0) {                                                                       \
+            D16_READ_B(cb_, 1, 0, 1);                                                   \
+            D16_READ_B(cb_, 1, 1, 1);                                                   \
+            D16_MMA(0, 0, 0, N0);                                                       \
+            D16_MIX(N0, N1 + RB2, 1);                                                   \
         }                                                                               \
         PL_FENCE();                                                                     \
-        D16_ISSUE_A1(ka_, sa_far, 1);                                                   \
-        if (H0) {                                                                       \
-            D16_READ_A(sa_cur, 1, 0, 0);                                                \
-            D16_READ_B(STG, 1, 2, 1);                                                   \
-            D16_READ_B(STG, 1, 3, 1);                                                   \
+        D16_ISSUE_FAR(1);                                                                 \
+        if (N0) {                                                                       \
+            D16_READ_A(ca_, 1, 0, N0, 0);                                            \
+            D16_READ_B(cb_, 1, 2, 1);                                                   \
+            D16_READ_B(cb_, 1, 3, 1);                                                   \
         }                                                                               \
-        if (H1) {                                                                       \
-            D16_MMA(0, 1, 1);                                                           \
-            D16_MIX(4 + RB2, 1);                                                        \
+        if (N1) {                                                                       \
+            D16_MMA(0, 1, N0, N1);                                                      \
+            D16_MIX(N1, N0 + RB2, 1);                                                   \
         }                                                                               \
         PL_FENCE();                                                                     \
-        D16_ISSUE_A1(ka_, sa_far, 2);                                                   \
-        D16_ISSUE_A1(ka_, sa_far, 3);                                                   \
-        if (H1) D16_READ_A(sa_cur, 1, 1, 1);                                            \
-        if (H0) {                                                                       \
-            D16_MMA(1, 0, 0);                                                           \
-            D16_MIX(H1 ? 4 : 1, 2);                                                     \
+        D16_ISSUE_FAR(2);                                                                 \
+        D16_ISSUE_FAR(3);                                                                 \
+        if (N1) D16_READ_A(ca_, 1, N0, N1, 1);                                       \
+        if (N0) {                                                                       \
+            D16_MMA(1, 0, 0, N0);                                                       \
+            D16_MIX(N0, N1 ? N1 : 1, 2);                                                \
         }                                                                               \
         PL_FENCE();                                                                     \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NIA) : "memory"); \
         __builtin_amdgcn_s_setprio(2);                                                  \
         PL_FENCE();                                                                     \
-        if (H0) {                                                                       \
-            D16_READ_B(STG ^ 1, 0, 0, 0);                                               \
-            D16_READ_A(sa_nxt, 0, 0, 0);                                                \
-            D16_READ_B(STG ^ 1, 0, 1, 0);                                               \
-            D16_READ_B(STG ^ 1, 0, 2, 0);                                               \
-            D16_READ_B(STG ^ 1, 0, 3, 0);                                               \
+        if (N0) {                                                                       \
+            D16_READ_B(nb_, 0, 0, 0);                                               \
+            D16_READ_A(na_, 0, 0, N0, 0);                                            \
+            D16_READ_B(nb_, 0, 1, 0);                                               \
+            D16_READ_B(nb_, 0, 2, 0);                                               \
+            D16_READ_B(nb_, 0, 3, 0);                                               \
         }                                                                               \
-        D16_ISSUE_B(min((kt_) + 2, nk - 1), STG);                                       \
-        if (H1) {                                                                       \
-            D16_MMA(1, 1, 1);                                                           \
-            D16_MIX_DMA();                                                              \
+        if (MIDROWS) D16_ISSUE_A(ka_, STG * A_STAGE)                                       \
+        else D16_ISSUE_B(ka_, STG * B_STAGE)                                            \
+        if (N1) {                                                                       \
+            D16_MMA(1, 1, N0, N1);                                                      \
+            D16_MIX_DMA(N0, N1);                                                        \
         }                                                                               \
         PL_FENCE();                                                                     \
-        sa_cur = sa_nxt;                                                                \
-        sa_nxt = sa_nxt == 2 * A_STAGE ? 0 : sa_nxt + A_STAGE;                          \
+        s_cur = s_nxt;                                                                  \
+        s_nxt = s_nxt == 2 * A_STAGE ? 0 : s_nxt + A_STAGE;                             \
     }
-#define D16_LOOP(H0, H1)                                                                \
+#define D16_LOOP(N0, N1)                                                                \
     {                                                                                   \
         int kt = 0;                                                                     \
-        for (; kt + 1 < nk; kt += 2) {                                                  \
-            D16_ITER(kt, 0, H0, H1);                                                    \
-            D16_ITER(kt + 1, 1, H0, H1);                                                \
+        if (N0) {                                                                       \
+            D16_READ_A(0, 0, 0, N0, 0);                                                 \
+            _Pragma("unroll") for (int j = 0; j < TN; ++j) D16_READ_B(0, 0, j, 0);      \
         }                                                                               \
-        if (kt < nk) D16_ITER(kt, 0, H0, H1);                                           \
+        for (; kt + 1 < nk; kt += 2) {                                                  \
+            D16_ITER(kt, 0, N0, N1);                                                    \
+            D16_ITER(kt + 1, 1, N0, N1);                                                \
+        }                                                                               \
+        if (kt < nk) D16_ITER(kt, 0, N0, N1);                                           \
     }
 
     D16_ISSUE_B(0, 0);
-    D16_ISSUE_B(min(1, nk - 1), 1);
+    D16_ISSUE_B(min(1, nk - 1), B_STAGE);
 #pragma unroll
     for (int j = 0; j < NIA; ++j) {
         const int64_t src = gather ? (int64_t)(a_idx[j] / p.a_row_div) : (int64_t)a_idx[j];
@@ -1338,21 +1381,26 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     D16_ISSUE_A(0, 0);
     D16_ISSUE_A(min(1, nk - 1), A_STAGE);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NIA) : "memory");
-    int sa_cur = 0, sa_nxt = A_STAGE;
-    // rows of the expert in this wave's 128-row share of the tile (wave-uniform)
-    const int wave_rows = count - (tc.mt * BM + wm * (BM / WM));
-    if (wave_rows > 64) {
-        D16_READ_A(sa_cur, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) D16_READ_B(0, 0, j, 0);
-        D16_LOOP(true, true);
+    int s_cur = 0, s_nxt = A_STAGE;
+    // rows of the expert in this wave's share of the tile (wave-uniform)
+    const int wave_row = tile_row + wm * wave_share;
+    int wave_rows = count - wave_row;
+    if constexpr (MIDROWS) {
+        wave_rows = wave_rows < wave_share ? wave_rows : wave_share;
+        switch (frags) {
+            case 8: D16_LOOP(4, 4) break;
+            case 7: D16_LOOP(4, 3) break;
+            case 6: D16_LOOP(3, 3) break;
+            case 5: D16_LOOP(3, 2) break;
+            case 4: D16_LOOP(2, 2) break;
+            default: D16_LOOP(1, 1) break;
+        }
+    } else if (wave_rows > 64) {
+        D16_LOOP(4, 4)
     } else if (wave_rows > 0) {
-        D16_READ_A(sa_cur, 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) D16_READ_B(0, 0, j, 0);
-        D16_LOOP(true, false);
+        D16_LOOP(4, 0)
     } else {
-        D16_LOOP(false, false);
+        D16_LOOP(0, 0)
     }
     __builtin_amdgcn_s_setprio(0);
     // the clamped loads of the last slabs may still be in flight; the epilogue reuses LDS
@@ -1361,6 +1409,8 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 #undef D16_ISSUE_A
 #undef D16_ISSUE_A1
 #undef D16_ISSUE_B
+#undef D16_ISSUE_B1
+#undef D16_ISSUE_FAR
 #undef D16_B_ROW
 #undef D16_READ_A
 #undef D16_READ_B
@@ -1372,27 +1422,27 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     {
         typedef AccView16<TM, TN, SWIGLU> View;
         constexpr int WSTAGE = epilogue_wstage_bytes<TO, View, DSILU>();
-        const int wrow = tc.mt * BM + wm * (BM / WM);
         const int ncol0 = SWIGLU ? tc.nt * HALF + wn * (BN / WN / 2) : tc.nt * BN + wn * (BN / WN);
         if constexpr (SAVEGU || DSILU) {
             constexpr int TSTAGE = SAVEGU ? kTransStageH : kTransStageD;
             static_assert(NW * (WSTAGE + TSTAGE) <= (3 * BM + 2 * BN) * 128, "epilogue staging exceeds the tile's LDS");
             TO* tout = static_cast<TO*>(p.t_out);
-            const int64_t tcol = tout ? (int64_t)p.t_col0[tc.e] + wrow : 0;
+            const int64_t tcol = tout ? (int64_t)p.t_col0[tc.e] + wave_row : 0;
             epilogue_view<TO, View, SWIGLU, SAVEGU, DSILU>(View{acc}, smem + wave * WSTAGE, static_cast<TO*>(p.out), p.ldo,
-                                                           (int64_t)row0 + wrow, count - wrow, ncol0, p.N_out, lane,
+                                                           (int64_t)row0 + wave_row, wave_rows, ncol0, p.N_out, lane,
                                                            static_cast<TO*>(p.gu_out), p.ld_gu, p.up_offset, tout,
                                                            p.ld_t, tcol, smem + NW * WSTAGE + wave * TSTAGE);
         } else {
             epilogue_view<TO, View, SWIGLU, SAVEGU, DSILU>(View{acc}, smem + wave * WSTAGE, static_cast<TO*>(p.out), p.ldo,
-                                                           (int64_t)row0 + wrow, count - wrow, ncol0, p.N_out, lane,
+                                                           (int64_t)row0 + wave_row, wave_rows, ncol0, p.N_out, lane,
                                                            static_cast<TO*>(p.gu_out), p.ld_gu, p.up_offset);
         }
     }
 #endif
 }
 
-template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false>
+template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
+          bool MIDROWS = false>
 __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) {
     // The body is a function of its own for one reason: a __restrict__ parameter that it reads through gives every
     // other memory access in it (the transposing LDS reads among them) "does not alias that parameter" metadata once
@@ -1401,7 +1451,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
     // the K-major variant is preceded by s_waitcnt vmcnt(0), i.e. waits for all of the slab loads just issued (the
     // plain 16-byte fragment reads carry type-based alias metadata and never had that wait): 27-37 % slower.
     extern __shared__ __align__(16) unsigned char smem_k[];
-    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM>(p, smem_k, p.row_count);
+    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS>(p, smem_k, p.row_count);
 }
 
 #undef PL_STORE
@@ -1412,6 +1462,10 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
 
 // LDS of the direct-to-LDS kernel: three activation stages and two weight stages of unpadded 128-byte rows.
 constexpr size_t dma_lds_bytes(int BM, int BN) { return (size_t)(3 * BM + 2 * BN) * 128; }
+
+// Rows per group on average below which the 16 x 16 x 32 kernel runs in its MIDROWS form (measured there).
+constexpr int64_t kMidRowsMaxAvg = 768;
+static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1) < kMidRowsMaxAvg; }
 
 template <typename T, typename TO, int BM, int BN, int WM, int WN, int SM, int SN, bool SWIGLU, bool DMA = false>
 static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
@@ -1438,11 +1492,17 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
         } else if constexpr (DMA) return grouped_gemm_dma_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
         else return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, kSliced>;
     }();
+    auto kern_mid = [] {       // groups of a few hundred rows
+        if constexpr (DMA && std::is_same<T, bf16_t>::value) return grouped_gemm_dma16_kernel<TO, SM, SN, SWIGLU, false, false, false, true>;
+        else if constexpr (DMA) return grouped_gemm_dma_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
+        else return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, kSliced>;
+    }();
     if (smem > 64 * 1024) {
         static LdsReservation reserved;      // one per tile configuration (this function is a template)
         hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern_general),
                                               reinterpret_cast<const void*>(kern_pipe),
-                                              reinterpret_cast<const void*>(kern_dma)}, (int)smem);
+                                              reinterpret_cast<const void*>(kern_dma),
+                                              reinterpret_cast<const void*>(kern_mid)}, (int)smem);
         if (e != hipSuccess) {
             set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
             return ATS_ERR_LAUNCH;
@@ -1466,7 +1526,7 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     }
     // the direct-to-LDS kernel addresses its operands with 32-bit lane offsets
     const bool dma_ok = DMA && p.K % BK == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0;
-    auto kern = dma_ok ? kern_dma : (p.K % BK == 0) ? kern_pipe : kern_general;
+    auto kern = dma_ok ? (mid_rows(max_rows, p.E) ? kern_mid : kern_dma) : (p.K % BK == 0) ? kern_pipe : kern_general;
     const size_t smem_launch = (!dma_ok && p.K % BK == 0) ? smem_staged : smem;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WM * WN * 64), smem_launch, s, p);
     return ATS_OK;
@@ -1481,8 +1541,10 @@ struct TileCost {
     float per_slab, per_tile;
     int min_tiles;
 };
-static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs) {
-    const int64_t avg = (max_rows + E - 1) / E;
+// spread: groups vary around their mean, so those of a mean just below a multiple of the tile height need one tile more.
+static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs, bool spread = false) {
+    const int64_t rows = spread && E > 1 ? max_rows + max_rows / 10 : max_rows;
+    const int64_t avg = (rows + E - 1) / E;
     const int64_t tiles = (int64_t)E * ((avg + c.rows - 1) / c.rows) * ((n_cols + c.cols - 1) / c.cols);
     const int64_t per_cu = (tiles + 255) / 256;
     return (float)(per_cu > c.min_tiles ? per_cu : c.min_tiles) * (k_slabs * c.per_slab + c.per_tile);
@@ -1555,8 +1617,10 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
                                         : TileCost{64, SWIGLU ? 32 : 64, 0.58f, 3.f, 1};
     constexpr TileCost kMid = kBf16 ? TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 0.58f : 1.05f, 5.f, 1}
                                     : TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 2.0f : 3.65f, 5.f, 1};
-    const float mid = tile_time(kMid, max_rows, E, p.N_out, nk);
-    const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? 1.45f : 7.3f, 7.f, 1}, max_rows, E, p.N_out, nk);
+    const float mid = tile_time(kMid, max_rows, E, p.N_out, nk, true);
+    // (the 16 x 16 x 32 kernel computes only the 32-row steps that a tile has; up to 192 rows its loads bound a slab)
+    const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? (avg <= 192 ? 1.3f : 1.45f) : 7.3f, 7.f, 1},
+                                max_rows, E, p.N_out, nk, true);
     const float least_large = mid < big ? mid : big;
     // (two full rounds of 256-row tiles: nothing is idle, and groups of unequal size fit them better; 8 experts with 20-45
     // rows each, gate/up [28672, 4096]: 343 us against 372 in 32-row tiles)
@@ -1564,7 +1628,10 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     if (big_tiles >= 512) {
     } else if (avg <= (kBf16 ? 192 : 256)) {
         const float small32 = tile_time(kSmall32, max_rows, E, p.N_out, nk);
-        const float small64 = tile_time(kSmall64, max_rows, E, p.N_out, nk);
+        // (a long K streams the weights from HBM: 8 groups x 128 rows, [4096, 14336]: 328 us against 258 in 128-row tiles)
+        TileCost c64 = kSmall64;
+        if (kBf16 && nk >= 128) c64.per_slab = 0.3f;
+        const float small64 = tile_time(c64, max_rows, E, p.N_out, nk);
         if (small32 < least_large && small32 <= small64)
             return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
         if (small64 < least_large) return launch_small<T, TO, 2, 2, 4, 1, SWIGLU>(p, max_rows, s);
@@ -1673,8 +1740,9 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
     p.n_tiles = (p.N_out + BN - 1) / BN;
     constexpr size_t smem = dma_lds_bytes(BM, BN);
     auto kern = grouped_gemm_dma16_kernel<TO, 4, 8, false, false, DSILU, true>;
+    auto kern_mid = grouped_gemm_dma16_kernel<TO, 4, 8, false, false, DSILU, true, !DSILU>;
     static LdsReservation reserved;
-    hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern)}, (int)smem);
+    hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern), reinterpret_cast<const void*>(kern_mid)}, (int)smem);
     if (e != hipSuccess) {
         set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
         return ATS_ERR_LAUNCH;
@@ -1688,7 +1756,7 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(512), smem, s, p);
+    hipLaunchKernelGGL(mid_rows(max_rows, p.E) ? kern_mid : kern, dim3((unsigned)blocks), dim3(512), smem, s, p);
     return ATS_OK;
 }
 
