@@ -20,6 +20,12 @@ class AtsError(RuntimeError):
     """A libats_gfx950 entry point returned an error code."""
 
 
+class Table(ctypes.Structure):
+    """ats_table of the C header."""
+    _fields_ = [("out", c_void_p), ("base", c_int64), ("stride", c_int64), ("index", c_void_p), ("n", c_int),
+                ("kind", c_int), ("wide", c_int)]
+
+
 _SIGNATURES = {
     "ats_version": (c_int, []),
     "ats_last_error_string": (c_char_p, []),
@@ -81,6 +87,7 @@ _SIGNATURES = {
     "ats_router_bwd_dw_workspace": (c_size_t, [c_int64, c_int, c_int]),
     "ats_router_bwd_dw": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t,
                                   c_void_p]),
+    "ats_fill_tables": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "ats_transpose_batched": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "ats_wgrad_padded_rows": (c_int64, [c_int64, c_int]),
     "ats_wgrad_plan": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p]),

@@ -155,8 +155,7 @@ class LinearFunction(Function):
         N = w.shape[0]
         dy = dy.to(x.dtype).contiguous()
         dx = dw = None
-        offsets = torch.tensor([0, T], dtype=torch.int32, device=x.device)
-        kept = offsets[1:].clone()
+        offsets, kept = ops._single_group(T, x.device)
         if ctx.needs_input_grad[0]:
             if DGRAD_FROM_FORWARD_WEIGHTS and ops.grouped_gemm_nn_supported(1, T, K, N, K, x.dtype):
                 dx = ops.grouped_gemm_nn(ops.weight_pointer_table([w]), K, offsets, kept, T, T, K, N, dy)
@@ -168,11 +167,7 @@ class LinearFunction(Function):
             ld = ops.wgrad_padded_rows(T, 1)
             dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
             xT = ops.transpose_grouped_rows(x, offsets, kept, T)
-            es = x.element_size()
-            a_ptrs = ks.long() * es + dyT.data_ptr()
-            b_ptrs = ks.long() * es + xT.data_ptr()
-            rs = torch.zeros(1, dtype=torch.int32, device=x.device)
-            rc = torch.full((1,), N, dtype=torch.int32, device=x.device)
+            a_ptrs, b_ptrs, rs, rc = ops.wgrad_tables(ks, N, dyT, xT)
             dw = ops.grouped_gemm_nt(b_ptrs, ld, K, rs, rc, N, N, K, ld, a_ptrs=a_ptrs, lda=ld, k_count=kc,
                                      dtype=x.dtype, out_dtype=x.dtype).to(ctx.param_dtype)
         return dx, dw
@@ -245,7 +240,7 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
     transposed copy, so only dy and the gathered x go through a transposing pass."""
     E = len(wd)
     H, I = x.shape[1], wd[0].shape[1]
-    dtype, dev = x.dtype, x.device
+    dtype = x.dtype
     if need_w and wplan is None:
         wplan = ops.wgrad_plan(kept)
     dguT = None
@@ -276,17 +271,13 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
     if need_w:
         ks, kc = wplan
         ld = ops.wgrad_padded_rows(rows, E)
-        es = x.element_size()
 
         def wgrad(lhs, rhs, M, N, gather=None, lhsT=None, rhsT=None):
             if lhsT is None:
                 lhsT = ops.transpose_grouped_rows(lhs, offsets, kept, rows)
             if rhsT is None:
                 rhsT = ops.transpose_grouped_rows(rhs, offsets, kept, rows, gather=gather, gather_div=k)
-            a_ptrs = ks.long() * es + lhsT.data_ptr()
-            b_ptrs = ks.long() * es + rhsT.data_ptr()
-            rs = torch.arange(E, dtype=torch.int32, device=dev) * M
-            rc = torch.full((E,), M, dtype=torch.int32, device=dev)
+            a_ptrs, b_ptrs, rs, rc = ops.wgrad_tables(ks, M, lhsT, rhsT)
             g = ops.grouped_gemm_nt(b_ptrs, ld, N, rs, rc, E * M, E * M, N, ld, a_ptrs=a_ptrs, lda=ld, k_count=kc,
                                     dtype=dtype, out_dtype=dtype)
             return g.view(E, M, N)

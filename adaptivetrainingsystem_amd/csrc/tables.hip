@@ -1,0 +1,69 @@
+// Address and row tables of grouped products, several per launch.
+//
+// The grouped kernels read their groups' base addresses and row ranges from device memory.  All of these tables are
+// affine in an index that follows from the group number (the group itself, the key/value matrix of a query head, the
+// slot of a head in a reduction buffer, an int32 read on the device), so one launch of one small workgroup per table
+// writes every table that a step needs.  Bound: the launch itself (about 5 us on the timeline of a stream).  Built from
+// torch expressions, each table was two or three launches and as many host calls of 4-6 us: a float32 transformer block
+// made 107 of its 250 launches for them.
+#include "ats_common.hpp"
+
+namespace ats {
+
+constexpr int kMaxTables = 20;
+struct TableArgs {
+    ats_table t[kMaxTables];
+    int Hq, Hkv, BHkv;
+};
+
+__global__ __launch_bounds__(64) void fill_tables_kernel(TableArgs a) {
+    const ats_table t = a.t[blockIdx.x];
+    for (int i = threadIdx.x; i < t.n; i += 64) {
+        int64_t x = 0;
+        switch (t.kind) {
+            case ATS_TABLE_INDEX: x = i; break;
+            case ATS_TABLE_KV_OF_HEAD: x = (i / a.Hq) * a.Hkv + (i % a.Hq) / (a.Hq / a.Hkv); break;
+            case ATS_TABLE_SLOT_OF_HEAD:
+                x = (i % a.Hq % (a.Hq / a.Hkv)) * a.BHkv + (i / a.Hq) * a.Hkv + (i % a.Hq) / (a.Hq / a.Hkv);
+                break;
+            case ATS_TABLE_HEAD_OF_SLOT: {
+                const int kv = i % a.BHkv;
+                x = (kv / a.Hkv) * a.Hq + (kv % a.Hkv) * (a.Hq / a.Hkv) + i / a.BHkv;
+                break;
+            }
+            case ATS_TABLE_FROM_ARRAY: x = t.index[i]; break;
+            default: break;      // ATS_TABLE_CONSTANT
+        }
+        const int64_t v = t.base + x * t.stride;
+        if (t.wide) static_cast<int64_t*>(t.out)[i] = v;
+        else static_cast<int32_t*>(t.out)[i] = (int32_t)v;
+    }
+}
+
+}  // namespace ats
+
+extern "C" int ats_fill_tables(const ats_table* tables, int n_tables, int batch, int q_heads, int kv_heads,
+                               ats_stream_t stream) {
+    using namespace ats;
+    ATS_REQUIRE(tables && n_tables >= 0 && n_tables <= kMaxTables, ATS_ERR_INVALID_ARG, "ats_fill_tables: %d tables (at most %d)",
+                n_tables, kMaxTables);
+    if (n_tables == 0) return ATS_OK;
+    TableArgs a{};
+    for (int i = 0; i < n_tables; ++i) {
+        const ats_table& t = tables[i];
+        const bool heads = t.kind == ATS_TABLE_KV_OF_HEAD || t.kind == ATS_TABLE_SLOT_OF_HEAD || t.kind == ATS_TABLE_HEAD_OF_SLOT;
+        ATS_REQUIRE(t.out && t.n >= 0 && t.kind >= ATS_TABLE_INDEX && t.kind <= ATS_TABLE_CONSTANT, ATS_ERR_INVALID_ARG,
+                    "ats_fill_tables: table %d: n=%d kind=%d or null output", i, t.n, t.kind);
+        ATS_REQUIRE(t.kind != ATS_TABLE_FROM_ARRAY || t.index, ATS_ERR_INVALID_ARG, "ats_fill_tables: table %d has no index array", i);
+        ATS_REQUIRE(!heads || (batch > 0 && kv_heads > 0 && q_heads > 0 && q_heads % kv_heads == 0 && t.n <= (int64_t)batch * q_heads),
+                    ATS_ERR_INVALID_ARG, "ats_fill_tables: table %d: %d entries of %d x %d heads (%d key/value heads)", i, t.n, batch,
+                    q_heads, kv_heads);
+        a.t[i] = t;
+    }
+    a.Hq = q_heads > 0 ? q_heads : 1;
+    a.Hkv = kv_heads > 0 ? kv_heads : 1;
+    a.BHkv = batch > 0 ? batch * a.Hkv : 1;
+    hipLaunchKernelGGL(fill_tables_kernel, dim3((unsigned)n_tables), dim3(64), 0, as_stream(stream), a);
+    ATS_CHECK_LAUNCH("ats_fill_tables");
+    return ATS_OK;
+}

@@ -288,6 +288,38 @@ def weight_pointer_table(weights: Sequence[torch.Tensor]) -> torch.Tensor:
     return table
 
 
+# kinds of fill_tables (see ats_fill_tables)
+TABLE_INDEX, TABLE_KV_OF_HEAD, TABLE_SLOT_OF_HEAD, TABLE_HEAD_OF_SLOT, TABLE_FROM_ARRAY, TABLE_CONSTANT = range(6)
+
+
+def fill_tables(device: torch.device, specs: Sequence[tuple], heads: Tuple[int, int, int] = (0, 0, 0)) -> list:
+    """Device tables base + x(i) * stride from one launch; a spec is (kind, n, base, stride, wide[, index]) and gives an
+    int64 (wide) or int32 tensor of n entries; heads = (batch, query heads, key/value heads)."""
+    most = max(spec[1] for spec in specs)
+    rows = torch.empty(len(specs), most, dtype=torch.int64, device=device)
+    at, arr, outs = rows.data_ptr(), (_lib.Table * len(specs))(), []
+    for i, (row, (kind, n, base, stride, wide, *index)) in enumerate(zip(rows.unbind(0), specs)):
+        if index:
+            _need_gpu(index[0])
+            if index[0].dtype != torch.int32 or index[0].numel() < n or not index[0].is_contiguous():
+                raise AtsError("fill_tables: the index array must be contiguous int32 with one entry per table entry")
+        arr[i] = (at + i * most * 8, base, stride, index[0].data_ptr() if index else None, n, kind, wide)
+        if not wide:
+            row = row.view(torch.int32)
+        outs.append(row if row.numel() == n else row[:n])
+    check(_lib.load().ats_fill_tables(arr, len(specs), *heads, _stream()), "ats_fill_tables")
+    return outs
+
+
+def wgrad_tables(k_start: torch.Tensor, M: int, lhsT: torch.Tensor, rhsT: torch.Tensor) -> list:
+    """(a_ptrs, b_ptrs, row_start, row_count) of the weight-gradient product of [*, padded] transposed operands: group e
+    contracts over the columns from k_start[e] and writes rows e * M .. + M."""
+    E, es = k_start.numel(), lhsT.element_size()
+    return fill_tables(k_start.device, [(TABLE_FROM_ARRAY, E, lhsT.data_ptr(), es, True, k_start),
+                                        (TABLE_FROM_ARRAY, E, rhsT.data_ptr(), es, True, k_start),
+                                        (TABLE_INDEX, E, 0, M, False), (TABLE_CONSTANT, E, M, 0, False)])
+
+
 def grouped_gateup_swiglu(a: torch.Tensor, w_gu_ptrs: torch.Tensor, row_start: torch.Tensor, row_count: torch.Tensor,
                           n_rows_out: int, max_rows: int, H: int, I: int, a_rows: Optional[torch.Tensor] = None,
                           a_row_div: int = 1) -> torch.Tensor:
@@ -880,8 +912,10 @@ def transpose_batched(mats: Sequence[torch.Tensor]) -> Tuple[list, torch.Tensor]
     buf = torch.empty(E, C, R, dtype=mats[0].dtype, device=mats[0].device)
     outs = [buf[e] for e in range(E)]
     in_tab = weight_pointer_table(list(mats))
-    out_tab = weight_pointer_table(outs)
-    aligned = all(m.data_ptr() % 16 == 0 for m in mats) and all(o.data_ptr() % 16 == 0 for o in outs)
+    # (written on the device: an upload of addresses that change from call to call would wait for the queue to drain)
+    step = C * R * buf.element_size()
+    out_tab, = fill_tables(buf.device, [(TABLE_INDEX, E, buf.data_ptr(), step, True)])
+    aligned = step % 16 == 0 and all(m.data_ptr() % 16 == 0 for m in mats)
     check(_lib.load().ats_transpose_batched(in_tab.data_ptr(), out_tab.data_ptr(), E, R, C, _tag(mats[0]), int(aligned),
                                             _stream()), "ats_transpose_batched")
     return outs, out_tab
@@ -922,7 +956,8 @@ def grouped_gemm_nt(b_ptrs: torch.Tensor, ldb: int, b_rows: int, row_start: torc
                     n_rows_out: int, max_rows: int, N: int, K: int, a: Optional[torch.Tensor] = None,
                     a_ptrs: Optional[torch.Tensor] = None, lda: Optional[int] = None,
                     a_rows: Optional[torch.Tensor] = None, a_row_div: int = 1, k_count: Optional[torch.Tensor] = None,
-                    dtype: Optional[torch.dtype] = None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                    dtype: Optional[torch.dtype] = None, out_dtype: Optional[torch.dtype] = None,
+                    out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[row_start[e]+m, :N] = A_e[m, :K_e] @ B_e[:N, :K_e]^T (see ats_grouped_gemm_nt)."""
     _need_gpu(a, a_ptrs, b_ptrs, row_start, row_count, a_rows, k_count)
     if (a is None) == (a_ptrs is None):
@@ -935,7 +970,10 @@ def grouped_gemm_nt(b_ptrs: torch.Tensor, ldb: int, b_rows: int, row_start: torc
         raise AtsError("grouped_gemm_nt: a_ptrs needs dtype and lda")
     out_dtype = dtype if out_dtype is None else out_dtype
     E = b_ptrs.numel()
-    out = torch.empty(n_rows_out, N, dtype=out_dtype, device=b_ptrs.device)
+    if out is None:
+        out = torch.empty(n_rows_out, N, dtype=out_dtype, device=b_ptrs.device)
+    elif out.shape != (n_rows_out, N) or out.dtype != out_dtype or not out.is_contiguous():
+        raise AtsError("grouped_gemm_nt: out must be a contiguous [n_rows_out, N] tensor of out_dtype")
     check(_lib.load().ats_grouped_gemm_nt(_ptr(a), _ptr(a_ptrs), int(lda), int(a.shape[0]) if a is not None else 0,
                                           _ptr(a_rows), int(a_row_div), b_ptrs.data_ptr(), int(ldb), int(b_rows),
                                           out.data_ptr(), N, row_start.data_ptr(), row_count.data_ptr(), _ptr(k_count),
@@ -1084,16 +1122,9 @@ def causal_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out:
 
 
 # --------------------------------------------------------------------------- float32 attention
-def _ptr_table(t: torch.Tensor, index: torch.Tensor, stride_elems: int) -> torch.Tensor:
-    """Device table of addresses t.data_ptr() + index * stride_elems * itemsize (no host round trip)."""
-    return index.to(torch.int64) * (stride_elems * t.element_size()) + t.data_ptr()
-
-
-def _transpose_to(src: torch.Tensor, src_index: torch.Tensor, dst: torch.Tensor, dst_index: torch.Tensor, R: int, C: int):
-    """Matrix src_index[n] ([R, C] contiguous inside src) -> matrix dst_index[n] ([C, R] inside dst)."""
-    n = src_index.numel()
-    in_tab, out_tab = _ptr_table(src, src_index, R * C), _ptr_table(dst, dst_index, R * C)   # both alive at the launch
-    check(_lib.load().ats_transpose_batched(in_tab.data_ptr(), out_tab.data_ptr(), n, R, C, _tag(src), 1, _stream()),
+def _transpose_tables(src: torch.Tensor, in_tab: torch.Tensor, out_tab: torch.Tensor, R: int, C: int):
+    """Matrix n at in_tab[n] ([R, C] contiguous) -> [C, R] at out_tab[n]; src gives the type."""
+    check(_lib.load().ats_transpose_batched(in_tab.data_ptr(), out_tab.data_ptr(), in_tab.numel(), R, C, _tag(src), 1, _stream()),
           "ats_transpose_batched")
 
 
@@ -1104,12 +1135,6 @@ def _pad_rows(t: torch.Tensor, rows: int) -> torch.Tensor:
     out = t.new_zeros(*t.shape[:-2], rows, t.shape[-1])
     out[..., :t.shape[-2], :] = t
     return out
-
-
-def _f32_groups(B: int, Hq: int, Hkv: int, dev):
-    e = torch.arange(B * Hq, device=dev)
-    kv_of = (e // Hq) * Hkv + (e % Hq) // (Hq // Hkv)            # the (batch, kv head) matrix of group (batch, q head)
-    return e, kv_of
 
 
 def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None,
@@ -1141,22 +1166,24 @@ def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Opti
     Lp, Lkp = (L + 3) // 4 * 4, (Lk + 3) // 4 * 4
     E = B * Hq
     qp, kp, vp = _pad_rows(q, Lp), _pad_rows(k, Lkp), _pad_rows(v, Lkp)
-    e, kv_of = _f32_groups(B, Hq, Hkv, dev)
-    row_start = (e * Lp).to(torch.int32)
-    row_count = torch.full((E,), Lp, dtype=torch.int32, device=dev)
+    vT = torch.empty(B * Hkv, D, Lkp, dtype=q.dtype, device=dev)
+    kv_bytes = Lkp * D * 4
+    row_start, row_count, k_tab, v_in, v_out, vT_tab = fill_tables(dev, [
+        (TABLE_INDEX, E, 0, Lp, False), (TABLE_CONSTANT, E, Lp, 0, False),
+        (TABLE_KV_OF_HEAD, E, kp.data_ptr(), kv_bytes, True), (TABLE_INDEX, B * Hkv, vp.data_ptr(), kv_bytes, True),
+        (TABLE_INDEX, B * Hkv, vT.data_ptr(), kv_bytes, True), (TABLE_KV_OF_HEAD, E, vT.data_ptr(), kv_bytes, True)],
+        (B, Hq, Hkv))
     # scores[e] = q[e] . k[kv_of[e]]^T
-    w = grouped_gemm_nt(_ptr_table(kp, kv_of, Lkp * D), D, Lkp, row_start, row_count, E * Lp, E * Lp, Lkp, D,
+    w = grouped_gemm_nt(k_tab, D, Lkp, row_start, row_count, E * Lp, E * Lp, Lkp, D,
                         a=qp.view(E * Lp, D))
     w_drop = torch.empty_like(w) if dropout_p > 0 else None
     check(lib.ats_attention_softmax_f32(w.data_ptr(), _ptr(w_drop), B, Hq, L, Lp, Lk, Lkp, scale, _ptr(key_bias),
                                         _ptr(pair_bias), pair_sb, pair_sh, float(dropout_p),
                                         int(dropout_seed) & 0xFFFFFFFFFFFFFFFF, _stream()), "ats_attention_softmax_f32")
     # out[e] = weights[e] . v[kv_of[e]]  (NT product against v^T)
-    vT = torch.empty(B * Hkv, D, Lkp, dtype=q.dtype, device=dev)
-    every_kv = torch.arange(B * Hkv, device=dev)
-    _transpose_to(vp, every_kv, vT, every_kv, Lkp, D)
+    _transpose_tables(vp, v_in, v_out, Lkp, D)
     used = w_drop if w_drop is not None else w
-    o = grouped_gemm_nt(_ptr_table(vT, kv_of, D * Lkp), Lkp, D, row_start, row_count, E * Lp, E * Lp, D, Lkp, a=used)
+    o = grouped_gemm_nt(vT_tab, Lkp, D, row_start, row_count, E * Lp, E * Lp, D, Lkp, a=used)
     out = o.view(B, Hq, Lp, D)[:, :, :L].transpose(1, 2).reshape(B, L, Hq * D)
     if return_weights:
         return out, (w, w_drop, qp, kp, vp)
@@ -1176,46 +1203,51 @@ def attention_f32_bwd(state, dout: torch.Tensor, B: int, Hq: int, Hkv: int, L: i
     scale = float(D ** -0.5 if scale is None else scale)
     Lp, Lkp = qp.shape[2], kp.shape[2]
     E, rep = B * Hq, Hq // Hkv
-    e, kv_of = _f32_groups(B, Hq, Hkv, dev)
-    row_start = (e * Lp).to(torch.int32)
-    row_count = torch.full((E,), Lp, dtype=torch.int32, device=dev)
     do = _pad_rows(dout.to(torch.float32).view(B, L, Hq, D).permute(0, 2, 1, 3), Lp)          # [B, Hq, Lp, D]
+    kT = torch.empty(B * Hkv, D, Lkp, dtype=w.dtype, device=dev)
+    doT, qT = (torch.empty(E, D, Lp, dtype=w.dtype, device=dev) for _ in range(2))
+    matT = torch.empty(E, Lkp, Lp, dtype=w.dtype, device=dev)       # of the weights, then of dS
+    ds = torch.empty(E * Lp, Lkp, dtype=w.dtype, device=dev)
+    used = w_drop if w_drop is not None else w
+    kv_bytes, q_bytes, s_bytes = Lkp * D * 4, Lp * D * 4, Lp * Lkp * 4
+    # dV and dK: per query head a product over the queries, written so that the `rep` heads of a kv head are
+    # `rep` slices of one buffer: group (b, hq) goes to slot (hq % rep) * (B * Hkv) + its kv matrix.  The b_ptrs and row
+    # tables of those products are read in slot order.
+    (row_start, row_count, v_tab, k_in, k_out, kT_tab, do_in, do_out, q_in, q_out, w_in, ds_in, mat_out, doT_tab, qT_tab,
+     slot_start, slot_count) = fill_tables(dev, [
+         (TABLE_INDEX, E, 0, Lp, False), (TABLE_CONSTANT, E, Lp, 0, False),
+         (TABLE_KV_OF_HEAD, E, vp.data_ptr(), kv_bytes, True),
+         (TABLE_INDEX, B * Hkv, kp.data_ptr(), kv_bytes, True), (TABLE_INDEX, B * Hkv, kT.data_ptr(), kv_bytes, True),
+         (TABLE_KV_OF_HEAD, E, kT.data_ptr(), kv_bytes, True),
+         (TABLE_INDEX, E, do.data_ptr(), q_bytes, True), (TABLE_INDEX, E, doT.data_ptr(), q_bytes, True),
+         (TABLE_INDEX, E, qp.data_ptr(), q_bytes, True), (TABLE_INDEX, E, qT.data_ptr(), q_bytes, True),
+         (TABLE_INDEX, E, used.data_ptr(), s_bytes, True), (TABLE_INDEX, E, ds.data_ptr(), s_bytes, True),
+         (TABLE_SLOT_OF_HEAD, E, matT.data_ptr(), s_bytes, True),
+         (TABLE_HEAD_OF_SLOT, E, doT.data_ptr(), q_bytes, True), (TABLE_HEAD_OF_SLOT, E, qT.data_ptr(), q_bytes, True),
+         (TABLE_INDEX, E, 0, Lkp, False), (TABLE_CONSTANT, E, Lkp, 0, False)],
+        (B, Hq, Hkv))
     # dP' = dO . V^T, then in place to dS (gradient of the raw scores)
-    ds = grouped_gemm_nt(_ptr_table(vp, kv_of, Lkp * D), D, Lkp, row_start, row_count, E * Lp, E * Lp, Lkp, D,
-                         a=do.view(E * Lp, D))
+    grouped_gemm_nt(v_tab, D, Lkp, row_start, row_count, E * Lp, E * Lp, Lkp, D, a=do.view(E * Lp, D), out=ds)
     check(lib.ats_attention_softmax_bwd_f32(w.data_ptr(), ds.data_ptr(), B, Hq, L, Lp, Lk, Lkp, scale, float(dropout_p),
                                             int(dropout_seed) & 0xFFFFFFFFFFFFFFFF, _stream()),
           "ats_attention_softmax_bwd_f32")
     # dQ = dS . K  (NT product against K^T)
-    every_kv = torch.arange(B * Hkv, device=dev)
-    kT = torch.empty(B * Hkv, D, Lkp, dtype=w.dtype, device=dev)
-    _transpose_to(kp, every_kv, kT, every_kv, Lkp, D)
-    dq = grouped_gemm_nt(_ptr_table(kT, kv_of, D * Lkp), Lkp, D, row_start, row_count, E * Lp, E * Lp, D, Lkp, a=ds)
+    _transpose_tables(kp, k_in, k_out, Lkp, D)
+    dq = grouped_gemm_nt(kT_tab, Lkp, D, row_start, row_count, E * Lp, E * Lp, D, Lkp, a=ds)
     dq = dq.view(B, Hq, Lp, D)[:, :, :L].contiguous()
-    # dV and dK: per query head a product over the queries, written so that the `rep` heads of a kv head are
-    # `rep` slices of one buffer: group (b, hq) goes to slot (hq % rep) * (B * Hkv) + its kv matrix
-    slot = (e % Hq % rep) * (B * Hkv) + kv_of
-    slot_count = torch.full((E,), Lkp, dtype=torch.int32, device=dev)
-    order = torch.empty(E, dtype=torch.int64, device=dev)
-    order[slot] = e                                   # group that owns slot s
-    doT = torch.empty(E, D, Lp, dtype=w.dtype, device=dev)
-    _transpose_to(do, e, doT, e, Lp, D)
-    qT = torch.empty(E, D, Lp, dtype=w.dtype, device=dev)
-    _transpose_to(qp, e, qT, e, Lp, D)
+    _transpose_tables(do, do_in, do_out, Lp, D)
+    _transpose_tables(qp, q_in, q_out, Lp, D)
 
-    def over_queries(mat: torch.Tensor, rhsT: torch.Tensor) -> torch.Tensor:
+    def over_queries(in_tab, rhsT_tab) -> torch.Tensor:
         """sum over the heads of a kv group of mat[e]^T . rhs[e]: mat [E*Lp, Lkp], rhsT [E, D, Lp] -> [B,Hkv,Lkp,D]."""
-        matT = torch.empty(E, Lkp, Lp, dtype=w.dtype, device=dev)
-        _transpose_to(mat, e, matT, slot, Lp, Lkp)
-        # b_ptrs and row tables are read in group order 0..E-1 = slot order here
-        parts = grouped_gemm_nt(_ptr_table(rhsT, order, D * Lp), Lp, D, (torch.arange(E, device=dev) * Lkp).to(torch.int32),
-                                slot_count, E * Lkp, E * Lkp, D, Lp, a=matT.view(E * Lkp, Lp))
+        _transpose_tables(matT, in_tab, mat_out, Lp, Lkp)
+        parts = grouped_gemm_nt(rhsT_tab, Lp, D, slot_start, slot_count, E * Lkp, E * Lkp, D, Lp, a=matT.view(E * Lkp, Lp))
         parts = parts.view(rep, B * Hkv * Lkp * D)
         total = sum_partials(parts, torch.float32) if rep > 1 else parts[0]
         return total.view(B, Hkv, Lkp, D)[:, :, :Lk].contiguous()
 
-    dv = over_queries(w_drop if w_drop is not None else w, doT)
-    dk = over_queries(ds, qT)
+    dv = over_queries(w_in, doT_tab)
+    dk = over_queries(ds_in, qT_tab)
     return dq, dk, dv
 
 

@@ -397,6 +397,19 @@ int ats_router_bwd_dx(const float* dlogits, const void* wg, const void* base, vo
 size_t ats_router_bwd_dw_workspace(int64_t T, int E, int H);
 int ats_router_bwd_dw(const float* dlogits, const void* x, float* dwg, int64_t T, int E, int H, int dtype,
                       void* workspace, size_t workspace_bytes, ats_stream_t stream);
+/* Up to 20 device tables in one launch: out[i] = base + x(i) * stride for i < n, as int64 (wide) or int32, x by kind:
+ * i itself; for attention groups i = batch * q_heads + head: the key/value matrix batch * kv_heads + head / rep of
+ * group i (rep = q_heads / kv_heads), its slot (head % rep) * batch * kv_heads + that matrix, and the group that owns
+ * slot i; an int32 device array; or 0.  Addresses and row ranges of the grouped products. */
+enum { ATS_TABLE_INDEX = 0, ATS_TABLE_KV_OF_HEAD = 1, ATS_TABLE_SLOT_OF_HEAD = 2, ATS_TABLE_HEAD_OF_SLOT = 3,
+       ATS_TABLE_FROM_ARRAY = 4, ATS_TABLE_CONSTANT = 5 };
+typedef struct {
+    void* out;
+    int64_t base, stride;
+    const int32_t* index;
+    int n, kind, wide;
+} ats_table;
+int ats_fill_tables(const ats_table* tables, int n_tables, int batch, int q_heads, int kv_heads, ats_stream_t stream);
 /* Transposes that make the contraction dimension contiguous for the backward GEMMs:
  * E matrices [R, C] -> [C, R]; and grouped rows [*, C] (row r of expert e, optionally
  * gathered as in ats_grouped_gateup_swiglu) -> [C, ld_out] where expert e owns the columns
