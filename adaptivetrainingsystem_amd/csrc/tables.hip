@@ -6,6 +6,8 @@
 // writes every table that a step needs.  Bound: the launch itself (about 5 us on the timeline of a stream).  Built from
 // torch expressions, each table was two or three launches and as many host calls of 4-6 us: a float32 transformer block
 // made 107 of its 250 launches for them.
+#include <string.h>
+
 #include "ats_common.hpp"
 
 namespace ats {
@@ -40,7 +42,34 @@ __global__ __launch_bounds__(64) void fill_tables_kernel(TableArgs a) {
     }
 }
 
+// Small host arrays (a list of tensor addresses and sizes) as launch arguments: a copy from pageable memory waits until
+// the queue has drained, which left the GPU idle between the backward of the loss and the gradient norm.
+constexpr int kUploadBytes = 3584;           // of the 4 KiB that the arguments of a launch can have
+struct UploadArgs {
+    uint64_t w[kUploadBytes / 8];
+};
+__global__ __launch_bounds__(64) void upload_kernel(UploadArgs a, uint64_t* __restrict__ dst, int words) {
+    for (int i = threadIdx.x; i < words; i += 64) dst[i] = a.w[i];
+}
+
 }  // namespace ats
+
+extern "C" int ats_upload_max_bytes(void) { return ats::kUploadBytes; }
+
+extern "C" int ats_upload(void* dst, const void* src, int bytes, ats_stream_t stream) {
+    using namespace ats;
+    ATS_REQUIRE(bytes >= 0 && bytes <= kUploadBytes && bytes % 8 == 0, ATS_ERR_INVALID_ARG,
+                "ats_upload: %d bytes (a multiple of 8, at most %d)", bytes, kUploadBytes);
+    if (bytes == 0) return ATS_OK;
+    ATS_REQUIRE(dst && src && (reinterpret_cast<uintptr_t>(dst) & 7u) == 0, ATS_ERR_INVALID_ARG,
+                "ats_upload: null pointer or unaligned destination");
+    UploadArgs a;
+    memcpy(a.w, src, (size_t)bytes);
+    memset(reinterpret_cast<char*>(a.w) + bytes, 0, sizeof(a.w) - (size_t)bytes);
+    hipLaunchKernelGGL(upload_kernel, dim3(1), dim3(64), 0, as_stream(stream), a, static_cast<uint64_t*>(dst), bytes / 8);
+    ATS_CHECK_LAUNCH("ats_upload");
+    return ATS_OK;
+}
 
 extern "C" int ats_fill_tables(const ats_table* tables, int n_tables, int batch, int q_heads, int kv_heads,
                                ats_stream_t stream) {

@@ -8,6 +8,7 @@ trains through it); per-token weights and bf16 logits / gradients are handled by
 """
 from __future__ import annotations
 
+from array import array
 from typing import Dict, Iterable, Optional
 
 import torch
@@ -33,16 +34,17 @@ class CrossEntropyFunction(Function):
         f32 = dict(dtype=torch.float32, device=dev)
         loss_tok, lse = torch.empty(T, **f32), torch.empty(T, **f32)
         correct, valid = torch.empty(T, **f32), torch.empty(T, **f32)
-        sums = torch.empty(5, **f32)
-        check(_lib.load().ats_cross_entropy_fwd(logits.data_ptr(), labels.data_ptr(), int(pad_id),
-                                                None if weights is None else weights.data_ptr(), loss_tok.data_ptr(),
-                                                lse.data_ptr(), correct.data_ptr(), valid.data_ptr(), sums.data_ptr(),
-                                                T, V, _DT[logits.dtype], _stream()), "ats_cross_entropy_fwd")
+        sums, loss, report = torch.empty(5, **f32), torch.empty((), **f32), torch.empty(4, **f32)
+        check(_lib.load().ats_cross_entropy_fwd_stats(logits.data_ptr(), labels.data_ptr(), int(pad_id),
+                                                      None if weights is None else weights.data_ptr(),
+                                                      loss_tok.data_ptr(), lse.data_ptr(), correct.data_ptr(),
+                                                      valid.data_ptr(), sums.data_ptr(), loss.data_ptr(),
+                                                      report.data_ptr(), T, V, _DT[logits.dtype], _stream()),
+              "ats_cross_entropy_fwd_stats")
         ctx.save_for_backward(logits, labels, lse, valid, sums, weights if weights is not None else sums.new_empty(0))
         ctx.has_weights = weights is not None
-        stats["sums"] = sums
-        stats["loss_tok"] = loss_tok
-        return sums[0] / torch.clamp(sums[1], min=1e-8)
+        stats["report"] = report
+        return loss
 
     @staticmethod
     def backward(ctx, dloss):
@@ -84,19 +86,21 @@ class FusedLoss:
                 raise AtsError("FusedLoss: loss_weights must have one entry per token")
         stats: Dict[str, torch.Tensor] = {}
         loss = CrossEntropyFunction.apply(lg, lb, w, int(pad_token_id), stats)
-        sums = stats["sums"]
-        n_valid = sums[4]
-        denom = torch.clamp(n_valid, min=1.0)
-        raw = sums[2] / denom                                  # unweighted mean over the valid tokens
-        any_valid = n_valid > 0
-        inf = torch.full_like(raw, float("inf"))
-        return {
-            "loss": loss,
-            "raw_loss": raw.detach(),
-            "perplexity": torch.where(any_valid, torch.exp(torch.clamp(raw.detach(), min=0.0, max=15.0)), inf),
-            "valid_tokens": n_valid.detach(),
-            "accuracy": (sums[3] / denom).detach(),
-        }
+        raw, perplexity, n_valid, accuracy = stats["report"].unbind(0)        # raw: unweighted mean over the valid tokens
+        return {"loss": loss, "raw_loss": raw, "perplexity": perplexity, "valid_tokens": n_valid, "accuracy": accuracy}
+
+
+def _upload_tables(ptrs: list, sizes: list, starts: list, dev: torch.device):
+    """Two int64 tables and one int32 table on the device, sent with launches instead of copies."""
+    host = array("q", ptrs + sizes)
+    host.frombytes(array("i", starts + [0] * (len(starts) % 2)).tobytes())
+    buf = torch.empty(len(host), dtype=torch.int64, device=dev)
+    lib, (src, n) = _lib.load(), host.buffer_info()
+    step = lib.ats_upload_max_bytes()
+    for off in range(0, n * 8, step):
+        check(lib.ats_upload(buf.data_ptr() + off, src + off, min(step, n * 8 - off), _stream()), "ats_upload")
+    k = len(ptrs)
+    return buf[:k], buf[k:2 * k], buf[2 * k:].view(torch.int32)
 
 
 class FusedGradClip:
@@ -130,7 +134,7 @@ class FusedGradClip:
             if g.numel():
                 groups.setdefault(g.dtype, []).append(g)
         self.total_params = sum(g.numel() for g in grads)
-        norm_out = torch.zeros(2, dtype=torch.float32, device=dev)
+        norm_out = None
         tables = []
         extra = None
         for dtype, gs in groups.items():
@@ -138,11 +142,9 @@ class FusedGradClip:
             starts = [0]
             for n in sizes:
                 starts.append(starts[-1] + (n + chunk - 1) // chunk)
-            ptrs = torch.tensor([g.data_ptr() for g in gs], dtype=torch.int64, device=dev)
-            sizes_t = torch.tensor(sizes, dtype=torch.int64, device=dev)
-            starts_t = torch.tensor(starts, dtype=torch.int32, device=dev)
+            ptrs, sizes_t, starts_t = _upload_tables([g.data_ptr() for g in gs], sizes, starts, dev)
             partial = torch.empty(max(starts[-1], 1), dtype=torch.float32, device=dev)
-            out = torch.zeros(2, dtype=torch.float32, device=dev)
+            out = torch.empty(2, dtype=torch.float32, device=dev)
             single = len(groups) == 1
             check(lib.ats_grad_norm_clip(ptrs.data_ptr(), sizes_t.data_ptr(), starts_t.data_ptr(), len(gs), starts[-1],
                                          _DT[dtype], None if extra is None else extra[1:].data_ptr(),
@@ -156,7 +158,7 @@ class FusedGradClip:
                 check(lib.ats_grad_norm_clip(ptrs.data_ptr(), sizes_t.data_ptr(), starts_t.data_ptr(), n, n_chunks,
                                              _DT[dtype], None, partial.data_ptr(), norm_out.data_ptr(), float(max_norm),
                                              2, _stream()), "ats_grad_norm_clip")
-        return norm_out[0]
+        return torch.zeros((), dtype=torch.float32, device=dev) if norm_out is None else norm_out[0]
 
     def __call__(self, parameters, max_norm) -> float:
         params = [p for p in parameters]

@@ -409,6 +409,10 @@ typedef struct {
     const int32_t* index;
     int n, kind, wide;
 } ats_table;
+/* Copies at most ats_upload_max_bytes() bytes of host memory to the device inside the arguments of a launch: in stream
+ * order, without waiting for the queue, and the host memory may change when the call returns.  dst 8-byte aligned. */
+int ats_upload_max_bytes(void);
+int ats_upload(void* dst, const void* src, int bytes, ats_stream_t stream);
 int ats_fill_tables(const ats_table* tables, int n_tables, int batch, int q_heads, int kv_heads, ats_stream_t stream);
 /* Transposes that make the contraction dimension contiguous for the backward GEMMs:
  * E matrices [R, C] -> [C, R]; and grouped rows [*, C] (row r of expert e, optionally
@@ -550,6 +554,11 @@ int ats_attention_softmax_bwd_f32(const float* weights, float* dp, int B, int Hq
 int ats_cross_entropy_fwd(const void* logits, const int64_t* labels, int64_t pad_id, const float* weights,
                           float* loss_tok, float* lse, float* correct, float* valid, float* sums, int64_t T,
                           int V, int dtype, ats_stream_t stream);
+/* As ats_cross_entropy_fwd, and with loss / stats not NULL also loss[0] = sums[0] / max(sums[1], 1e-8) and stats = mean
+ * loss over the valid tokens, its perplexity exp(clamp(mean, 0, 15)) (inf without valid tokens), their number, accuracy. */
+int ats_cross_entropy_fwd_stats(const void* logits, const int64_t* labels, int64_t pad_id, const float* weights,
+                                float* loss_tok, float* lse, float* correct, float* valid, float* sums, float* loss,
+                                float* stats, int64_t T, int V, int dtype, ats_stream_t stream);
 /* Gradient of sums[0] / max(sums[1], 1e-8) w.r.t. the logits, times the device scalar scale[0]:
  * dlogits[t,v] = scale * w_t * valid_t / max(sums[1], 1e-8) * (exp(z - lse_t) - [v == label_t]).
  * (The reference's fused loss returns a value without a graph; its fallback uses autograd.) */
