@@ -259,6 +259,25 @@ struct RopeCacheTarget {
     int64_t pos;
 };
 
+static int rope_run(const char* name, float sin_sign, const ats::RopeSeg& q, const ats::RopeSeg& k, const ats::RopeSeg& v3,
+                    const float* cos_tab, const float* sin_tab, int table_stride, int B, int L, int D, int pos_offset, int dtype,
+                    ats_stream_t stream) {
+    using namespace ats;
+    const int V = dtype == ATS_F32 ? 4 : 8;
+    auto seg_ok = [&](const RopeSeg& sgm) {
+        return sgm.heads == 0 || (aligned16(sgm.in) && aligned16(sgm.out) && sgm.sb % V == 0 && sgm.sh % V == 0 &&
+                                  sgm.sl % V == 0 && sgm.ob % V == 0 && sgm.oh % V == 0 && sgm.ol % V == 0);
+    };
+    const int half = D / 2;
+    const bool vec_ok = half % V == 0 && half / V <= kWave && seg_ok(q) && seg_ok(k) && seg_ok(v3);
+    if (dtype == ATS_F32)
+        launch_rope<float>(q, k, v3, cos_tab, sin_tab, table_stride, B, L, D, pos_offset, vec_ok, sin_sign, as_stream(stream));
+    else
+        launch_rope<bf16_t>(q, k, v3, cos_tab, sin_tab, table_stride, B, L, D, pos_offset, vec_ok, sin_sign, as_stream(stream));
+    ATS_CHECK_LAUNCH(name);
+    return ATS_OK;
+}
+
 static int rope_apply(const char* name, float sin_sign, const void* q_in, const void* k_in, void* q_out, void* k_out,
                       const float* cos_tab, const float* sin_tab, int table_stride, int table_len, int B, int Hq,
                       int Hkv, int L, int D, int pos_offset, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb,
@@ -287,19 +306,32 @@ static int rope_apply(const char* name, float sin_sign, const void* q_in, const 
         v3.ob = cache->cb, v3.oh = cache->ch, v3.ol = cache->cl;
         v3.rotate = 0;
     }
-    const int V = dtype == ATS_F32 ? 4 : 8;
-    auto seg_ok = [&](const RopeSeg& sgm) {
-        return sgm.heads == 0 || (aligned16(sgm.in) && aligned16(sgm.out) && sgm.sb % V == 0 && sgm.sh % V == 0 &&
-                                  sgm.sl % V == 0 && sgm.ob % V == 0 && sgm.oh % V == 0 && sgm.ol % V == 0);
-    };
-    const int half = D / 2;
-    const bool vec_ok = half % V == 0 && half / V <= kWave && seg_ok(q) && seg_ok(k) && seg_ok(v3);
-    if (dtype == ATS_F32)
-        launch_rope<float>(q, k, v3, cos_tab, sin_tab, table_stride, B, L, D, pos_offset, vec_ok, sin_sign, as_stream(stream));
-    else
-        launch_rope<bf16_t>(q, k, v3, cos_tab, sin_tab, table_stride, B, L, D, pos_offset, vec_ok, sin_sign, as_stream(stream));
-    ATS_CHECK_LAUNCH(name);
-    return ATS_OK;
+    return rope_run(name, sin_sign, q, k, v3, cos_tab, sin_tab, table_stride, B, L, D, pos_offset, dtype, stream);
+}
+
+extern "C" int ats_rope_strided(const void* const* in, void* const* out, const int64_t* in_strides, const int64_t* out_strides,
+                                const float* cos_tab, const float* sin_tab, int table_stride, int table_len, int B,
+                                const int* heads, int L, int D, int pos_offset, int inverse, int dtype, ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_rope_strided";
+    ATS_REQUIRE(in && out && in_strides && out_strides && heads, ATS_ERR_INVALID_ARG, "%s: null argument array", name);
+    ATS_REQUIRE(B >= 0 && heads[0] >= 0 && heads[1] >= 0 && heads[2] >= 0 && L >= 0 && D > 0 && D % 2 == 0, ATS_ERR_INVALID_ARG,
+                "%s: B=%d heads=%d/%d/%d L=%d D=%d", name, B, heads[0], heads[1], heads[2], L, D);
+    ATS_REQUIRE(dtype == ATS_F32 || dtype == ATS_BF16, ATS_ERR_UNSUPPORTED, "%s: dtype tag %d", name, dtype);
+    if (B == 0 || L == 0 || heads[0] + heads[1] + heads[2] == 0) return ATS_OK;
+    ATS_REQUIRE(cos_tab && sin_tab && table_stride >= D / 2, ATS_ERR_INVALID_ARG,
+                "%s: table pointers/stride (stride=%d, need >= %d)", name, table_stride, D / 2);
+    ATS_REQUIRE(pos_offset >= 0 && (int64_t)pos_offset + L <= table_len, ATS_ERR_INVALID_ARG,
+                "%s: positions %d..%d exceed table length %d", name, pos_offset, pos_offset + L - 1, table_len);
+    RopeSeg seg[3];
+    for (int i = 0; i < 3; ++i) {
+        ATS_REQUIRE(heads[i] == 0 || (in[i] && out[i]), ATS_ERR_INVALID_ARG, "%s: null tensor pointer", name);
+        seg[i] = rope_seg(in[i], out[i], in_strides[3 * i], in_strides[3 * i + 1], in_strides[3 * i + 2], heads[i], L, D);
+        seg[i].ob = out_strides[3 * i], seg[i].oh = out_strides[3 * i + 1], seg[i].ol = out_strides[3 * i + 2];
+    }
+    seg[2].rotate = 0;
+    return rope_run(name, inverse ? -1.0f : 1.0f, seg[0], seg[1], seg[2], cos_tab, sin_tab, table_stride, B, L, D, pos_offset,
+                    dtype, stream);
 }
 
 extern "C" int ats_rope_fwd(const void* q_in, const void* k_in, void* q_out, void* k_out, const float* cos_tab,

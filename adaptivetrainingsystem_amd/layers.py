@@ -256,19 +256,17 @@ class GroupedQueryAttention(nn.Module):
         x2 = x.reshape(B * L, H).contiguous()
         grad = torch.is_grad_enabled() and _wants_grad(x, self.q_proj.weight, self.k_proj.weight, self.v_proj.weight,
                                                        self.o_proj.weight)
+        # positions 0..L-1 also when a cache is passed, as the reference does (model.py:690-698)
+        cos, sin = self.rope(L, x.device)
         if grad:
             lin = ag.LinearFunction.apply
-            q = lin(x2, self.q_proj.weight).view(B, L, nh, D).transpose(1, 2)
-            k = lin(x2, self.k_proj.weight).view(B, L, nkv, D).transpose(1, 2)
-            v = lin(x2, self.v_proj.weight).view(B, L, nkv, D).transpose(1, 2)
+            q, k, v = ag.QKVRoPEFunction.apply(x2, self.q_proj.weight, self.k_proj.weight, self.v_proj.weight, cos, sin, B, L, D)
         else:
             # one product with the three weights stacked (a copy kept until a weight changes): a third of the
             # launches, which is what a decoding step is made of; q, k, v are column ranges of its output
             lin = lambda a, w: ops.linear_nt(a, _as_dtype(w, a.dtype))
             qkv = ops.linear_nt(x2, self._stacked_qkv(x.dtype)).view(B, L, nh + 2 * nkv, D).transpose(1, 2)
             q, k, v = qkv[:, :nh], qkv[:, nh:nh + nkv], qkv[:, nh + nkv:]
-        # positions 0..L-1 also when a cache is passed, as the reference does (model.py:690-698)
-        cos, sin = self.rope(L, x.device)
         if past_key_value is not None:
             k_cache, v_cache = past_key_value
             if (k_cache.dim() != 4 or k_cache.shape[0] != B or k_cache.shape[1] != nkv or k_cache.shape[3] != D
@@ -278,7 +276,8 @@ class GroupedQueryAttention(nn.Module):
             # the rotation writes the new keys, and the values beside them, straight behind the cache
             q, k, v = self._extend_cache(k_cache, v_cache, q, k, v, cos, sin)
         else:
-            q, k = ag.RoPEFunction.apply(q, k, cos, sin, 0) if grad else ops.rope(q, k, cos, sin, 0)
+            if not grad:
+                q, k = ops.rope(q, k, cos, sin, 0)
             if past_key_value is not None:
                 k = torch.cat([k_cache.to(k.dtype), k], dim=2)
                 v = torch.cat([v_cache.to(v.dtype), v], dim=2)

@@ -8,6 +8,7 @@ GPU; there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+from array import array
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -115,6 +116,38 @@ def rope(q: torch.Tensor, k: Optional[torch.Tensor], cos: torch.Tensor, sin: tor
                                      sin.data_ptr(), cos.stride(0), cos.shape[0], B, Hq, Hkv, L, D,
                                      int(position_offset), qsb, qsh, qsl, ksb, ksh, ksl, _tag(q), _stream()), name)
     return q_out, k_out
+
+
+def rope_strided(ins: Sequence[Optional[torch.Tensor]], outs: Sequence[Optional[torch.Tensor]], cos: torch.Tensor,
+                 sin: torch.Tensor, position_offset: int = 0, inverse: bool = False) -> None:
+    """Rotates ins[0], ins[1] into outs[0], outs[1] and copies ins[2] into outs[2] (None: no such segment), one launch; all
+    [B, heads, L, D] of one type with any strides but that of D."""
+    _need_gpu(*ins, *outs, cos, sin)
+    given = [t for t in ins if t is not None]
+    B, _, L, D = given[0].shape
+    src, dst, ss, ds, heads = [], [], [], [], []
+    for i, o in zip(ins, outs):
+        if i is None:
+            src.append(None), dst.append(None), heads.append(0)
+            ss += [0, 0, 0]
+            ds += [0, 0, 0]
+            continue
+        if i.dim() != 4 or i.shape != o.shape or i.shape[0] != B or i.shape[2] != L or i.shape[3] != D \
+                or i.dtype != given[0].dtype or o.dtype != i.dtype or o.stride(3) != 1:
+            raise AtsError(f"rope_strided: segment {tuple(i.shape)}/{i.dtype} -> {tuple(o.shape)}/{o.dtype}")
+        i, *strides = _bhl_strides(i)
+        given.append(i)                              # (a copy stays alive until the launch is queued)
+        src.append(i.data_ptr()), dst.append(o.data_ptr()), heads.append(i.shape[1])
+        ss += strides
+        ds += o.stride()[:3]
+    if cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != sin.shape or cos.dim() != 2:
+        raise AtsError("rope_strided: cos/sin must be float32 2-D tables of equal shape")
+    if cos.stride(1) != 1 or sin.stride(1) != 1 or cos.stride(0) != sin.stride(0):
+        cos, sin = cos.contiguous(), sin.contiguous()
+    check(_lib.load().ats_rope_strided((ctypes.c_void_p * 3)(*src), (ctypes.c_void_p * 3)(*dst), (ctypes.c_int64 * 9)(*ss),
+                                       (ctypes.c_int64 * 9)(*ds), cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[0],
+                                       B, (ctypes.c_int * 3)(*heads), L, D, int(position_offset), int(inverse),
+                                       _tag(given[0]), _stream()), "ats_rope_strided")
 
 
 def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
@@ -309,6 +342,57 @@ def fill_tables(device: torch.device, specs: Sequence[tuple], heads: Tuple[int, 
         outs.append(row if row.numel() == n else row[:n])
     check(_lib.load().ats_fill_tables(arr, len(specs), *heads, _stream()), "ats_fill_tables")
     return outs
+
+
+def upload(words: array, device: torch.device) -> torch.Tensor:
+    """An int64 array on the device, sent with launches instead of a copy that waits for the queue."""
+    lib, (src, n) = _lib.load(), words.buffer_info()
+    buf = torch.empty(n, dtype=torch.int64, device=device)
+    step = lib.ats_upload_max_bytes()
+    for off in range(0, n * 8, step):
+        check(lib.ats_upload(buf.data_ptr() + off, src + off, min(step, n * 8 - off), _stream()), "ats_upload")
+    return buf
+
+
+def wgrad_slices(M: int, N: int, rows: int) -> int:
+    """K slices of a weight gradient [M, N] over `rows` bfloat16 rows.  Its 256 x 256 tiles are few (16 of a [1024, 1024]
+    gradient) and its K long: slices over workgroups, added in float32, fill the chip.  Least estimated time in microseconds:
+    rounds of 256 CUs, 1.45 per 64-row slab and 7 per tile, and the partial results written and read at 5 TB/s.  Measured,
+    one slice | the rule's: 16384 rows [1024, 4096] 342 | 117 (four), [2048, 2048] 342 | 117 (four), [2048, 4096] 344 | 208
+    (two; four 226), [4096, 4096] 384 | (two 407); 2048 rows [2048, 2048] 56 | 51 (two; four 44); 512 rows [2048, 4096]
+    25 | (two 41)."""
+    tiles, slabs = -(-M // 256) * -(-N // 256), -(-rows // 64)
+    best, slices = None, 1
+    for s in range(1, 17):
+        if s > 1 and slabs < 8 * s:
+            break
+        t = -(-tiles * s // 256) * (-(-slabs // s) * 1.45 + 7.0) + (s * M * N * 8 / 5e6 + 6.0 if s > 1 else 0.0)
+        if best is None or t < 0.95 * best:
+            best, slices = t, s
+    return slices
+
+
+def wgrad_dense(lhsT: torch.Tensor, rhsT: torch.Tensor, rows: int) -> torch.Tensor:
+    """lhsT @ rhsT^T over the first `rows` columns (zero padded to a multiple of 64) of two contiguous transposed operands
+    [M, ld], [N, ld]: the weight gradient of a linear layer."""
+    _need_gpu(lhsT, rhsT)
+    (M, ld), N, es, dtype = lhsT.shape, rhsT.shape[0], lhsT.element_size(), lhsT.dtype
+    slices = wgrad_slices(M, N, rows) if dtype == torch.bfloat16 and (M * N) % 8 == 0 else 1
+    slabs = max(1, -(-rows // 64))
+    per = -(-slabs // slices)
+    slices = -(-slabs // per)
+    tab = array("q", [lhsT.data_ptr() + i * per * 64 * es for i in range(slices)] +
+                [rhsT.data_ptr() + i * per * 64 * es for i in range(slices)])
+    rc = [i * M for i in range(slices)] + [M] * slices + [min(per, slabs - i * per) * 64 for i in range(slices)]
+    tab.frombytes(array("i", rc + [0] * (len(rc) % 2)).tobytes())
+    buf = upload(tab, lhsT.device)
+    r32 = buf[2 * slices:].view(torch.int32)
+    parts = grouped_gemm_nt(buf[slices:2 * slices], ld, N, r32[:slices], r32[slices:2 * slices], slices * M, slices * M, N, ld,
+                            a_ptrs=buf[:slices], lda=ld, k_count=r32[2 * slices:3 * slices], dtype=dtype,
+                            out_dtype=dtype if slices == 1 else torch.float32)
+    if slices == 1:
+        return parts
+    return sum_partials(parts.view(slices, M * N), dtype).view(M, N)
 
 
 def wgrad_tables(k_start: torch.Tensor, M: int, lhsT: torch.Tensor, rhsT: torch.Tensor) -> list:

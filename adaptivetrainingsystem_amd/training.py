@@ -14,7 +14,7 @@ from typing import Dict, Iterable, Optional
 import torch
 from torch.autograd import Function
 
-from . import _lib
+from . import _lib, ops
 from ._lib import ATS_BF16, ATS_F32, AtsError, check
 
 _DT = {torch.float32: ATS_F32, torch.bfloat16: ATS_BF16}
@@ -94,11 +94,7 @@ def _upload_tables(ptrs: list, sizes: list, starts: list, dev: torch.device):
     """Two int64 tables and one int32 table on the device, sent with launches instead of copies."""
     host = array("q", ptrs + sizes)
     host.frombytes(array("i", starts + [0] * (len(starts) % 2)).tobytes())
-    buf = torch.empty(len(host), dtype=torch.int64, device=dev)
-    lib, (src, n) = _lib.load(), host.buffer_info()
-    step = lib.ats_upload_max_bytes()
-    for off in range(0, n * 8, step):
-        check(lib.ats_upload(buf.data_ptr() + off, src + off, min(step, n * 8 - off), _stream()), "ats_upload")
+    buf = ops.upload(host, dev)
     k = len(ptrs)
     return buf[:k], buf[k:2 * k], buf[2 * k:].view(torch.int32)
 

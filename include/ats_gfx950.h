@@ -80,6 +80,12 @@ int ats_rope_fwd(const void* q_in, const void* k_in, void* q_out, void* k_out, c
                  const float* sin_tab, int table_stride, int table_len, int B, int Hq, int Hkv, int L,
                  int D, int pos_offset, int64_t q_sb, int64_t q_sh, int64_t q_sl, int64_t k_sb,
                  int64_t k_sh, int64_t k_sl, int dtype, ats_stream_t stream);
+/* The rotation of ats_rope_fwd (inverse != 0: of ats_rope_bwd) on the segments 0 and 1, and a plain copy of segment 2, in
+ * one launch and between any layouts: heads[i] heads each, element strides {batch, head, position} per segment on both
+ * sides.  The gradients of a stacked query/key/value projection leave it in the projection's own layout. */
+int ats_rope_strided(const void* const* in, void* const* out, const int64_t* in_strides, const int64_t* out_strides,
+                     const float* cos_tab, const float* sin_tab, int table_stride, int table_len, int B, const int* heads,
+                     int L, int D, int pos_offset, int inverse, int dtype, ats_stream_t stream);
 /* ats_rope_fwd whose rotated keys, and the values beside them, are appended to a key / value cache instead of
  * going into tensors of their own: the in-place form of torch.cat([past_key, k], dim=2) /
  * torch.cat([past_value, v], dim=2) in GroupedQueryAttention.forward (model.py:700-704) for a cache buffer
