@@ -40,6 +40,9 @@ _SIGNATURES = {
     "ats_route_topk_workspace": (c_size_t, [c_int64, c_int]),
     "ats_route_topk": (c_int, [c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p, c_void_p, c_void_p,
                                c_void_p, c_void_p, c_float, c_void_p, c_size_t, c_void_p]),
+    "ats_route_plan_supported": (c_int, [c_int64, c_int, c_int]),
+    "ats_route_plan": (c_int, [c_void_p, c_int64, c_int, c_int, c_float, c_int] + [c_void_p] * 5 +
+                       [c_float, c_void_p, c_size_t, c_int] + [c_void_p] * 9),
     "ats_dispatch_plan_workspace": (c_size_t, [c_int64, c_int, c_int]),
     "ats_dispatch_plan": (c_int, [c_void_p, c_int, c_int64, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -15,42 +15,13 @@
 #include <limits.h>
 
 #include "ats_common.hpp"
+#include "dispatch_plan.hpp"
 
 // Products and sums below must round separately (the reference computes them as separate
 // tensor ops); the HIP default would contract a*b+c into one fused multiply-add.
 #pragma clang fp contract(off)
 
 namespace ats {
-
-constexpr int kPlanChunk = 256;      // assignments per block of the multi-block plan (64 per wave: one step)
-constexpr int kPlanSingle = 1024;    // largest plan done by one block alone (256 per wave: four steps)
-constexpr int kPlanMaxE = 1024;
-
-template <typename IdxT>
-__device__ __forceinline__ int load_expert(const IdxT* idx, int64_t a, int64_t n, int E, bool* bad) {
-    if (a >= n) return -1;
-    const long long e = (long long)idx[a];
-    if (e < 0 || e >= E) {
-        *bad = true;
-        return -1;
-    }
-    return (int)e;
-}
-
-// step 1: counts of one chunk into LDS (s_cnt[w*E + e] per wave), returns via LDS
-template <typename IdxT, int PERWAVE>
-__device__ void chunk_wave_counts(const IdxT* idx, int64_t n, int E, int64_t chunk_base, int* s_cnt, bool* bad) {
-    const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < 4 * E; i += 256) s_cnt[i] = 0;
-    __syncthreads();
-    for (int step = 0; step < PERWAVE / kWave; ++step) {
-        const int64_t a = chunk_base + wave * PERWAVE + step * kWave + lane;
-        const int e = load_expert(idx, a, n, E, bad);
-        if (e >= 0) atomicAdd(&s_cnt[wave * E + e], 1);
-    }
-    __syncthreads();
-}
 
 template <typename IdxT>
 __global__ __launch_bounds__(256) void plan_hist_kernel(const IdxT* __restrict__ idx, int64_t n, int E,
@@ -65,137 +36,11 @@ __global__ __launch_bounds__(256) void plan_hist_kernel(const IdxT* __restrict__
     if (blockIdx.x == 0 && threadIdx.x == 0) status[0] = 0;
 }
 
-// step 2 (one block): chunk_hist -> exclusive chunk bases (in place), hist, kept, offsets.  chunk_hist is
-// [E, nchunks]: an expert's chunk counts lie side by side, so the lanes of a scanning wave read one line.
-// A wave scans four experts at a time: 64 chunks per pass with a prefix sum over the wave, the carry
-// runs across passes.
-__device__ void scan_totals(int32_t* chunk_hist, int nchunks, int E, int C, int32_t* hist, int32_t* kept,
-                            int32_t* offsets, int* s_tot) {
-    const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
-    const int nwaves = blockDim.x >> 6;
-    constexpr int U = 4;   // experts scanned together by a wave (their loads are issued back to back)
-    constexpr int P = 2;   // passes of 64 chunks whose loads are issued together
-    for (int e0 = wave * U; e0 < E; e0 += nwaves * U) {
-        int carry[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) carry[u] = 0;
-        for (int base = 0; base < nchunks; base += P * kWave) {
-            int v[P][U];
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                const int c = base + q * kWave + lane;
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    v[q][u] = (c < nchunks && e0 + u < E) ? chunk_hist[(int64_t)(e0 + u) * nchunks + c] : 0;
-            }
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                const int c = base + q * kWave + lane;
-                if (base + q * kWave >= nchunks) break;      // wave-uniform
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int incl = wave_inclusive_scan(v[q][u]);
-                    if (c < nchunks && e0 + u < E) chunk_hist[(int64_t)(e0 + u) * nchunks + c] = carry[u] + incl - v[q][u];
-                    carry[u] += __builtin_amdgcn_readlane(incl, kWave - 1);
-                }
-            }
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (e0 + u < E) {
-                    hist[e0 + u] = carry[u];
-                    const int kp = carry[u] < C ? carry[u] : C;
-                    kept[e0 + u] = kp;
-                    s_tot[e0 + u] = kp;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // offsets = exclusive prefix sums of the kept counts: the first wave, 64 experts per step
-    if (wave == 0) {
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += kWave) {
-            const int e = e0 + lane;
-            const int kp = e < E ? s_tot[e] : 0;
-            const int incl = wave_inclusive_scan(kp);
-            if (e < E) offsets[e] = run + incl - kp;
-            run += __builtin_amdgcn_readlane(incl, kWave - 1);
-        }
-        if (lane == 0) offsets[E] = run;
-    }
-    __syncthreads();
-}
-
 __global__ __launch_bounds__(1024) void plan_scan_kernel(int32_t* __restrict__ chunk_hist, int nchunks, int E, int C,
                                                         int32_t* __restrict__ hist, int32_t* __restrict__ kept,
                                                         int32_t* __restrict__ offsets) {
     extern __shared__ int s_tot[];
     scan_totals(chunk_hist, nchunks, E, C, hist, kept, offsets, s_tot);
-}
-
-// step 3: ranks of one chunk.  s_cnt holds the per-wave counts of this chunk
-// (from chunk_wave_counts); they are turned into per-wave running bases.
-template <typename IdxT, int PERWAVE>
-__device__ void chunk_rank_and_write(const IdxT* idx, int64_t n, int k, int E, int C, int64_t chunk_base,
-                                     const int32_t* chunk_excl /* this chunk's entry of expert 0 */, int chunk_pitch,
-                                     const int32_t* offsets, int* s_cnt, int32_t* slot, int32_t* token_map,
-                                     int32_t* row_src, int32_t* row_of) {
-    const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
-    // per-wave running base = chunk base + counts of the earlier waves
-    for (int e = threadIdx.x; e < E; e += 256) {
-        int run = chunk_excl[(int64_t)e * chunk_pitch];
-        for (int w = 0; w < 4; ++w) {
-            const int v = s_cnt[w * E + e];
-            s_cnt[w * E + e] = run;
-            run += v;
-        }
-    }
-    __syncthreads();
-    int* my_base = s_cnt + wave * E;
-    const unsigned long long lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    // up to 64 experts: lane l keeps the running base of expert l in a register, so the loop below touches no LDS
-    const bool in_regs = E <= kWave;
-    int base_reg = (in_regs && lane < E) ? my_base[lane] : 0;
-    for (int step = 0; step < PERWAVE / kWave; ++step) {
-        const int64_t a = chunk_base + wave * PERWAVE + step * kWave + lane;
-        bool bad = false;
-        const int e = load_expert(idx, a, n, E, &bad);
-        int rank = -1;
-        unsigned long long remaining = __ballot(e >= 0);
-        while (remaining) {
-            // the leader and its expert are the same in all lanes: scalar reads instead of shuffles
-            const int leader = __builtin_amdgcn_readfirstlane(__ffsll((long long)remaining) - 1);
-            const int le = __builtin_amdgcn_readlane(e, leader);
-            const unsigned long long same = __ballot(e == le);
-            const int n_same = __popcll(same);
-            if (in_regs) {
-                const int b = __builtin_amdgcn_readlane(base_reg, le);
-                if (e == le) rank = b + __popcll(same & lt_mask);
-                if (lane == le) base_reg += n_same;
-            } else {
-                if (e == le) rank = my_base[le] + __popcll(same & lt_mask);
-                // all lanes have read my_base[le]; the leader advances it for the next step
-                if (lane == leader) my_base[le] += n_same;
-            }
-            remaining &= ~same;
-        }
-        if (a < n) {
-            if (e >= 0 && rank < C) {
-                const int row = offsets[e] + rank;
-                slot[a] = rank;
-                token_map[(int64_t)e * C + rank] = (int32_t)a;
-                row_src[row] = (int32_t)a;
-                row_of[a] = row;
-            } else {
-                slot[a] = -1;
-                row_of[a] = -1;
-            }
-        }
-    }
 }
 
 template <typename IdxT>
@@ -357,38 +202,14 @@ __global__ __launch_bounds__(256) void plan_fused_kernel(const IdxT* __restrict_
     for (int64_t i = total + (int64_t)blockIdx.x * 256 + threadIdx.x; i < row_src_len; i += stride) row_src[i] = -1;
 }
 
-// Whole plan in one block (n <= kPlanSingle).
 template <typename IdxT>
-__global__ __launch_bounds__(256) void plan_single_kernel(const IdxT* idx, int64_t n, int k, int E,
-                                                          int C, int32_t* chunk_hist,
-                                                          int32_t* hist, int32_t* kept,
-                                                          int32_t* offsets, int32_t* slot,
-                                                          int32_t* token_map,
-                                                          int32_t* row_src, int32_t* row_of,
+__global__ __launch_bounds__(256) void plan_single_kernel(const IdxT* idx, int64_t n, int k, int E, int C, int32_t* hist,
+                                                          int32_t* kept, int32_t* offsets, int32_t* slot,
+                                                          int32_t* token_map, int32_t* row_src, int32_t* row_of,
                                                           int64_t row_src_len, int32_t* status) {
     extern __shared__ int s_all[];
-    int* s_cnt = s_all;          // [4*E]
-    int* s_tot = s_all + 4 * E;  // [E]
-    bool bad = false;
-    chunk_wave_counts<IdxT, kPlanSingle / 4>(idx, n, E, 0, s_cnt, &bad);
-    if (threadIdx.x == 0) status[0] = 0;
-    __syncthreads();
-    if (bad) status[0] = 1;
-    for (int e = threadIdx.x; e < E; e += 256)
-        chunk_hist[e] = s_cnt[e] + s_cnt[E + e] + s_cnt[2 * E + e] + s_cnt[3 * E + e];
-    __syncthreads();
-    scan_totals(chunk_hist, 1, E, C, hist, kept, offsets, s_tot);
-    __threadfence_block();
-    chunk_rank_and_write<IdxT, kPlanSingle / 4>(idx, n, k, E, C, 0, chunk_hist, 1, offsets, s_cnt, slot, token_map, row_src,
-                                                row_of);
-    const int64_t ec = (int64_t)E * C;
-    for (int64_t i = threadIdx.x; i < ec; i += 256) {
-        const int e = (int)(i / C);
-        const int pos = (int)(i - (int64_t)e * C);
-        if (pos >= kept[e]) token_map[i] = -1;
-    }
-    const int total = offsets[E];
-    for (int64_t i = total + threadIdx.x; i < row_src_len; i += 256) row_src[i] = -1;
+    plan_single_block<IdxT>(idx, nullptr, n, k, E, C, hist, kept, offsets, slot, token_map, row_src, row_of, row_src_len,
+                            status, s_all);
 }
 
 // ------------------------------------------------------------------ row gather
@@ -832,14 +653,15 @@ extern "C" int ats_dispatch_plan(const void* idx, int idx_dtype, int64_t T, int 
         ATS_CHECK_LAUNCH("ats_dispatch_plan(fused)");
         return ATS_OK;
     }
+    const size_t smem_single = ((size_t)6 * E + 1) * sizeof(int);
     if (single) {
         if (idx_dtype == ATS_IDX_I32)
-            hipLaunchKernelGGL((plan_single_kernel<int32_t>), dim3(1), dim3(256), smem, s,
-                               static_cast<const int32_t*>(idx), n, k, E, C, chunk_hist, hist, kept, offsets, slot,
+            hipLaunchKernelGGL((plan_single_kernel<int32_t>), dim3(1), dim3(256), smem_single, s,
+                               static_cast<const int32_t*>(idx), n, k, E, C, hist, kept, offsets, slot,
                                token_map, row_src, row_of, row_src_len, status);
         else
-            hipLaunchKernelGGL((plan_single_kernel<int64_t>), dim3(1), dim3(256), smem, s,
-                               static_cast<const int64_t*>(idx), n, k, E, C, chunk_hist, hist, kept, offsets, slot,
+            hipLaunchKernelGGL((plan_single_kernel<int64_t>), dim3(1), dim3(256), smem_single, s,
+                               static_cast<const int64_t*>(idx), n, k, E, C, hist, kept, offsets, slot,
                                token_map, row_src, row_of, row_src_len, status);
         ATS_CHECK_LAUNCH("ats_dispatch_plan(single)");
         return ATS_OK;

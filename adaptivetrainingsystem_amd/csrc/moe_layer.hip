@@ -63,15 +63,24 @@ extern "C" int ats_moe_forward(const void* x, const void* gate, const float* gat
 
     int rc = ats_router_logits(x, gate, gate_bias, logits, T, H, E, dtype, stream);
     if (rc != ATS_OK) return rc;
-    rc = ats_route_topk(logits, T, E, k, temperature, variant, i32(ATS_MOE_LAYOUT_INDICES), w, i32(ATS_MOE_LAYOUT_ROUTED),
-                        static_cast<float*>(at(ATS_MOE_LAYOUT_PROB_COLSUM)), aux, load_balancing_weight,
-                        at(ATS_MOE_LAYOUT_ROUTE_WS), route_ws, stream);
-    if (rc != ATS_OK) return rc;
-    rc = ats_dispatch_plan(i32(ATS_MOE_LAYOUT_INDICES), ATS_IDX_I32, T, k, E, C, i32(ATS_MOE_LAYOUT_SLOT),
-                           i32(ATS_MOE_LAYOUT_TOKEN_MAP), i32(ATS_MOE_LAYOUT_HIST), i32(ATS_MOE_LAYOUT_KEPT),
-                           i32(ATS_MOE_LAYOUT_OFFSETS), i32(ATS_MOE_LAYOUT_ROW_SRC), i32(ATS_MOE_LAYOUT_ROW_OF),
-                           i32(ATS_MOE_LAYOUT_STATUS), at(ATS_MOE_LAYOUT_PLAN_WS), plan_ws, stream);
-    if (rc != ATS_OK) return rc;
+    if (ats_route_plan_supported(T, E, k)) {
+        rc = ats_route_plan(logits, T, E, k, temperature, variant, i32(ATS_MOE_LAYOUT_INDICES), w, i32(ATS_MOE_LAYOUT_ROUTED),
+                            static_cast<float*>(at(ATS_MOE_LAYOUT_PROB_COLSUM)), aux, load_balancing_weight,
+                            at(ATS_MOE_LAYOUT_ROUTE_WS), route_ws, C, i32(ATS_MOE_LAYOUT_SLOT), i32(ATS_MOE_LAYOUT_TOKEN_MAP),
+                            i32(ATS_MOE_LAYOUT_HIST), i32(ATS_MOE_LAYOUT_KEPT), i32(ATS_MOE_LAYOUT_OFFSETS),
+                            i32(ATS_MOE_LAYOUT_ROW_SRC), i32(ATS_MOE_LAYOUT_ROW_OF), i32(ATS_MOE_LAYOUT_STATUS), stream);
+        if (rc != ATS_OK) return rc;
+    } else {
+        rc = ats_route_topk(logits, T, E, k, temperature, variant, i32(ATS_MOE_LAYOUT_INDICES), w, i32(ATS_MOE_LAYOUT_ROUTED),
+                            static_cast<float*>(at(ATS_MOE_LAYOUT_PROB_COLSUM)), aux, load_balancing_weight,
+                            at(ATS_MOE_LAYOUT_ROUTE_WS), route_ws, stream);
+        if (rc != ATS_OK) return rc;
+        rc = ats_dispatch_plan(i32(ATS_MOE_LAYOUT_INDICES), ATS_IDX_I32, T, k, E, C, i32(ATS_MOE_LAYOUT_SLOT),
+                               i32(ATS_MOE_LAYOUT_TOKEN_MAP), i32(ATS_MOE_LAYOUT_HIST), i32(ATS_MOE_LAYOUT_KEPT),
+                               i32(ATS_MOE_LAYOUT_OFFSETS), i32(ATS_MOE_LAYOUT_ROW_SRC), i32(ATS_MOE_LAYOUT_ROW_OF),
+                               i32(ATS_MOE_LAYOUT_STATUS), at(ATS_MOE_LAYOUT_PLAN_WS), plan_ws, stream);
+        if (rc != ATS_OK) return rc;
+    }
     const int32_t* const offsets = i32(ATS_MOE_LAYOUT_OFFSETS);
     const int32_t* const kept = i32(ATS_MOE_LAYOUT_KEPT);
     rc = ats_grouped_gateup_swiglu(x, T, i32(ATS_MOE_LAYOUT_ROW_SRC), k, w_gu, h, offsets, kept, E, rows, H, I, dtype, stream);

@@ -18,6 +18,7 @@
 #include <math.h>
 
 #include "ats_common.hpp"
+#include "dispatch_plan.hpp"
 
 namespace ats {
 
@@ -441,15 +442,16 @@ __global__ __launch_bounds__(256) void route_topk_wave_kernel(const float* __res
     }
 }
 
+// One workgroup of 256 threads; smem_raw: 6 * E floats of LDS.
 template <int VPL>
-__global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
-                                                         float temperature, int variant, int G, int iters,
-                                                         int32_t* __restrict__ idx_out, float* __restrict__ w_out,
-                                                         int32_t* __restrict__ part_hist,
-                                                         float* __restrict__ part_colsum, float lbw,
-                                                         int32_t* __restrict__ hist, float* __restrict__ colsum,
-                                                         float* __restrict__ aux) {
-    extern __shared__ unsigned char smem_raw[];
+__device__ __forceinline__ void route_topk_block(const float* __restrict__ logits, int64_t T, int E, int k,
+                                                 float temperature, int variant, int G, int iters,
+                                                 int32_t* idx_out, float* __restrict__ w_out,
+                                                 int32_t* __restrict__ part_hist,
+                                                 float* __restrict__ part_colsum, float lbw,
+                                                 int32_t* __restrict__ hist, float* __restrict__ colsum,
+                                                 float* __restrict__ aux, unsigned char* smem_raw,
+                                                 int* s_idx = nullptr) {
     int* s_hist = reinterpret_cast<int*>(smem_raw);            // [E]
     float* s_col = reinterpret_cast<float*>(s_hist + E);        // [4][E]  (then [E] terms of the auxiliary loss)
     const bool want_stats = part_hist != nullptr;
@@ -580,6 +582,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
         if (tok_ok && is_sel) {
             idx_out[t * k + gl] = sel_idx;
             w_out[t * k + gl] = wsel;
+            if (s_idx) s_idx[t * k + gl] = sel_idx;
         }
     }
     if (want_stats) {
@@ -614,11 +617,50 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
             __syncthreads();
             if (threadIdx.x == 0 && aux) {
                 float sum = 0.f;
+#pragma unroll 8
                 for (int e = 0; e < E; ++e) sum += s_term[e];
                 aux[0] = fminf(sum * (float)E * lbw, 1.0f);
             }
         }
     }
+}
+
+template <int VPL>
+__global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
+                                                         float temperature, int variant, int G, int iters,
+                                                         int32_t* __restrict__ idx_out, float* __restrict__ w_out,
+                                                         int32_t* __restrict__ part_hist,
+                                                         float* __restrict__ part_colsum, float lbw,
+                                                         int32_t* __restrict__ hist, float* __restrict__ colsum,
+                                                         float* __restrict__ aux) {
+    extern __shared__ unsigned char smem_raw[];
+    route_topk_block<VPL>(logits, T, E, k, temperature, variant, G, iters, idx_out, w_out, part_hist, part_colsum, lbw, hist,
+                          colsum, aux, smem_raw);
+}
+
+// Decoding steps: the routing pass of all tokens and the dispatch plan in one workgroup.  Both are chains of a few
+// dependent memory and LDS round trips that one workgroup walks.  3 tokens, 64 experts: two launches 15.0 us, one launch
+// 13.8, with the choices handed on in LDS and the plan's own round trips through global memory gone 9.2.
+struct PlanOut {
+    int C;
+    int32_t *hist, *kept, *offsets, *slot, *token_map, *row_src, *row_of, *status;
+    int64_t row_src_len;
+};
+template <int VPL>
+__global__ __launch_bounds__(256) void route_plan_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
+                                                         float temperature, int variant, int G, int iters, int32_t* idx_out,
+                                                         float* __restrict__ w_out, int32_t* __restrict__ part_hist,
+                                                         float* __restrict__ part_colsum, float lbw,
+                                                         int32_t* __restrict__ hist, float* __restrict__ colsum,
+                                                         float* __restrict__ aux, PlanOut p) {
+    extern __shared__ unsigned char smem_raw[];
+    int* s_plan = reinterpret_cast<int*>(smem_raw) + 6 * E;      // [6 * E + 1], then the choices
+    int* s_idx = s_plan + 6 * E + 1;
+    route_topk_block<VPL>(logits, T, E, k, temperature, variant, G, iters, idx_out, w_out, part_hist, part_colsum, lbw, hist,
+                          colsum, aux, smem_raw, s_idx);
+    __syncthreads();      // the choices are written
+    plan_single_block<int32_t>(nullptr, s_idx, T * k, k, E, p.C, p.hist, p.kept, p.offsets, p.slot, p.token_map, p.row_src,
+                               p.row_of, p.row_src_len, p.status, s_plan);
 }
 
 // Reduces the per-block partials in a fixed order and evaluates the auxiliary loss.
@@ -805,5 +847,50 @@ extern "C" int ats_route_topk(const float* logits, int64_t T, int E, int k, floa
                            part_col, nblocks, E, T, k, load_balancing_weight, hist, prob_colsum, aux);
         ATS_CHECK_LAUNCH("ats_route_topk(finalize)");
     }
+    return ATS_OK;
+}
+
+extern "C" int ats_route_plan_supported(int64_t T, int E, int k) {
+    using namespace ats;
+    if (T <= 0 || E <= 0 || E > kPlanMaxE || k <= 0 || k > E || k > kRouteMaxK || T * (int64_t)k > kPlanSingle) return 0;
+    int G, iters;
+    return route_grid(T, E, &G, &iters) == 1 ? 1 : 0;
+}
+
+extern "C" int ats_route_plan(const float* logits, int64_t T, int E, int k, float temperature, int variant, int32_t* idx_out,
+                              float* w_out, int32_t* routed, float* prob_colsum, float* aux, float load_balancing_weight,
+                              void* route_workspace, size_t route_workspace_bytes, int C, int32_t* slot, int32_t* token_map,
+                              int32_t* hist, int32_t* kept, int32_t* offsets, int32_t* row_src, int32_t* row_of,
+                              int32_t* status, ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_route_plan";
+    ATS_REQUIRE(ats_route_plan_supported(T, E, k), ATS_ERR_UNSUPPORTED, "%s: T=%lld E=%d k=%d (one workgroup's tokens, at most %d "
+                "assignments)", name, (long long)T, E, k, kPlanSingle);
+    ATS_REQUIRE(variant == ATS_ROUTE_SOFTMAX_TOPK || variant == ATS_ROUTE_TOPK_SOFTMAX, ATS_ERR_INVALID_ARG, "%s: variant %d", name,
+                variant);
+    ATS_REQUIRE(temperature > 0.f, ATS_ERR_INVALID_ARG, "%s: temperature %g", name, temperature);
+    ATS_REQUIRE(C > 0 && (int64_t)E * C < (int64_t)INT_MAX, ATS_ERR_INVALID_ARG, "%s: C=%d", name, C);
+    ATS_REQUIRE(logits && idx_out && w_out && routed && prob_colsum && slot && token_map && hist && kept && offsets && row_src &&
+                    row_of && status, ATS_ERR_INVALID_ARG, "%s: null pointer", name);
+    const size_t need = (size_t)E * (sizeof(int32_t) + sizeof(float));
+    ATS_REQUIRE(route_workspace && route_workspace_bytes >= need, ATS_ERR_WORKSPACE, "%s: workspace of %zu bytes, need %zu", name,
+                route_workspace_bytes, need);
+    int G, iters;
+    route_grid(T, E, &G, &iters);
+    int32_t* part_hist = static_cast<int32_t*>(route_workspace);
+    float* part_col = reinterpret_cast<float*>(part_hist + E);
+    int64_t len = T * k < (int64_t)E * C ? T * k : (int64_t)E * C;
+    const PlanOut p{C, hist, kept, offsets, slot, token_map, row_src, row_of, status, len};
+    hipStream_t s = as_stream(stream);
+    const size_t smem = ((size_t)12 * E + 1 + (size_t)(T * k)) * sizeof(float);
+    const int vpl = (E + G - 1) / G;
+#define ATS_ROUTE_PLAN(V_)                                                                                                    \
+    hipLaunchKernelGGL((route_plan_kernel<V_>), dim3(1), dim3(256), smem, s, logits, T, E, k, temperature, variant, G, iters, \
+                       idx_out, w_out, part_hist, part_col, load_balancing_weight, routed, prob_colsum, aux, p)
+    if (vpl <= 1) ATS_ROUTE_PLAN(1);
+    else if (vpl <= 4) ATS_ROUTE_PLAN(4);
+    else ATS_ROUTE_PLAN(16);
+#undef ATS_ROUTE_PLAN
+    ATS_CHECK_LAUNCH(name);
     return ATS_OK;
 }

@@ -153,6 +153,15 @@ int ats_dispatch_plan_static(const void* idx, int idx_dtype, int64_t T, int k, i
                              int32_t* offsets, int32_t* row_src, int32_t* row_of, int32_t* status,
                              ats_stream_t stream);
 
+/* ats_route_topk and ats_dispatch_plan of a decoding step in one launch of one workgroup, the same results bit for bit
+ * (routed: the histogram of ats_route_topk); for the sizes that ats_route_plan_supported accepts.  A workspace
+ * of 8 * E bytes. */
+int ats_route_plan_supported(int64_t T, int E, int k);
+int ats_route_plan(const float* logits, int64_t T, int E, int k, float temperature, int variant, int32_t* idx_out,
+                   float* w_out, int32_t* routed, float* prob_colsum, float* aux, float load_balancing_weight,
+                   void* route_workspace, size_t route_workspace_bytes, int C, int32_t* slot, int32_t* token_map,
+                   int32_t* hist, int32_t* kept, int32_t* offsets, int32_t* row_src, int32_t* row_of, int32_t* status,
+                   ats_stream_t stream);
 /* out[r,:] = src[map[r] / div, :] or zeros when map[r] < 0; r in [0, n_rows).
  * With map = token_map and div = k this fills expert_inputs[E,C,H]
  * (moe_cuda_wrapper.py:306-322); with div = 1 it is a plain row gather. */
