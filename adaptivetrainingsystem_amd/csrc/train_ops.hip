@@ -26,15 +26,18 @@ __device__ __forceinline__ float exp_split(float x) {
     return fmaf(p * e, 0.693147182464599609375f, p);
 }
 
-// exp(x - ref), x and ref of one row.  Float32 rows through exp_split.  bfloat16 rows have twice the elements per byte, and
-// with eight operations each the forward pass was bound by them (16376 x 32000: 262 us, 185 with these two): one rounding of
-// (x - ref) log2(e), and the product with a ref common to the whole row.
+// exp(x - ref), x and ref of one row, x <= ref.  Float32 rows through exp_split.  bfloat16 rows have twice the elements per
+// byte, and with eight operations each the forward pass was bound by them (16376 x 32000: 262 us, 185 with these two): one
+// rounding of (x - ref) log2(e), and the product with a ref common to the whole row.  Near the end of the type's range (a
+// mask of the lowest value) that product overflows; there x - ref is 0 or so far below it that exp2 without the factor gives
+// the same 1 or 0.
 template <typename T>
 struct RowExp {
-    float ref;
-    __device__ __forceinline__ explicit RowExp(float r) : ref(sizeof(T) == 2 ? r * 1.4426950408889634f : r) {}
+    float scale, ref;
+    __device__ __forceinline__ explicit RowExp(float r)
+        : scale(fabsf(r) > 1e38f ? 1.f : 1.4426950408889634f), ref(sizeof(T) == 2 ? r * scale : r) {}
     __device__ __forceinline__ float operator()(float x) const {
-        if (sizeof(T) == 2) return __builtin_amdgcn_exp2f(fmaf(x, 1.4426950408889634f, -ref));
+        if (sizeof(T) == 2) return __builtin_amdgcn_exp2f(fmaf(x, scale, -ref));
         return exp_split(x - ref);
     }
 };

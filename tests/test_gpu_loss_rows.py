@@ -44,6 +44,34 @@ def test_nan_is_not_lost_among_masked_logits(gpu, V):
     assert out["loss"].item() == 5.0                               # 0 for the first token, the substitute 10 for the second
 
 
+@pytest.mark.parametrize("V", [40, 1000, 4099, 32000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_masks_of_the_lowest_value(gpu, V, dtype):
+    """Logits masked with the type's lowest value, in part of a row and in all of it, and logits of the highest."""
+    from adaptivetrainingsystem_amd.training import FusedLoss
+    low, high = torch.finfo(dtype).min, torch.finfo(dtype).max
+    z = torch.randn(4, V, generator=torch.Generator().manual_seed(8)).to(dtype)
+    z[0, 3:] = low                                                 # whole threads see masked elements only
+    z[1, :-2] = low
+    z[2] = low
+    z[3, ::2] = high
+    labels = torch.tensor([1, V - 1, 5, 4])
+    ref = torch.nn.functional.log_softmax(z.double(), dim=-1)
+    z = z.to(gpu).requires_grad_()
+    for t in range(4):
+        z.grad = None
+        out = FusedLoss()(z[t:t + 1], labels[t:t + 1].to(gpu))
+        out["loss"].backward()
+        if t < 2:
+            want = -ref[t, labels[t]].item()
+            assert abs(out["loss"].item() - want) <= 2e-6 * max(1.0, want)
+        # at the ends of the range the float32 log-sum-exp has no room for log(V): the loss is 0 and every probability 1
+        p = ref[t].exp() if t < 2 else (z[t].detach().double().cpu() == (low if t == 2 else high)).double()
+        p[labels[t]] -= 1.0
+        err = (z.grad[t].double().cpu() - p).abs().max().item() / p.abs().max().item()
+        assert err <= (1e-5 if dtype == torch.float32 else 2 ** -8), (t, err)
+
+
 def test_upload(gpu):
     from adaptivetrainingsystem_amd import _lib
     lib = _lib.load()
