@@ -74,6 +74,7 @@ struct GroupedArgs {
     void* t_out;
     int64_t ld_t;
     const int32_t* t_col0;
+    int tile_rows;          // MIDROWS instance: most rows of a tile (0: the tile's own height)
 };
 
 constexpr int kRowPitch = 144;  // bytes per staged row: 128 data + 16 pad
@@ -1045,7 +1046,8 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 //   383   642 -> 635 -> 622  |  324 -> 314 -> 306  |  286 -> 295 -> 287
 //   1024 1469 -> 1498 -> 1493 |  815 -> 819 -> 819 |  629 -> 641 -> 639
 //   4096 5473 -> 5520 -> 5556 | 2734 -> 2765 -> 2773 | 2380 -> 2413 -> 2442
-// so launches below kMidRowsMaxAvg rows per group take it.  Sums over K are in the same order in both instances.
+// so launches below kMidRowsMaxAvg rows per group take it, and those of one group at any height that dense_tile_rows finds.
+// Sums over K are in the same order in both instances.
 //
 // A 64-element slab is two 32-element k-steps; the wave's rows are up to two halves of up to four 16-row fragments.
 // A slab is four phases of up to 16 MFMAs, (k-step, row half) = (0,0) (0,1) (1,0) (1,1); fragments live in two
@@ -1105,7 +1107,8 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
     TileCoord tc;
-    if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, BM, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0, &tc)) return;
+    const int most_rows = MIDROWS && p.tile_rows ? p.tile_rows : BM;
+    if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, most_rows, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0, &tc)) return;
     const int count = row_count[tc.e];
     const int row0 = p.row_start[tc.e];
     const int K = p.k_count ? p.k_count[tc.e] : p.K;
@@ -1121,7 +1124,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     // ---- rows of this tile: row_base .. + 2 * wave_share, wave row wm taking the wm-th share
     int frags = TM;                     // 16-row fragments per wave
     if constexpr (MIDROWS) {
-        const int m_tiles = (count + BM - 1) / BM;
+        const int m_tiles = (count + most_rows - 1) / most_rows;
         const int f = ((count + m_tiles - 1) / m_tiles + 31) / 32;
         frags = __builtin_amdgcn_readfirstlane(f > 4 ? f : (f > 2 ? 4 : 2));
     }
@@ -1466,6 +1469,29 @@ constexpr size_t dma_lds_bytes(int BM, int BN) { return (size_t)(3 * BM + 2 * BN
 // Rows per group on average below which the 16 x 16 x 32 kernel runs in its MIDROWS form (measured there).
 constexpr int64_t kMidRowsMaxAvg = 768;
 static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1) < kMidRowsMaxAvg; }
+// Tile height of a bfloat16 launch with one group (its row count is exact), 0 for the full 256 rows.  An XCD takes whole
+// supertiles of 32 tiles and its 32 CUs hold one tile each, so a launch lasts as many rounds as there are supertiles per XCD,
+// and lower tiles pay where they turn a round that is mostly empty into work for all CUs.  Microseconds per 64-element slab
+// by height as measured (a round of K = 4096: 256 rows 94, 224: 84, 192: 76, 160: 60, 128: 54).  Rows x [N, K], 256-row tiles ->
+// the rule's: 5331 x [4096, 4096] 188 -> 153 us (192), x [6144, 4096] 248 -> 222 (192), 3000 x [4096, 4096] 95 -> 80 (192),
+// 1500 x [4096, 4096] 78 -> 59 (128), 4200 x [2048, 2048] 53 -> 38 (160), 8000 x [3072, 2048] 98 -> 91 (224), 1000 x
+// [6144, 4096] 93 -> 58 (128); 2048 x [6144, 4096] stays (97; 128 rows 113).  Sums over K are in the same order.
+static int dense_tile_rows(int64_t rows, int n_tiles, int k_slabs, int sm, int sn) {
+    float best = 0.f;
+    int best_rows = 0;
+    for (int h : {256, 224, 192, 160, 128}) {
+        const int64_t m_tiles = (rows + h - 1) / h;
+        const int64_t height = ((rows + m_tiles - 1) / m_tiles + 31) / 32 * 32;     // tiles of a group have one height
+        const float per_slab = height > 224 ? 1.36f : height > 192 ? 1.2f : height > 160 ? 1.08f : height > 128 ? 0.84f : 0.75f;
+        const int64_t rounds = ((m_tiles + sm - 1) / sm * ((n_tiles + sn - 1) / sn) + kNumXcd - 1) / kNumXcd;
+        const float t = (float)rounds * (k_slabs * per_slab + 7.f);
+        if (h == 256 || t < 0.97f * best) {
+            best = t;
+            best_rows = h == 256 ? 0 : h;
+        }
+    }
+    return best_rows;
+}
 
 template <typename T, typename TO, int BM, int BN, int WM, int WN, int SM, int SN, bool SWIGLU, bool DMA = false>
 static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
@@ -1519,14 +1545,18 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     p.sn = SN;
     if (SM == 4 && SN == 8) pick_supertile(p.n_tiles, &p.sm, &p.sn);
     p.aligned_bands = max_rows / (p.E > 0 ? p.E : 1) >= kAlignedBandsMinAvgRows ? 1 : 0;
-    const int64_t blocks = grid_blocks(max_rows * splits, p.E * splits, BM, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0);
+    // the direct-to-LDS kernel addresses its operands with 32-bit lane offsets
+    const bool dma_ok = DMA && p.K % BK == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0;
+    p.tile_rows = 0;
+    if (dma_ok && std::is_same<T, bf16_t>::value && p.E == 1)
+        p.tile_rows = dense_tile_rows(max_rows, p.n_tiles, p.K / BK, p.sm, p.sn);
+    const int64_t blocks = grid_blocks(max_rows * splits, p.E * splits, p.tile_rows ? p.tile_rows : BM, p.n_tiles, p.sm, p.sn,
+                                       p.aligned_bands != 0);
     if (blocks > 0x7fffffffLL) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;
     }
-    // the direct-to-LDS kernel addresses its operands with 32-bit lane offsets
-    const bool dma_ok = DMA && p.K % BK == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0;
-    auto kern = dma_ok ? (mid_rows(max_rows, p.E) ? kern_mid : kern_dma) : (p.K % BK == 0) ? kern_pipe : kern_general;
+    auto kern = dma_ok ? (p.tile_rows || mid_rows(max_rows, p.E) ? kern_mid : kern_dma) : (p.K % BK == 0) ? kern_pipe : kern_general;
     const size_t smem_launch = (!dma_ok && p.K % BK == 0) ? smem_staged : smem;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WM * WN * 64), smem_launch, s, p);
     return ATS_OK;
