@@ -45,20 +45,13 @@ class RoPEFunction(Function):
     def forward(ctx, q, k, cos, sin, position_offset):
         ctx.save_for_backward(cos, sin)
         ctx.position_offset = position_offset
-        # heads behind positions in memory, as projections leave them: the gradients then get that layout too
-        ctx.bhl = [t is not None and not t.is_contiguous() and t.transpose(1, 2).is_contiguous() for t in (q, k)]
         q_out, k_out = ops.rope(q, k, cos, sin, position_offset)
         return q_out, k_out
 
     @staticmethod
     def backward(ctx, dq, dk):
         cos, sin = ctx.saved_tensors
-        if not any(ctx.bhl):
-            gq, gk = ops.rope(dq, dk, cos, sin, ctx.position_offset, inverse=True)
-        else:
-            gq, gk = (None if d is None else torch.empty_like(d.transpose(1, 2), memory_format=torch.contiguous_format).transpose(1, 2)
-                      if bhl else torch.empty_like(d, memory_format=torch.contiguous_format) for d, bhl in zip((dq, dk), ctx.bhl))
-            ops.rope_strided((dq, dk, None), (gq, gk, None), cos, sin, ctx.position_offset, inverse=True)
+        gq, gk = ops.rope(dq, dk, cos, sin, ctx.position_offset, inverse=True)
         return gq, gk, None, None, None
 
 
