@@ -202,14 +202,14 @@ __global__ __launch_bounds__(256) void plan_fused_kernel(const IdxT* __restrict_
     for (int64_t i = total + (int64_t)blockIdx.x * 256 + threadIdx.x; i < row_src_len; i += stride) row_src[i] = -1;
 }
 
-template <typename IdxT>
-__global__ __launch_bounds__(256) void plan_single_kernel(const IdxT* idx, int64_t n, int k, int E, int C, int32_t* hist,
+template <typename IdxT, int NW>
+__global__ __launch_bounds__(NW * 64) void plan_single_kernel(const IdxT* idx, int64_t n, int k, int E, int C, int32_t* hist,
                                                           int32_t* kept, int32_t* offsets, int32_t* slot,
                                                           int32_t* token_map, int32_t* row_src, int32_t* row_of,
                                                           int64_t row_src_len, int32_t* status) {
     extern __shared__ int s_all[];
-    plan_single_block<IdxT>(idx, nullptr, n, k, E, C, hist, kept, offsets, slot, token_map, row_src, row_of, row_src_len,
-                            status, s_all);
+    plan_single_block<IdxT, NW>(idx, nullptr, n, k, E, C, hist, kept, offsets, slot, token_map, row_src, row_of, row_src_len,
+                                status, s_all);
 }
 
 // ------------------------------------------------------------------ row gather
@@ -597,16 +597,22 @@ extern "C" int ats_dispatch_plan(const void* idx, int idx_dtype, int64_t T, int 
         ATS_CHECK_LAUNCH("ats_dispatch_plan(fused)");
         return ATS_OK;
     }
-    const size_t smem_single = ((size_t)6 * E + 1) * sizeof(int);
     if (single) {
-        if (idx_dtype == ATS_IDX_I32)
-            hipLaunchKernelGGL((plan_single_kernel<int32_t>), dim3(1), dim3(256), smem_single, s,
-                               static_cast<const int32_t*>(idx), n, k, E, C, hist, kept, offsets, slot,
-                               token_map, row_src, row_of, row_src_len, status);
-        else
-            hipLaunchKernelGGL((plan_single_kernel<int64_t>), dim3(1), dim3(256), smem_single, s,
-                               static_cast<const int64_t*>(idx), n, k, E, C, hist, kept, offsets, slot,
-                               token_map, row_src, row_of, row_src_len, status);
+        // 16 waves walk one step of 64 assignments each, four walk up to four (64 experts, 1020
+        // assignments 9.7 -> 5.6 us, 576 8.1 -> 4.7)
+        const bool wide = n > 256 && E <= 128;
+        const size_t smem_single = ((size_t)((wide ? 16 : 4) + 2) * E + 1) * sizeof(int);
+#define ATS_PLAN_SINGLE(T_, W_)                                                                                        \
+    hipLaunchKernelGGL((plan_single_kernel<T_, W_>), dim3(1), dim3(W_ * 64), smem_single, s, static_cast<const T_*>(idx), n, k, \
+                       E, C, hist, kept, offsets, slot, token_map, row_src, row_of, row_src_len, status)
+        if (idx_dtype == ATS_IDX_I32) {
+            if (wide) ATS_PLAN_SINGLE(int32_t, 16);
+            else ATS_PLAN_SINGLE(int32_t, 4);
+        } else {
+            if (wide) ATS_PLAN_SINGLE(int64_t, 16);
+            else ATS_PLAN_SINGLE(int64_t, 4);
+        }
+#undef ATS_PLAN_SINGLE
         ATS_CHECK_LAUNCH("ats_dispatch_plan(single)");
         return ATS_OK;
     }

@@ -1,12 +1,12 @@
 // Device parts of the dispatch plan that its kernels share: counts of a chunk, totals over chunks, ranks inside a chunk,
-// and the whole plan of up to kPlanSingle assignments in one workgroup of 256 threads.
+// and the whole plan of up to kPlanSingle assignments in one workgroup.
 #pragma once
 #include "ats_common.hpp"
 
 namespace ats {
 
 constexpr int kPlanChunk = 256;      // assignments per block of the multi-block plan (64 per wave: one step)
-constexpr int kPlanSingle = 1024;    // largest plan done by one block alone (256 per wave: four steps)
+constexpr int kPlanSingle = 1024;    // largest plan done by one block alone (four waves: 256 each, four steps)
 constexpr int kPlanMaxE = 1024;
 
 template <typename IdxT>
@@ -163,17 +163,18 @@ __device__ void chunk_rank_and_write(const IdxT* idx, int64_t n, int k, int E, i
 
 // Whole plan in one block (n <= kPlanSingle).  A chain of dependent steps, so what passes between them stays in registers
 // (the expert ids) and LDS (counts, kept, offsets) instead of going through global memory, and waves and steps without
-// assignments are skipped: 18 assignments to 64 experts take about 2 us behind the routing pass, 6.3 before.  s_all: 6 * E + 1 integers of LDS.
+// assignments are skipped: 18 assignments to 64 experts take about 2 us behind the routing pass, 6.3 before.  NW: waves of
+// the block.  s_all: (NW + 2) * E + 1 integers of LDS.
 // s_idx: the ids again in LDS, or nullptr.
-template <typename IdxT>
+template <typename IdxT, int NW>
 __device__ __forceinline__ void plan_single_block(const IdxT* idx, const int* s_idx, int64_t n, int k, int E, int C,
                                                   int32_t* hist, int32_t* kept, int32_t* offsets, int32_t* slot,
                                                   int32_t* token_map, int32_t* row_src, int32_t* row_of,
                                                   int64_t row_src_len, int32_t* status, int* s_all) {
-    int* s_cnt = s_all;              // [4 * E] counts, then running bases, per wave
-    int* s_kept = s_all + 4 * E;     // [E]
-    int* s_off = s_all + 5 * E;      // [E + 1]
-    constexpr int S = kPlanSingle / 4 / kWave;
+    int* s_cnt = s_all;                    // [NW * E] counts, then running bases, per wave
+    int* s_kept = s_all + NW * E;          // [E]
+    int* s_off = s_all + (NW + 1) * E;     // [E + 1]
+    constexpr int S = kPlanSingle / NW / kWave;
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int ids[S];
@@ -188,16 +189,16 @@ __device__ __forceinline__ void plan_single_block(const IdxT* idx, const int* s_
             ids[st] = load_expert(idx, a, n, E, &bad);
         }
     }
-    for (int i = threadIdx.x; i < 4 * E; i += 256) s_cnt[i] = 0;
+    for (int i = threadIdx.x; i < NW * E; i += NW * 64) s_cnt[i] = 0;
     __syncthreads();
 #pragma unroll
     for (int st = 0; st < S; ++st)
         if (ids[st] >= 0) atomicAdd(&s_cnt[wave * E + ids[st]], 1);
     const int any_bad = __syncthreads_or(bad ? 1 : 0);
     if (threadIdx.x == 0) status[0] = any_bad;
-    for (int e = threadIdx.x; e < E; e += 256) {
+    for (int e = threadIdx.x; e < E; e += NW * 64) {
         int run = 0;                 // per-wave running base = counts of the earlier waves
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < NW; ++w) {
             const int v = s_cnt[w * E + e];
             s_cnt[w * E + e] = run;
             run += v;
@@ -260,11 +261,11 @@ __device__ __forceinline__ void plan_single_block(const IdxT* idx, const int* s_
         }
     }
     const int ec = E * C;            // (below 2^31: checked on the host)
-    for (int i = threadIdx.x; i < ec; i += 256) {
+    for (int i = threadIdx.x; i < ec; i += NW * 64) {
         const int e = (int)((unsigned)i / (unsigned)C);
         if (i - e * C >= s_kept[e]) token_map[i] = -1;
     }
-    for (int64_t i = s_off[E] + threadIdx.x; i < row_src_len; i += 256) row_src[i] = -1;
+    for (int64_t i = s_off[E] + threadIdx.x; i < row_src_len; i += NW * 64) row_src[i] = -1;
 }
 
 }  // namespace ats

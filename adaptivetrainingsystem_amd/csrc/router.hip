@@ -43,6 +43,7 @@ constexpr int kGateKC = 128;  // k elements consumed per wave per step
 // A step's 16 x 128 elements of x and, tile after tile, of the gate reach the MFMA operand layout through a
 // wave-private piece of LDS (see gate_gemm_bf16_flat_kernel: coalesced loads of whole cache lines instead of
 // 16 rows x 64 bytes per instruction); a wave's LDS accesses complete in order, so no barrier is involved.
+// gridDim.y > 1 (NT = 1): an expert tile per workgroup.
 template <int NT, int KW, bool PF>
 __global__ __launch_bounds__(KW * 64) void gate_gemm_bf16_kernel(const bf16_t* __restrict__ x,
                                                                const bf16_t* __restrict__ wg,
@@ -58,6 +59,7 @@ __global__ __launch_bounds__(KW * 64) void gate_gemm_bf16_kernel(const bf16_t* _
     const int lrow = lane >> 4;     // loader view: row 4 j + lrow of a 16-row tile ...
     const int lchunk = lane & 15;   // ... and 16-byte chunk of the step's 256-byte row piece
     const int64_t t0 = (int64_t)blockIdx.x * 16;
+    const int e0 = NT == 1 ? (int)blockIdx.y * 16 : 0;
 
     // this wave's k range (whole steps; the tail is handled by predicates)
     const int steps_total = (H + kGateKC - 1) / kGateKC;
@@ -91,7 +93,7 @@ __global__ __launch_bounds__(KW * 64) void gate_gemm_bf16_kernel(const bf16_t* _
         }                                                                                              \
         _Pragma("unroll") for (int n = 0; n < NT; ++n) {                                               \
             _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                            \
-                const int e = n * 16 + 4 * j + lrow;                                                   \
+                const int e = e0 + n * 16 + 4 * j + lrow;                                              \
                 b[buf_][n][j] = zero4;                                                                 \
                 if (e < E && kk < H) b[buf_][n][j] = *reinterpret_cast<const u32x4_t*>(wg + (int64_t)e * H + kk); \
             }                                                                                          \
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(KW * 64) void gate_gemm_bf16_kernel(const bf16_t* _
         const int n = i >> 8;
         const int row = (i & 255) >> 4;
         const int col = i & 15;
-        const int e = n * 16 + col;
+        const int e = e0 + n * 16 + col;
         const int64_t t = t0 + row;
         if (t < T && e < E) {
             float v = reinterpret_cast<const float*>(stage[0][0])[i];
@@ -352,6 +354,8 @@ __device__ __forceinline__ bool key_before(float va, int ia, float vb, int ib) {
 }
 
 constexpr int kRouteMaxK = 16;
+constexpr int kRouteWideMaxE = 128;     // most experts of the 16-wave workgroups (LDS)
+constexpr int kRouteOnePasses = 16;     // one workgroup takes all tokens up to that many passes of four waves
 
 // Selection key of key_before as an unsigned number: larger key = earlier in the order.  NaN is the largest
 // key, -0 counts as +0, and 0 is below every value (used for lanes that hold no candidate).
@@ -442,8 +446,10 @@ __global__ __launch_bounds__(256) void route_topk_wave_kernel(const float* __res
     }
 }
 
-// One workgroup of 256 threads; smem_raw: 6 * E floats of LDS.
-template <int VPL>
+// One workgroup of NW waves; smem_raw: (NW + 2) * E floats of LDS.  Where a token fills a wave (32 < E <= 64) the arg-max
+// rounds are those of route_topk_wave_kernel: a maximum over DPP steps and three scalar reads instead of six exchanges of a
+// value, an id and a probability.
+template <int VPL, int NW>
 __device__ __forceinline__ void route_topk_block(const float* __restrict__ logits, int64_t T, int E, int k,
                                                  float temperature, int variant, int G, int iters,
                                                  int32_t* idx_out, float* __restrict__ w_out,
@@ -453,17 +459,17 @@ __device__ __forceinline__ void route_topk_block(const float* __restrict__ logit
                                                  float* __restrict__ aux, unsigned char* smem_raw,
                                                  int* s_idx = nullptr) {
     int* s_hist = reinterpret_cast<int*>(smem_raw);            // [E]
-    float* s_col = reinterpret_cast<float*>(s_hist + E);        // [4][E]  (then [E] terms of the auxiliary loss)
+    float* s_col = reinterpret_cast<float*>(s_hist + E);        // [NW][E]  (then [E] terms of the auxiliary loss)
     const bool want_stats = part_hist != nullptr;
     const int lane = lane_id();
     const int wave = threadIdx.x >> 6;
     const int gl = lane & (G - 1);          // lane inside the group
     const int grp = lane / G;               // group inside the wave
     const int groups_per_wave = kWave / G;
-    const int groups_per_block = 4 * groups_per_wave;
+    const int groups_per_block = NW * groups_per_wave;
 
     if (want_stats) {
-        for (int i = threadIdx.x; i < E; i += 256) s_hist[i] = 0;
+        for (int i = threadIdx.x; i < E; i += NW * 64) s_hist[i] = 0;
         __syncthreads();
     }
     float col[VPL];
@@ -526,6 +532,7 @@ __device__ __forceinline__ void route_topk_block(const float* __restrict__ logit
         }
         // k rounds of group-wide arg-max
         unsigned taken = 0;   // bit i: v[i] already selected
+        unsigned key = gl < E ? route_order_key(sv[0]) : 0u;      // of a token that fills its wave
         float sel_term = 0.f; // lane j < k of the group keeps choice j: its unnormalised weight ...
         int sel_idx = 0;      // ... and expert id
         float tot = 0.f, first_val = 0.f;
@@ -533,15 +540,22 @@ __device__ __forceinline__ void route_topk_block(const float* __restrict__ logit
             float bv = neg_inf;
             int bi = INT_MAX;
             float bp = 0.f;
+            if (VPL == 1 && G == kWave) {
+                const unsigned best = wave_max_u32(key);
+                bi = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(key == best)) - 1);
+                bv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sv[0]), bi));
+                bp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p[0]), bi));
+                if (lane == bi) key = 0u;
+            } else {
 #pragma unroll
-            for (int i = 0; i < VPL; ++i) {
-                const int e = gl + i * G;
-                if (e < E && !((taken >> i) & 1u) && key_before(sv[i], e, bv, bi)) {
-                    bv = sv[i];
-                    bi = e;
-                    bp = p[i];
+                for (int i = 0; i < VPL; ++i) {
+                    const int e = gl + i * G;
+                    if (e < E && !((taken >> i) & 1u) && key_before(sv[i], e, bv, bi)) {
+                        bv = sv[i];
+                        bi = e;
+                        bp = p[i];
+                    }
                 }
-            }
 #define ROUTE_MERGE_STEP(S_)                                                       \
     if (G > (1 << (S_))) {                                                         \
         const float ov = butterfly_partner_f32<S_>(bv);                            \
@@ -553,17 +567,18 @@ __device__ __forceinline__ void route_topk_block(const float* __restrict__ logit
             bp = op;                                                               \
         }                                                                          \
     }
-            ROUTE_MERGE_STEP(0)
-            ROUTE_MERGE_STEP(1)
-            ROUTE_MERGE_STEP(2)
-            ROUTE_MERGE_STEP(3)
-            ROUTE_MERGE_STEP(4)
-            ROUTE_MERGE_STEP(5)
+                ROUTE_MERGE_STEP(0)
+                ROUTE_MERGE_STEP(1)
+                ROUTE_MERGE_STEP(2)
+                ROUTE_MERGE_STEP(3)
+                ROUTE_MERGE_STEP(4)
+                ROUTE_MERGE_STEP(5)
 #undef ROUTE_MERGE_STEP
-            // owner marks its value as used
+                // owner marks its value as used
 #pragma unroll
-            for (int i = 0; i < VPL; ++i)
-                if (gl + i * G == bi) taken |= 1u << i;
+                for (int i = 0; i < VPL; ++i)
+                    if (gl + i * G == bi) taken |= 1u << i;
+            }
             // the round's choice is the same in every lane of the group, so the normaliser of the weights is
             // summed here, in rank order, instead of being gathered afterwards
             if (j == 0) first_val = bv;
@@ -595,19 +610,24 @@ __device__ __forceinline__ void route_topk_block(const float* __restrict__ logit
             if (grp == 0 && e < E) s_col[wave * E + e] = c;
         }
         __syncthreads();
+        auto col_sum = [&](int e) {
+            float c = s_col[e];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) c += s_col[w * E + e];
+            return c;
+        };
         if (gridDim.x > 1) {
-            for (int e = threadIdx.x; e < E; e += 256) {
+            for (int e = threadIdx.x; e < E; e += NW * 64) {
                 part_hist[(int64_t)blockIdx.x * E + e] = s_hist[e];
-                part_colsum[(int64_t)blockIdx.x * E + e] =
-                    ((s_col[e] + s_col[E + e]) + s_col[2 * E + e]) + s_col[3 * E + e];
+                part_colsum[(int64_t)blockIdx.x * E + e] = col_sum(e);
             }
         } else {
             // one block holds every token (a decoding step): its partials are the totals, so the statistics
             // and the auxiliary loss are finished here, with route_finalize_kernel's arithmetic
-            float* s_term = s_col + 4 * E;
-            for (int e = threadIdx.x; e < E; e += 256) {
+            float* s_term = s_col + NW * E;
+            for (int e = threadIdx.x; e < E; e += NW * 64) {
                 const int hsum = s_hist[e];
-                const float csum = ((s_col[e] + s_col[E + e]) + s_col[2 * E + e]) + s_col[3 * E + e];
+                const float csum = col_sum(e);
                 hist[e] = hsum;
                 colsum[e] = csum;
                 const float usage = (float)hsum / (float)((double)T * k + 1e-9);
@@ -625,8 +645,8 @@ __device__ __forceinline__ void route_topk_block(const float* __restrict__ logit
     }
 }
 
-template <int VPL>
-__global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
+template <int VPL, int NW>
+__global__ __launch_bounds__(NW * 64) void route_topk_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
                                                          float temperature, int variant, int G, int iters,
                                                          int32_t* __restrict__ idx_out, float* __restrict__ w_out,
                                                          int32_t* __restrict__ part_hist,
@@ -634,32 +654,34 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
                                                          int32_t* __restrict__ hist, float* __restrict__ colsum,
                                                          float* __restrict__ aux) {
     extern __shared__ unsigned char smem_raw[];
-    route_topk_block<VPL>(logits, T, E, k, temperature, variant, G, iters, idx_out, w_out, part_hist, part_colsum, lbw, hist,
-                          colsum, aux, smem_raw);
+    route_topk_block<VPL, NW>(logits, T, E, k, temperature, variant, G, iters, idx_out, w_out, part_hist, part_colsum, lbw, hist,
+                              colsum, aux, smem_raw);
 }
 
 // Decoding steps: the routing pass of all tokens and the dispatch plan in one workgroup.  Both are chains of a few
 // dependent memory and LDS round trips that one workgroup walks.  3 tokens, 64 experts: two launches 15.0 us, one launch
-// 13.8, with the choices handed on in LDS and the plan's own round trips through global memory gone 9.2.
+// 13.8, with the choices handed on in LDS and the plan's own round trips through global memory gone 9.2, with the scalar
+// arg-max 6.2.  With 16 waves from the second pass of four on: 16 tokens 23.1 -> 8.1, 64 tokens 81.1 -> 16.9; 8 experts,
+// 500 tokens 31.4 -> 14.2.
 struct PlanOut {
     int C;
     int32_t *hist, *kept, *offsets, *slot, *token_map, *row_src, *row_of, *status;
     int64_t row_src_len;
 };
-template <int VPL>
-__global__ __launch_bounds__(256) void route_plan_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
+template <int VPL, int NW>
+__global__ __launch_bounds__(NW * 64) void route_plan_kernel(const float* __restrict__ logits, int64_t T, int E, int k,
                                                          float temperature, int variant, int G, int iters, int32_t* idx_out,
                                                          float* __restrict__ w_out, int32_t* __restrict__ part_hist,
                                                          float* __restrict__ part_colsum, float lbw,
                                                          int32_t* __restrict__ hist, float* __restrict__ colsum,
                                                          float* __restrict__ aux, PlanOut p) {
     extern __shared__ unsigned char smem_raw[];
-    int* s_plan = reinterpret_cast<int*>(smem_raw) + 6 * E;      // [6 * E + 1], then the choices
-    int* s_idx = s_plan + 6 * E + 1;
-    route_topk_block<VPL>(logits, T, E, k, temperature, variant, G, iters, idx_out, w_out, part_hist, part_colsum, lbw, hist,
-                          colsum, aux, smem_raw, s_idx);
+    int* s_plan = reinterpret_cast<int*>(smem_raw) + (NW + 2) * E;      // [(NW + 2) * E + 1], then the choices
+    int* s_idx = s_plan + (NW + 2) * E + 1;
+    route_topk_block<VPL, NW>(logits, T, E, k, temperature, variant, G, iters, idx_out, w_out, part_hist, part_colsum, lbw, hist,
+                              colsum, aux, smem_raw, s_idx);
     __syncthreads();      // the choices are written
-    plan_single_block<int32_t>(nullptr, s_idx, T * k, k, E, p.C, p.hist, p.kept, p.offsets, p.slot, p.token_map, p.row_src,
+    plan_single_block<int32_t, NW>(nullptr, s_idx, T * k, k, E, p.C, p.hist, p.kept, p.offsets, p.slot, p.token_map, p.row_src,
                                p.row_of, p.row_src_len, p.status, s_plan);
 }
 
@@ -722,23 +744,32 @@ __global__ __launch_bounds__(1024) void route_finalize_kernel(const int32_t* __r
     }
 }
 
-static int route_grid(int64_t T, int E, int* G_out, int* iters_out) {
-    int G = 1;
-    while (G < E && G < kWave) G <<= 1;
-    const int groups_per_block = 4 * (kWave / G);
-    int64_t iters = (T + (int64_t)512 * groups_per_block - 1) / ((int64_t)512 * groups_per_block);
-    if (iters < 1) iters = 1;
-    if (iters > 64) iters = 64;
-    const int64_t per_block = (int64_t)groups_per_block * iters;
-    *G_out = G;
-    // few tokens: one block takes them all in up to 16 passes and finishes the statistics itself
-    const int64_t passes = (T + groups_per_block - 1) / groups_per_block;
-    if (passes <= 16) {
-        *iters_out = (int)(passes < 1 ? 1 : passes);
-        return 1;
+// Workgroups of a routing pass; waves of a workgroup, lanes per token and passes per workgroup beside it.
+struct RouteGrid {
+    int blocks, waves, G, iters;
+};
+static RouteGrid route_grid(int64_t T, int E) {
+    RouteGrid g;
+    g.G = 1;
+    while (g.G < E && g.G < kWave) g.G <<= 1;
+    const int groups_per_wave = kWave / g.G;
+    auto passes = [&](int waves) { return (T + (int64_t)waves * groups_per_wave - 1) / ((int64_t)waves * groups_per_wave); };
+    // few tokens: one workgroup takes them all and finishes the statistics itself, with 16 waves where four would need
+    // several passes, each a chain of a few thousand cycles (64 tokens, 64 experts, top 6: 77 -> 14.5 us with the scalar
+    // arg-max, 16 tokens 20.8 -> 5.3; 512 tokens, 8 experts, top 2: 25.6 -> 10.4, 128 tokens 8.1 -> 4.5)
+    g.waves = 4;
+    if (passes(4) <= kRouteOnePasses) {
+        if (E <= kRouteWideMaxE && passes(4) > 1) g.waves = 16;
+        g.blocks = 1;
+        g.iters = (int)(passes(g.waves) < 1 ? 1 : passes(g.waves));
+        return g;
     }
-    *iters_out = (int)iters;
-    return (int)((T + per_block - 1) / per_block);
+    const int groups_per_block = 4 * groups_per_wave;
+    int64_t iters = (T + (int64_t)512 * groups_per_block - 1) / ((int64_t)512 * groups_per_block);
+    g.iters = (int)(iters < 1 ? 1 : iters > 64 ? 64 : iters);
+    const int64_t per_block = (int64_t)groups_per_block * g.iters;
+    g.blocks = (int)((T + per_block - 1) / per_block);
+    return g;
 }
 
 }  // namespace ats
@@ -767,6 +798,11 @@ extern "C" int ats_router_logits(const void* x, const void* wg, const float* bia
             hipLaunchKernelGGL(gate_gemm_bf16_flat_kernel, dim3(blocks), dim3(512), 0, s, xp, wp, bias, logits, T, H, E);
         else if (nt <= 1)
             hipLaunchKernelGGL((gate_gemm_bf16_kernel<1, 8, false>), dim3(blocks), dim3(512), 0, s, xp, wp, bias, logits, T, H, E);
+        // few tokens against more expert tiles: a workgroup per tile shortens the chain of loads that one workgroup walks
+        // through all gate rows (the same order of accumulation, the same bits).  64 experts, H 2048, microseconds one
+        // workgroup | one per tile: 3 tokens 6.9 | 4.8, 64 7.2 | 5.2, 1024 8.8 | 5.6, 4096 10.4 | 15.2 (x is read per tile)
+        else if (nt > 2 && T <= 1024)
+            hipLaunchKernelGGL((gate_gemm_bf16_kernel<1, 4, true>), dim3(blocks, nt), dim3(256), 0, s, xp, wp, bias, logits, T, H, E);
         else if (nt <= 2)
             hipLaunchKernelGGL((gate_gemm_bf16_kernel<2, 4, true>), dim3(blocks), dim3(256), 0, s, xp, wp, bias, logits, T, H, E);
         else if (nt <= 4)
@@ -790,9 +826,7 @@ extern "C" int ats_router_logits(const void* x, const void* wg, const float* bia
 extern "C" size_t ats_route_topk_workspace(int64_t T, int E) {
     using namespace ats;
     if (T <= 0 || E <= 0) return 0;
-    int G, iters;
-    const int nblocks = route_grid(T, E, &G, &iters);
-    return (size_t)nblocks * E * (sizeof(int32_t) + sizeof(float));
+    return (size_t)route_grid(T, E).blocks * E * (sizeof(int32_t) + sizeof(float));
 }
 
 extern "C" int ats_route_topk(const float* logits, int64_t T, int E, int k, float temperature, int variant,
@@ -812,8 +846,8 @@ extern "C" int ats_route_topk(const float* logits, int64_t T, int E, int k, floa
     ATS_REQUIRE(stats || aux == nullptr, ATS_ERR_INVALID_ARG, "ats_route_topk: aux needs hist and prob_colsum");
     if (T == 0) return ATS_OK;
     ATS_REQUIRE(logits && idx_out && w_out, ATS_ERR_INVALID_ARG, "ats_route_topk: null pointer");
-    int G, iters;
-    const int nblocks = route_grid(T, E, &G, &iters);
+    const RouteGrid g = route_grid(T, E);
+    const int nblocks = g.blocks;
     int32_t* part_hist = nullptr;
     float* part_col = nullptr;
     if (stats) {
@@ -824,23 +858,20 @@ extern "C" int ats_route_topk(const float* logits, int64_t T, int E, int k, floa
         part_col = reinterpret_cast<float*>(part_hist + (size_t)nblocks * E);
     }
     hipStream_t s = as_stream(stream);
-    const size_t smem = (size_t)E * 6 * sizeof(float);
-    const int vpl = (E + G - 1) / G;
-    if (G == kWave && vpl <= 1 && nblocks > 1)
+    const size_t smem = (size_t)E * (g.waves + 2) * sizeof(float);
+    const int vpl = (E + g.G - 1) / g.G;
+#define ATS_ROUTE_TOPK(V_, W_)                                                                                              \
+    hipLaunchKernelGGL((route_topk_kernel<V_, W_>), dim3(nblocks), dim3(W_ * 64), smem, s, logits, T, E, k, temperature,    \
+                       variant, g.G, g.iters, idx_out, w_out, part_hist, part_col, load_balancing_weight, hist, prob_colsum, aux)
+    if (g.G == kWave && vpl <= 1 && nblocks > 1)
         hipLaunchKernelGGL(route_topk_wave_kernel, dim3(nblocks), dim3(256), smem, s, logits, T, E, k, temperature,
-                           variant, iters, idx_out, w_out, part_hist, part_col);
-    else if (vpl <= 1)
-        hipLaunchKernelGGL((route_topk_kernel<1>), dim3(nblocks), dim3(256), smem, s, logits, T, E, k, temperature,
-                           variant, G, iters, idx_out, w_out, part_hist, part_col, load_balancing_weight, hist,
-                           prob_colsum, aux);
-    else if (vpl <= 4)
-        hipLaunchKernelGGL((route_topk_kernel<4>), dim3(nblocks), dim3(256), smem, s, logits, T, E, k, temperature,
-                           variant, G, iters, idx_out, w_out, part_hist, part_col, load_balancing_weight, hist,
-                           prob_colsum, aux);
-    else
-        hipLaunchKernelGGL((route_topk_kernel<16>), dim3(nblocks), dim3(256), smem, s, logits, T, E, k, temperature,
-                           variant, G, iters, idx_out, w_out, part_hist, part_col, load_balancing_weight, hist,
-                           prob_colsum, aux);
+                           variant, g.iters, idx_out, w_out, part_hist, part_col);
+    else if (vpl <= 1 && g.waves > 4) ATS_ROUTE_TOPK(1, 16);
+    else if (vpl <= 1) ATS_ROUTE_TOPK(1, 4);
+    else if (vpl <= 4 && g.waves > 4) ATS_ROUTE_TOPK(4, 16);
+    else if (vpl <= 4) ATS_ROUTE_TOPK(4, 4);
+    else ATS_ROUTE_TOPK(16, 4);
+#undef ATS_ROUTE_TOPK
     ATS_CHECK_LAUNCH("ats_route_topk");
     if (stats && nblocks > 1) {
         hipLaunchKernelGGL(route_finalize_kernel, dim3(1), dim3(1024), (size_t)(E + 2048) * sizeof(float), s, part_hist,
@@ -853,8 +884,7 @@ extern "C" int ats_route_topk(const float* logits, int64_t T, int E, int k, floa
 extern "C" int ats_route_plan_supported(int64_t T, int E, int k) {
     using namespace ats;
     if (T <= 0 || E <= 0 || E > kPlanMaxE || k <= 0 || k > E || k > kRouteMaxK || T * (int64_t)k > kPlanSingle) return 0;
-    int G, iters;
-    return route_grid(T, E, &G, &iters) == 1 ? 1 : 0;
+    return route_grid(T, E).blocks == 1 ? 1 : 0;
 }
 
 extern "C" int ats_route_plan(const float* logits, int64_t T, int E, int k, float temperature, int variant, int32_t* idx_out,
@@ -875,21 +905,22 @@ extern "C" int ats_route_plan(const float* logits, int64_t T, int E, int k, floa
     const size_t need = (size_t)E * (sizeof(int32_t) + sizeof(float));
     ATS_REQUIRE(route_workspace && route_workspace_bytes >= need, ATS_ERR_WORKSPACE, "%s: workspace of %zu bytes, need %zu", name,
                 route_workspace_bytes, need);
-    int G, iters;
-    route_grid(T, E, &G, &iters);
+    const RouteGrid g = route_grid(T, E);
     int32_t* part_hist = static_cast<int32_t*>(route_workspace);
     float* part_col = reinterpret_cast<float*>(part_hist + E);
     int64_t len = T * k < (int64_t)E * C ? T * k : (int64_t)E * C;
     const PlanOut p{C, hist, kept, offsets, slot, token_map, row_src, row_of, status, len};
     hipStream_t s = as_stream(stream);
-    const size_t smem = ((size_t)12 * E + 1 + (size_t)(T * k)) * sizeof(float);
-    const int vpl = (E + G - 1) / G;
-#define ATS_ROUTE_PLAN(V_)                                                                                                    \
-    hipLaunchKernelGGL((route_plan_kernel<V_>), dim3(1), dim3(256), smem, s, logits, T, E, k, temperature, variant, G, iters, \
-                       idx_out, w_out, part_hist, part_col, load_balancing_weight, routed, prob_colsum, aux, p)
-    if (vpl <= 1) ATS_ROUTE_PLAN(1);
-    else if (vpl <= 4) ATS_ROUTE_PLAN(4);
-    else ATS_ROUTE_PLAN(16);
+    const size_t smem = ((size_t)(2 * (g.waves + 2)) * E + 1 + (size_t)(T * k)) * sizeof(float);
+    const int vpl = (E + g.G - 1) / g.G;
+#define ATS_ROUTE_PLAN(V_, W_)                                                                                                \
+    hipLaunchKernelGGL((route_plan_kernel<V_, W_>), dim3(1), dim3(W_ * 64), smem, s, logits, T, E, k, temperature, variant,   \
+                       g.G, g.iters, idx_out, w_out, part_hist, part_col, load_balancing_weight, routed, prob_colsum, aux, p)
+    if (vpl <= 1 && g.waves > 4) ATS_ROUTE_PLAN(1, 16);
+    else if (vpl <= 1) ATS_ROUTE_PLAN(1, 4);
+    else if (vpl <= 4 && g.waves > 4) ATS_ROUTE_PLAN(4, 16);
+    else if (vpl <= 4) ATS_ROUTE_PLAN(4, 4);
+    else ATS_ROUTE_PLAN(16, 4);
 #undef ATS_ROUTE_PLAN
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;
