@@ -1091,11 +1091,12 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // c ^ f(r), f(r) = (r % 4) | ((r / 8) % 4) << 2: the 16 row pieces that one read instruction touches fall on 16
 // different slots, i.e. on all banks once.
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
-          bool MIDROWS = false>
+          bool MIDROWS = false, bool SLICED = false>
 __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, unsigned char* smem,
                                                          const int32_t* __restrict__ row_count) {
 #if defined(__HIP_DEVICE_COMPILE__)
     static_assert(!BKM || (!SWIGLU && !SAVEGU), "the K-major weight layout serves the plain product and the dgrad epilogue");
+    static_assert(!SLICED || (MIDROWS && !SWIGLU && !BKM), "slices of K need a linear epilogue");
     typedef bf16_t T;
     constexpr int BM = 256, BN = 256, WM = 2, WN = 4;
     constexpr int NW = WM * WN;
@@ -1114,12 +1115,19 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 
     TileCoord tc;
     const int most_rows = MIDROWS && p.tile_rows ? p.tile_rows : BM;
-    if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, most_rows, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0, &tc)) return;
+    int split = 0;                      // slice of K of this tile
+    if constexpr (SLICED) {
+        if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, most_rows, p.n_tiles, p.sm, p.sn, false, &tc, p.k_splits, &split)) return;
+        split = __builtin_amdgcn_readfirstlane(split);
+    } else {
+        if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, most_rows, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0, &tc)) return;
+    }
     const int count = row_count[tc.e];
     const int row0 = p.row_start[tc.e];
-    const int K = p.k_count ? p.k_count[tc.e] : p.K;
-    const T* Bexp = static_cast<const T*>(p.b[tc.e]);
-    const T* A = static_cast<const T*>(p.a_ptrs ? p.a_ptrs[tc.e] : p.a);
+    const int K = SLICED ? p.k_slice : p.k_count ? p.k_count[tc.e] : p.K;
+    const int64_t k_first = SLICED ? (int64_t)split * p.k_slice : 0;
+    const T* Bexp = static_cast<const T*>(p.b[tc.e]) + k_first;
+    const T* A = static_cast<const T*>(p.a_ptrs ? p.a_ptrs[tc.e] : p.a) + k_first;
     const int arow0 = p.a_ptrs ? 0 : row0;
 
     const int tid = threadIdx.x;
@@ -1442,7 +1450,8 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
                                                            static_cast<TO*>(p.gu_out), p.ld_gu, p.up_offset, tout,
                                                            p.ld_t, tcol, smem + NW * WSTAGE + wave * TSTAGE);
         } else {
-            epilogue_view<TO, View, SWIGLU, SAVEGU, DSILU>(View{acc}, smem + wave * WSTAGE, static_cast<TO*>(p.out), p.ldo,
+            TO* const out = static_cast<TO*>(p.out) + (SLICED ? (int64_t)split * p.part_stride : 0);
+            epilogue_view<TO, View, SWIGLU, SAVEGU, DSILU>(View{acc}, smem + wave * WSTAGE, out, p.ldo,
                                                            (int64_t)row0 + wave_row, wave_rows, ncol0, p.N_out, lane,
                                                            static_cast<TO*>(p.gu_out), p.ld_gu, p.up_offset);
         }
@@ -1451,7 +1460,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 }
 
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
-          bool MIDROWS = false>
+          bool MIDROWS = false, bool SLICED = false>
 __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) {
     // The body is a function of its own for one reason: a __restrict__ parameter that it reads through gives every
     // other memory access in it (the transposing LDS reads among them) "does not alias that parameter" metadata once
@@ -1460,7 +1469,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
     // the K-major variant is preceded by s_waitcnt vmcnt(0), i.e. waits for all of the slab loads just issued (the
     // plain 16-byte fragment reads carry type-based alias metadata and never had that wait): 27-37 % slower.
     extern __shared__ __align__(16) unsigned char smem_k[];
-    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS>(p, smem_k, p.row_count);
+    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS, SLICED>(p, smem_k, p.row_count);
 }
 
 #undef PL_STORE
@@ -1568,6 +1577,33 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     return ATS_OK;
 }
 
+// K in slices over workgroups on the direct-to-LDS tile, groups of 21 .. 256 rows: float32 partial results.  A down projection
+// of few experts has half a round of these tiles or less (8 x [4096, 14336]: 128), and a CU takes 1.2-1.4 us per slab of
+// K whatever the other half of the chip does; two slices make it a full round: 200 rows per expert 314 -> 165 us.  The 32
+// and 64-row sliced tiles it replaces for several groups read every weight once per 64 rows (200 rows: 517 us).
+static int launch_mid_sliced(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
+    GroupedArgs p = p0;
+    p.n_tiles = (p.N_out + 255) / 256;
+    constexpr size_t smem = dma_lds_bytes(256, 256);
+    auto kern = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, false, true, true>;
+    static LdsReservation reserved;
+    hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern)}, (int)smem);
+    if (e != hipSuccess) {
+        set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
+        return ATS_ERR_LAUNCH;
+    }
+    pick_supertile(p.n_tiles, &p.sm, &p.sn);
+    p.aligned_bands = 0;
+    p.tile_rows = 0;
+    const int64_t blocks = grid_blocks(max_rows * p.k_splits, p.E * p.k_splits, 256, p.n_tiles, p.sm, p.sn, false);
+    if (blocks > 0x7fffffffLL) {
+        set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
+        return ATS_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(512), smem, s, p);
+    return ATS_OK;
+}
+
 // Time of a launch on one tile configuration, in microseconds, from the number of tiles that the busiest CU gets:
 // every tile costs per_slab for each 128-byte slab of K (with the CU's other resident tiles running beside it) and
 // per_tile for its set-up and epilogue.  min_tiles: below that many tiles per CU nothing hides the latency of a slab,
@@ -1610,6 +1646,12 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     if constexpr (!SWIGLU) {
         // K in slices over workgroups: 32-row tiles, 64-row tiles where up to 64 rows can stream the weights once
         if (p.k_splits > 1) {
+            if constexpr (kBf16) {
+                // (with fewer tiles than half of the CUs the small tiles below spread the work further)
+                if (E > 1 && avg > 20 && p.k_slice % 64 == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0 && !p.k_count &&
+                    (int64_t)E * ((p.N_out + 255) / 256) * p.k_splits >= 128)
+                    return launch_mid_sliced(p, max_rows, s);
+            }
             return avg > 32 ? launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s)
                             : launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
         }
