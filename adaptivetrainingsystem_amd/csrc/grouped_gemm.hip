@@ -1035,8 +1035,9 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // LDS was busy 60 % of this kernel's cycles with that conflict; without it the prefill step is 0.45 % faster.
 //
 // MIDROWS: the instance for groups of a few hundred rows.  A group is cut into as few tiles as possible, all of one
-// height (a multiple of 32 rows), and a tile's rows are dealt evenly to the two wave rows, so that every SIMD has the
-// same, smallest number of MFMAs; with 256-row tiles and the rest, a group of 192 rows kept one wave of a SIMD at 128
+// height (a multiple of 16 rows), and a tile's rows are dealt to the two wave rows, which differ by one fragment where their
+// number is odd: a SIMD has a wave of each, so every SIMD has the same, smallest number of MFMAs (heights in steps of 32
+// instead of 16: 8 experts with 358-407 rows each, gate/up 603 against 584 us, down 292 against 288); with 256-row tiles and the rest, a group of 192 rows kept one wave of a SIMD at 128
 // rows beside one at 64.  There the weights also come from HBM instead of from the L2 of an XCD that four or more
 // row tiles share, so the three-stage ring is the weights' and the activations have the two stages (the roles in
 // the phases below trade places).  Rows per group, gate/up [28672, 4096] x 8 | down [4096, 14336] x 8 | gate/up
@@ -1135,15 +1136,17 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;
 
-    // ---- rows of this tile: row_base .. + 2 * wave_share, wave row wm taking the wm-th share
-    int frags = TM;                     // 16-row fragments per wave
+    // ---- rows of this tile: the upper wave row takes the first share of them, the lower one the rest
+    int frags = TM;                     // 16-row fragments of this wave
+    int share0 = 128, share1 = 128;     // rows of the two wave rows
     if constexpr (MIDROWS) {
         const int m_tiles = (count + most_rows - 1) / most_rows;
-        const int f = ((count + m_tiles - 1) / m_tiles + 31) / 32;
-        frags = __builtin_amdgcn_readfirstlane(f > 4 ? f : (f > 2 ? 4 : 2));
+        const int f = __builtin_amdgcn_readfirstlane(((count + m_tiles - 1) / m_tiles + 15) / 16);
+        share0 = (f + 1) / 2 * 16;
+        share1 = f > 1 ? f / 2 * 16 : 16;
+        frags = (wm == 0 ? share0 : share1) / 16;
     }
-    const int wave_share = frags * 16;
-    const int tile_row = tc.mt * 2 * wave_share;
+    const int tile_row = tc.mt * (share0 + share1);
 
     // ---- load descriptors and lane offsets: instruction j of this wave covers rows (j*NW + wave)*8 .. +8
     constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
@@ -1162,7 +1165,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     for (int j = 0; j < NIA; ++j) {
         // stage rows 0 .. 127 belong to wave row 0, the others to wave row 1; rows that nobody has repeat the last one
         const int r = (j * NW + wave) * 8 + drow;
-        int m = (r & 127) < wave_share ? tile_row + (r >> 7) * wave_share + (r & 127) : count - 1;
+        int m = (r & 127) < (r < 128 ? share0 : share1) ? tile_row + (r >> 7) * share0 + (r & 127) : count - 1;
         m = m < count ? m : count - 1;
         a_idx[j] = gather ? p.a_rows[arow0 + m] : m - tile_row;
     }
@@ -1400,16 +1403,17 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NIA) : "memory");
     int s_cur = 0, s_nxt = A_STAGE;
     // rows of the expert in this wave's share of the tile (wave-uniform)
-    const int wave_row = tile_row + wm * wave_share;
+    const int wave_row = tile_row + wm * share0;
     int wave_rows = count - wave_row;
     if constexpr (MIDROWS) {
-        wave_rows = wave_rows < wave_share ? wave_rows : wave_share;
+        wave_rows = wave_rows < frags * 16 ? wave_rows : frags * 16;
         switch (frags) {
             case 8: D16_LOOP(4, 4) break;
             case 7: D16_LOOP(4, 3) break;
             case 6: D16_LOOP(3, 3) break;
             case 5: D16_LOOP(3, 2) break;
             case 4: D16_LOOP(2, 2) break;
+            case 3: D16_LOOP(2, 1) break;
             default: D16_LOOP(1, 1) break;
         }
     } else if (wave_rows > 64) {
@@ -1487,17 +1491,20 @@ static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1
 // Tile height of a bfloat16 launch with one group (its row count is exact), 0 for the full 256 rows.  An XCD takes whole
 // supertiles of 32 tiles and its 32 CUs hold one tile each, so a launch lasts as many rounds as there are supertiles per XCD,
 // and lower tiles pay where they turn a round that is mostly empty into work for all CUs.  Microseconds per 64-element slab
-// by height as measured (a round of K = 4096: 256 rows 94, 224: 84, 192: 76, 160: 60, 128: 54).  Rows x [N, K], 256-row tiles ->
-// the rule's: 5331 x [4096, 4096] 188 -> 153 us (192), x [6144, 4096] 248 -> 222 (192), 3000 x [4096, 4096] 95 -> 80 (192),
-// 1500 x [4096, 4096] 78 -> 59 (128), 4200 x [2048, 2048] 53 -> 38 (160), 8000 x [3072, 2048] 98 -> 91 (224), 1000 x
-// [6144, 4096] 93 -> 58 (128); 2048 x [6144, 4096] stays (97; 128 rows 113).  Sums over K are in the same order.
+// by height as measured (a round of K = 4096: 256 rows 94, 224: 84, 192: 76, 160: 60, 128: 54; odd multiples of 16 between).
+// Rows x [N, K], 256-row tiles -> heights in steps of 32 -> in steps of 16: 5331 x [4096, 4096] 188 -> 143 -> 134 us, x
+// [6144, 4096] 248 -> 207 -> 200, 4200 x [4096, 4096] 123 -> 116, 10000 x [6144, 4096] 369 -> 346, 5331 x [3072, 2048] 67 -> 62,
+// 3000 x [4096, 4096] 95 -> 76 -> 74, 1500 x [4096, 4096] 78 -> 58 -> 56, 1000 x [6144, 4096] 93 -> 57 -> 56; 2048 x [6144, 4096]
+// stays (92; 128 rows 113).  Weights stored [K][N] take the same heights: 1000 x [4096, 4096] 90 -> 55, 300 x 55 -> 49, 5331 x
+// 176 -> 136, x [6144, 4096] 238 -> 202, 2048 x [2048, 2048] 50 -> 32.  Sums over K are in the same order.
 static int dense_tile_rows(int64_t rows, int n_tiles, int k_slabs, int sm, int sn) {
     float best = 0.f;
     int best_rows = 0;
-    for (int h : {256, 224, 192, 160, 128}) {
+    constexpr float kPerSlab[] = {0.75f, 0.80f, 0.86f, 0.97f, 1.08f, 1.14f, 1.20f, 1.28f, 1.36f};     // 128, 144, .. 256 rows
+    for (int h = 256; h >= 128; h -= 16) {
         const int64_t m_tiles = (rows + h - 1) / h;
-        const int64_t height = ((rows + m_tiles - 1) / m_tiles + 31) / 32 * 32;     // tiles of a group have one height
-        const float per_slab = height > 224 ? 1.36f : height > 192 ? 1.2f : height > 160 ? 1.08f : height > 128 ? 0.84f : 0.75f;
+        const int64_t height = ((rows + m_tiles - 1) / m_tiles + 15) / 16 * 16;     // tiles of a group have one height
+        const float per_slab = kPerSlab[height > 128 ? (height - 128) / 16 : 0];
         const int64_t rounds = ((m_tiles + sm - 1) / sm * ((n_tiles + sn - 1) / sn) + kNumXcd - 1) / kNumXcd;
         const float t = (float)rounds * (k_slabs * per_slab + 7.f);
         if (h == 256 || t < 0.97f * best) {
@@ -1613,9 +1620,10 @@ struct TileCost {
     float per_slab, per_tile;
     int min_tiles;
 };
-// spread: groups vary around their mean, so those of a mean just below a multiple of the tile height need one tile more.
+// spread: groups vary around their mean, so those of a mean just below a multiple of the tile height need one tile more (64
+// experts of 108 rows on average, 81-140: gate/up 182 us in 128-row tiles, 161 in 256-row ones; of 94 rows 167 both).
 static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs, bool spread = false) {
-    const int64_t rows = spread && E > 1 ? max_rows + max_rows / 10 : max_rows;
+    const int64_t rows = spread && E > 1 ? max_rows + max_rows / 5 : max_rows;
     const int64_t avg = (rows + E - 1) / E;
     const int64_t tiles = (int64_t)E * ((avg + c.rows - 1) / c.rows) * ((n_cols + c.cols - 1) / c.cols);
     const int64_t per_cu = (tiles + 255) / 256;
@@ -1697,7 +1705,7 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     constexpr TileCost kMid = kBf16 ? TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 0.58f : 1.05f, 5.f, 1}
                                     : TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 2.0f : 3.65f, 5.f, 1};
     const float mid = tile_time(kMid, max_rows, E, p.N_out, nk, true);
-    // (the 16 x 16 x 32 kernel computes only the 32-row steps that a tile has; up to 192 rows its loads bound a slab)
+    // (the 16 x 16 x 32 kernel computes only the 16-row fragments that a tile has; up to 192 rows its loads bound a slab)
     const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? (avg <= 192 ? 1.3f : 1.45f) : 7.3f, 7.f, 1},
                                 max_rows, E, p.N_out, nk, true);
     const float least_large = mid < big ? mid : big;
@@ -1831,12 +1839,13 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
     p.sn = 8;
     pick_supertile(p.n_tiles, &p.sm, &p.sn);
     p.aligned_bands = max_rows / (p.E > 0 ? p.E : 1) >= kAlignedBandsMinAvgRows ? 1 : 0;
-    const int64_t blocks = grid_blocks(max_rows, p.E, BM, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0);
+    if (!DSILU && p.E == 1) p.tile_rows = dense_tile_rows(max_rows, p.n_tiles, p.K / 64, p.sm, p.sn);
+    const int64_t blocks = grid_blocks(max_rows, p.E, p.tile_rows ? p.tile_rows : BM, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0);
     if (blocks > 0x7fffffffLL) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(mid_rows(max_rows, p.E) ? kern_mid : kern, dim3((unsigned)blocks), dim3(512), smem, s, p);
+    hipLaunchKernelGGL(p.tile_rows || mid_rows(max_rows, p.E) ? kern_mid : kern, dim3((unsigned)blocks), dim3(512), smem, s, p);
     return ATS_OK;
 }
 
