@@ -287,8 +287,9 @@ def _ffn_forward(x, wgu, wd, offsets, kept, rows, row_src, k, want_wgrad=False):
 
 
 def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x, need_w, hT=None, wplan=None):
-    """Gradients of _ffn_forward: dx_rows [rows, H] (or None), dWgu [E, 2I, H], dWd [E, H, I] (or None).
-    dgrad multiplies by per-step transposed copies of the weights; wgrad multiplies the transposed,
+    """Gradients of _ffn_forward: dx_rows [rows, H] (or None; float32 [slices, rows, H], to be added, where the product cut
+    K), dWgu [E, 2I, H], dWd [E, H, I] (or None).
+    dgrad reads the weights as the forward holds them (float32 and sizes off its grid: per-step transposed copies); wgrad multiplies the transposed,
     zero-padded activations of each expert (K = its padded row count).  h may be None when hT, its transposed
     copy from the forward kernel, is given; the fused bfloat16 dgrad kernel likewise hands back dgu and its
     transposed copy, so only dy and the gathered x go through a transposing pass."""
@@ -298,28 +299,45 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
     if need_w and wplan is None:
         wplan = ops.wgrad_plan(kept)
     dguT = None
+
+    def from_forward_weights(ws, N, K, grad):
+        """grad [rows, K] against the forward's own [K, N] weights: [rows, N], float32 [slices, rows, N] where K is cut, or
+        None where a transposed copy of the weights is the better way."""
+        slices = ops.grouped_gemm_nn_slices(E, rows, N, K, N, dtype) if DGRAD_FROM_FORWARD_WEIGHTS else 0
+        if slices == 0:
+            return None
+        tab = ops.weight_pointer_table(list(ws))
+        if rows // E > 256:
+            return ops.grouped_gemm_nn(tab, N, offsets, kept, rows, rows, N, K, grad)
+        return ops.grouped_gemm_nn_sliced(tab, N, offsets, kept, rows, rows, N, K, grad, slices)
+
+    dh = None
     t_col0 = wplan[0] if need_w and FUSE_TRANSPOSED_COPIES else None
     if DGRAD_FROM_FORWARD_WEIGHTS and ops.grouped_down_dgrad_dsilu_supported(E, rows, H, I, dtype, transposed_weights=False):
         # prefill-sized bfloat16 groups: one kernel, reading the down weights as the forward holds them
         pair = ops.grouped_down_dgrad_dsilu(dy, ops.weight_pointer_table(list(wd)), gu, offsets, kept, rows, H, I,
                                             t_col0=t_col0, transposed_weights=False)
     else:
-        wdT, tab_dT = ops.transpose_batched(wd)                  # [I, H] per expert; kept alive until return
         pair = None
+        dh = from_forward_weights(wd, I, H, dy)
+    if pair is None and dh is None:
+        wdT, tab_dT = ops.transpose_batched(wd)                  # [I, H] per expert; kept alive until return
         if _fused_grid(dtype, E, rows, I):
             pair = ops.grouped_down_dgrad_dsilu(dy, tab_dT, gu, offsets, kept, rows, H, I, t_col0=t_col0)   # one kernel
     dgu = None
     if pair is not None:
         dgu, dguT = pair
     if dgu is None:                                              # smaller groups, float32: two kernels
-        dh = ops.grouped_gemm_nt(tab_dT, H, I, offsets, kept, rows, rows, I, H, a=dy)
+        if dh is None:
+            dh = ops.grouped_gemm_nt(tab_dT, H, I, offsets, kept, rows, rows, I, H, a=dy)
+        elif dh.dim() == 3:
+            dh = ops.sum_partials(dh, dtype)
         dgu = torch.empty_like(gu)
         ops.silu_mul_bwd(gu[:, :I], gu[:, I:], dh, da=dgu[:, :I], db=dgu[:, I:], rows_dev=offsets[-1:])
     dx_rows = dwgu = dwd = None
     if need_x:
-        if DGRAD_FROM_FORWARD_WEIGHTS and ops.grouped_gemm_nn_supported(E, rows, H, 2 * I, H, dtype):
-            dx_rows = ops.grouped_gemm_nn(ops.weight_pointer_table(list(wgu)), H, offsets, kept, rows, rows, H, 2 * I, dgu)
-        else:
+        dx_rows = from_forward_weights(wgu, H, 2 * I, dgu)
+        if dx_rows is None:
             wguT, tab_guT = ops.transpose_batched(wgu)           # [H, 2I] per expert
             dx_rows = ops.grouped_gemm_nt(tab_guT, 2 * I, H, offsets, kept, rows, rows, H, 2 * I, a=dgu)
     if need_w:
@@ -372,6 +390,8 @@ class ExpertFFNFunction(Function):
         need_x, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         dx, dwgu, dwd = _ffn_backward(dy.to(x.dtype).contiguous(), x, ctx.wgu, ctx.wd, gu, h, offsets, kept,
                                       x.shape[0], None, 1, need_x, need_w, hT=hT, wplan=wplan)
+        if dx is not None and dx.dim() == 3:
+            dx = ops.sum_partials(dx, x.dtype)
         return (dx, dwgu[0].to(ctx.param_dtypes[0]) if need_w else None,
                 dwd[0].to(ctx.param_dtypes[1]) if need_w else None)
 
@@ -454,7 +474,11 @@ class MoEFunction(Function):
                                                need_w, hT=hT, wplan=wplan)
             if need_x:
                 ones = torch.ones(T, k, dtype=torch.float32, device=dev)
-                dx = ops.combine(dx_rows, row_of, ones, T, k, out_dtype=dtype)
+                if dx_rows.dim() == 3 and k <= 8:
+                    dx = ops.combine_partials(dx_rows, row_of, ones, T, k, dtype)
+                else:
+                    dx_rows = ops.sum_partials(dx_rows, dtype) if dx_rows.dim() == 3 else dx_rows
+                    dx = ops.combine(dx_rows, row_of, ones, T, k, out_dtype=dtype)
         else:
             dw = torch.zeros(T, k, dtype=torch.float32, device=dev)
             dx = torch.zeros(T, H, dtype=dtype, device=dev) if need_x else None

@@ -1097,7 +1097,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
                                                          const int32_t* __restrict__ row_count) {
 #if defined(__HIP_DEVICE_COMPILE__)
     static_assert(!BKM || (!SWIGLU && !SAVEGU), "the K-major weight layout serves the plain product and the dgrad epilogue");
-    static_assert(!SLICED || (MIDROWS && !SWIGLU && !BKM), "slices of K need a linear epilogue");
+    static_assert(!SLICED || (MIDROWS && !SWIGLU && !DSILU), "slices of K need a linear epilogue");
     typedef bf16_t T;
     constexpr int BM = 256, BN = 256, WM = 2, WN = 4;
     constexpr int NW = WM * WN;
@@ -1127,7 +1127,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     const int row0 = p.row_start[tc.e];
     const int K = SLICED ? p.k_slice : p.k_count ? p.k_count[tc.e] : p.K;
     const int64_t k_first = SLICED ? (int64_t)split * p.k_slice : 0;
-    const T* Bexp = static_cast<const T*>(p.b[tc.e]) + k_first;
+    const T* Bexp = static_cast<const T*>(p.b[tc.e]) + (BKM ? k_first * p.ldb : k_first);
     const T* A = static_cast<const T*>(p.a_ptrs ? p.a_ptrs[tc.e] : p.a) + k_first;
     const int arow0 = p.a_ptrs ? 0 : row0;
 
@@ -1588,11 +1588,12 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
 // of few experts has half a round of these tiles or less (8 x [4096, 14336]: 128), and a CU takes 1.2-1.4 us per slab of
 // K whatever the other half of the chip does; two slices make it a full round: 200 rows per expert 314 -> 165 us.  The 32
 // and 64-row sliced tiles it replaces for several groups read every weight once per 64 rows (200 rows: 517 us).
+template <bool BKM = false>
 static int launch_mid_sliced(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     GroupedArgs p = p0;
     p.n_tiles = (p.N_out + 255) / 256;
     constexpr size_t smem = dma_lds_bytes(256, 256);
-    auto kern = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, false, true, true>;
+    auto kern = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, BKM, true, true>;
     static LdsReservation reserved;
     hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern)}, (int)smem);
     if (e != hipSuccess) {
@@ -1658,7 +1659,7 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
                 // (with fewer tiles than half of the CUs the small tiles below spread the work further)
                 if (E > 1 && avg > 20 && p.k_slice % 64 == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0 && !p.k_count &&
                     (int64_t)E * ((p.N_out + 255) / 256) * p.k_splits >= 128)
-                    return launch_mid_sliced(p, max_rows, s);
+                    return launch_mid_sliced<>(p, max_rows, s);
             }
             return avg > 32 ? launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s)
                             : launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
@@ -2089,6 +2090,82 @@ extern "C" int ats_grouped_gemm_nn(const void* a, int64_t lda, int64_t a_num_row
     hipStream_t s = as_stream(stream);
     const int rc = out_dtype == ATS_F32 ? launch_kmajor<float, false>(p, max_rows, s)
                                         : launch_kmajor<bf16_t, false>(p, max_rows, s);
+    if (rc != ATS_OK) return rc;
+    ATS_CHECK_LAUNCH(name);
+    return ATS_OK;
+}
+
+// Slices of K with which a product against [K][N] weights is to run, 0 where multiplying by a transposed copy is the
+// faster one or the only one.  Above 256 rows per group it is ats_grouped_gemm_nn.  Below, the 256-column tiles of a few
+// experts leave CUs idle, so K is cut (launch_mid_sliced); the estimate holds both routes against each other: a CU takes
+// 1.3 us per slab and 7 per tile, partial results are written and read at 5 TB/s, a copy is made at 5.2 TB/s and
+// multiplied at 4.6.  Training pass of 8 experts, top 2, [28672, 4096] and [4096, 14336], copies -> this: 256 tokens 3445 ->
+// 2124 us, 588 tokens 3851 -> 2557, 760 tokens 4050 -> 2742 (the copies alone were 1100).
+extern "C" int ats_grouped_gemm_nn_slices(int E, int64_t max_rows, int N, int K, int64_t ldb, int dtype) {
+    using namespace ats;
+    if (N <= 0 || K <= 0 || E <= 0 || max_rows <= 0 || dtype != ATS_BF16) return 0;
+    if (!kmajor_supported(E, max_rows, N, K, ldb, -1)) return 0;
+    const int64_t avg = (max_rows + E - 1) / E;
+    if (max_rows / E > 256) return 1;
+    const double weights = 2.0 * E * N * K;      // bytes
+    const int64_t tiles = (int64_t)E * ((N + 255) / 256) * (E > 1 && avg > 232 ? 3 : 2) / 2;
+    // (the unsliced launch of more than 192 rows never had a copy to make)
+    double best = max_rows / E > 192 ? 1e30 : weights * (2 / 5.2e6 + 1 / 4.6e6) + 5.;
+    int slices = 0;
+    for (int s = 1; s <= 16; s *= 2) {
+        if (s > 1 && (K % (s * 64) != 0 || K / s < 512)) break;
+        const double t = (double)((tiles * s + 255) / 256) * (K / 64 / s * 1.3 + 7.) + (s > 1 ? 8. * max_rows * N * s / 5e6 + 4. : 0.);
+        if (t < 0.97 * best) {
+            best = t;
+            slices = s;
+        }
+    }
+    return slices;
+}
+
+// out: k_splits = 1: [rows, ldo = N] of out_dtype; more: float32 partial results [k_splits][part_rows][N].
+extern "C" int ats_grouped_gemm_nn_sliced(const void* a, int64_t lda, const void* const* b_ptrs, int64_t ldb, void* out,
+                                          int64_t part_rows, const int32_t* row_start, const int32_t* row_count, int E,
+                                          int64_t max_rows, int N, int K, int k_splits, int dtype, int out_dtype,
+                                          ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_grouped_gemm_nn_sliced";
+    ATS_REQUIRE(E > 0 && E <= 4096 && max_rows >= 0 && N > 0 && K > 0 && part_rows >= max_rows, ATS_ERR_INVALID_ARG,
+                "%s: E=%d max_rows=%lld part_rows=%lld N=%d K=%d", name, E, (long long)max_rows, (long long)part_rows, N, K);
+    ATS_REQUIRE(dtype == ATS_BF16 && (out_dtype == ATS_F32 || (out_dtype == ATS_BF16 && k_splits == 1)), ATS_ERR_UNSUPPORTED,
+                "%s: dtype tags %d -> %d (bfloat16 operands; slices give float32)", name, dtype, out_dtype);
+    ATS_REQUIRE(a && b_ptrs && out && row_start && row_count, ATS_ERR_INVALID_ARG, "%s: null pointer", name);
+    ATS_REQUIRE(lda % 8 == 0 && lda >= K, ATS_ERR_UNSUPPORTED, "%s: K=%d lda=%lld must describe 16-byte aligned rows", name, K,
+                (long long)lda);
+    ATS_REQUIRE(aligned16(a) && aligned16(out), ATS_ERR_INVALID_ARG, "%s: operands must be 16-byte aligned", name);
+    ATS_REQUIRE(k_splits >= 1 && k_splits <= 64 && K % (k_splits * 64) == 0, ATS_ERR_UNSUPPORTED,
+                "%s: K=%d is not %d slices of whole 64-element slabs", name, K, k_splits);
+    if (max_rows == 0) return ATS_OK;
+    ATS_REQUIRE(kmajor_supported(E, max_rows, N, K, ldb, -1) && max_rows / E <= 256, ATS_ERR_UNSUPPORTED,
+                "%s: up to 256 rows per expert on average, N and ldb multiples of 8 and one expert's weights within 4 GiB "
+                "(E=%d max_rows=%lld N=%d K=%d ldb=%lld)", name, E, (long long)max_rows, N, K, (long long)ldb);
+    GroupedArgs p{};
+    p.a = a;
+    p.a_row_div = 1;
+    p.lda = lda;
+    p.b = b_ptrs;
+    p.ldb = ldb;
+    p.out = out;
+    p.ldo = N;
+    p.row_start = row_start;
+    p.row_count = row_count;
+    p.E = E;
+    p.K = K;
+    p.N_out = N;
+    p.k_splits = k_splits;
+    p.k_slice = K / k_splits;
+    p.part_stride = part_rows * N;
+    p.a_extent_bytes = 0xffffffffu;
+    p.b_extent_bytes = extent32(K, ldb, 2);
+    hipStream_t s = as_stream(stream);
+    const int rc = k_splits > 1 ? launch_mid_sliced<true>(p, max_rows, s)
+                   : out_dtype == ATS_F32 ? launch_kmajor<float, false>(p, max_rows, s)
+                                          : launch_kmajor<bf16_t, false>(p, max_rows, s);
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;

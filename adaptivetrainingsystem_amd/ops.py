@@ -1115,6 +1115,32 @@ def grouped_gemm_nn(b_ptrs: torch.Tensor, ldb: int, row_start: torch.Tensor, row
     return out
 
 
+def grouped_gemm_nn_slices(E: int, max_rows: int, N: int, K: int, ldb: int, dtype: torch.dtype) -> int:
+    """Slices of K for a product against weights stored [K, ldb]; 0: multiply by a transposed copy."""
+    if dtype != torch.bfloat16:
+        return 0
+    return int(_lib.load().ats_grouped_gemm_nn_slices(int(E), int(max_rows), int(N), int(K), int(ldb), _DT[dtype]))
+
+
+def grouped_gemm_nn_sliced(b_ptrs: torch.Tensor, ldb: int, row_start: torch.Tensor, row_count: torch.Tensor, n_rows_out: int,
+                           max_rows: int, N: int, K: int, a: torch.Tensor, k_splits: int) -> torch.Tensor:
+    """grouped_gemm_nn for groups of up to 256 rows on average: the product [n_rows_out, N], or with more than one slice of
+    K the float32 partial results [k_splits, n_rows_out, N]."""
+    _need_gpu(a, b_ptrs, row_start, row_count)
+    a = _rows_2d(a, "grouped_gemm_nn_sliced")
+    if a.shape[0] < max_rows or n_rows_out < max_rows:
+        raise AtsError("grouped_gemm_nn_sliced: fewer rows than max_rows")
+    E = b_ptrs.numel()
+    shape, dtype = ((n_rows_out, N), a.dtype) if k_splits == 1 else ((k_splits, n_rows_out, N), torch.float32)
+    out = torch.empty(shape, dtype=dtype, device=b_ptrs.device)
+    check(_lib.load().ats_grouped_gemm_nn_sliced(a.data_ptr(), int(a.stride(0)), b_ptrs.data_ptr(), int(ldb), out.data_ptr(),
+                                                 int(n_rows_out), row_start.data_ptr(), row_count.data_ptr(), E,
+                                                 int(max_rows), int(N), int(K), int(k_splits), _DT[a.dtype], _DT[dtype],
+                                                 _stream()),
+          "ats_grouped_gemm_nn_sliced")
+    return out
+
+
 # --------------------------------------------------------------------------- attention
 def _key_bias(key_bias, B: int, Lk: int, q: torch.Tensor, who: str):
     if key_bias is None:

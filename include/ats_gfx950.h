@@ -463,6 +463,15 @@ int ats_grouped_gemm_nn(const void* a, int64_t lda, int64_t a_num_rows, const in
                         const void* const* b_ptrs, int64_t ldb, void* out, int64_t ldo, const int32_t* row_start,
                         const int32_t* row_count, int E, int64_t max_rows, int N, int K, int dtype, int out_dtype,
                         ats_stream_t stream);
+/* The same product for groups of up to 256 rows on average, K cut into k_splits equal slices of whole 64-element
+ * slabs: float32 partial results [k_splits][part_rows][N] that ats_sum_partials or ats_combine_partials add, or with
+ * k_splits = 1 the product itself, [part_rows][N] of out_dtype.  ..._slices: the number of slices to use; 1 also for
+ * larger groups, which are ats_grouped_gemm_nn's; 0: transpose and call ats_grouped_gemm_nt. */
+int ats_grouped_gemm_nn_slices(int E, int64_t max_rows, int N, int K, int64_t ldb, int dtype);
+int ats_grouped_gemm_nn_sliced(const void* a, int64_t lda, const void* const* b_ptrs, int64_t ldb, void* out,
+                               int64_t part_rows, const int32_t* row_start, const int32_t* row_count, int E,
+                               int64_t max_rows, int N, int K, int k_splits, int dtype, int out_dtype,
+                               ats_stream_t stream);
 
 /* ---- Causal grouped-query attention (forward) -----------------------------------
  * Replaces GroupedQueryAttention._standard_attention / _flash_attention

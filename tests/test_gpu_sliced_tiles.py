@@ -49,3 +49,37 @@ def test_layer_with_sliced_down_projection(gpu, T):
     ref = ref["out"] if isinstance(ref, dict) else ref[0]
     err = (out.cpu().double() - ref.double().view(out.shape)).norm() / ref.double().norm()
     assert err <= 1.2e-2      # h and y are rounded to bfloat16 (2^-9 each), measured 3e-3
+
+
+# the same against weights stored [K][N]: columns that are no multiple of the tile, slices of one slab and of several, groups
+# on both sides of a fragment, of one tile and of two, without rows
+@pytest.mark.parametrize("counts,N,K,S", [([33, 1, 0, 200, 256, 17, 64, 127], 264, 1024, 2), ([257, 30, 31, 32], 72, 512, 8),
+                                          ([40, 500, 1, 12], 1000, 320, 5), ([5], 520, 128, 1), ([190, 16, 0, 15], 8, 192, 1)])
+def test_sliced_product_with_k_major_weights(gpu, counts, N, K, S):
+    print("case sliced k-major", counts, N, K, S, flush=True)
+    from adaptivetrainingsystem_amd import ops
+    g = torch.Generator().manual_seed(sum(counts) + N)
+    E, rows, ldb = len(counts), sum(counts), N + 8
+    a = (torch.randn(rows, K, generator=g) * 0.5).bfloat16()
+    w = [(torch.randn(K, ldb, generator=g) * 0.05).bfloat16() for _ in range(E)]
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    start = torch.tensor(off[:-1], dtype=torch.int32, device=gpu)
+    count = torch.tensor(counts, dtype=torch.int32, device=gpu)
+    w_gpu = [t.to(gpu) for t in w]
+    out = ops.grouped_gemm_nn_sliced(ops.weight_pointer_table(w_gpu), ldb, start, count, rows, rows, N, K, a.to(gpu), S).cpu()
+    n = K // S
+    for s in range(S):
+        ref = torch.cat([a[off[e]:off[e + 1], s * n:(s + 1) * n].double() @ w[e][s * n:(s + 1) * n, :N].double() for e in range(E)])
+        bound = 4e-7 * (a[:, s * n:(s + 1) * n].double().abs().sum(1).max() * max(t.abs().max().double() for t in w))
+        if S == 1:
+            bound = bound + 2.0 ** -8 * ref.abs().max()      # one rounding to bfloat16
+        assert ((out if S == 1 else out[s]).double() - ref).abs().max() <= bound
+
+
+def test_rule_of_k_major_slices(gpu):
+    from adaptivetrainingsystem_amd import ops
+    rule = lambda *a: ops.grouped_gemm_nn_slices(*a, torch.bfloat16)
+    assert rule(8, 650, 4096, 28672, 4096) == 2 and rule(8, 650, 14336, 4096, 14336) == 1
+    assert rule(8, 8 * 300, 4096, 28672, 4096) == 1 and rule(8, 8 * 200, 4096, 28672, 4096) >= 1
+    assert rule(8, 650, 4100, 28672, 4100) == 0 and rule(8, 650, 4096, 28672 + 32, 4096) == 0 and rule(8, 0, 4096, 4096, 4096) == 0
+    assert ops.grouped_gemm_nn_slices(8, 650, 4096, 28672, 4096, torch.float32) == 0
