@@ -115,11 +115,18 @@ class AttentionFunction(Function):
 
 
 class AttentionF32Function(Function):
-    """The float32 route of the attention (ops.attention_f32): same arguments as AttentionFunction; the softmax
-    weights are kept for the backward, as autograd keeps them for the reference."""
+    """The float32 route of the attention: same arguments as AttentionFunction.  Where the kernels without materialised
+    scores take the call, the inputs, the output and two numbers per row are kept for the backward; otherwise the softmax
+    weights, as autograd keeps them for the reference (ops.attention_f32)."""
 
     @staticmethod
     def forward(ctx, q, k, v, scale, key_bias=None, pair_bias=None, dropout_p=0.0, dropout_seed=0):
+        ctx.fused = ops.attention_f32_fused_supported(q, k, v, pair_bias, dropout_p)
+        ctx.scale = scale
+        if ctx.fused:
+            out, stats = ops.attention_f32_fused(q, k, v, scale, key_bias)
+            ctx.save_for_backward(q, k, v, out, stats, key_bias)
+            return out
         out, state = ops.attention_f32(q, k, v, scale, key_bias=key_bias, pair_bias=pair_bias, dropout_p=dropout_p,
                                        dropout_seed=dropout_seed, return_weights=True)
         w, w_drop, qp, kp, vp = state
@@ -130,8 +137,12 @@ class AttentionF32Function(Function):
 
     @staticmethod
     def backward(ctx, dout):
+        saved = ctx.saved_tensors
+        if ctx.fused:
+            q, k, v, out, stats, key_bias = saved
+            return (*ops.attention_f32_fused_bwd(q, k, v, out, stats, dout, ctx.scale, key_bias), None, None, None, None, None)
         B, Hq, Hkv, L, Lk, D, scale, p, seed = ctx.meta
-        dq, dk, dv = ops.attention_f32_bwd(ctx.saved_tensors, dout.contiguous(), B, Hq, Hkv, L, Lk, D, scale, p, seed)
+        dq, dk, dv = ops.attention_f32_bwd(saved, dout.contiguous(), B, Hq, Hkv, L, Lk, D, scale, p, seed)
         return dq, dk, dv, None, None, None, None, None
 
 

@@ -1295,6 +1295,8 @@ def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Opti
     if pair_bias is not None:
         pair_bias, pair_sb, pair_sh = _pair_bias(pair_bias, B, Hq, L, Lk, q, "attention_f32")
     scale = float(D ** -0.5 if scale is None else scale)
+    if not return_weights and attention_f32_fused_supported(q, k, v, pair_bias, dropout_p):
+        return attention_f32_fused(q, k, v, scale, key_bias, want_stats=False)[0]
     dev = q.device
     lib = _lib.load()
     Lp, Lkp = (L + 3) // 4 * 4, (Lk + 3) // 4 * 4
@@ -1322,6 +1324,49 @@ def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Opti
     if return_weights:
         return out, (w, w_drop, qp, kp, vp)
     return out
+
+
+def attention_f32_fused_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pair_bias: Optional[torch.Tensor],
+                                  dropout_p: float) -> bool:
+    """Whether the kernels without materialised scores take this call (csrc/attention_f32_fused.hip)."""
+    return (pair_bias is None and dropout_p == 0.0 and q.shape[3] in (64, 128) and q.shape[2] > 0 and q.shape[0] > 0
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (q, k, v)))
+
+
+def attention_f32_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, key_bias: Optional[torch.Tensor],
+                        want_stats: bool = True) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """attention_f32 in one launch: out [B, L, Hq*D] and, for the backward pass, the maximum and the reciprocal sum of
+    every row [B*Hq, L, 2]."""
+    _need_gpu(q, k, v)
+    B, Hq, L, D = q.shape
+    Hkv, Lk = k.shape[1], k.shape[2]
+    key_bias = _key_bias(key_bias, B, Lk, q, "attention_f32")
+    out = torch.empty(B, L, Hq * D, dtype=torch.float32, device=q.device)
+    stats = torch.empty(B * Hq, L, 2, dtype=torch.float32, device=q.device) if want_stats else None
+    check(_lib.load().ats_attention_f32_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _ptr(stats), B, Hq, Hkv,
+                                            L, Lk, D, float(scale), _ptr(key_bias), _stream()), "ats_attention_f32_fwd")
+    return out, stats
+
+
+def attention_f32_fused_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, stats: torch.Tensor,
+                            dout: torch.Tensor, scale: float, key_bias: Optional[torch.Tensor]):
+    """Gradients of attention_f32_fused: (dq, dk, dv) in two launches."""
+    _need_gpu(q, k, v, out, stats, dout)
+    B, Hq, L, D = q.shape
+    Hkv, Lk = k.shape[1], k.shape[2]
+    if dout.shape != out.shape or dout.dtype != torch.float32:
+        raise AtsError("attention_f32_fused_bwd: dout must be float32 of the output's shape")
+    dout = dout.contiguous()
+    if dout.data_ptr() % 16:
+        dout = dout.clone()
+    key_bias = _key_bias(key_bias, B, Lk, q, "attention_f32")
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    delta = torch.empty(B * Hq * L, dtype=torch.float32, device=q.device)
+    check(_lib.load().ats_attention_f32_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), stats.data_ptr(),
+                                            dout.data_ptr(), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B,
+                                            Hq, Hkv, L, Lk, D, float(scale), _ptr(key_bias), _stream()),
+          "ats_attention_f32_bwd")
+    return dq, dk, dv
 
 
 def attention_f32_bwd(state, dout: torch.Tensor, B: int, Hq: int, Hkv: int, L: int, Lk: int, D: int,

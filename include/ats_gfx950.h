@@ -562,6 +562,16 @@ int ats_attention_softmax_f32(float* scores, float* weights_drop, int B, int Hq,
 int ats_attention_softmax_bwd_f32(const float* weights, float* dp, int B, int Hq, int L, int Lp, int Lk, int ld,
                                   float scale, float dropout_p, uint64_t dropout_seed, ats_stream_t stream);
 
+/* The same attention without materialised scores: D = 64 or 128, contiguous q [B,Hq,L,D], k, v [B,Hkv,Lk,D], no dropout, no
+ * per-pair mask (key_bias [B,Lk] or NULL as above).  out [B,L,Hq*D]; stats (may be NULL without a backward pass)
+ * [B*Hq,L][2] receives a row's maximum and the reciprocal of its sum.  _bwd: dout laid out like out, delta is scratch of
+ * B*Hq*L floats; dq, dk, dv laid out like q, k, v. */
+int ats_attention_f32_fwd(const float* q, const float* k, const float* v, float* out, float* stats, int B, int Hq, int Hkv,
+                          int L, int Lk, int D, float scale, const float* key_bias, ats_stream_t stream);
+int ats_attention_f32_bwd(const float* q, const float* k, const float* v, const float* out, const float* stats,
+                          const float* dout, float* delta, float* dq, float* dk, float* dv, int B, int Hq, int Hkv, int L,
+                          int Lk, int D, float scale, const float* key_bias, ats_stream_t stream);
+
 /* ---- Training-step ops beside the sparse layer --------------------------------
  * Fused cross-entropy + accuracy.  Replaces fused_cross_entropy_accuracy_launcher
  * (Src/Main_Scripts/training/fused_loss.cu:179-214); numerics follow FusedLoss._pytorch_fallback
