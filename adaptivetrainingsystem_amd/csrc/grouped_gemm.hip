@@ -26,6 +26,8 @@
 //   grouped_gemm_stream_kernel    decode-sized groups: a stream of weights, see grouped_gemm_stream.hpp.
 //   grouped_gemm_small_kernel     32 and 64-row tiles for launches whose large tiles would leave most CUs idle, see
 //                                 grouped_gemm_small.hpp.
+//   grouped_gemm_short_kernel     weight gradients over a few hundred rows per expert: stores bound, see
+//                                 grouped_gemm_short.hpp.
 //   grouped_gemm_kernel           general fallback for K that is not a multiple of a slab (bounds-checked loads).
 #include <math.h>
 
@@ -146,6 +148,7 @@ struct AccView16 {
 // instruction.  Instead every wave transposes 32-row blocks of its sub-tile through a private LDS
 // region and writes whole rows: 16 bytes per lane, 128-byte lines fully covered.
 // wstage: this wave's private region, 32 * (columns * sizeof(TO) + 16) bytes.
+// STREAM: the results leave with non-temporal stores.
 // SAVEGU (with SWIGLU): the gate and up accumulators themselves also go to gu[row, col] and gu[row, up_off + col]
 // (what the backward pass of a training step needs), through the same staging region.
 // DSILU (without SWIGLU): the tile is dh, the gradient of h = silu(g) * u; instead of storing it, every lane reads
@@ -177,7 +180,7 @@ constexpr int epilogue_wstage_bytes() {
     return DSILU && sizeof(TO) == 2 && View::kCols == 64 && View::kBlocks == 4
                ? 32 * 128 : 32 * (View::kCols * (int)sizeof(TO) + 16);
 }
-template <typename TO, typename View, bool SWIGLU, bool SAVEGU = false, bool DSILU = false>
+template <typename TO, typename View, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool STREAM = false>
 __device__ __forceinline__ void epilogue_view(const View av, unsigned char* wstage, TO* out, int64_t ldo,
                                               int64_t row_base, int rows_valid, int ncol0, int n_out, int lane,
                                               TO* gu = nullptr, int64_t ldgu = 0, int up_off = 0,
@@ -296,8 +299,11 @@ __device__ __forceinline__ void epilogue_view(const View av, unsigned char* wsta
                     }
                 }
             } else {
-                if (m_local < rows_valid && col < n_out)
-                    *reinterpret_cast<u32x4_t*>(out + (row_base + m_local) * ldo + col) = data;
+                if (m_local < rows_valid && col < n_out) {
+                    u32x4_t* const to = reinterpret_cast<u32x4_t*>(out + (row_base + m_local) * ldo + col);
+                    if constexpr (STREAM) __builtin_nontemporal_store(data, to);
+                    else *to = data;
+                }
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1482,6 +1488,12 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
 #undef PL_FENCE
 #undef PL_MIX_READS
 
+}  // namespace ats
+
+#include "grouped_gemm_short.hpp"
+
+namespace ats {
+
 // LDS of the direct-to-LDS kernel: three activation stages and two weight stages of unpadded 128-byte rows.
 constexpr size_t dma_lds_bytes(int BM, int BN) { return (size_t)(3 * BM + 2 * BN) * 128; }
 
@@ -1667,6 +1679,11 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     }
     // (with a K per group, p.K is the bound on their sum)
     const int nk = p.k_count ? (p.K / E + BK - 1) / BK : (p.K + BK - 1) / BK;
+    if constexpr (kBf16 && !SWIGLU && std::is_same<TO, bf16_t>::value) {
+        // weight gradients over up to 512 padded rows per group that are large enough to fill the chip four deep
+        if (p.k_count && !p.a_rows && nk <= 8 && (int64_t)E * ((avg + kShortBM - 1) / kShortBM) * ((p.N_out + kShortBN - 1) / kShortBN) >= 2048)
+            return launch_short(p, max_rows, s);
+    }
     // Few rows per group: a stream of weights (E == 1: the row count is exact; several groups vary around their mean, and
     // a group beyond 32 rows reads its weights twice).  Measured, microseconds, weights from HBM, against the register-
     // staged 32-row tiles with two slabs in flight that this kernel replaced:
