@@ -149,7 +149,7 @@ class AttentionF32Function(Function):
 class LinearFunction(Function):
     """y = x @ weight^T for x [T, K], weight [N, K] (a bias-free nn.Linear) through the grouped GEMM kernels
     with one group: dgrad reads the weight as it is where the K-major kernel applies (bfloat16, more than 192
-    rows) and multiplies by a transposed copy otherwise, wgrad multiplies the transposed activations."""
+    rows) and multiplies by a transposed copy otherwise, wgrad reads both operands as they are (bfloat16) or transposed."""
 
     @staticmethod
     def forward(ctx, x, weight):
@@ -174,9 +174,12 @@ class LinearFunction(Function):
                 wT, tab = ops.transpose_batched([w])             # [K, N]; kept alive until the GEMM is queued
                 dx = ops.grouped_gemm_nt(tab, N, K, offsets, kept, T, T, K, N, a=dy)
         if ctx.needs_input_grad[1]:
-            dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
-            xT = ops.transpose_grouped_rows(x, offsets, kept, T)
-            dw = ops.wgrad_dense(dyT, xT, T).to(ctx.param_dtype)
+            if ops.wgrad_linear_supported(dy, x):
+                dw = ops.wgrad_linear(dy, x).to(ctx.param_dtype)
+            else:
+                dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
+                xT = ops.transpose_grouped_rows(x, offsets, kept, T)
+                dw = ops.wgrad_dense(dyT, xT, T).to(ctx.param_dtype)
         return dx, dw
 
 
@@ -184,7 +187,7 @@ class QKVRoPEFunction(Function):
     """q, k, v [B, heads, L, D] of a self-attention sub-layer from x [B*L, K] and the bias-free projections: one product with
     the stacked weights, then one launch that rotates q and k and lays out v.  Backward: one launch puts the three
     gradients, rotated back, side by side, so that the data gradient is one product (its sum over the three projections
-    stays in float32) and x is transposed once for the weight gradients; k and v share one of those.  Saved are the
+    stays in float32); k and v share one weight gradient.  Saved are the
     parameters, not their stacked copy (50 MB a layer at hidden 4096): it is made again for the data gradient (40 us).
     Against three linear layers and a rotation, 8 x 2048 x 4096 bfloat16 forward and backward: the sub-layer 5588 -> 4665 us."""
 
@@ -223,17 +226,21 @@ class QKVRoPEFunction(Function):
                 wT, tab = ops.transpose_batched([w], tab)        # [K, N]; kept alive until the GEMM is queued
                 dx = ops.grouped_gemm_nt(tab, N, K, offsets, kept, T, T, K, N, a=dy)
         if any(ctx.needs_input_grad[1:4]):
-            dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
-            xT = ops.transpose_grouped_rows(x, offsets, kept, T)
             nq, nk = nh * D, nkv * D
+            if ops.wgrad_linear_supported(dy, x) and nk % 8 == 0:
+                wgrad = lambda lo, hi, heights=None: ops.wgrad_linear(dy[:, lo:hi], x, heights)
+            else:
+                dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
+                xT = ops.transpose_grouped_rows(x, offsets, kept, T)
+                wgrad = lambda lo, hi, heights=None: ops.wgrad_dense(dyT[lo:hi], xT, T, heights)
             if ctx.needs_input_grad[1]:
-                dws[0] = ops.wgrad_dense(dyT[:nq], xT, T)
+                dws[0] = wgrad(0, nq)
             if ctx.needs_input_grad[2] and ctx.needs_input_grad[3]:
-                dws[1:] = ops.wgrad_dense(dyT[nq:], xT, T, (nk, nk))
+                dws[1:] = wgrad(nq, N, (nk, nk))
             elif ctx.needs_input_grad[2]:
-                dws[1] = ops.wgrad_dense(dyT[nq:nq + nk], xT, T)
+                dws[1] = wgrad(nq, nq + nk)
             elif ctx.needs_input_grad[3]:
-                dws[2] = ops.wgrad_dense(dyT[nq + nk:], xT, T)
+                dws[2] = wgrad(nq + nk, N)
             dws = [None if g is None else g.to(dt) for g, dt in zip(dws, ctx.param_dtypes)]
         return (dx, *dws, None, None, None, None, None)
 

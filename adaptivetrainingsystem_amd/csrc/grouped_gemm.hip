@@ -1097,13 +1097,18 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // bits.  The 32-byte chunks of a row are swizzled on the global side, chunk c of stage row r lands in slot
 // c ^ f(r), f(r) = (r % 4) | ((r / 8) % 4) << 2: the 16 row pieces that one read instruction touches fall on 16
 // different slots, i.e. on all banks once.
+//
+// AKM: the other operand is stored [K][rows] as well (one group; p.b is the operand itself, p.K its exact number of rows): the
+// weight gradient of a linear layer from the gradients and activations as they lie, tokens along the rows, without
+// transposed copies.  The same slabs, swizzle and transposing reads; same bits as the product of transposed copies.
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
-          bool MIDROWS = false, bool SLICED = false>
+          bool MIDROWS = false, bool SLICED = false, bool AKM = false>
 __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, unsigned char* smem,
                                                          const int32_t* __restrict__ row_count) {
 #if defined(__HIP_DEVICE_COMPILE__)
     static_assert(!BKM || (!SWIGLU && !SAVEGU), "the K-major weight layout serves the plain product and the dgrad epilogue");
     static_assert(!SLICED || (MIDROWS && !SWIGLU && !DSILU), "slices of K need a linear epilogue");
+    static_assert(!AKM || (BKM && MIDROWS && !DSILU), "both operands K-major: the plain product in tiles of equal height");
     typedef bf16_t T;
     constexpr int BM = 256, BN = 256, WM = 2, WN = 4;
     constexpr int NW = WM * WN;
@@ -1131,10 +1136,11 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     }
     const int count = row_count[tc.e];
     const int row0 = p.row_start[tc.e];
-    const int K = SLICED ? p.k_slice : p.k_count ? p.k_count[tc.e] : p.K;
     const int64_t k_first = SLICED ? (int64_t)split * p.k_slice : 0;
-    const T* Bexp = static_cast<const T*>(p.b[tc.e]) + (BKM ? k_first * p.ldb : k_first);
-    const T* A = static_cast<const T*>(p.a_ptrs ? p.a_ptrs[tc.e] : p.a) + k_first;
+    const int K = AKM ? (int)(SLICED && k_first + p.k_slice < p.K ? p.k_slice : p.K - k_first)
+                  : SLICED ? p.k_slice : p.k_count ? p.k_count[tc.e] : p.K;
+    const T* Bexp = (AKM ? reinterpret_cast<const T*>(p.b) : static_cast<const T*>(p.b[tc.e])) + (BKM ? k_first * p.ldb : k_first);
+    const T* A = static_cast<const T*>(p.a_ptrs ? p.a_ptrs[tc.e] : p.a) + (AKM ? k_first * p.lda : k_first);
     const int arow0 = p.a_ptrs ? 0 : row0;
 
     const int tid = threadIdx.x;
@@ -1157,11 +1163,14 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     // ---- load descriptors and lane offsets: instruction j of this wave covers rows (j*NW + wave)*8 .. +8
     constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
     const bool gather = p.a_rows != nullptr;
-    const T* a_base = gather ? A : A + ((int64_t)arow0 + (int64_t)tile_row) * p.lda;
+    const T* a_base = gather || AKM ? A : A + ((int64_t)arow0 + (int64_t)tile_row) * p.lda;
+    // AKM: the descriptors end with the last of the K rows, what lies behind it reads as zero
+    const uint32_t a_extent = AKM ? (uint32_t)(((int64_t)(K - 1) * p.lda + count) * ES) : p.a_extent_bytes;
+    const uint32_t b_extent = AKM ? (uint32_t)(((int64_t)(K - 1) * p.ldb + p.N_out) * ES) : p.b_extent_bytes;
     const __amdgpu_buffer_rsrc_t rsrc_a =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a_base), 0, (int)p.a_extent_bytes, kRsrcFlags);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a_base), 0, (int)a_extent, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rsrc_b =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(Bexp), 0, (int)p.b_extent_bytes, kRsrcFlags);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(Bexp), 0, (int)b_extent, kRsrcFlags);
     const int drow = lane >> 3;
     const int dchunk = (lane & 7) ^ drow;
     unsigned ao[NIA], bo[NIB];
@@ -1169,6 +1178,16 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     int a_idx[NIA];
 #pragma unroll
     for (int j = 0; j < NIA; ++j) {
+        if constexpr (AKM) {
+            // as the K-major weights below, columns 0 .. 127 of a stage for wave row 0, the others for wave row 1
+            const int r = 2 * (j * NW + wave) + (lane >> 5);
+            const int f = (r & 3) | (((r >> 3) & 3) << 2);
+            const int col = ((lane & 31) ^ (f << 1)) * 8;
+            int m = (col & 127) < (col < 128 ? share0 : share1) ? tile_row + (col >> 7) * share0 + (col & 127) : count - 8;
+            m = m <= count - 8 ? m : count - 8;
+            ao[j] = (unsigned)(((int64_t)r * p.lda + m) * ES);
+            continue;
+        }
         // stage rows 0 .. 127 belong to wave row 0, the others to wave row 1; rows that nobody has repeat the last one
         const int r = (j * NW + wave) * 8 + drow;
         int m = (r & 127) < (r < 128 ? share0 : share1) ? tile_row + (r >> 7) * share0 + (r & 127) : count - 1;
@@ -1209,7 +1228,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    const int nk = K * ES / 128;
+    const int nk = AKM ? (K + 63) / 64 : K * ES / 128;
 
     // ---- fragment addresses: one register per k-step and operand; fragments and weight stages by offset
     const int frow = lane & 15;
@@ -1228,7 +1247,14 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     typedef short tr4_t __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) tr4_t* lds_tr_ptr_t;
     typedef __attribute__((address_space(3))) unsigned char* lds_u8_t;
-    lds_u8_t fb_tr[TN];
+    lds_u8_t fb_tr[TN], fa_tr[AKM ? TM : 1];
+    if constexpr (AKM) {      // fragment i of a wave's eight: column block 8 wm + i
+        const int t4 = frow >> 2;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+            fa_tr[i] = (lds_u8_t)smem + (8 * kgrp + t4) * 512 + 8 * (frow & 3) +
+                       (((((2 * wm + (i >> 2)) ^ kgrp) & 3) << 2) | ((i & 3) ^ t4)) * 32;
+    }
     if constexpr (BKM) {
         const int t4 = frow >> 2;
         const int base0 = B_BASE + (8 * kgrp + t4) * 512 + 8 * (frow & 3) + (((wn ^ kgrp) & 3) << 2) * 32;
@@ -1236,32 +1262,44 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
         for (int j = 0; j < TN; ++j) fb_tr[j] = (lds_u8_t)smem + base0 + ((j ^ t4) * 32);
     }
     const int b_slab = BKM ? (int)(p.ldb * 128) : 128;   // bytes from one slab of the weight operand to the next
+    const int a_slab = AKM ? (int)(p.lda * 128) : 128;
     constexpr int RB2 = BKM ? 4 : 2;   // read instructions of two weight fragments
+    constexpr int RA = AKM ? 2 : 1;    // read instructions of an activation fragment
     u32x4_t fa[2][4], fb[2][TN];
 
+// AKM: the advance along K is part of the lane offset, which the descriptor's end is checked against (the scalar offset is
+// not); otherwise it is the scalar offset.
+#define D16_LOAD(rsrc_, dst_, off_, adv_)                                                              \
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_, (lds_ptr_t)(dst_), 16, (off_) + (AKM ? (unsigned)(adv_) : 0u), \
+                                             AKM ? 0 : (adv_), 0, 0)
+#define D16_ISSUE_A1(kt_, aoff_, j_) D16_LOAD(rsrc_a, dma_a + (aoff_) + (j_) * NW * 1024, ao[j_], (kt_) * a_slab)
+#define D16_ISSUE_B1(kt_, boff_, j_) D16_LOAD(rsrc_b, dma_b + (boff_) + (j_) * NW * 1024, bo[j_], (kt_) * b_slab)
 #define D16_ISSUE_A(kt_, aoff_)                                                                        \
     {                                                                                                  \
-        const int soff = (kt_) * 128;                                                                  \
+        const int adv = (kt_) * a_slab;                                                                \
         _Pragma("unroll") for (int j = 0; j < NIA; ++j)                                                \
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                  \
-                rsrc_a, (lds_ptr_t)(dma_a + (aoff_) + j * NW * 1024), 16, ao[j], soff, 0, 0);          \
+            D16_LOAD(rsrc_a, dma_a + (aoff_) + j * NW * 1024, ao[j], adv);                             \
     }
-#define D16_ISSUE_A1(kt_, aoff_, j_)                                                                   \
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(dma_a + (aoff_) + (j_) * NW * 1024), 16, \
-                                             ao[j_], (kt_) * 128, 0, 0)
-#define D16_ISSUE_B1(kt_, boff_, j_)                                                                   \
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(dma_b + (boff_) + (j_) * NW * 1024), 16, \
-                                             bo[j_], (kt_) * b_slab, 0, 0)
 #define D16_ISSUE_B(kt_, boff_)                                                                        \
     {                                                                                                  \
-        const int soff = (kt_) * b_slab;                                                               \
+        const int adv = (kt_) * b_slab;                                                                \
         _Pragma("unroll") for (int j = 0; j < NIB; ++j)                                                \
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                  \
-                rsrc_b, (lds_ptr_t)(dma_b + (boff_) + j * NW * 1024), 16, bo[j], soff, 0, 0); \
+            D16_LOAD(rsrc_b, dma_b + (boff_) + j * NW * 1024, bo[j], adv);                             \
     }
 #define D16_B_ROW(j_) (SWIGLU ? ((j_) < TN / 2 ? (j_) * 16 : HALF + ((j_) - TN / 2) * 16) : (j_) * 16)
 #define D16_READ_A(aoff_, ks_, f0_, nf_, buf_)                                                         \
-    {                                                                                                  \
+    if constexpr (AKM) {                                                                               \
+        _Pragma("unroll") for (int i = 0; i < (nf_); ++i) {                                            \
+            union {                                                                                    \
+                tr4_t t[2];                                                                            \
+                u32x4_t u;                                                                             \
+            } cv_;                                                                                     \
+            const lds_u8_t pa_ = fa_tr[(AKM ? (f0_) + i : 0)] + (aoff_) + (ks_) * (32 * 512);          \
+            cv_.t[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr_t)(pa_));                   \
+            cv_.t[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr_t)(pa_ + 4 * 512));         \
+            fa[buf_][i] = cv_.u;                                                                       \
+        }                                                                                              \
+    } else {                                                                                                  \
         const unsigned char* fa_ = fa_addr[ks_] + (aoff_) + (f0_) * 2048;                              \
         _Pragma("unroll") for (int i = 0; i < (nf_); ++i)                                              \
             fa[buf_][i] = *reinterpret_cast<const u32x4_t*>(fa_ + i * 2048);                           \
@@ -1311,7 +1349,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
         __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);                            \
     }                                                                                   \
     _Pragma("unroll") for (int g_ = 0; g_ < (nf0_); ++g_) {                             \
-        __builtin_amdgcn_sched_group_barrier(SG_DS_RD, 1, 0);                           \
+        __builtin_amdgcn_sched_group_barrier(SG_DS_RD, RA, 0);                          \
         __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);                            \
     }                                                                                   \
     _Pragma("unroll") for (int g_ = 0; g_ < 4; ++g_) {                                  \
@@ -1341,7 +1379,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
             D16_READ_B(cb_, 1, 0, 1);                                                   \
             D16_READ_B(cb_, 1, 1, 1);                                                   \
             D16_MMA(0, 0, 0, N0);                                                       \
-            D16_MIX(N0, N1 + RB2, 1);                                                   \
+            D16_MIX(N0, N1 * RA + RB2, 1);                                                   \
         }                                                                               \
         PL_FENCE();                                                                     \
         D16_ISSUE_FAR(1);                                                                 \
@@ -1352,7 +1390,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
         }                                                                               \
         if (N1) {                                                                       \
             D16_MMA(0, 1, N0, N1);                                                      \
-            D16_MIX(N1, N0 + RB2, 1);                                                   \
+            D16_MIX(N1, N0 * RA + RB2, 1);                                                   \
         }                                                                               \
         PL_FENCE();                                                                     \
         D16_ISSUE_FAR(2);                                                                 \
@@ -1360,7 +1398,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
         if (N1) D16_READ_A(ca_, 1, N0, N1, 1);                                       \
         if (N0) {                                                                       \
             D16_MMA(1, 0, 0, N0);                                                       \
-            D16_MIX(N0, N1 ? N1 : 1, 2);                                                \
+            D16_MIX(N0, N1 ? N1 * RA : 1, 2);                                                \
         }                                                                               \
         PL_FENCE();                                                                     \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NIA) : "memory"); \
@@ -1400,7 +1438,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     D16_ISSUE_B(0, 0);
     D16_ISSUE_B(min(1, nk - 1), B_STAGE);
 #pragma unroll
-    for (int j = 0; j < NIA; ++j) {
+    for (int j = 0; j < NIA && !AKM; ++j) {
         const int64_t src = gather ? (int64_t)(a_idx[j] / p.a_row_div) : (int64_t)a_idx[j];
         ao[j] = (unsigned)(src * p.lda * ES + dchunk * 16);
     }
@@ -1433,6 +1471,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     // the clamped loads of the last slabs may still be in flight; the epilogue reuses LDS
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #undef D16_LOOP
+#undef D16_LOAD
 #undef D16_ISSUE_A
 #undef D16_ISSUE_A1
 #undef D16_ISSUE_B
@@ -1470,7 +1509,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 }
 
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
-          bool MIDROWS = false, bool SLICED = false>
+          bool MIDROWS = false, bool SLICED = false, bool AKM = false>
 __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) {
     // The body is a function of its own for one reason: a __restrict__ parameter that it reads through gives every
     // other memory access in it (the transposing LDS reads among them) "does not alias that parameter" metadata once
@@ -1479,7 +1518,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
     // the K-major variant is preceded by s_waitcnt vmcnt(0), i.e. waits for all of the slab loads just issued (the
     // plain 16-byte fragment reads carry type-based alias metadata and never had that wait): 27-37 % slower.
     extern __shared__ __align__(16) unsigned char smem_k[];
-    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS, SLICED>(p, smem_k, p.row_count);
+    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS, SLICED, AKM>(p, smem_k, p.row_count);
 }
 
 #undef PL_STORE
@@ -1867,6 +1906,32 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
     return ATS_OK;
 }
 
+// Weight gradient of a linear layer, out[m, n] = sum_t a[t, m] b[t, n]: tiles and slices as launch_cfg takes them for the
+// product of transposed copies.
+template <typename TO, bool SLICED>
+static int launch_tn(const GroupedArgs& p0, int64_t rows, hipStream_t s) {
+    GroupedArgs p = p0;
+    p.n_tiles = (p.N_out + 255) / 256;
+    constexpr size_t smem = dma_lds_bytes(256, 256);
+    auto kern = grouped_gemm_dma16_kernel<TO, 4, 8, false, false, false, true, true, SLICED, true>;
+    static LdsReservation reserved;
+    hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern)}, (int)smem);
+    if (e != hipSuccess) {
+        set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
+        return ATS_ERR_LAUNCH;
+    }
+    pick_supertile(p.n_tiles, &p.sm, &p.sn);
+    p.aligned_bands = 0;
+    p.tile_rows = SLICED ? 0 : dense_tile_rows(rows, p.n_tiles, (p.K + 63) / 64, p.sm, p.sn);
+    const int64_t blocks = grid_blocks(rows * p.k_splits, p.k_splits, p.tile_rows ? p.tile_rows : 256, p.n_tiles, p.sm, p.sn, false);
+    if (blocks > 0x7fffffffLL) {
+        set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
+        return ATS_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(512), smem, s, p);
+    return ATS_OK;
+}
+
 // Bytes reachable from a buffer descriptor, or 0 when they do not fit its 32-bit range.
 static uint32_t extent32(int64_t rows, int64_t row_elems, int elem_size) {
     if (rows <= 0 || rows > (int64_t)0xffffffffLL / (row_elems * elem_size)) return 0;
@@ -2183,6 +2248,48 @@ extern "C" int ats_grouped_gemm_nn_sliced(const void* a, int64_t lda, const void
     const int rc = k_splits > 1 ? launch_mid_sliced<true>(p, max_rows, s)
                    : out_dtype == ATS_F32 ? launch_kmajor<float, false>(p, max_rows, s)
                                           : launch_kmajor<bf16_t, false>(p, max_rows, s);
+    if (rc != ATS_OK) return rc;
+    ATS_CHECK_LAUNCH(name);
+    return ATS_OK;
+}
+
+extern "C" int ats_wgrad_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void* out, int64_t T, int M, int N,
+                            int slab_slices, const int32_t* row_start, const int32_t* row_count, int dtype, int out_dtype,
+                            ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_wgrad_tn";
+    ATS_REQUIRE(T > 0 && T <= 0x7fffffc0 && M > 0 && N > 0 && lda >= M && ldb >= N && slab_slices >= 1 && slab_slices <= 64,
+                ATS_ERR_INVALID_ARG, "%s: T=%lld M=%d N=%d lda=%lld ldb=%lld slices=%d", name, (long long)T, M, N, (long long)lda,
+                (long long)ldb, slab_slices);
+    ATS_REQUIRE(dtype == ATS_BF16 && (slab_slices > 1 ? out_dtype == ATS_F32 : out_dtype == ATS_BF16), ATS_ERR_UNSUPPORTED,
+                "%s: dtype tags %d -> %d (bfloat16 operands; bfloat16 out, float32 with slices)", name, dtype, out_dtype);
+    ATS_REQUIRE(a && b && out && row_start && row_count, ATS_ERR_INVALID_ARG, "%s: null pointer", name);
+    // (offsets of a whole last slab have to fit 32 bits: a wrapped one would not be seen as lying past the end)
+    const int64_t padded = (T + 63) / 64 * 64;
+    ATS_REQUIRE(M % 8 == 0 && N % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned16(a) && aligned16(b) && aligned16(out) &&
+                    extent32_ok(padded, lda, 2) && extent32_ok(padded, ldb, 2),
+                ATS_ERR_UNSUPPORTED, "%s: M=%d N=%d lda=%lld ldb=%lld must describe 16-byte aligned rows within 4 GiB", name, M,
+                N, (long long)lda, (long long)ldb);
+    GroupedArgs p{};
+    p.a = a;
+    p.a_row_div = 1;
+    p.lda = lda;
+    p.b = static_cast<const void* const*>(b);
+    p.ldb = ldb;
+    p.out = out;
+    p.ldo = N;
+    p.row_start = row_start;
+    p.row_count = row_count;
+    p.E = 1;
+    p.K = (int)T;
+    p.N_out = N;
+    const int64_t slabs = padded / 64, per = (slabs + slab_slices - 1) / slab_slices;
+    p.k_splits = (int)((slabs + per - 1) / per);
+    ATS_REQUIRE(p.k_splits == slab_slices, ATS_ERR_INVALID_ARG, "%s: %lld slabs do not make %d slices", name, (long long)slabs, slab_slices);
+    p.k_slice = (int)per * 64;
+    p.part_stride = (int64_t)M * N;
+    hipStream_t s = as_stream(stream);
+    const int rc = slab_slices > 1 ? launch_tn<float, true>(p, M, s) : launch_tn<bf16_t, false>(p, M, s);
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;

@@ -400,11 +400,39 @@ def wgrad_dense(lhsT: torch.Tensor, rhsT: torch.Tensor, rows: int, heights: Opti
     parts = grouped_gemm_nt(buf[slices:2 * slices], ld, N, r32[:slices], r32[slices:2 * slices], slices * M, slices * M, N, ld,
                             a_ptrs=buf[:slices], lda=ld, k_count=r32[2 * slices:3 * slices], dtype=dtype,
                             out_dtype=dtype if slices == 1 else torch.float32)
+    return _wgrad_result(parts, slices, M, N, dtype, heights)
+
+
+def _wgrad_result(parts: torch.Tensor, slices: int, M: int, N: int, dtype: torch.dtype, heights: Optional[Sequence[int]]):
     if heights is None:
         return parts if slices == 1 else sum_partials(parts.view(slices, M * N), dtype).view(M, N)
     if slices == 1:
         return [part.clone() for part in parts.split(list(heights))]
     return [sum_partials(part, dtype) for part in parts.view(slices, M, N).split(list(heights), dim=1)]
+
+
+def wgrad_linear_supported(dy: torch.Tensor, x: torch.Tensor) -> bool:
+    """Whether wgrad_linear takes these operands: bfloat16, 16-byte aligned rows within 4 GiB."""
+    return dy.dtype == torch.bfloat16 and x.dtype == dy.dtype and all(
+        t.dim() == 2 and t.shape[0] > 0 and t.shape[1] > 0 and t.shape[1] % 8 == 0 and t.stride(1) == 1
+        and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+        and (t.shape[0] + 63) * t.stride(0) * 2 < 1 << 32 for t in (dy, x))
+
+
+def wgrad_linear(dy: torch.Tensor, x: torch.Tensor, heights: Optional[Sequence[int]] = None):
+    """dy^T @ x for dy [T, M] and x [T, N] with rows of any stride, as they lie: the weight gradient of a linear layer; the
+    bits of wgrad_dense on transposed copies, and its heights."""
+    _need_gpu(dy, x)
+    if not wgrad_linear_supported(dy, x) or dy.shape[0] != x.shape[0]:
+        raise AtsError("wgrad_linear: bfloat16 [T, M], [T, N] of 16-byte aligned rows within 4 GiB")
+    (T, M), N, dtype = dy.shape, x.shape[1], dy.dtype
+    slabs = -(-T // 64)
+    slices = -(-slabs // -(-slabs // wgrad_slices(M, N, T)))
+    start, count = _single_group(M, x.device)
+    parts = torch.empty(slices * M, N, dtype=dtype if slices == 1 else torch.float32, device=x.device)
+    check(_lib.load().ats_wgrad_tn(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), parts.data_ptr(), T, M, N, slices,
+                                   start.data_ptr(), count.data_ptr(), _DT[dtype], _DT[parts.dtype], _stream()), "ats_wgrad_tn")
+    return _wgrad_result(parts, slices, M, N, dtype, heights)
 
 
 def wgrad_tables(k_start: torch.Tensor, M: int, lhsT: torch.Tensor, rhsT: torch.Tensor) -> list:

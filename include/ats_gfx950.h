@@ -463,7 +463,15 @@ int ats_grouped_gemm_nn(const void* a, int64_t lda, int64_t a_num_rows, const in
                         const void* const* b_ptrs, int64_t ldb, void* out, int64_t ldo, const int32_t* row_start,
                         const int32_t* row_count, int E, int64_t max_rows, int N, int K, int dtype, int out_dtype,
                         ats_stream_t stream);
-/* The same product for groups of up to 256 rows on average, K cut into k_splits equal slices of whole 64-element
+/* Weight gradient of a linear layer from operands as they lie: out[m, n] = sum_t a[t, m] * b[t, n], a [T, lda >= M] and
+ * b [T, ldb >= N] bfloat16 with 16-byte aligned rows (autograd's weight gradient of nn.Linear).  slab_slices = 1: out [M, N]
+ * bfloat16; more: float32 partial results [slab_slices][M][N] over equal runs of 64-row slabs (the last one may be shorter,
+ * none empty).  row_start / row_count: device integers 0 and M.  Any T; same bits as ats_grouped_gemm_nt on transposed,
+ * zero-padded copies. */
+int ats_wgrad_tn(const void* a, int64_t lda, const void* b, int64_t ldb, void* out, int64_t T, int M, int N, int slab_slices,
+                 const int32_t* row_start, const int32_t* row_count, int dtype, int out_dtype, ats_stream_t stream);
+
+/* ats_grouped_gemm_nn for groups of up to 256 rows on average, K cut into k_splits equal slices of whole 64-element
  * slabs: float32 partial results [k_splits][part_rows][N] that ats_sum_partials or ats_combine_partials add, or with
  * k_splits = 1 the product itself, [part_rows][N] of out_dtype.  ..._slices: the number of slices to use; 1 also for
  * larger groups, which are ats_grouped_gemm_nn's; 0: transpose and call ats_grouped_gemm_nt. */
