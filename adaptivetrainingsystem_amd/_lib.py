@@ -6,7 +6,9 @@ call fails, an exception is raised.  There is no PyTorch or CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
+import threading
 from ctypes import c_char_p, c_double, c_float, c_int, c_int64, c_uint64, c_size_t, c_void_p
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libats_gfx950.so")
@@ -194,6 +196,32 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+_native = None
+_native_lock = threading.Lock()
+
+
+def native():
+    """The compiled host side of the shortest calls (csrc/torch_binding.cpp); loaded once, raises if it has not been built.
+    Its functions return None for calls that the general path is to take."""
+    global _native
+    if _native is not None:
+        return _native
+    with _native_lock:
+        if _native is not None:
+            return _native
+        load()
+        import torch  # noqa: F401  (its libraries come first)
+        path = os.path.join(os.path.dirname(LIB_PATH), "_ats_torch.so")
+        if not os.path.exists(path):
+            raise AtsError(f"{path} is missing: build it with `python -m adaptivetrainingsystem_amd.build`")
+        spec = importlib.util.spec_from_file_location("_ats_torch", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.set_error(AtsError)
+        _native = module
+    return _native
 
 
 def last_error() -> str:

@@ -1,4 +1,5 @@
-"""Builds libats_gfx950.so (hand-written HIP kernels + C ABI) with hipcc for gfx950.
+"""Builds libats_gfx950.so (hand-written HIP kernels + C ABI) with hipcc for gfx950, and _ats_torch.so (the host side of
+its shortest calls) with the C++ compiler.
 
 The library is built in-tree (adaptivetrainingsystem_amd/lib/) so that it travels
 with the source tree; nothing is compiled at import time.
@@ -16,6 +17,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(PKG_DIR, "csrc")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libats_gfx950.so")
+BINDING_PATH = os.path.join(LIB_DIR, "_ats_torch.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -35,6 +37,25 @@ def sources():
     return sorted(glob.glob(os.path.join(CSRC_DIR, "*.hip")))
 
 
+def _compile_binding(obj: str):
+    """Starts the compilation of the host side of the short calls (csrc/torch_binding.cpp), plain C++ against torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no C++ compiler found (set CXX)")
+    # (the first two are what the HIP headers ask of a compiler that is not hipcc)
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           "-DTORCH_EXTENSION_NAME=_ats_torch", *("-I" + d for d in include_paths(device_type="cuda")),
+           "-I" + sysconfig.get_paths()["include"], "-c", os.path.join(CSRC_DIR, "torch_binding.cpp"), "-o", obj]
+    link = [cxx, "-shared", obj, "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch", "-ltorch_python", "-L" + LIB_DIR, "-l:libats_gfx950.so", "-Wl,-rpath,$ORIGIN"]
+    return cmd, link
+
+
 def build_library(verbose: bool = True, jobs: int = 6) -> str:
     """Compiles every .hip source to an object (in parallel) and links the shared library."""
     hipcc = find_hipcc()
@@ -43,6 +64,9 @@ def build_library(verbose: bool = True, jobs: int = 6) -> str:
     os.makedirs(obj_dir, exist_ok=True)
     compile_flags = [f for f in HIPCC_FLAGS if f != "-shared"]
     procs, objs = [], []
+    binding_obj = os.path.join(obj_dir, "torch_binding.o")
+    binding_cmd, binding_link = _compile_binding(binding_obj)
+    procs.append(("torch_binding.cpp", subprocess.Popen(binding_cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     for src in sources():
         obj = os.path.join(obj_dir, os.path.basename(src)[:-4] + ".o")
         objs.append(obj)
@@ -72,6 +96,9 @@ def build_library(verbose: bool = True, jobs: int = 6) -> str:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
     os.replace(tmp, LIB_PATH)
+    tmp = BINDING_PATH + ".tmp"
+    subprocess.check_call([*binding_link, "-o", tmp])
+    os.replace(tmp, BINDING_PATH)
     return LIB_PATH
 
 

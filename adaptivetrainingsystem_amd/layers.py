@@ -37,7 +37,7 @@ import torch.nn as nn
 from . import autograd as ag
 from . import ops
 from .profiling import stage, timer_context
-from ._lib import ROUTE_SOFTMAX_TOPK, ROUTE_TOPK_SOFTMAX, AtsError
+from ._lib import ROUTE_SOFTMAX_TOPK, ROUTE_TOPK_SOFTMAX, AtsError, native
 
 
 # float16 activations: the gfx950 kernels take float32 and bfloat16.  The reference's fused wrappers convert
@@ -77,6 +77,9 @@ class RMSNorm(nn.Module):
         if x.shape[-1] != self.dim:
             raise AtsError(f"RMSNorm: last dimension {x.shape[-1]} != {self.dim}")
         w = self.weight if self.elementwise_affine else None
+        y = native().rmsnorm(x, w, self.eps)
+        if y is not None:
+            return y
         if _is_f16(x, w):
             xf, wf = _f32(x), _f32(w)
             y = ag.RMSNormFunction.apply(xf, wf, self.eps) if _wants_grad(xf, wf) else ops.rmsnorm(xf, wf, self.eps)
@@ -106,6 +109,9 @@ class FusedRMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.float32_output and x.dtype != torch.float32:
             x = x.float()
+        y = native().rmsnorm(x, self.weight, self.eps)
+        if y is not None:
+            return y
         if _is_f16(x, self.weight):
             xf, wf = _f32(x), _f32(self.weight)
             y = ag.RMSNormFunction.apply(xf, wf, self.eps) if _wants_grad(xf, wf) else ops.rmsnorm(xf, wf, self.eps)
@@ -163,6 +169,10 @@ class RotaryEmbedding(nn.Module):
 def apply_rotary_pos_emb(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
                          sin: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """q [B,Hq,L,D], k [B,Hkv,L,D], cos/sin [L, D] -> rotated (q, k) in the input dtype."""
+    if k is not None:
+        r = native().rope(q, k, cos, sin, 0)
+        if r is not None:
+            return r
     if _is_f16(q, k):
         qo, ko = apply_rotary_pos_emb(_f32(q), _f32(k), cos, sin)
         return qo.to(q.dtype), ko.to(k.dtype)
@@ -187,6 +197,10 @@ class FusedRoPE(nn.Module):
         if self.cos_cache.device != q.device:
             self.cos_cache = self.cos_cache.to(q.device)
             self.sin_cache = self.sin_cache.to(q.device)
+        if k is not None:
+            r = native().rope(q, k, self.cos_cache, self.sin_cache, position_offset)
+            if r is not None:
+                return r
         if _is_f16(q, k):
             qo, ko = self.forward(_f32(q), _f32(k), position_offset)
             return qo.to(q.dtype), ko.to(k.dtype)

@@ -157,6 +157,9 @@ def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Te
     """rope(q, k) with the rotated keys, and the values beside them, written into the cache buffers
     k_cache / v_cache [B, Hkv, capacity, D] at positions cache_pos .. cache_pos + L - 1 (one launch instead of the
     rotation and two strided copies).  Returns the rotated q as a new contiguous tensor."""
+    done = _lib.native().rope_append(q, k, v, cos, sin, k_cache, v_cache, cache_pos, position_offset)
+    if done is not None:
+        return done
     _need_gpu(q, k, v, cos, sin, k_cache, v_cache)
     if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape or k_cache.dim() != 4 or v_cache.shape != k_cache.shape:
         raise AtsError("rope_append: q, k, v [batch, heads, seq, head_dim] and two caches of one shape")
@@ -1225,6 +1228,10 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: O
     key); causal_attention_bwd given the same seed sees the same mask.
     split_keys=False keeps the single-pass kernel where few rows against many keys would otherwise be cut
     into key ranges.  Returns out [B, L, Hq*D] (and lse [B,Hq,L] float32 if asked)."""
+    if not return_lse and key_bias is None and pair_bias is None and dropout_p == 0.0:
+        done = _lib.native().attention(q, k, v, q.shape[-1] ** -0.5 if scale is None else scale, split_keys)
+        if done is not None:
+            return done
     _need_gpu(q, k, v)
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or q.dtype != torch.bfloat16 or k.dtype != q.dtype or v.dtype != q.dtype:
         raise AtsError("causal_attention: q, k, v must be 4-D bfloat16 tensors [batch, heads, seq, head_dim]")
@@ -1502,6 +1509,9 @@ def linear_nt(x: torch.Tensor, weight: torch.Tensor, table: Optional[torch.Tenso
     # ([4096, 4096] x 16 rows: 10.3 us against 14.2 with the slices and their sum), and a short K leaves its small tiles
     # less to do than the sum costs ([2048, 2048] x 64 rows: 8.8 against 11.3).
     splits = down_k_splits(1, T, N, K, x.dtype) if T > 32 and K * x.element_size() > 4096 and K % 8 == 0 and N % 8 == 0 else 1
+    done = _lib.native().linear(x, table, start, count, N, splits)
+    if done is not None:
+        return done
     if splits > 1:      # a few rows against a whole weight matrix: slices of K keep every CU streaming
         return sum_partials(grouped_down_splitk(x, table, start, count, T, N, K, splits), x.dtype)
     return grouped_gemm_nt(table, K, N, start, count, T, T, N, K, a=x)
