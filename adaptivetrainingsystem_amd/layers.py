@@ -290,7 +290,13 @@ class GroupedQueryAttention(nn.Module):
             # the rotation writes the new keys, and the values beside them, straight behind the cache
             q, k, v = self._extend_cache(k_cache, v_cache, q, k, v, cos, sin)
         else:
-            if not grad:
+            if not grad and use_cache and past_key_value is None:
+                # the cache of a prompt: one launch rotates q and k and lays the values beside the keys (3 x 1777 tokens 525 ->
+                # 517 us, 80 tokens 54 -> 42)
+                k_new, v_new = (torch.empty(B, nkv, L, D, dtype=x.dtype, device=x.device) for _ in range(2))
+                q = ops.rope_append(q, k, v, cos, sin, k_new, v_new, 0, 0)
+                k, v = k_new, v_new
+            elif not grad:
                 q, k = ops.rope(q, k, cos, sin, 0)
             if past_key_value is not None:
                 k = torch.cat([k_cache.to(k.dtype), k], dim=2)
