@@ -63,6 +63,12 @@ _SIGNATURES = {
     "ats_grouped_gemm_nn_supported": (c_int, [c_int, c_int64, c_int, c_int, c_int64, c_int]),
     "ats_grouped_gemm_nn": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int, c_void_p, c_int64, c_void_p, c_int64,
                                     c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_void_p]),
+    "ats_grouped_gemm_nn_f32_supported": (c_int, [c_int, c_int64, c_int, c_int]),
+    "ats_grouped_gemm_nn_f32": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int64,
+                                        c_int, c_int, c_void_p]),
+    "ats_grouped_wgrad_f32_supported": (c_int, [c_int, c_int64, c_int, c_int]),
+    "ats_grouped_wgrad_f32": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
+                                      c_int64, c_int, c_int, c_void_p]),
     "ats_wgrad_tn": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_void_p,
                              c_int, c_int, c_void_p]),
     "ats_grouped_gemm_nn_slices": (c_int, [c_int, c_int64, c_int, c_int, c_int64, c_int]),

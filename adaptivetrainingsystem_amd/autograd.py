@@ -170,12 +170,16 @@ class LinearFunction(Function):
         if ctx.needs_input_grad[0]:
             if DGRAD_FROM_FORWARD_WEIGHTS and ops.grouped_gemm_nn_supported(1, T, K, N, K, x.dtype):
                 dx = ops.grouped_gemm_nn(ops.weight_pointer_table([w]), K, offsets, kept, T, T, K, N, dy)
+            elif DGRAD_FROM_FORWARD_WEIGHTS and x.dtype == torch.float32 and ops.grouped_gemm_nn_f32_supported(1, T, K, N):
+                dx = ops.grouped_gemm_nn_f32(ops.weight_pointer_table([w]), K, offsets, kept, T, K, N, dy)
             else:
                 wT, tab = ops.transpose_batched([w])             # [K, N]; kept alive until the GEMM is queued
                 dx = ops.grouped_gemm_nt(tab, N, K, offsets, kept, T, T, K, N, a=dy)
         if ctx.needs_input_grad[1]:
             if ops.wgrad_linear_supported(dy, x):
                 dw = ops.wgrad_linear(dy, x).to(ctx.param_dtype)
+            elif ops.wgrad_f32_supported(dy, x):
+                dw = ops.wgrad_f32(dy, x).to(ctx.param_dtype)
             else:
                 dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
                 xT = ops.transpose_grouped_rows(x, offsets, kept, T)
@@ -222,6 +226,8 @@ class QKVRoPEFunction(Function):
             tab = ops.address_table(w)
             if DGRAD_FROM_FORWARD_WEIGHTS and ops.grouped_gemm_nn_supported(1, T, K, N, K, x.dtype):
                 dx = ops.grouped_gemm_nn(tab, K, offsets, kept, T, T, K, N, dy)
+            elif DGRAD_FROM_FORWARD_WEIGHTS and x.dtype == torch.float32 and ops.grouped_gemm_nn_f32_supported(1, T, K, N):
+                dx = ops.grouped_gemm_nn_f32(tab, K, offsets, kept, T, K, N, dy)
             else:
                 wT, tab = ops.transpose_batched([w], tab)        # [K, N]; kept alive until the GEMM is queued
                 dx = ops.grouped_gemm_nt(tab, N, K, offsets, kept, T, T, K, N, a=dy)
@@ -229,6 +235,11 @@ class QKVRoPEFunction(Function):
             nq, nk = nh * D, nkv * D
             if ops.wgrad_linear_supported(dy, x) and nk % 8 == 0:
                 wgrad = lambda lo, hi, heights=None: ops.wgrad_linear(dy[:, lo:hi], x, heights)
+            elif ops.wgrad_f32_supported(dy[:, :nk], x) and ops.wgrad_f32_supported(dy[:, :nq], x):
+                def wgrad(lo, hi, heights=None):
+                    if heights is None:
+                        return ops.wgrad_f32(dy[:, lo:hi], x)
+                    return [ops.wgrad_f32(dy[:, lo + i * nk:lo + (i + 1) * nk], x) for i in range(2)]
             else:
                 dyT = ops.transpose_grouped_rows(dy, offsets, kept, T)
                 xT = ops.transpose_grouped_rows(x, offsets, kept, T)
@@ -283,12 +294,12 @@ def _fused_grid(dtype, E, rows, n):
 
 def _ffn_forward(x, wgu, wd, offsets, kept, rows, row_src, k, want_wgrad=False):
     """Expert FFN over the grouped rows, keeping the gate/up pre-activations for the backward pass.
-    Returns (gu [rows, 2I], h [rows, I], y [rows, H], hT, wplan): with want_wgrad, wplan = the weight-gradient
+    Returns (gu [rows, 2I], h [rows, I], y [rows, H], hT, wplan): with want_wgrad, in bfloat16, wplan = the weight-gradient
     layout of these groups (ops.wgrad_plan) and, where the fused bfloat16 kernel runs, hT = h already transposed
     into it by that kernel (the backward pass then keeps hT instead of h); otherwise None."""
     H, I = x.shape[1], wd[0].shape[1]
     tab_gu, tab_d = ops.weight_pointer_table(wgu), ops.weight_pointer_table(wd)
-    wplan = ops.wgrad_plan(kept) if want_wgrad and rows > 0 else None
+    wplan = ops.wgrad_plan(kept) if want_wgrad and rows > 0 and x.dtype != torch.float32 else None
     hT = None
     both = None
     if _fused_grid(x.dtype, len(wd), rows, 2 * I):
@@ -319,13 +330,16 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
     E = len(wd)
     H, I = x.shape[1], wd[0].shape[1]
     dtype = x.dtype
-    if need_w and wplan is None:
+    f32_rows = need_w and h is not None and ops.wgrad_f32_supported(dy, h, E) and ops.wgrad_f32_supported(gu, x, E)
+    if need_w and wplan is None and not f32_rows:
         wplan = ops.wgrad_plan(kept)
     dguT = None
 
     def from_forward_weights(ws, N, K, grad):
         """grad [rows, K] against the forward's own [K, N] weights: [rows, N], float32 [slices, rows, N] where K is cut, or
         None where a transposed copy of the weights is the better way."""
+        if DGRAD_FROM_FORWARD_WEIGHTS and dtype == torch.float32 and ops.grouped_gemm_nn_f32_supported(E, rows, N, K):
+            return ops.grouped_gemm_nn_f32(ops.weight_pointer_table(list(ws)), N, offsets, kept, rows, N, K, grad)
         slices = ops.grouped_gemm_nn_slices(E, rows, N, K, N, dtype) if DGRAD_FROM_FORWARD_WEIGHTS else 0
         if slices == 0:
             return None
@@ -335,7 +349,7 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
         return ops.grouped_gemm_nn_sliced(tab, N, offsets, kept, rows, rows, N, K, grad, slices)
 
     dh = None
-    t_col0 = wplan[0] if need_w and FUSE_TRANSPOSED_COPIES else None
+    t_col0 = wplan[0] if wplan is not None and need_w and FUSE_TRANSPOSED_COPIES else None
     if DGRAD_FROM_FORWARD_WEIGHTS and ops.grouped_down_dgrad_dsilu_supported(E, rows, H, I, dtype, transposed_weights=False):
         # prefill-sized bfloat16 groups: one kernel, reading the down weights as the forward holds them
         pair = ops.grouped_down_dgrad_dsilu(dy, ops.weight_pointer_table(list(wd)), gu, offsets, kept, rows, H, I,
@@ -363,7 +377,10 @@ def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x
         if dx_rows is None:
             wguT, tab_guT = ops.transpose_batched(wgu)           # [H, 2I] per expert
             dx_rows = ops.grouped_gemm_nt(tab_guT, 2 * I, H, offsets, kept, rows, rows, H, 2 * I, a=dgu)
-    if need_w:
+    if f32_rows:
+        dwd = ops.wgrad_f32(dy, h, offsets, kept)
+        dwgu = ops.wgrad_f32(dgu, x, offsets, kept, b_rows=row_src, b_row_div=k)
+    elif need_w:
         ks, kc = wplan
         ld = ops.wgrad_padded_rows(rows, E)
 

@@ -77,6 +77,11 @@ struct GroupedArgs {
     int64_t ld_t;
     const int32_t* t_col0;
     int tile_rows;          // MIDROWS instance: most rows of a tile (0: the tile's own height)
+    // float32 products with both operands K-major: output rows of every group, first row of K per group (null: 0), optional
+    // gather of the second operand's rows; p.b is that operand itself
+    int uniform_rows, b_row_div;
+    const int32_t* k_start;
+    const int32_t* b_rows;
 };
 
 constexpr int kRowPitch = 144;  // bytes per staged row: 128 data + 16 pad
@@ -1906,6 +1911,31 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
     return ATS_OK;
 }
 
+// Float32 products against K-major operands on the small tiles, in microseconds, and what a transposing pass costs.  The
+// tiles' constants are those of launch_grouped, a tenth more per slab for the 4-byte fragment reads (and less per tile for
+// short sums, of which several share a CU).  Copies and their product -> operands as they lie:
+//   weight gradients, rows x [M, N]: 512 x [512, 512] 47 -> 8; 2000 x [512, 512] 75 -> 22; 2048 x [2048, 2048] 225 -> 185;
+//     2048 x [4096, 4096] 503 (650); 8 x 128 x [2816, 512] 63 -> 46; 8 x 500 x [2816, 512] 153 -> 132; 8 x 500 x [4096, 1024] 299 (355)
+//   data gradients, rows x [N, K]: 512 x [512, 1024] 41 -> 11; 2000 x [512, 1024] 41 -> 29; 2048 x [2048, 2048] 209 -> 159;
+//     4096 x [4096, 4096] 961 (1196); 8 x 128 x [512, 2816] 56 -> 37; 8 x 250 x [1408, 512] 61 -> 46
+static float small_kmajor_time(int64_t max_rows, int E, int N, int K, bool* wide) {
+    const int nk = (K + 31) / 32;
+    const float t32 = tile_time(TileCost{32, 32, 0.20f, 1.5f, 1}, max_rows, E, N, nk);
+    const float t64 = tile_time(TileCost{64, 64, 0.64f, 1.6f, 1}, max_rows, E, N, nk);
+    *wide = t64 < t32;
+    return *wide ? t64 : t32;
+}
+// The product of copies: their passes at 4 TB/s and 4 us each, then the least of the tiles that launch_grouped has for it.
+static float transposed_time(int64_t max_rows, int E, int N, int K, int64_t copied, int copies) {
+    const int nk = (K + 31) / 32;
+    float best = tile_time(TileCost{256, 256, 7.3f, 25.f, 1}, max_rows, E, N, nk);      // (62 us for five slabs)
+    for (const TileCost& c : {TileCost{128, 256, 3.65f, 5.f, 1}, TileCost{64, 64, 0.58f, 3.f, 1}, TileCost{32, 32, 0.18f, 1.5f, 1}}) {
+        const float t = tile_time(c, max_rows, E, N, nk);
+        if (t < best) best = t;
+    }
+    return best + (float)copied * 8.f / 4e6f + 4.f * copies;
+}
+
 // Weight gradient of a linear layer, out[m, n] = sum_t a[t, m] b[t, n]: tiles and slices as launch_cfg takes them for the
 // product of transposed copies.
 template <typename TO, bool SLICED>
@@ -2248,6 +2278,92 @@ extern "C" int ats_grouped_gemm_nn_sliced(const void* a, int64_t lda, const void
     const int rc = k_splits > 1 ? launch_mid_sliced<true>(p, max_rows, s)
                    : out_dtype == ATS_F32 ? launch_kmajor<float, false>(p, max_rows, s)
                                           : launch_kmajor<bf16_t, false>(p, max_rows, s);
+    if (rc != ATS_OK) return rc;
+    ATS_CHECK_LAUNCH(name);
+    return ATS_OK;
+}
+
+extern "C" int ats_grouped_gemm_nn_f32_supported(int E, int64_t max_rows, int N, int K) {
+    using namespace ats;
+    bool wide;
+    if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || N % 4 != 0 || K % 4 != 0) return 0;
+    return small_kmajor_time(max_rows, E, N, K, &wide) <= transposed_time(max_rows, E, N, K, (int64_t)E * N * K, 1) ? 1 : 0;
+}
+extern "C" int ats_grouped_gemm_nn_f32(const float* a, int64_t lda, const void* const* b_ptrs, int64_t ldb, float* out, int64_t ldo,
+                                       const int32_t* row_start, const int32_t* row_count, int E, int64_t max_rows, int N, int K,
+                                       ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_grouped_gemm_nn_f32";
+    ATS_REQUIRE(E > 0 && E <= 4096 && max_rows >= 0 && N > 0 && K > 0, ATS_ERR_INVALID_ARG, "%s: E=%d max_rows=%lld N=%d K=%d",
+                name, E, (long long)max_rows, N, K);
+    ATS_REQUIRE(a && b_ptrs && out && row_start && row_count && aligned16(a) && aligned16(out), ATS_ERR_INVALID_ARG,
+                "%s: null or misaligned pointer", name);
+    ATS_REQUIRE(N % 4 == 0 && K % 4 == 0 && lda % 4 == 0 && lda >= K && ldb % 4 == 0 && ldb >= N && ldo % 4 == 0 && ldo >= N,
+                ATS_ERR_UNSUPPORTED, "%s: N=%d K=%d lda=%lld ldb=%lld ldo=%lld must describe 16-byte aligned rows", name, N, K,
+                (long long)lda, (long long)ldb, (long long)ldo);
+    if (max_rows == 0) return ATS_OK;
+    GroupedArgs p{};
+    p.a = a;
+    p.a_row_div = 1;
+    p.lda = lda;
+    p.b = b_ptrs;
+    p.ldb = ldb;
+    p.out = out;
+    p.ldo = ldo;
+    p.row_start = row_start;
+    p.row_count = row_count;
+    p.E = E;
+    p.K = K;
+    p.N_out = N;
+    bool wide;
+    small_kmajor_time(max_rows, E, N, K, &wide);
+    const int rc = wide ? launch_small<float, float, 2, 2, 4, 1, false, false, true>(p, max_rows, as_stream(stream))
+                        : launch_small<float, float, 1, 1, 4, 1, false, false, true>(p, max_rows, as_stream(stream));
+    if (rc != ATS_OK) return rc;
+    ATS_CHECK_LAUNCH(name);
+    return ATS_OK;
+}
+
+// (max_k: bound on the sum over the groups)
+extern "C" int ats_grouped_wgrad_f32_supported(int E, int64_t max_k, int M, int N) {
+    using namespace ats;
+    bool wide;
+    if (E <= 0 || max_k <= 0 || max_k > 0x7fffffff || M <= 0 || N <= 0 || M % 4 != 0 || N % 4 != 0) return 0;
+    const int k = (int)((max_k + E - 1) / E);
+    return small_kmajor_time((int64_t)E * M, E, N, k, &wide) <=
+                   transposed_time((int64_t)E * M, E, N, k + 16, max_k * ((int64_t)M + N), 2) ? 1 : 0;
+}
+extern "C" int ats_grouped_wgrad_f32(const float* a, int64_t lda, const float* b, int64_t ldb, const int32_t* b_rows, int b_row_div,
+                                     float* out, const int32_t* k_start, const int32_t* k_count, int E, int64_t max_k, int M, int N,
+                                     ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_grouped_wgrad_f32";
+    ATS_REQUIRE(E > 0 && E <= 4096 && max_k >= 0 && max_k <= 0x7fffffff && M > 0 && N > 0 && (E == 1 || (k_start && k_count)),
+                ATS_ERR_INVALID_ARG, "%s: E=%d max_k=%lld M=%d N=%d", name, E, (long long)max_k, M, N);
+    ATS_REQUIRE(a && b && out && aligned16(a) && aligned16(b) && aligned16(out) && (!b_rows || b_row_div > 0), ATS_ERR_INVALID_ARG,
+                "%s: null or misaligned pointer", name);
+    ATS_REQUIRE(M % 4 == 0 && N % 4 == 0 && lda % 4 == 0 && lda >= M && ldb % 4 == 0 && ldb >= N, ATS_ERR_UNSUPPORTED,
+                "%s: M=%d N=%d lda=%lld ldb=%lld must describe 16-byte aligned rows", name, M, N, (long long)lda, (long long)ldb);
+    GroupedArgs p{};
+    p.a = a;
+    p.a_row_div = 1;
+    p.lda = lda;
+    p.b = reinterpret_cast<const void* const*>(b);
+    p.ldb = ldb;
+    p.b_rows = b_rows;
+    p.b_row_div = b_rows ? b_row_div : 1;
+    p.out = out;
+    p.ldo = N;
+    p.k_start = k_start;
+    p.k_count = k_count;
+    p.uniform_rows = M;
+    p.E = E;
+    p.K = (int)max_k;
+    p.N_out = N;
+    bool wide;
+    small_kmajor_time((int64_t)E * M, E, N, (int)((max_k + E - 1) / E), &wide);
+    const int rc = wide ? launch_small<float, float, 2, 2, 4, 1, false, true, true>(p, (int64_t)E * M, as_stream(stream))
+                        : launch_small<float, float, 1, 1, 4, 1, false, true, true>(p, (int64_t)E * M, as_stream(stream));
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;

@@ -10,6 +10,13 @@
 // 128-byte row pieces in, MFMA fragments out; a wave's LDS accesses complete in order, so there is no barrier in the
 // loop) while the next slab is in flight.  Results leave through LDS as 16-byte (8-byte for bfloat16) stores.  No
 // atomics: the result does not depend on timing.  Any K that is a multiple of 16 bytes.
+//
+// BKM (float32): the weights are stored [K][N], the reduction index along their rows, as the data gradient of a linear layer
+// finds them; AKM: the other operand too, [K][rows] (the weight gradient: tokens along the rows of both, the rows of the
+// second one optionally gathered).  A slab is then 32 rows of K, staged as it lies, and a lane's four reduction steps are four
+// 4-byte reads instead of one of 16: the same values in the same order as from a transposed copy, without the copy.  In AKM
+// every group has p.uniform_rows output rows, so no table is read.  512 rows
+// x [512, 1024] with the copy 41 -> 11 us.
 #pragma once
 
 namespace ats {
@@ -26,7 +33,7 @@ struct SmallTile {
     static constexpr int kLds = kWaves * (kStage > kRed ? kStage : kRed);
 };
 
-template <typename T, typename TO, int TM, int TN, int KW, int WG, bool SWIGLU>
+template <typename T, typename TO, int TM, int TN, int KW, int WG, bool SWIGLU, bool AKM = false, bool BKM = false>
 __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(GroupedArgs p) {
     typedef SmallTile<T, TO, TM, TN, KW, WG, SWIGLU> Tile;
     constexpr int BM = Tile::BM, BN = Tile::BN;
@@ -38,14 +45,24 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
 
     extern __shared__ __align__(16) unsigned char smem[];
 
+    static_assert(!AKM || BKM, "K-major rows come with K-major weights");
+    static_assert(!BKM || (sizeof(T) == 4 && !SWIGLU), "K-major operands: the plain float32 product");
     TileCoord tc;
-    if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, Tile::kRows, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0, &tc)) return;
-    const int count = p.row_count[tc.e];
-    const int row0 = p.row_start[tc.e];
+    if constexpr (AKM) {
+        const int per = (p.uniform_rows + Tile::kRows - 1) / Tile::kRows * p.n_tiles;
+        tc.e = blockIdx.x / per;
+        tc.mt = blockIdx.x % per / p.n_tiles;
+        tc.nt = blockIdx.x % per % p.n_tiles;
+    } else {
+        if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, Tile::kRows, p.n_tiles, p.sm, p.sn, p.aligned_bands != 0, &tc)) return;
+    }
+    const int count = AKM ? p.uniform_rows : p.row_count[tc.e];
+    const int64_t row0 = AKM ? (int64_t)tc.e * count : p.row_start[tc.e];
     const int K = p.k_count ? p.k_count[tc.e] : p.K;
-    const T* Bexp = static_cast<const T*>(p.b[tc.e]);
+    const int k_row0 = AKM && p.k_start ? p.k_start[tc.e] : 0;
+    const T* Bexp = AKM ? reinterpret_cast<const T*>(p.b) : static_cast<const T*>(p.b[tc.e]);
     const T* A = static_cast<const T*>(p.a_ptrs ? p.a_ptrs[tc.e] : p.a);
-    const int arow0 = p.a_ptrs ? 0 : row0;
+    const int64_t arow0 = p.a_ptrs ? 0 : row0;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -58,7 +75,7 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
     // rows past the end of the group or of N repeat the last one (their results are never stored)
     const T* ap[NIA];
 #pragma unroll
-    for (int i = 0; i < NIA; ++i) {
+    for (int i = 0; i < NIA && !AKM; ++i) {
         int m = m0 + i * 8 + lrow;
         m = m < count ? m : count - 1;
         int64_t src = arow0 + m;
@@ -66,8 +83,12 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
         ap[i] = A + src * p.lda + lchunk * VEC;
     }
     const T* bp[NIB];
+    // K-major: lanes per row of a slab, rows per load instruction; columns past the end repeat the last four (never stored)
+    constexpr int CA = BM / 4, RA = 64 / CA, PA = BM * 4 + 16, CB = BN / 4, RB = 64 / CB, PB = BN * 4 + 16;
+    const T* const akm = A + min(m0 + lane % CA * 4, count - 4);
+    const T* const bkm = Bexp + min(n0 + lane % CB * 4, p.N_out - 4);
 #pragma unroll
-    for (int i = 0; i < NIB; ++i) {
+    for (int i = 0; i < NIB && !BKM; ++i) {
         const int rb = i * 8 + lrow;
         int n = n0 + (SWIGLU && rb >= HALF ? rb - HALF : rb);
         n = n < p.N_out ? n : p.N_out - 1;
@@ -94,16 +115,39 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
         const int koff = slab * BK;
         const bool ok = koff + lchunk * VEC < K;    // false only in the last slab of a ragged K
 #pragma unroll
-        for (int i = 0; i < NIA; ++i) ra[i] = ok ? *reinterpret_cast<const u32x4_t*>(ap[i] + koff) : zero4;
+        for (int i = 0; i < NIA; ++i) {
+            if constexpr (AKM) {
+                const int k = koff + i * RA + lane / CA;
+                ra[i] = k < K ? *reinterpret_cast<const u32x4_t*>(akm + ((int64_t)k_row0 + k) * p.lda) : zero4;
+            } else ra[i] = ok ? *reinterpret_cast<const u32x4_t*>(ap[i] + koff) : zero4;
+        }
 #pragma unroll
-        for (int i = 0; i < NIB; ++i) rb[i] = ok ? *reinterpret_cast<const u32x4_t*>(bp[i] + koff) : zero4;
+        for (int i = 0; i < NIB; ++i) {
+            if constexpr (BKM) {
+                const int k = koff + i * RB + lane / CB;
+                int64_t r = (int64_t)k_row0 + k;
+                if (AKM && p.b_rows && k < K) r = p.b_rows[r] / p.b_row_div;
+                rb[i] = k < K ? *reinterpret_cast<const u32x4_t*>(bkm + r * p.ldb) : zero4;
+            } else rb[i] = ok ? *reinterpret_cast<const u32x4_t*>(bp[i] + koff) : zero4;
+        }
+    };
+    // four reduction steps of a lane from a slab as it lies
+    auto column = [&](const unsigned char* at, int pitch, int ks) {
+        u32x4_t f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            f[c] = *reinterpret_cast<const uint32_t*>(at + (8 * ks + 4 * (lane >> 5) + c) * pitch + (lane & 31) * 4);
+        return f;
     };
     if (kw < nk) load(kw);
     for (int s = kw; s < nk; s += KW) {
 #pragma unroll
-        for (int i = 0; i < NIA; ++i) *reinterpret_cast<u32x4_t*>(st_at + i * 8 * kRowPitch) = ra[i];
+        for (int i = 0; i < NIA; ++i)
+            *reinterpret_cast<u32x4_t*>(AKM ? stage + (i * RA + lane / CA) * PA + lane % CA * 16 : st_at + i * 8 * kRowPitch) = ra[i];
 #pragma unroll
-        for (int i = 0; i < NIB; ++i) *reinterpret_cast<u32x4_t*>(st_at + (BM + i * 8) * kRowPitch) = rb[i];
+        for (int i = 0; i < NIB; ++i)
+            *reinterpret_cast<u32x4_t*>(BKM ? stage + BM * kRowPitch + (i * RB + lane / CB) * PB + lane % CB * 16
+                                            : st_at + (BM + i * 8) * kRowPitch) = rb[i];
         // other lanes' pieces are read below: nothing may move across (the wave's LDS accesses themselves are in order)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (s + KW < nk) load(s + KW);
@@ -111,10 +155,13 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
         for (int ks = 0; ks < 4; ++ks) {
             u32x4_t fa[TM], fb[TN];
 #pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const u32x4_t*>(fr_at + i * 32 * kRowPitch + ks * 32);
+            for (int i = 0; i < TM; ++i)
+                fa[i] = AKM ? column(stage + i * 128, PA, ks)
+                            : *reinterpret_cast<const u32x4_t*>(fr_at + i * 32 * kRowPitch + ks * 32);
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                fb[j] = *reinterpret_cast<const u32x4_t*>(fr_at + (BM + j * 32) * kRowPitch + ks * 32);
+                fb[j] = BKM ? column(stage + BM * kRowPitch + j * 128, PB, ks)
+                            : *reinterpret_cast<const u32x4_t*>(fr_at + (BM + j * 32) * kRowPitch + ks * 32);
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -173,12 +220,13 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
     }
 }
 
-template <typename T, typename TO, int TM, int TN, int KW, int WG, bool SWIGLU>
+template <typename T, typename TO, int TM, int TN, int KW, int WG, bool SWIGLU, bool AKM = false, bool BKM = false>
 static int launch_small(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
     typedef SmallTile<T, TO, TM, TN, KW, WG, SWIGLU> Tile;
     GroupedArgs p = p0;
     p.n_tiles = (p.N_out + Tile::kTileCols - 1) / Tile::kTileCols;
-    auto kern = grouped_gemm_small_kernel<T, TO, TM, TN, KW, WG, SWIGLU>;
+    static_assert(!BKM || 32 * (Tile::BN * 4 + 16) <= Tile::BN * kRowPitch, "a slab as it lies fits the room of its rows");
+    auto kern = grouped_gemm_small_kernel<T, TO, TM, TN, KW, WG, SWIGLU, AKM, BKM>;
     if (Tile::kLds > 64 * 1024) {
         static LdsReservation reserved;
         hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern)}, Tile::kLds);
@@ -189,7 +237,8 @@ static int launch_small(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) 
     }
     pick_supertile(p.n_tiles, &p.sm, &p.sn);
     p.aligned_bands = 0;
-    const int64_t blocks = grid_blocks(max_rows, p.E, Tile::kRows, p.n_tiles, p.sm, p.sn, false);
+    const int64_t blocks = AKM ? (int64_t)p.E * ((p.uniform_rows + Tile::kRows - 1) / Tile::kRows) * p.n_tiles
+                               : grid_blocks(max_rows, p.E, Tile::kRows, p.n_tiles, p.sm, p.sn, false);
     if (blocks > 0x7fffffffLL) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;

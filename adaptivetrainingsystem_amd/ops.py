@@ -1172,6 +1172,50 @@ def grouped_gemm_nn_sliced(b_ptrs: torch.Tensor, ldb: int, row_start: torch.Tens
     return out
 
 
+def grouped_gemm_nn_f32_supported(E: int, max_rows: int, N: int, K: int) -> bool:
+    """Whether a float32 product against [K, N] weights is faster read as they lie than through a transposed copy."""
+    return bool(_lib.load().ats_grouped_gemm_nn_f32_supported(int(E), int(max_rows), int(N), int(K)))
+
+
+def grouped_gemm_nn_f32(b_ptrs: torch.Tensor, ldb: int, row_start: torch.Tensor, row_count: torch.Tensor, max_rows: int, N: int,
+                        K: int, a: torch.Tensor) -> torch.Tensor:
+    """grouped_gemm_nn in float32 on the small tiles: [max_rows, N]."""
+    _need_gpu(a, b_ptrs, row_start, row_count)
+    a = _rows_2d(a, "grouped_gemm_nn_f32")
+    if a.dtype != torch.float32 or a.shape[0] < max_rows or a.shape[1] < K:
+        raise AtsError("grouped_gemm_nn_f32: a must be float32 [rows, K]")
+    out = torch.empty(max_rows, N, dtype=torch.float32, device=a.device)
+    check(_lib.load().ats_grouped_gemm_nn_f32(a.data_ptr(), a.stride(0), b_ptrs.data_ptr(), int(ldb), out.data_ptr(), N,
+                                              row_start.data_ptr(), row_count.data_ptr(), b_ptrs.numel(), int(max_rows), int(N),
+                                              int(K), _stream()), "ats_grouped_gemm_nn_f32")
+    return out
+
+
+def wgrad_f32_supported(a: torch.Tensor, b: torch.Tensor, E: int = 1) -> bool:
+    """Whether wgrad_f32 takes these rows (float32, 16-byte aligned) and is faster than the product of transposed copies."""
+    return all(t.dtype == torch.float32 and t.dim() == 2 and t.shape[0] > 0 and t.shape[1] % 4 == 0 and t.stride(1) == 1
+               and t.stride(0) >= t.shape[1] and t.stride(0) % 4 == 0 and t.data_ptr() % 16 == 0 for t in (a, b)) \
+        and bool(_lib.load().ats_grouped_wgrad_f32_supported(int(E), a.shape[0], a.shape[1], b.shape[1]))
+
+
+def wgrad_f32(a: torch.Tensor, b: torch.Tensor, k_start: Optional[torch.Tensor] = None, k_count: Optional[torch.Tensor] = None,
+              b_rows: Optional[torch.Tensor] = None, b_row_div: int = 1) -> torch.Tensor:
+    """a^T @ b for rows as they lie, a [R, M], b [R, N]; per group [E, M, N] over the k_count[e] rows from k_start[e] where
+    these are given, with b's row r taken from b_rows[r] // b_row_div if a gather table is given."""
+    _need_gpu(a, b, k_start, k_count, b_rows)
+    if not wgrad_f32_supported(a, b, 1 if k_count is None else k_count.numel()):
+        raise AtsError("wgrad_f32: float32 rows of 16-byte multiples, of sizes that the small tiles serve")
+    if b_rows is None and k_count is None and a.shape[0] != b.shape[0]:
+        raise AtsError("wgrad_f32: a and b must have the same number of rows")
+    (R, M), N = a.shape, b.shape[1]
+    E = 1 if k_count is None else k_count.numel()
+    out = torch.empty((M, N) if k_count is None else (E, M, N), dtype=torch.float32, device=a.device)
+    check(_lib.load().ats_grouped_wgrad_f32(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), _ptr(b_rows), int(b_row_div),
+                                            out.data_ptr(), _ptr(k_start), _ptr(k_count), E, R, M, N, _stream()),
+          "ats_grouped_wgrad_f32")
+    return out
+
+
 # --------------------------------------------------------------------------- attention
 def _key_bias(key_bias, B: int, Lk: int, q: torch.Tensor, who: str):
     if key_bias is None:

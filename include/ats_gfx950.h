@@ -463,6 +463,20 @@ int ats_grouped_gemm_nn(const void* a, int64_t lda, int64_t a_num_rows, const in
                         const void* const* b_ptrs, int64_t ldb, void* out, int64_t ldo, const int32_t* row_start,
                         const int32_t* row_count, int E, int64_t max_rows, int N, int K, int dtype, int out_dtype,
                         ats_stream_t stream);
+/* Float32 products against operands as training holds them, on the tiles for small products; ..._supported: whether that is
+ * faster than ats_grouped_gemm_nt on transposed copies (rows of 16-byte multiples).  Same bits as the sliced tiles on copies.
+ * _nn_f32: out[row_start[e]+m, n] = sum_k A_e[m,k] * B_e[k,n], B_e = b_ptrs[e] ([K, ldb >= N]).
+ * _wgrad_f32: out[e][m][n] = sum over the k_count[e] rows from k_start[e] of a[r, m] * b[r or b_rows[r] / b_row_div, n], zero
+ * for a group without rows; max_k bounds the sum of the counts; E = 1 may leave k_start / k_count NULL (rows 0 .. max_k). */
+int ats_grouped_gemm_nn_f32_supported(int E, int64_t max_rows, int N, int K);
+int ats_grouped_gemm_nn_f32(const float* a, int64_t lda, const void* const* b_ptrs, int64_t ldb, float* out, int64_t ldo,
+                            const int32_t* row_start, const int32_t* row_count, int E, int64_t max_rows, int N, int K,
+                            ats_stream_t stream);
+int ats_grouped_wgrad_f32_supported(int E, int64_t max_k, int M, int N);
+int ats_grouped_wgrad_f32(const float* a, int64_t lda, const float* b, int64_t ldb, const int32_t* b_rows, int b_row_div,
+                          float* out, const int32_t* k_start, const int32_t* k_count, int E, int64_t max_k, int M, int N,
+                          ats_stream_t stream);
+
 /* Weight gradient of a linear layer from operands as they lie: out[m, n] = sum_t a[t, m] * b[t, n], a [T, lda >= M] and
  * b [T, ldb >= N] bfloat16 with 16-byte aligned rows (autograd's weight gradient of nn.Linear).  slab_slices = 1: out [M, N]
  * bfloat16; more: float32 partial results [slab_slices][M][N] over equal runs of 64-row slabs (the last one may be shorter,
