@@ -467,17 +467,28 @@ static bool launch_combine(const void* y, const int32_t* row_of, const float* w,
 }
 
 // out[i] = sum over the n_parts partial results of parts[s * part_stride + i], added in slice order.
-template <typename TO>
+template <typename TO, int U>
 __global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ parts, int n_parts,
                                                            int64_t part_stride, TO* __restrict__ out, int64_t n4) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
-        float4 acc = *reinterpret_cast<const float4*>(parts + i * 4);
-        for (int s = 1; s < n_parts; ++s) {
-            const float4 v = *reinterpret_cast<const float4*>(parts + s * part_stride + i * 4);
-            acc.x += v.x;
-            acc.y += v.y;
-            acc.z += v.z;
-            acc.w += v.w;
+        // U slices are asked for together (8 x [64, 4096] 3.1 -> 2.8 us); the order of the additions is that of the slices
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int s0 = 0; s0 < n_parts; s0 += U) {
+            float4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int s = s0 + u < n_parts ? s0 + u : n_parts - 1;
+                v[u] = *reinterpret_cast<const float4*>(parts + s * part_stride + i * 4);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (s0 + u < n_parts) {
+                    const bool first = s0 + u == 0;
+                    acc.x = first ? v[u].x : acc.x + v[u].x;
+                    acc.y = first ? v[u].y : acc.y + v[u].y;
+                    acc.z = first ? v[u].z : acc.z + v[u].z;
+                    acc.w = first ? v[u].w : acc.w + v[u].w;
+                }
         }
         if constexpr (sizeof(TO) == 2) {
             uint2 u;
@@ -506,12 +517,14 @@ extern "C" int ats_sum_partials(const float* parts, int n_parts, int64_t part_st
     const int64_t n4 = n / 4;
     int64_t blocks = (n4 + 255) / 256;
     if (blocks > 4096) blocks = 4096;
+    auto kern_f32 = n_parts <= 2 ? sum_partials_kernel<float, 2> : n_parts <= 4 ? sum_partials_kernel<float, 4> : sum_partials_kernel<float, 8>;
+    auto kern_bf16 = n_parts <= 2 ? sum_partials_kernel<bf16_t, 2> : n_parts <= 4 ? sum_partials_kernel<bf16_t, 4> : sum_partials_kernel<bf16_t, 8>;
     if (out_dtype == ATS_F32)
-        hipLaunchKernelGGL((sum_partials_kernel<float>), dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), parts,
-                           n_parts, part_stride, static_cast<float*>(out), n4);
+        hipLaunchKernelGGL(kern_f32, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), parts, n_parts, part_stride,
+                           static_cast<float*>(out), n4);
     else
-        hipLaunchKernelGGL((sum_partials_kernel<bf16_t>), dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), parts,
-                           n_parts, part_stride, static_cast<bf16_t*>(out), n4);
+        hipLaunchKernelGGL(kern_bf16, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), parts, n_parts, part_stride,
+                           static_cast<bf16_t*>(out), n4);
     ATS_CHECK_LAUNCH("ats_sum_partials");
     return ATS_OK;
 }

@@ -1,5 +1,6 @@
 // RMSNorm forward for gfx950.  HBM-bound: every element is read once and
-// written once.  One wave64 owns one row at a time, keeps the whole row in
+// written once.  One wave64 (a workgroup for long rows and for few rows) owns
+// one row at a time, keeps the whole row in
 // registers as 16-byte vectors (so x is fetched exactly once), reduces the sum
 // of squares with cross-lane shuffles, and writes 16 bytes per lane.  The
 // weight vector is fetched once per block into LDS as float32, behind the
@@ -44,17 +45,14 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
     // weights: once per block, a 16-byte load or two per thread instead of up to eight per lane of every wave,
     // converted to float32 into LDS, from where every wave picks up its slices.  Later rows are fetched two
     // rows (one row) ahead.  [8192, 2048] bf16 with float32 weights: 13.3 -> 11.6 us.
-    constexpr bool kPrefetch = NV <= 8;
+    static_assert(NV <= 8, "longer rows have a workgroup each");
     constexpr bool kTwoAhead = NV <= 4;
-    constexpr int NP = kPrefetch ? NV : 1;
     constexpr int NP2 = kTwoAhead ? NV : 1;
-    uint4 cur[NP], nxt[NP2];
-    if (kPrefetch) {
+    uint4 cur[NV], nxt[NP2];
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int v = lane + i * kWave;
-            if (wave < rows && v < nvec) cur[kPrefetch ? i : 0] = stream_load(reinterpret_cast<const uint4*>(x + wave * H) + v);
-        }
+    for (int i = 0; i < NV; ++i) {
+        const int v = lane + i * kWave;
+        if (wave < rows && v < nvec) cur[i] = stream_load(reinterpret_cast<const uint4*>(x + wave * H) + v);
     }
     if (kTwoAhead) {
 #pragma unroll
@@ -66,7 +64,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
     }
     float wreg[NV][V];
     if (HAS_W && !kTwoAhead) {
-        // long rows: every wave loads its own slices (measured at [16384, 4096]: 46.5 us against 48.7 through LDS)
+        // long rows: every wave loads its own slices
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int v = lane + i * kWave;
@@ -106,8 +104,8 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
         if (kTwoAhead) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
-                raw[i] = cur[kPrefetch ? i : 0];
-                cur[kPrefetch ? i : 0] = nxt[kTwoAhead ? i : 0];
+                raw[i] = cur[i];
+                cur[i] = nxt[kTwoAhead ? i : 0];
             }
             if (row + 2 * nwaves < rows) {
                 const uint4* xn = reinterpret_cast<const uint4*>(x + (row + 2 * nwaves) * H);
@@ -117,23 +115,16 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
                     if (v < nvec) nxt[kTwoAhead ? i : 0] = stream_load(xn + v);
                 }
             }
-        } else if (kPrefetch) {
+        } else {
 #pragma unroll
-            for (int i = 0; i < NV; ++i) raw[i] = cur[kPrefetch ? i : 0];
+            for (int i = 0; i < NV; ++i) raw[i] = cur[i];
             if (row + nwaves < rows) {
                 const uint4* xn = reinterpret_cast<const uint4*>(x + (row + nwaves) * H);
 #pragma unroll
                 for (int i = 0; i < NV; ++i) {
                     const int v = lane + i * kWave;
-                    if (v < nvec) cur[kPrefetch ? i : 0] = stream_load(xn + v);
+                    if (v < nvec) cur[i] = stream_load(xn + v);
                 }
-            }
-        } else {
-            const uint4* xr = reinterpret_cast<const uint4*>(x + row * H);
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int v = lane + i * kWave;
-                if (v < nvec) raw[i] = stream_load(xr + v);
             }
         }
         float ss = 0.f;
@@ -161,6 +152,70 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
                     float t = f[j] * r;
                     if (HAS_W) t = t * wreg[i][j];
                     f[j] = t;
+                }
+                stream_store(yr + v, Elem<T>::pack(f));
+            }
+        }
+    }
+}
+
+// A workgroup per row.  Few rows (decoding steps): what a launch takes is one row's chain of loads, arithmetic and stores, a
+// quarter as long here as in a wave.  Long rows: a wave holds 64 .. 128 values and weights per lane, too many registers to
+// keep the memory busy; here they are 4 .. 16.  Wave per row -> this, microseconds, buffers from HBM above 1024 rows:
+//   bfloat16 [64, 4096] 4.9 -> 2.9   [512, 2048] 4.2 -> 3.1   [4096, 2048]  9.5 ->  8.3   [8192, 2048] 10.9 (13.7)
+//            [512, 4096] 5.5 -> 3.6  [4096, 4096] 14.8 -> 13.0   [16384, 4096] 47.6 -> 44.3 (6.1 TB/s)
+//   float32  [64, 4096] 10.2 -> 3.4  [512, 4096] 11.5 -> 5.9   [4096, 4096] 31.2 -> 23.4  [16384, 4096] 135 -> 88
+//            [512, 2048] 4.3 -> 3.8  [2048, 2048]  7.1 (7.4)
+template <typename T, typename WT, int NV, bool HAS_W>
+__global__ __launch_bounds__(256) void rmsnorm_row_block_kernel(const T* __restrict__ x, const WT* __restrict__ w,
+                                                                T* __restrict__ y, int64_t rows, int H, float eps) {
+    constexpr int V = Elem<T>::kVec;
+    __shared__ float s_part[4];
+    const int nvec = H / V;
+    uint4 raw[NV], nxt[NV];
+    float wreg[NV][V];
+    auto fetch = [&](int64_t row, uint4(&to)[NV]) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int v = threadIdx.x + i * 256;
+            to[i] = v < nvec ? stream_load(reinterpret_cast<const uint4*>(x + row * H) + v) : make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
+    fetch(blockIdx.x, nxt);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int v = threadIdx.x + i * 256;
+        if (HAS_W && v < nvec) load_weight_vec<WT, V>(w + (int64_t)v * V, wreg[i]);
+    }
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        uint4* yr = reinterpret_cast<uint4*>(y + row * H);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) raw[i] = nxt[i];
+        if (row + gridDim.x < rows) fetch(row + gridDim.x, nxt);
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            float f[V];
+            Elem<T>::unpack(raw[i], f);
+#pragma unroll
+            for (int j = 0; j < V; ++j) ss += f[j] * f[j];
+        }
+        ss = wave_sum(ss);
+        __syncthreads();
+        if (lane_id() == 0) s_part[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+        const float r = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int v = threadIdx.x + i * 256;
+            if (v < nvec) {
+                float f[V];
+                Elem<T>::unpack(raw[i], f);
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    f[j] *= r;
+                    if (HAS_W) f[j] *= wreg[i][j];
                 }
                 stream_store(yr + v, Elem<T>::pack(f));
             }
@@ -215,6 +270,22 @@ static int launch_rmsnorm(const void* x, const void* w, void* y, int64_t rows, i
         return ATS_OK;
     }
     const int per_lane = (H / V + kWave - 1) / kWave;
+    // A workgroup per row where it was measured to be the faster: rows of more than 512 vectors, bfloat16 rows of more than 256 with
+    // bfloat16 weights (float32 weights, twice the row's bytes, pay for themselves in a wave that keeps them: [2048, 4096]
+    // 8.1 against 9.0 us), few rows of at least two vectors per lane.
+    constexpr int kRmsRowBlocks = 2048;      // resident workgroups, eight to a CU, that keep their weights from row to row
+    const int64_t most = per_lane > 8 ? INT64_MAX : per_lane < 2 ? 0 : V == 4 ? 512 : per_lane <= 4 ? 4096
+                         : HAS_W && sizeof(WT) == 4 ? 1024 : INT64_MAX;
+    if (rows <= most) {
+        const unsigned grid = (unsigned)(rows < kRmsRowBlocks ? rows : kRmsRowBlocks);
+#define ATS_RMS_ROW(NV)                                                                                               \
+    hipLaunchKernelGGL((rmsnorm_row_block_kernel<T, WT, NV, HAS_W>), dim3(grid), dim3(256), 0, s, xp, wp, yp, rows, H, eps)
+        if (per_lane <= 4) ATS_RMS_ROW(1);
+        else if (per_lane <= 8) ATS_RMS_ROW(2);
+        else ATS_RMS_ROW(4);
+#undef ATS_RMS_ROW
+        return ATS_OK;
+    }
     const size_t wl = HAS_W ? (size_t)H * sizeof(float) : 0;      // the block's weights as float32 (rows of up to 4 vectors per lane)
 #define ATS_RMS_CASE(NV)                                                                            \
     hipLaunchKernelGGL((rmsnorm_rows_kernel<T, WT, NV, HAS_W>), dim3(blocks), dim3(256), wl, s, xp, wp, \
@@ -222,8 +293,7 @@ static int launch_rmsnorm(const void* x, const void* w, void* y, int64_t rows, i
     if (per_lane <= 1) ATS_RMS_CASE(1);
     else if (per_lane <= 2) ATS_RMS_CASE(2);
     else if (per_lane <= 4) ATS_RMS_CASE(4);
-    else if (per_lane <= 8) ATS_RMS_CASE(8);
-    else ATS_RMS_CASE(16);
+    else ATS_RMS_CASE(8);
 #undef ATS_RMS_CASE
     return ATS_OK;
 }
