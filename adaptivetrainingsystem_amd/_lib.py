@@ -37,6 +37,7 @@ _SIGNATURES = {
                              c_int, c_int, c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int,
                              c_void_p]),
     "ats_rope_fwd_append": (c_int, [c_void_p] * 8 + [c_int] * 8 + [c_int64] * 14 + [c_int, c_void_p]),
+    "ats_rope_sum_append": (c_int, [c_void_p, c_int, c_int64] + [c_void_p] * 5 + [c_int] * 7 + [c_int64] * 5 + [c_int, c_void_p]),
     "ats_rope_strided": (c_int, [c_void_p] * 6 + [c_int] * 3 + [c_void_p] + [c_int] * 5 + [c_void_p]),
     "ats_router_logits": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "ats_route_topk_workspace": (c_size_t, [c_int64, c_int]),

@@ -204,6 +204,35 @@ std::optional<Tensor> linear(const Tensor& x, const Tensor& table, const Tensor&
     return out;
 }
 
+// linear of stacked q, k, v weights with splits > 1, its sum fused with rope_append: x [B * L, K] -> rotated q [B, Hq, L, D]
+std::optional<Tensor> linear_rope_append(const Tensor& x, const Tensor& table, const Tensor& start, const Tensor& count, int64_t splits,
+                                         const Tensor& cos, const Tensor& sin, const Tensor& k_cache, const Tensor& v_cache,
+                                         int64_t cache_pos, int64_t Hq, int64_t L) {
+    auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    if (!on_gpu(x) || !served(x.scalar_type()) || x.dim() != 2 || !x.is_contiguous() || x.numel() == 0 || !tables_ok(cos, sin) ||
+        !heads_ok(k_cache) || !heads_ok(v_cache) || k_cache.scalar_type() != x.scalar_type() ||
+        v_cache.scalar_type() != x.scalar_type() || v_cache.sizes() != k_cache.sizes() || v_cache.strides() != k_cache.strides() ||
+        k_cache.size(0) * L != x.size(0) || k_cache.size(3) % 8 || k_cache.stride(0) % 4 || k_cache.stride(1) % 4 ||
+        k_cache.stride(2) % 4 || cos.stride(0) % 4 || !aligned(k_cache) || !aligned(v_cache) || !aligned(cos) || !aligned(sin) ||
+        transformed())
+        return {};
+    const int64_t T = x.size(0), K = x.size(1), B = k_cache.size(0), Hkv = k_cache.size(1), D = k_cache.size(3);
+    const int64_t N = (Hq + 2 * Hkv) * D;
+    at::AutoDispatchBelowADInplaceOrView below;
+    Tensor qo = at::empty({B, Hq, L, D}, x.options());
+    Tensor parts = at::empty({splits, T, N}, x.options().dtype(at::kFloat));
+    float* const p = static_cast<float*>(parts.data_ptr());
+    check(ats_grouped_down_splitk(x.data_ptr(), static_cast<const void* const*>(table.data_ptr()), p,
+                                  static_cast<const int32_t*>(start.data_ptr()), static_cast<const int32_t*>(count.data_ptr()), 1, T, T,
+                                  (int)N, (int)K, (int)splits, tag(x), stream()), "ats_grouped_down_splitk");
+    check(ats_rope_sum_append(p, (int)splits, T * N, qo.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                              static_cast<const float*>(cos.data_ptr()), static_cast<const float*>(sin.data_ptr()),
+                              (int)cos.stride(0), (int)cos.size(0), (int)B, (int)Hq, (int)Hkv, (int)L, (int)D, k_cache.stride(0),
+                              k_cache.stride(1), k_cache.stride(2), cache_pos, k_cache.size(2), tag(x), stream()),
+          "ats_rope_sum_append");
+    return qo;
+}
+
 // causal attention without masks, dropout or log-sum-exp
 std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool split_keys) {
     if (!heads_ok(q) || !heads_ok(k) || !heads_ok(v) || q.scalar_type() != at::kBFloat16 || k.scalar_type() != q.scalar_type() ||
@@ -234,5 +263,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("rope", &rope);
     m.def("rope_append", &rope_append);
     m.def("linear", &linear);
+    m.def("linear_rope_append", &linear_rope_append);
     m.def("attention", &attention);
 }

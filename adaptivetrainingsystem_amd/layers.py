@@ -279,8 +279,16 @@ class GroupedQueryAttention(nn.Module):
             # one product with the three weights stacked (a copy kept until a weight changes): a third of the
             # launches, which is what a decoding step is made of; q, k, v are column ranges of its output
             lin = lambda a, w: ops.linear_nt(a, _as_dtype(w, a.dtype))
-            qkv = ops.linear_nt(x2, self._stacked_qkv(x.dtype)).view(B, L, nh + 2 * nkv, D).transpose(1, 2)
-            q, k, v = qkv[:, :nh], qkv[:, nh:nh + nkv], qkv[:, nh + nkv:]
+            stacked = self._stacked_qkv(x.dtype)
+
+            def project():
+                qkv = ops.linear_nt(x2, stacked).view(B, L, nh + 2 * nkv, D).transpose(1, 2)
+                return qkv[:, :nh], qkv[:, nh:nh + nkv], qkv[:, nh + nkv:]
+
+            def append(k_buf, v_buf, pos):
+                """The projections; the rotated q, the rotated keys and the values at pos in the two buffers."""
+                q = ops.linear_rope_append(x2, stacked, cos, sin, k_buf, v_buf, pos, L)
+                return ops.rope_append(*project(), cos, sin, k_buf, v_buf, pos, 0) if q is None else q
         if past_key_value is not None:
             k_cache, v_cache = past_key_value
             if (k_cache.dim() != 4 or k_cache.shape[0] != B or k_cache.shape[1] != nkv or k_cache.shape[3] != D
@@ -288,15 +296,15 @@ class GroupedQueryAttention(nn.Module):
                 raise AtsError(f"GroupedQueryAttention: cache shapes {tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
         if past_key_value is not None and use_cache and not grad:
             # the rotation writes the new keys, and the values beside them, straight behind the cache
-            q, k, v = self._extend_cache(k_cache, v_cache, q, k, v, cos, sin)
+            q, k, v = self._extend_cache(k_cache, v_cache, L, x, append)
         else:
             if not grad and use_cache and past_key_value is None:
                 # the cache of a prompt: one launch rotates q and k and lays the values beside the keys (3 x 1777 tokens 525 ->
                 # 517 us, 80 tokens 54 -> 42)
-                k_new, v_new = (torch.empty(B, nkv, L, D, dtype=x.dtype, device=x.device) for _ in range(2))
-                q = ops.rope_append(q, k, v, cos, sin, k_new, v_new, 0, 0)
-                k, v = k_new, v_new
+                k, v = (torch.empty(B, nkv, L, D, dtype=x.dtype, device=x.device) for _ in range(2))
+                q = append(k, v, 0)
             elif not grad:
+                q, k, v = project()
                 q, k = ops.rope(q, k, cos, sin, 0)
             if past_key_value is not None:
                 k = torch.cat([k_cache.to(k.dtype), k], dim=2)
@@ -363,7 +371,7 @@ class GroupedQueryAttention(nn.Module):
         self._state["qkv_key"] = None
         self._state["qkv"] = None
 
-    def _extend_cache(self, k_cache, v_cache, q, k_new, v_new, cos, sin):
+    def _extend_cache(self, k_cache, v_cache, L, x, append):
         """The rotated q, and the cache followed by the new rows (keys rotated, values as they are), as the
         reference's rotation and torch.cat give them (model.py:690-704), without
         copying the cache on every step: the tensors handed back are the first rows of buffers
@@ -372,11 +380,10 @@ class GroupedQueryAttention(nn.Module):
         place (its length must be the buffer's fill), so continuing twice from one cache copies as cat does;
         any other cache tensor is copied into a fresh buffer whose capacity is 1.5 x the new length."""
         B, nkv, Lp, D = k_cache.shape
-        L = k_new.shape[2]
         st = self._state["kv"]
         cap_strides = lambda cap: (nkv * cap * D, cap * D, D, 1)
         if (st is not None and Lp == st["length"] and Lp + L <= st["capacity"]
-                and k_cache.dtype == k_new.dtype and v_cache.dtype == v_new.dtype
+                and k_cache.dtype == x.dtype and v_cache.dtype == x.dtype
                 and k_cache.data_ptr() == st["k_ptr"] and v_cache.data_ptr() == st["v_ptr"]
                 and k_cache.stride() == cap_strides(st["capacity"]) and v_cache.stride() == cap_strides(st["capacity"])
                 and k_cache.untyped_storage().nbytes() >= st["nbytes"]
@@ -388,11 +395,11 @@ class GroupedQueryAttention(nn.Module):
         else:
             self._state["kv_copies"] += 1
             cap = Lp + L + max(64, (Lp + L) // 2)
-            k_buf = torch.empty(B, nkv, cap, D, dtype=k_new.dtype, device=k_new.device)
-            v_buf = torch.empty(B, nkv, cap, D, dtype=v_new.dtype, device=v_new.device)
+            k_buf = torch.empty(B, nkv, cap, D, dtype=x.dtype, device=x.device)
+            v_buf = torch.empty(B, nkv, cap, D, dtype=x.dtype, device=x.device)
             k_buf[:, :, :Lp].copy_(k_cache)
             v_buf[:, :, :Lp].copy_(v_cache)
-        q = ops.rope_append(q, k_new, v_new, cos, sin, k_buf, v_buf, Lp, 0)
+        q = append(k_buf, v_buf, Lp)
         self._state["kv"] = {"k_ptr": k_buf.data_ptr(), "v_ptr": v_buf.data_ptr(), "capacity": cap, "length": Lp + L,
                            "nbytes": k_buf.numel() * k_buf.element_size()}
         return q, k_buf[:, :, :Lp + L], v_buf[:, :, :Lp + L]

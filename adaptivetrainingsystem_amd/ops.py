@@ -1537,6 +1537,27 @@ def _single_group(T: int, device: torch.device):
     return pair
 
 
+def _linear_slices(T: int, N: int, K: int, dtype: torch.dtype) -> int:
+    # 33-256 rows against a long K: slices of K over workgroups.  Up to 32 rows the plain launch streams the weights itself
+    # ([4096, 4096] x 16 rows: 10.3 us against 14.2 with the slices and their sum), and a short K leaves its small tiles
+    # less to do than the sum costs ([2048, 2048] x 64 rows: 8.8 against 11.3).
+    return down_k_splits(1, T, N, K, dtype) if T > 32 and K * dtype.itemsize > 4096 and K % 8 == 0 and N % 8 == 0 else 1
+
+
+def linear_rope_append(x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,
+                       v_cache: torch.Tensor, cache_pos: int, seq: int) -> Optional[torch.Tensor]:
+    """linear_nt(x [batch * seq, K], weight [(Hq + 2 Hkv) * D, K]) and rope_append of its columns: where the product runs in
+    slices of K one launch adds them up, rotates and appends (the same bits).  None where it does not."""
+    T, K = x.shape
+    N, D = weight.shape[0], k_cache.shape[3]
+    splits = _linear_slices(T, N, K, x.dtype)
+    if splits == 1 or not x.is_cuda or weight.dtype != x.dtype or not weight.is_contiguous():
+        return None
+    start, count = _single_group(T, x.device)
+    return _lib.native().linear_rope_append(x, weight_pointer_table([weight]), start, count, splits, cos, sin, k_cache, v_cache,
+                                            cache_pos, N // D - 2 * k_cache.shape[1], seq)
+
+
 def linear_nt(x: torch.Tensor, weight: torch.Tensor, table: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [T, K] @ weight[N, K]^T through the grouped GEMM kernels with a single group.  table: the (contiguous) weight's
     address on the device where the caller has it."""
@@ -1549,10 +1570,7 @@ def linear_nt(x: torch.Tensor, weight: torch.Tensor, table: Optional[torch.Tenso
     if table is None:
         table = weight_pointer_table([weight])
     start, count = _single_group(T, x.device)
-    # 33-256 rows against a long K: slices of K over workgroups.  Up to 32 rows the plain launch streams the weights itself
-    # ([4096, 4096] x 16 rows: 10.3 us against 14.2 with the slices and their sum), and a short K leaves its small tiles
-    # less to do than the sum costs ([2048, 2048] x 64 rows: 8.8 against 11.3).
-    splits = down_k_splits(1, T, N, K, x.dtype) if T > 32 and K * x.element_size() > 4096 and K % 8 == 0 and N % 8 == 0 else 1
+    splits = _linear_slices(T, N, K, x.dtype)
     done = _lib.native().linear(x, table, start, count, N, splits)
     if done is not None:
         return done

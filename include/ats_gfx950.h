@@ -101,6 +101,14 @@ int ats_rope_fwd_append(const void* q_in, const void* k_in, const void* v_in, vo
                         int64_t v_sh, int64_t v_sl, int64_t cache_sb, int64_t cache_sh, int64_t cache_sl,
                         int64_t cache_pos, int64_t cache_capacity, int dtype, ats_stream_t stream);
 
+/* ats_sum_partials and ats_rope_fwd_append (pos_offset 0) in one launch, the same results bit for bit: parts
+ * [n_parts][B * L][(Hq + 2 Hkv) * D] float32, heads of q, then k, then v, D a multiple of 8, 16-byte aligned pointers, cache
+ * strides and table_stride multiples of 4. */
+int ats_rope_sum_append(const float* parts, int n_parts, int64_t part_stride, void* q_out, void* k_cache, void* v_cache,
+                        const float* cos_tab, const float* sin_tab, int table_stride, int table_len, int B, int Hq, int Hkv,
+                        int L, int D, int64_t cache_sb, int64_t cache_sh, int64_t cache_sl, int64_t cache_pos,
+                        int64_t cache_capacity, int dtype, ats_stream_t stream);
+
 /* ---- Router -------------------------------------------------------------
  * logits[T,E] (float32) = x[T,H] . wg[E,H]^T (+ bias[E] if not NULL): the
  * nn.Linear(H, E, bias=False) gate of model.py:1124,1169. */
