@@ -271,7 +271,10 @@ __global__ __launch_bounds__(512) void gate_gemm_bf16_flat_kernel(const bf16_t* 
     }
 }
 
-// One wave per token, 8 experts at a time.  Works for every dtype / shape.
+// One wave per token, 8 experts at a time.  Works for every dtype / shape.  What bounds it is the latency of its loads (a
+// token's row and the gate rows, these from L2): those of four steps are asked for together, without a branch per expert (beyond
+// the last expert its row is read again), and added in the order of the steps.  float32 of width 512 and 8 experts:
+// 512 tokens 21.5 -> 7.7 us, with it a training step of 2000 tokens 1452 -> 1405.
 template <typename T>
 __global__ __launch_bounds__(256) void gate_gemm_generic_kernel(const T* __restrict__ x, const T* __restrict__ wg,
                                                                 const float* __restrict__ bias,
@@ -286,12 +289,27 @@ __global__ __launch_bounds__(256) void gate_gemm_generic_kernel(const T* __restr
             float acc[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[j] = 0.f;
-            for (int h = lane; h < H; h += kWave) {
+            const T* wr[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) wr[j] = wg + (int64_t)min(e0 + j, E - 1) * H;
+            int h = lane;
+            for (; h + 3 * kWave < H; h += 4 * kWave) {
+                float xv[4], wv[4][8];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    xv[u] = Elem<T>::load(xr + h + u * kWave);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) wv[u][j] = Elem<T>::load(wr[j] + h + u * kWave);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) acc[j] += xv[u] * wv[u][j];
+            }
+            for (; h < H; h += kWave) {
                 const float xv = Elem<T>::load(xr + h);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if (e0 + j < E) acc[j] += xv * Elem<T>::load(wg + (int64_t)(e0 + j) * H + h);
-                }
+                for (int j = 0; j < 8; ++j) acc[j] += xv * Elem<T>::load(wr[j] + h);
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
