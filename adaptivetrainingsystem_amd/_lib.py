@@ -128,6 +128,9 @@ _SIGNATURES = {
     "ats_attention_fwd": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p,
                                   c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p,
                                   c_size_t, c_void_p]),
+    "ats_attention_fwd_rope_supported": (c_int, [c_int] * 6),
+    "ats_attention_fwd_rope": (c_int, [c_void_p] + [c_int64] * 3 + [c_void_p] * 2 + [c_int] * 2 + [c_void_p] + [c_int64] * 2 +
+                               [c_void_p] + [c_int64] * 3 + [c_void_p] + [c_int] * 6 + [c_float, c_void_p]),
     "ats_attention_fwd_ex": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p,
                                      c_void_p, c_int64, c_int64, c_float, c_uint64, c_void_p, c_void_p, c_int, c_int, c_int,
                                      c_int, c_int, c_int, c_float, c_void_p, c_size_t, c_void_p]),

@@ -494,14 +494,37 @@ struct PipeSeq {
 // K runs one tile ahead of V: at the start of iteration t the loads of K(t+2) and V(t+1) are issued into the
 // stages that K(t) and V(t-1) occupied (everybody was done with them at the barrier that ended iteration
 // t-1) and have the whole iteration to land; two stages each, 4 x 16 KiB at head_dim 128.
-template <int D, bool BIAS, int NT>
+// With ROPE a tile's queries arrive unrotated, in the strides of the projection that wrote them, and are rotated here: a lane's
+// fragments hold both halves of its elements' pairs, so the rotation needs the tables and nothing else, and the rotated q makes no
+// trip through memory (rounded as the separate rotation rounds it, the same bits).  3 x 1777 tokens of 32 + 16 heads of 128: the
+// rotation 26.4 -> 10.5 us (keys and values are left to it), the attention 141 -> 145-150 (rows of q 12 KB apart).
+struct RopeQ {
+    const float* cos_tab;
+    const float* sin_tab;
+    int table_stride;
+    int64_t sb, sh, sl;      // element strides of q: batch, head, position
+};
+
+__device__ __forceinline__ void rotate_pairs(au32x4_t& lo, au32x4_t& hi, const float* cs, const float* sn) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float a0 = __uint_as_float(lo[j] << 16), a1 = __uint_as_float(lo[j] & 0xffff0000u);
+        const float b0 = __uint_as_float(hi[j] << 16), b1 = __uint_as_float(hi[j] & 0xffff0000u);
+        const float c0 = cs[2 * j], c1 = cs[2 * j + 1], s0 = sn[2 * j], s1 = sn[2 * j + 1];
+        lo[j] = pack_bf16x2(a0 * c0 - b0 * s0, a1 * c1 - b1 * s1);
+        hi[j] = pack_bf16x2(a0 * s0 + b0 * c0, a1 * s1 + b1 * c1);
+    }
+}
+
+template <int D, bool BIAS, int NT, bool ROPE>
 __device__ __forceinline__ void attention_q_tile_pipe(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                       int64_t k_sb, int64_t k_sh, const bf16_t* __restrict__ v,
                                                       int64_t v_sb, int v_sl, int64_t v_sh,
                                                       const float* __restrict__ key_bias, bf16_t* __restrict__ out,
                                                       float* __restrict__ lse, int Hq, int Hkv, int L, int Lk,
                                                       float scale_log2, int qt, int head, int b, bool pack,
-                                                      unsigned char* smem) {
+                                                      const RopeQ& rope, unsigned char* smem) {
     typedef __attribute__((address_space(3))) void* lds_ptr_t;
     typedef __attribute__((address_space(3))) unsigned char* lds_u8_t;
     typedef __attribute__((address_space(3))) au32x4_t* lds_v4_t;
@@ -545,13 +568,26 @@ __device__ __forceinline__ void attention_q_tile_pipe(const bf16_t* __restrict__
     const int hq = pack ? hkv * rep + row_clamped % rp : head;
     const bool row_valid = row < n_rows;
 
-    const bf16_t* qp = q + ((int64_t)(b * Hq + hq) * L + q_clamped) * D;
+    const bf16_t* qp = ROPE ? q + b * rope.sb + hq * rope.sh + q_clamped * rope.sl : q + ((int64_t)(b * Hq + hq) * L + q_clamped) * D;
     const bf16_t* kbase = k + b * k_sb + hkv * k_sh;
     const bf16_t* vbase = v + b * v_sb + hkv * v_sh;
 
     au32x4_t qf[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const au32x4_t*>(qp + s * 16 + g * 8);
+    // (the tables' columns land with the first tiles: a rotation here would be a trip to memory of its own)
+    float cs[ROPE ? KS / 2 : 1][8], sn[ROPE ? KS / 2 : 1][8];
+    if constexpr (ROPE) {
+        const float* const cp = rope.cos_tab + (int64_t)q_clamped * rope.table_stride + g * 8;
+        const float* const sp = rope.sin_tab + (int64_t)q_clamped * rope.table_stride + g * 8;
+#pragma unroll
+        for (int s = 0; s < KS / 2; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; j += 4) {
+                *reinterpret_cast<float4*>(&cs[s][j]) = *reinterpret_cast<const float4*>(cp + s * 16 + j);
+                *reinterpret_cast<float4*>(&sn[s][j]) = *reinterpret_cast<const float4*>(sp + s * 16 + j);
+            }
+    }
 
     const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<bf16_t*>(kbase), 0, (int)((int64_t)Lk * D * 2), 0x00020000);
@@ -637,6 +673,10 @@ __device__ __forceinline__ void attention_q_tile_pipe(const bf16_t* __restrict__
     if (has_bias && tid < kAttBN) s_bias[tid] = tid < Lk ? bias_row[tid] * 1.4426950408889634f : 0.f;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     PIPE_CLEAR_V_TAIL(0, 0)
+    if constexpr (ROPE) {
+#pragma unroll
+        for (int s = 0; s < KS / 2; ++s) rotate_pairs(qf[s], qf[s + KS / 2], cs[s], sn[s]);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
     for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
@@ -793,13 +833,13 @@ __device__ __forceinline__ void attention_q_tile_pipe(const bf16_t* __restrict__
 // Consecutive ids go to different XCDs; the blocks of one (batch, kv head) are kept on one XCD so that
 // its K and V stay in that XCD's L2.  Two waves per SIMD (register budget 256): one wave's softmax runs
 // in the shadow of the other's MFMAs.
-template <int D, bool BIAS, int NT>
+template <int D, bool BIAS, int NT, bool ROPE>
 __global__ __launch_bounds__(NT, 512 / NT) void attention_fwd_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                             int64_t k_sb, int64_t k_sh,
                                                             const bf16_t* __restrict__ v, int64_t v_sb, int v_sl, int64_t v_sh,
                                                             const float* __restrict__ key_bias, bf16_t* __restrict__ out,
                                                             float* __restrict__ lse, int Hq, int Hkv, int L, int Lk,
-                                                            float scale_log2, int B, int pack) {
+                                                            float scale_log2, int B, int pack, RopeQ rope) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kAttBM = att_rows_per_block(NT);
     const int heads_per_group = pack ? 1 : Hq / Hkv;     // packed: the group's heads share the rows of a tile
@@ -823,8 +863,8 @@ __global__ __launch_bounds__(NT, 512 / NT) void attention_fwd_kernel(const bf16_
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
         if (half && pair == qt_long) break;   // an odd tile count leaves the middle tile on its own
-        attention_q_tile_pipe<D, BIAS, NT>(q, k, k_sb, k_sh, v, v_sb, v_sl, v_sh, key_bias, out, lse, Hq, Hkv, L, Lk,
-                                           scale_log2, half ? pair : qt_long, head, b, pack != 0, smem);
+        attention_q_tile_pipe<D, BIAS, NT, ROPE>(q, k, k_sb, k_sh, v, v_sb, v_sl, v_sh, key_bias, out, lse, Hq, Hkv, L, Lk,
+                                                 scale_log2, half ? pair : qt_long, head, b, pack != 0, rope, smem);
     }
 }
 
@@ -1013,6 +1053,50 @@ bool make_attention_extra(const char* who, const float* bias_qk, int64_t bias_sb
     }
     return true;
 }
+// The tiles of attention_fwd_kernel; rope: queries to be rotated as they are loaded (no key bias then).
+static int launch_attention_fwd(const char* name, const void* q, const void* k, int64_t k_sb, int64_t k_sh, const void* v, int64_t v_sb,
+                                int64_t v_sl, int64_t v_sh, const float* key_bias, void* out, float* lse, int B, int Hq, int Hkv, int L,
+                                int Lk, int D, float scale_log2, const RopeQ* rope, hipStream_t s) {
+    const int nt = L >= 4096 ? 512 : 256;
+    const int kAttBM = att_rows_per_block(nt);
+    const int pack = (L < kAttBM && Hq > Hkv) ? 1 : 0;
+    const int64_t n_blocks = pack ? (int64_t)((((int64_t)L * (Hq / Hkv) + kAttBM - 1) / kAttBM + 1) / 2) * Hkv * B
+                                  : (int64_t)(((L + kAttBM - 1) / kAttBM + 1) / 2) * Hq * B;
+    ATS_REQUIRE(n_blocks <= 0x7fffffff, ATS_ERR_UNSUPPORTED, "%s: %lld workgroups", name, (long long)n_blocks);
+    const dim3 grid((unsigned)n_blocks);
+    static LdsReservation reserved_lds[12];      // one per kernel instance
+    auto launch = [&](auto kernel, int smem, LdsReservation& reserved) -> int {
+        if (smem > 64 * 1024) {
+            hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kernel)}, smem);
+            ATS_REQUIRE(e == hipSuccess, ATS_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", name, smem,
+                        hipGetErrorString(e));
+        }
+        hipLaunchKernelGGL(kernel, grid, dim3(nt), smem, s, static_cast<const bf16_t*>(q),
+                           static_cast<const bf16_t*>(k), k_sb, k_sh, static_cast<const bf16_t*>(v), v_sb, (int)v_sl, v_sh,
+                           key_bias,
+                           static_cast<bf16_t*>(out), lse, Hq, Hkv, L, Lk, scale_log2, B, pack, rope ? *rope : RopeQ{});
+        return ATS_OK;
+    };
+    // K tile, V tile (two stages each, rows unpadded) and, with a bias, two stages of one float per key
+    const int smem = 4 * kAttBN * D * 2 + (key_bias ? 2 * kAttBN * 4 : 0);
+    if (rope) {
+        if (D == 128) return nt == 256 ? launch(attention_fwd_kernel<128, false, 256, true>, smem, reserved_lds[8])
+                                       : launch(attention_fwd_kernel<128, false, 512, true>, smem, reserved_lds[9]);
+        return nt == 256 ? launch(attention_fwd_kernel<64, false, 256, true>, smem, reserved_lds[10])
+                         : launch(attention_fwd_kernel<64, false, 512, true>, smem, reserved_lds[11]);
+    }
+    if (D == 128 && nt == 256)
+        return key_bias ? launch(attention_fwd_kernel<128, true, 256, false>, smem, reserved_lds[0])
+                        : launch(attention_fwd_kernel<128, false, 256, false>, smem, reserved_lds[1]);
+    if (D == 128)
+        return key_bias ? launch(attention_fwd_kernel<128, true, 512, false>, smem, reserved_lds[2])
+                        : launch(attention_fwd_kernel<128, false, 512, false>, smem, reserved_lds[3]);
+    if (nt == 256)
+        return key_bias ? launch(attention_fwd_kernel<64, true, 256, false>, smem, reserved_lds[4])
+                        : launch(attention_fwd_kernel<64, false, 256, false>, smem, reserved_lds[5]);
+    return key_bias ? launch(attention_fwd_kernel<64, true, 512, false>, smem, reserved_lds[6])
+                    : launch(attention_fwd_kernel<64, false, 512, false>, smem, reserved_lds[7]);
+}
 }  // namespace ats
 
 extern "C" int ats_attention_fwd(const void* q, const void* k, int64_t k_sb, int64_t k_sh, const void* v, int64_t v_sb,
@@ -1137,42 +1221,43 @@ extern "C" int ats_attention_fwd_ex(const void* q, const void* k, int64_t k_sb, 
         return ATS_OK;
     }
     if (L * (int64_t)(Hq / Hkv) <= kDecRows) return launch_decode(1, 0, nullptr);
-    const int nt = L >= 4096 ? 512 : 256;
-    const int kAttBM = att_rows_per_block(nt);
-    const int pack = (L < kAttBM && Hq > Hkv) ? 1 : 0;
-    const int64_t n_blocks = pack ? (int64_t)((((int64_t)L * (Hq / Hkv) + kAttBM - 1) / kAttBM + 1) / 2) * Hkv * B
-                                  : (int64_t)(((L + kAttBM - 1) / kAttBM + 1) / 2) * Hq * B;
-    ATS_REQUIRE(n_blocks <= 0x7fffffff, ATS_ERR_UNSUPPORTED, "ats_attention_fwd: %lld workgroups", (long long)n_blocks);
-    const dim3 grid((unsigned)n_blocks);
-    static LdsReservation reserved_lds[8];      // one per kernel instance
-    auto launch = [&](auto kernel, int smem, LdsReservation& reserved) -> int {
-        if (smem > 64 * 1024) {
-            hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kernel)}, smem);
-            ATS_REQUIRE(e == hipSuccess, ATS_ERR_LAUNCH, "ats_attention_fwd: cannot reserve %d bytes of LDS: %s", smem,
-                        hipGetErrorString(e));
-        }
-        hipLaunchKernelGGL(kernel, grid, dim3(nt), smem, as_stream(stream), static_cast<const bf16_t*>(q),
-                           static_cast<const bf16_t*>(k), k_sb, k_sh, static_cast<const bf16_t*>(v), v_sb, (int)v_sl, v_sh,
-                           key_bias,
-                           static_cast<bf16_t*>(out), lse, Hq, Hkv, L, Lk, scale_log2, B, pack);
-        return ATS_OK;
-    };
-    // K tile, V tile (two stages each, rows unpadded) and, with a bias, two stages of one float per key
-    const int smem = 4 * kAttBN * D * 2 + (key_bias ? 2 * kAttBN * 4 : 0);
-    int rc;
-    if (D == 128 && nt == 256)
-        rc = key_bias ? launch(attention_fwd_kernel<128, true, 256>, smem, reserved_lds[0])
-                      : launch(attention_fwd_kernel<128, false, 256>, smem, reserved_lds[1]);
-    else if (D == 128)
-        rc = key_bias ? launch(attention_fwd_kernel<128, true, 512>, smem, reserved_lds[2])
-                      : launch(attention_fwd_kernel<128, false, 512>, smem, reserved_lds[3]);
-    else if (nt == 256)
-        rc = key_bias ? launch(attention_fwd_kernel<64, true, 256>, smem, reserved_lds[4])
-                      : launch(attention_fwd_kernel<64, false, 256>, smem, reserved_lds[5]);
-    else
-        rc = key_bias ? launch(attention_fwd_kernel<64, true, 512>, smem, reserved_lds[6])
-                      : launch(attention_fwd_kernel<64, false, 512>, smem, reserved_lds[7]);
+    const int rc = launch_attention_fwd("ats_attention_fwd", q, k, k_sb, k_sh, v, v_sb, v_sl, v_sh, key_bias, out, lse, B, Hq, Hkv, L, Lk,
+                                        D, scale_log2, nullptr, as_stream(stream));
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH("ats_attention_fwd");
+    return ATS_OK;
+}
+
+// Whether a call without masks, dropout or log-sum-exp runs on attention_fwd_kernel (neither decoding rows nor ranges of keys).
+extern "C" int ats_attention_fwd_rope_supported(int B, int Hq, int Hkv, int L, int Lk, int D) {
+    using namespace ats;
+    int part_len = 0;
+    return (D == 64 || D == 128) && B > 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && L > 0 && Lk >= L &&
+           L * (int64_t)(Hq / Hkv) > kDecRows && attention_split_plan(B, Hq, Hkv, L, Lk, D, &part_len) <= 1 &&
+           (int64_t)Lk * D * 2 < 0x7fffffffLL ? 1 : 0;
+}
+
+extern "C" int ats_attention_fwd_rope(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const float* cos_tab,
+                                      const float* sin_tab, int table_stride, int table_len, const void* k, int64_t k_sb, int64_t k_sh,
+                                      const void* v, int64_t v_sb, int64_t v_sl, int64_t v_sh, void* out, int B, int Hq, int Hkv, int L,
+                                      int Lk, int D, float scale, ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_attention_fwd_rope";
+    ATS_REQUIRE(ats_attention_fwd_rope_supported(B, Hq, Hkv, L, Lk, D), ATS_ERR_UNSUPPORTED, "%s: B=%d Hq=%d Hkv=%d L=%d Lk=%d D=%d",
+                name, B, Hq, Hkv, L, Lk, D);
+    ATS_REQUIRE(scale > 0.f && L <= table_len && table_stride >= D / 2 && table_stride % 4 == 0, ATS_ERR_INVALID_ARG,
+                "%s: scale=%g, %d positions, table of %d (stride %d)", name, scale, L, table_len, table_stride);
+    ATS_REQUIRE(q && k && v && out && cos_tab && sin_tab && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) &&
+                    aligned16(cos_tab) && aligned16(sin_tab), ATS_ERR_INVALID_ARG, "%s: null or misaligned pointer", name);
+    ATS_REQUIRE(q_sb % 8 == 0 && q_sh % 8 == 0 && q_sl % 8 == 0 && q_sb >= 0 && q_sh >= 0 && q_sl >= 0 && k_sb % 8 == 0 &&
+                    k_sh % 8 == 0 && k_sb >= 0 && k_sh >= 0 && v_sl >= D && v_sl % 8 == 0 && v_sb % 8 == 0 && v_sh % 8 == 0 &&
+                    v_sb >= 0 && v_sh >= 0, ATS_ERR_INVALID_ARG, "%s: strides must be multiples of 8 elements", name);
+    ATS_REQUIRE(((int64_t)Lk * v_sl + D) * 2 < 0x7fffffffLL, ATS_ERR_UNSUPPORTED,
+                "%s: %d keys (one head's K or V must stay under 2 GiB)", name, Lk);
+    const RopeQ rope{cos_tab, sin_tab, table_stride, q_sb, q_sh, q_sl};
+    const int rc = launch_attention_fwd(name, q, k, k_sb, k_sh, v, v_sb, v_sl, v_sh, nullptr, out, nullptr, B, Hq, Hkv, L, Lk, D,
+                                        scale * 1.4426950408889634f, &rope, as_stream(stream));
+    if (rc != ATS_OK) return rc;
+    ATS_CHECK_LAUNCH(name);
     return ATS_OK;
 }

@@ -255,6 +255,35 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
     return out;
 }
 
+// causal attention of a prompt on its stacked projections qkv [B * L, (Hq + 2 Hkv) * D]: keys rotated (with the values beside them:
+// the prompt's cache), queries rotated as the attention loads them -> out, k, v
+std::optional<std::tuple<Tensor, Tensor, Tensor>> prompt_attention(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t B,
+                                                                   int64_t Hkv, int64_t D, double scale, bool keep_values) {
+    auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    if (!on_gpu(qkv) || qkv.scalar_type() != at::kBFloat16 || !qkv.is_contiguous() || !tables_ok(cos, sin) || cos.stride(0) % 4 ||
+        !aligned(qkv) || !aligned(cos) || !aligned(sin) || transformed())
+        return {};
+    const int64_t L = qkv.size(0) / B, N = qkv.size(1), Hq = N / D - 2 * Hkv;
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor rows = qkv.view({B, L, N / D, D}).transpose(1, 2);
+    const Tensor k_in = rows.narrow(1, Hq, Hkv), v_in = rows.narrow(1, Hq + Hkv, Hkv);
+    const Tensor k = at::empty({B, Hkv, L, D}, qkv.options());
+    const Tensor v = keep_values ? at::empty({B, Hkv, L, D}, qkv.options()) : v_in;
+    const float* const c = static_cast<const float*>(cos.data_ptr());
+    const float* const s = static_cast<const float*>(sin.data_ptr());
+    const void* in[3] = {nullptr, k_in.data_ptr(), v_in.data_ptr()};
+    void* to[3] = {nullptr, k.data_ptr(), v.data_ptr()};
+    const int64_t is[9] = {0, 0, 0, L * N, D, N, L * N, D, N}, os[9] = {0, 0, 0, Hkv * L * D, L * D, D, Hkv * L * D, L * D, D};
+    const int heads[3] = {0, (int)Hkv, keep_values ? (int)Hkv : 0};
+    check(ats_rope_strided(in, to, is, os, c, s, (int)cos.stride(0), (int)cos.size(0), (int)B, heads, (int)L, (int)D, 0, 0, tag(qkv),
+                           stream()), "ats_rope_strided");
+    Tensor out = at::empty({B, L, Hq * D}, qkv.options());
+    check(ats_attention_fwd_rope(qkv.data_ptr(), L * N, D, N, c, s, (int)cos.stride(0), (int)cos.size(0), k.data_ptr(), k.stride(0),
+                                 k.stride(1), v.data_ptr(), v.stride(0), v.stride(2), v.stride(1), out.data_ptr(), (int)B, (int)Hq,
+                                 (int)Hkv, (int)L, (int)L, (int)D, (float)scale, stream()), "ats_attention_fwd_rope");
+    return std::make_tuple(out, k, v);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -265,4 +294,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("linear", &linear);
     m.def("linear_rope_append", &linear_rope_append);
     m.def("attention", &attention);
+    m.def("prompt_attention", &prompt_attention);
 }

@@ -1305,6 +1305,21 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: O
     return (out, lse) if return_lse else out
 
 
+def prompt_attention_supported(x: torch.Tensor, weight: torch.Tensor, B: int, L: int, Hq: int, Hkv: int, D: int) -> bool:
+    """Whether the attention of a prompt x [B * L, K] projected by weight rotates its queries itself (prompt_attention): a product
+    in slices of K has its rotation in the sum of the slices."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == x.dtype
+            and bool(_lib.load().ats_attention_fwd_rope_supported(B, Hq, Hkv, L, L, D))
+            and _linear_slices(B * L, weight.shape[0], x.shape[1], x.dtype) == 1)
+
+
+def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, B: int, Hkv: int, D: int, scale: float,
+                     keep_values: bool):
+    """rope and causal_attention of the stacked projections qkv [B * L, (Hq + 2 Hkv) * D]: (out [B, L, Hq * D], rotated k, v),
+    v contiguous with keep_values and a view of qkv without; None for operands that the launches do not read as they are."""
+    return _lib.native().prompt_attention(qkv, cos, sin, B, Hkv, D, scale, keep_values)
+
+
 def causal_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, lse: torch.Tensor,
                          dout: torch.Tensor, scale: Optional[float] = None, key_bias: Optional[torch.Tensor] = None,
                          pair_bias: Optional[torch.Tensor] = None, dropout_p: float = 0.0, dropout_seed: int = 0):

@@ -547,6 +547,15 @@ int ats_attention_fwd_ex(const void* q, const void* k, int64_t k_sb, int64_t k_s
                          int Hkv, int L, int Lk, int D, float scale, void* workspace, size_t workspace_bytes,
                          ats_stream_t stream);
 
+/* ats_attention_fwd of queries that ats_rope_fwd (pos_offset 0) would have rotated first, rotated as they are loaded: q in any
+ * batch / head / position strides (multiples of 8 elements), the same results bit for bit.  For calls that fill query tiles
+ * (see _supported: more than the decoding rows, keys not cut into ranges); table_stride a multiple of 4. */
+int ats_attention_fwd_rope_supported(int B, int Hq, int Hkv, int L, int Lk, int D);
+int ats_attention_fwd_rope(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, const float* cos_tab, const float* sin_tab,
+                           int table_stride, int table_len, const void* k, int64_t k_sb, int64_t k_sh, const void* v, int64_t v_sb,
+                           int64_t v_sl, int64_t v_sh, void* out, int B, int Hq, int Hkv, int L, int Lk, int D, float scale,
+                           ats_stream_t stream);
+
 /* ---- Causal grouped-query attention (backward) ----------------------------------
  * The reference leaves this gradient to autograd (model.py:757-839 under torch.autograd); the kernels
  * recompute the probabilities from the forward's log-sum-exp and form
