@@ -52,7 +52,55 @@ __global__ __launch_bounds__(64) void upload_kernel(UploadArgs a, uint64_t* __re
     for (int i = threadIdx.x; i < words; i += 64) dst[i] = a.w[i];
 }
 
+// Several matrices of one width below each other, and the address of the result where a grouped product reads it.  Bound by the
+// bytes: a workgroup moves 16 KB at a time, four 16-byte loads per lane in flight, with ordinary stores (the product behind it
+// reads them).  Projections of hidden 4096, 32 + 16 heads (50 MB): 18.5 us against 39.5 for torch's concatenation and 4.7 for the
+// launch that wrote the address.
+constexpr int kMaxStack = 8;
+struct StackArgs {
+    const uint4* src[kMaxStack];
+    int64_t first[kMaxStack], n[kMaxStack];      // 16-byte units
+};
+__global__ __launch_bounds__(256) void stack_rows_kernel(StackArgs a, uint4* __restrict__ out, int64_t* __restrict__ address) {
+    const uint4* __restrict__ const src = a.src[blockIdx.y];
+    uint4* const dst = out + a.first[blockIdx.y];
+    const int64_t n = a.n[blockIdx.y];
+    if (address && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *address = (int64_t)reinterpret_cast<uintptr_t>(out);
+    for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 1024) {
+        uint4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = src[min(i + 256 * u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + 256 * u < n) dst[i + 256 * u] = v[u];
+    }
+}
+
 }  // namespace ats
+
+extern "C" int ats_stack_rows(const void* const* src, const int64_t* bytes, int n, void* out, int64_t* address, ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_stack_rows";
+    ATS_REQUIRE(src && bytes && n >= 1 && n <= kMaxStack && out && aligned16(out), ATS_ERR_INVALID_ARG,
+                "%s: %d matrices (at most %d), null or misaligned pointer", name, n, kMaxStack);
+    StackArgs a{};
+    int64_t first = 0, most = 0;
+    for (int i = 0; i < n; ++i) {
+        ATS_REQUIRE(src[i] && aligned16(src[i]) && bytes[i] > 0 && bytes[i] % 16 == 0, ATS_ERR_INVALID_ARG,
+                    "%s: matrix %d of %lld bytes (16-byte aligned, a multiple of 16)", name, i, (long long)bytes[i]);
+        a.src[i] = static_cast<const uint4*>(src[i]);
+        a.first[i] = first;
+        a.n[i] = bytes[i] / 16;
+        first += a.n[i];
+        most = a.n[i] > most ? a.n[i] : most;
+    }
+    int64_t blocks = (most + 1023) / 1024;
+    if (blocks > 2048) blocks = 2048;
+    hipLaunchKernelGGL(stack_rows_kernel, dim3((unsigned)blocks, (unsigned)n), dim3(256), 0, as_stream(stream), a,
+                       static_cast<uint4*>(out), address);
+    ATS_CHECK_LAUNCH(name);
+    return ATS_OK;
+}
 
 extern "C" int ats_upload_max_bytes(void) { return ats::kUploadBytes; }
 

@@ -354,6 +354,23 @@ def address_table(t: torch.Tensor) -> torch.Tensor:
     return upload(array("q", [t.data_ptr()]), t.device)
 
 
+def stack_weights(ws: Sequence[torch.Tensor]) -> Tuple[torch.Tensor, torch.Tensor]:
+    """torch.cat(ws, dim=0) of weights of one type and width, and the address table of the result."""
+    w0 = ws[0]
+    if len(ws) > 8 or not all(w.is_cuda and w.is_contiguous() and w.dim() == 2 and w.dtype == w0.dtype and w.device == w0.device
+                              and w.shape[1] == w0.shape[1] and w.numel() > 0 and w.numel() * w.element_size() % 16 == 0
+                              and w.data_ptr() % 16 == 0 for w in ws):
+        out = torch.cat(list(ws), dim=0)
+        return out, address_table(out)
+    n = len(ws)
+    out = torch.empty(sum(w.shape[0] for w in ws), w0.shape[1], dtype=w0.dtype, device=w0.device)
+    table = torch.empty(1, dtype=torch.int64, device=w0.device)
+    check(_lib.load().ats_stack_rows((ctypes.c_void_p * n)(*[w.data_ptr() for w in ws]),
+                                     (ctypes.c_int64 * n)(*[w.numel() * w.element_size() for w in ws]), n, out.data_ptr(),
+                                     table.data_ptr(), _stream()), "ats_stack_rows")
+    return out, table
+
+
 def upload(words: array, device: torch.device) -> torch.Tensor:
     """An int64 array on the device, sent with launches instead of a copy that waits for the queue."""
     lib, (src, n) = _lib.load(), words.buffer_info()

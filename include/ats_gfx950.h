@@ -427,6 +427,9 @@ typedef struct {
     const int32_t* index;
     int n, kind, wide;
 } ats_table;
+/* out = the n (at most 8) matrices src[i] of bytes[i] one behind the other, all 16-byte aligned and of a multiple of 16 bytes;
+ * *address (on the device, may be NULL) = out, the one-entry pointer table of a grouped product. */
+int ats_stack_rows(const void* const* src, const int64_t* bytes, int n, void* out, int64_t* address, ats_stream_t stream);
 /* Copies at most ats_upload_max_bytes() bytes of host memory to the device inside the arguments of a launch: in stream
  * order, without waiting for the queue, and the host memory may change when the call returns.  dst 8-byte aligned. */
 int ats_upload_max_bytes(void);
