@@ -1914,16 +1914,15 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
 // Float32 products against K-major operands on the small tiles, in microseconds, and what a transposing pass costs.  The
 // tiles' constants are those of launch_grouped, a tenth more per slab for the 4-byte fragment reads (and less per tile for
 // short sums, of which several share a CU).  Copies and their product -> operands as they lie:
-//   weight gradients, rows x [M, N]: 512 x [512, 512] 47 -> 8; 2000 x [512, 512] 75 -> 22; 2048 x [2048, 2048] 225 -> 185;
+//   weight gradients, rows x [M, N]: 512 x [512, 512] 47 -> 8; 2000 x [512, 512] 75 -> 21; 2048 x [2048, 2048] 225 -> 162;
 //     2048 x [4096, 4096] 503 (650); 8 x 128 x [2816, 512] 63 -> 46; 8 x 500 x [2816, 512] 153 -> 132; 8 x 500 x [4096, 1024] 299 (355)
-//   data gradients, rows x [N, K]: 512 x [512, 1024] 41 -> 11; 2000 x [512, 1024] 41 -> 29; 2048 x [2048, 2048] 209 -> 159;
-//     4096 x [4096, 4096] 961 (1196); 8 x 128 x [512, 2816] 56 -> 37; 8 x 250 x [1408, 512] 61 -> 46
-static float small_kmajor_time(int64_t max_rows, int E, int N, int K, bool* wide) {
+//   data gradients, rows x [N, K]: 512 x [512, 1024] 41 -> 11; 2000 x [512, 1024] 41 -> 29; 2048 x [2048, 2048] 209 -> 160;
+//     4096 x [4096, 4096] 961 (1196); 8 x 128 x [512, 2816] 56 -> 37; 8 x 250 x [1408, 512] 61 -> 43
+static float small_kmajor_time(int64_t max_rows, int E, int N, int K) {
     const int nk = (K + 31) / 32;
     const float t32 = tile_time(TileCost{32, 32, 0.20f, 1.5f, 1}, max_rows, E, N, nk);
     const float t64 = tile_time(TileCost{64, 64, 0.64f, 1.6f, 1}, max_rows, E, N, nk);
-    *wide = t64 < t32;
-    return *wide ? t64 : t32;
+    return t64 < t32 ? t64 : t32;
 }
 // The product of copies: their passes at 4 TB/s and 4 us each, then the least of the tiles that launch_grouped has for it.
 static float transposed_time(int64_t max_rows, int E, int N, int K, int64_t copied, int copies) {
@@ -1934,6 +1933,23 @@ static float transposed_time(int64_t max_rows, int E, int N, int K, int64_t copi
         if (t < best) best = t;
     }
     return best + (float)copied * 8.f / 4e6f + 4.f * copies;
+}
+// 64 rows and columns per tile, or 32 (the same bits)?  Groups of unequal rows (uneven) end in half a tile on average, which
+// decides where a CU gets two or three tiles; a CU holds four workgroups of the small tile, two of the large one.  The constants
+// reproduce these within a tenth, microseconds with 64 | 32:
+//   weight gradients, 8 groups, rows in all x [2816, 512]: 500 51 | 43, 1024 64 | 59, 2000 98 | 91, 4000 145 | 153 (second operand
+//     gathered; with the row numbers read where they are needed instead of a slab ahead 56, 72, 117, 192 in 64 rows)
+//   data gradients, 8 groups, rows in all x [512, 2816]: 1024 51 | 51, 2000 113 | 80, 4000 170 | 142; x [1408, 512]: 1024 39 | 26,
+//     2000 50 | 43, 4000 81 | 76; one group 2048 x [2048, 2048] 166 | 175
+static bool kmajor_wide(int64_t max_rows, int E, int N, int K, bool uneven) {
+    const int nk = (K + 31) / 32;
+    const double avg = (double)max_rows / E;
+    auto time = [&](int tile, double per_slab, double per_tile, int min_tiles) {
+        const double rows = uneven ? avg / tile + 0.5 : (double)(((int64_t)ceil(avg) + tile - 1) / tile);
+        const int64_t per_cu = (int64_t)ceil(E * rows * ((N + tile - 1) / tile) / 256.);
+        return (per_cu > min_tiles ? per_cu : min_tiles) * (nk * per_slab + per_tile);
+    };
+    return time(64, 0.62, 3.3, 1) < time(32, 0.17, 0.65, 2);
 }
 
 // Weight gradient of a linear layer, out[m, n] = sum_t a[t, m] b[t, n]: tiles and slices as launch_cfg takes them for the
@@ -2285,9 +2301,8 @@ extern "C" int ats_grouped_gemm_nn_sliced(const void* a, int64_t lda, const void
 
 extern "C" int ats_grouped_gemm_nn_f32_supported(int E, int64_t max_rows, int N, int K) {
     using namespace ats;
-    bool wide;
     if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || N % 4 != 0 || K % 4 != 0) return 0;
-    return small_kmajor_time(max_rows, E, N, K, &wide) <= transposed_time(max_rows, E, N, K, (int64_t)E * N * K, 1) ? 1 : 0;
+    return small_kmajor_time(max_rows, E, N, K) <= transposed_time(max_rows, E, N, K, (int64_t)E * N * K, 1) ? 1 : 0;
 }
 extern "C" int ats_grouped_gemm_nn_f32(const float* a, int64_t lda, const void* const* b_ptrs, int64_t ldb, float* out, int64_t ldo,
                                        const int32_t* row_start, const int32_t* row_count, int E, int64_t max_rows, int N, int K,
@@ -2315,10 +2330,9 @@ extern "C" int ats_grouped_gemm_nn_f32(const float* a, int64_t lda, const void* 
     p.E = E;
     p.K = K;
     p.N_out = N;
-    bool wide;
-    small_kmajor_time(max_rows, E, N, K, &wide);
-    const int rc = wide ? launch_small<float, float, 2, 2, 4, 1, false, false, true>(p, max_rows, as_stream(stream))
-                        : launch_small<float, float, 1, 1, 4, 1, false, false, true>(p, max_rows, as_stream(stream));
+    const int rc = kmajor_wide(max_rows, E, N, K, E > 1)
+                       ? launch_small<float, float, 2, 2, 4, 1, false, false, true>(p, max_rows, as_stream(stream))
+                       : launch_small<float, float, 1, 1, 4, 1, false, false, true>(p, max_rows, as_stream(stream));
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;
@@ -2327,10 +2341,9 @@ extern "C" int ats_grouped_gemm_nn_f32(const float* a, int64_t lda, const void* 
 // (max_k: bound on the sum over the groups)
 extern "C" int ats_grouped_wgrad_f32_supported(int E, int64_t max_k, int M, int N) {
     using namespace ats;
-    bool wide;
     if (E <= 0 || max_k <= 0 || max_k > 0x7fffffff || M <= 0 || N <= 0 || M % 4 != 0 || N % 4 != 0) return 0;
     const int k = (int)((max_k + E - 1) / E);
-    return small_kmajor_time((int64_t)E * M, E, N, k, &wide) <=
+    return small_kmajor_time((int64_t)E * M, E, N, k) <=
                    transposed_time((int64_t)E * M, E, N, k + 16, max_k * ((int64_t)M + N), 2) ? 1 : 0;
 }
 extern "C" int ats_grouped_wgrad_f32(const float* a, int64_t lda, const float* b, int64_t ldb, const int32_t* b_rows, int b_row_div,
@@ -2360,10 +2373,9 @@ extern "C" int ats_grouped_wgrad_f32(const float* a, int64_t lda, const float* b
     p.E = E;
     p.K = (int)max_k;
     p.N_out = N;
-    bool wide;
-    small_kmajor_time((int64_t)E * M, E, N, (int)((max_k + E - 1) / E), &wide);
-    const int rc = wide ? launch_small<float, float, 2, 2, 4, 1, false, true, true>(p, (int64_t)E * M, as_stream(stream))
-                        : launch_small<float, float, 1, 1, 4, 1, false, true, true>(p, (int64_t)E * M, as_stream(stream));
+    const int rc = kmajor_wide((int64_t)E * M, E, N, (int)((max_k + E - 1) / E), false)
+                       ? launch_small<float, float, 2, 2, 4, 1, false, true, true>(p, (int64_t)E * M, as_stream(stream))
+                       : launch_small<float, float, 1, 1, 4, 1, false, true, true>(p, (int64_t)E * M, as_stream(stream));
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;

@@ -111,23 +111,29 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
     unsigned char* const st_at = stage + lrow * kRowPitch + lchunk * 16;
     const unsigned char* const fr_at = stage + (lane & 31) * kRowPitch + (lane >> 5) * 16;
 
+    // K-major: rows past K repeat the last one and are cleared on their way into LDS, so that no load has a branch of its own;
+    // the gathered rows' numbers are asked for a slab ahead of the rows
+    int rn[NIB];
+    auto rows_of = [&](int slab) {
+#pragma unroll
+        for (int i = 0; i < NIB; ++i) rn[i] = p.b_rows[k_row0 + min(slab * BK + i * RB + lane / CB, K - 1)];
+    };
+    const bool gathered = AKM && p.b_rows;
     auto load = [&](int slab) {
         const int koff = slab * BK;
         const bool ok = koff + lchunk * VEC < K;    // false only in the last slab of a ragged K
 #pragma unroll
         for (int i = 0; i < NIA; ++i) {
             if constexpr (AKM) {
-                const int k = koff + i * RA + lane / CA;
-                ra[i] = k < K ? *reinterpret_cast<const u32x4_t*>(akm + ((int64_t)k_row0 + k) * p.lda) : zero4;
+                const int k = min(koff + i * RA + lane / CA, K - 1);
+                ra[i] = *reinterpret_cast<const u32x4_t*>(akm + ((int64_t)k_row0 + k) * p.lda);
             } else ra[i] = ok ? *reinterpret_cast<const u32x4_t*>(ap[i] + koff) : zero4;
         }
 #pragma unroll
         for (int i = 0; i < NIB; ++i) {
             if constexpr (BKM) {
-                const int k = koff + i * RB + lane / CB;
-                int64_t r = (int64_t)k_row0 + k;
-                if (AKM && p.b_rows && k < K) r = p.b_rows[r] / p.b_row_div;
-                rb[i] = k < K ? *reinterpret_cast<const u32x4_t*>(bkm + r * p.ldb) : zero4;
+                const int64_t r = gathered ? rn[i] / p.b_row_div : (int64_t)k_row0 + min(koff + i * RB + lane / CB, K - 1);
+                rb[i] = *reinterpret_cast<const u32x4_t*>(bkm + r * p.ldb);
             } else rb[i] = ok ? *reinterpret_cast<const u32x4_t*>(bp[i] + koff) : zero4;
         }
     };
@@ -139,8 +145,20 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
             f[c] = *reinterpret_cast<const uint32_t*>(at + (8 * ks + 4 * (lane >> 5) + c) * pitch + (lane & 31) * 4);
         return f;
     };
-    if (kw < nk) load(kw);
+    if (kw < nk) {
+        if (gathered) rows_of(kw);
+        load(kw);
+        if (gathered && kw + KW < nk) rows_of(kw + KW);
+    }
     for (int s = kw; s < nk; s += KW) {
+        if (BKM && (s + 1) * BK > K) {
+#pragma unroll
+            for (int i = 0; i < NIA; ++i)
+                if (AKM && s * BK + i * RA + lane / CA >= K) ra[i] = zero4;
+#pragma unroll
+            for (int i = 0; i < NIB; ++i)
+                if (s * BK + i * RB + lane / CB >= K) rb[i] = zero4;
+        }
 #pragma unroll
         for (int i = 0; i < NIA; ++i)
             *reinterpret_cast<u32x4_t*>(AKM ? stage + (i * RA + lane / CA) * PA + lane % CA * 16 : st_at + i * 8 * kRowPitch) = ra[i];
@@ -150,7 +168,10 @@ __global__ __launch_bounds__(KW* WG* WG * 64) void grouped_gemm_small_kernel(Gro
                                             : st_at + (BM + i * 8) * kRowPitch) = rb[i];
         // other lanes' pieces are read below: nothing may move across (the wave's LDS accesses themselves are in order)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (s + KW < nk) load(s + KW);
+        if (s + KW < nk) {
+            load(s + KW);
+            if (gathered && s + 2 * KW < nk) rows_of(s + 2 * KW);
+        }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             u32x4_t fa[TM], fb[TN];
