@@ -114,6 +114,7 @@ _SIGNATURES = {
     "ats_grouped_gemm_nt": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int, c_void_p, c_int64, c_int64,
                                     c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_int,
                                     c_int, c_int, c_void_p]),
+    "ats_linear_nt": (c_int, [c_void_p] * 5 + [c_int64] + [c_int] * 3 + [c_void_p]),
     "ats_stack_rows": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p]),
     "ats_upload_max_bytes": (c_int, []),
     "ats_upload": (c_int, [c_void_p, c_void_p, c_int, c_void_p]),

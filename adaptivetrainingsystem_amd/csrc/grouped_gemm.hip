@@ -2593,6 +2593,50 @@ extern "C" int ats_grouped_gemm_nt(const void* a, const void* const* a_ptrs, int
     return ATS_OK;
 }
 
+// A linear layer: one group whose results no grouped launch has to repeat, so that float32 sums may be cut into slices of K at
+// any number of rows (up to 256 launch_grouped does so itself).  Two of the 64-row workgroups share a CU: an odd third costs as
+// much as a fourth.  [N, K] x rows, all of K in a wave -> slices, microseconds (half the error: four chains instead of one):
+//   [1024, 512] x 512 18 -> 10, x 1000 18 -> 15, x 2000 28 -> 27; [512, 1408] x 512 40 -> 13, x 2000 40 -> 33;
+//   [2048, 2048] x 257 58 -> 42, x 700 91 -> 76, x 1500 140 (147), x 2000 193 -> 160; x 4096 240 in 256-row tiles
+extern "C" int ats_linear_nt(const void* x, const void* const* w, void* out, const int32_t* row_start, const int32_t* row_count,
+                             int64_t T, int N, int K, int dtype, ats_stream_t stream) {
+    using namespace ats;
+    const char* name = "ats_linear_nt";
+    if (dtype == ATS_F32 && T > 256 && T <= 0x7fffffff && N > 0 && K > 0 && N % 4 == 0 && K % 4 == 0 && x && w && out && row_start &&
+        row_count && aligned16(x) && aligned16(out)) {
+        const int nk = (K + 31) / 32;
+        const int64_t tiles = ((T + 63) / 64) * ((N + 63) / 64);
+        const float t64 = (float)(tiles <= 256 ? 1 : (tiles + 511) / 512 * 2) * (nk * 0.58f + 3.f);
+        const float t32 = tile_time(TileCost{32, 32, 0.18f, 1.5f, 1}, T, 1, N, nk);
+        float others = tile_time(TileCost{64, 64, 0.74f, 3.f, 1}, T, 1, N, nk);
+        for (const TileCost& c : {TileCost{128, 256, 3.65f, 5.f, 1}, TileCost{256, 256, 7.3f, 7.f, 1}}) {
+            const float t = tile_time(c, T, 1, N, nk);
+            if (t < others) others = t;
+        }
+        if (t32 < others || t64 < others) {
+            GroupedArgs p{};
+            p.a = x;
+            p.a_row_div = 1;
+            p.lda = p.ldb = K;
+            p.b = w;
+            p.out = out;
+            p.ldo = N;
+            p.row_start = row_start;
+            p.row_count = row_count;
+            p.E = 1;
+            p.K = K;
+            p.N_out = N;
+            const int rc = t32 <= t64 ? launch_small<float, float, 1, 1, 4, 1, false>(p, T, as_stream(stream))
+                                      : launch_small<float, float, 2, 2, 4, 1, false>(p, T, as_stream(stream));
+            if (rc != ATS_OK) return rc;
+            ATS_CHECK_LAUNCH(name);
+            return ATS_OK;
+        }
+    }
+    return ats_grouped_gemm_nt(x, nullptr, K, T, nullptr, 1, w, K, N, out, N, row_start, row_count, nullptr, 1, T, N, K, dtype, dtype,
+                               stream);
+}
+
 // Device-side view of the tile schedule: one wave per block id evaluates decode_tile_wave (the search the GEMM
 // kernels run) and writes {expert, m_tile, n_tile, slice}, or -1s where the block owns no tile.
 namespace ats {

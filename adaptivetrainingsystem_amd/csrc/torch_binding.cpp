@@ -198,8 +198,7 @@ std::optional<Tensor> linear(const Tensor& x, const Tensor& table, const Tensor&
               "ats_grouped_down_splitk");
         check(ats_sum_partials(p, (int)splits, T * N, out.data_ptr(), T * N, tag(x), stream()), "ats_sum_partials");
     } else {
-        check(ats_grouped_gemm_nt(x.data_ptr(), nullptr, K, T, nullptr, 1, b, K, N, out.data_ptr(), N, rs, rc, nullptr, 1, T, (int)N,
-                                  (int)K, tag(x), tag(x), stream()), "ats_grouped_gemm_nt");
+        check(ats_linear_nt(x.data_ptr(), b, out.data_ptr(), rs, rc, T, (int)N, (int)K, tag(x), stream()), "ats_linear_nt");
     }
     return out;
 }

@@ -1608,4 +1608,7 @@ def linear_nt(x: torch.Tensor, weight: torch.Tensor, table: Optional[torch.Tenso
         return done
     if splits > 1:      # a few rows against a whole weight matrix: slices of K keep every CU streaming
         return sum_partials(grouped_down_splitk(x, table, start, count, T, N, K, splits), x.dtype)
-    return grouped_gemm_nt(table, K, N, start, count, T, T, N, K, a=x)
+    out = torch.empty(T, N, dtype=x.dtype, device=x.device)
+    check(_lib.load().ats_linear_nt(x.data_ptr(), table.data_ptr(), out.data_ptr(), start.data_ptr(), count.data_ptr(), T, N, K,
+                                    _tag(x), _stream()), "ats_linear_nt")
+    return out

@@ -462,6 +462,10 @@ int ats_grouped_gemm_nt(const void* a, const void* const* a_ptrs, int64_t lda, i
                         int64_t b_rows, void* out, int64_t ldo, const int32_t* row_start,
                         const int32_t* row_count, const int32_t* k_count, int E, int64_t max_rows, int N,
                         int K, int dtype, int out_dtype, ats_stream_t stream);
+/* The product of a linear layer, out [T, N] = x [T, K] . W^T with W = w[0] [N, K]; row_start = {0}, row_count = {T} on the device.
+ * ats_grouped_gemm_nt of one group, except that float32 sums may be cut along K (another order of additions, shorter chains). */
+int ats_linear_nt(const void* x, const void* const* w, void* out, const int32_t* row_start, const int32_t* row_count, int64_t T,
+                  int N, int K, int dtype, ats_stream_t stream);
 /* Grouped product against weights stored with the reduction index along their rows:
  * out[row_start[e]+m, n] = sum_k A_e[m,k] * B_e[k,n], B_e = b_ptrs[e] ([K, ldb >= N]).
  * The data gradient of a linear layer, dX = dY . W with W = [out_features, in_features] as the forward holds it
