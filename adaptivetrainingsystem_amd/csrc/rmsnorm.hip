@@ -159,19 +159,23 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
     }
 }
 
-// A workgroup per row.  Few rows (decoding steps): what a launch takes is one row's chain of loads, arithmetic and stores, a
-// quarter as long here as in a wave.  Long rows: a wave holds 64 .. 128 values and weights per lane, too many registers to
-// keep the memory busy; here they are 4 .. 16.  Wave per row -> this, microseconds, buffers from HBM above 1024 rows:
-//   bfloat16 [64, 4096] 4.9 -> 2.9   [512, 2048] 4.2 -> 3.1   [4096, 2048]  9.5 ->  8.3   [8192, 2048] 10.9 (13.7)
-//            [512, 4096] 5.5 -> 3.6  [4096, 4096] 14.8 -> 13.0   [16384, 4096] 47.6 -> 44.3 (6.1 TB/s)
-//   float32  [64, 4096] 10.2 -> 3.4  [512, 4096] 11.5 -> 5.9   [4096, 4096] 31.2 -> 23.4  [16384, 4096] 135 -> 88
-//            [512, 2048] 4.3 -> 3.8  [2048, 2048]  7.1 (7.4)
+// A workgroup per row.  Few rows (decoding steps): what a launch takes is one row's chain of loads, arithmetic and stores, and
+// four waves load, scale and store it.  Long rows: a wave holds 64 .. 128 values and weights per lane, too many registers to
+// keep the memory busy; here they are 4 .. 16.  The squares are added up in the order of rmsnorm_rows_kernel and of the backward
+// pass, every wave walking the whole row in LDS: a row has the same bits whatever the number of rows beside it, and the
+// scale that the gradient recomputes is the forward's.  (Four partial sums, one per wave, made the launch 0.2-0.4 us shorter, 0-5 %
+// of the time of many rows.)  Wave per row -> this, microseconds, buffers from HBM above 1024 rows:
+//   bfloat16 [64, 4096] 5.0 -> 3.7   [512, 2048] 4.5 -> 3.6   [4096, 2048]  9.6 ->  8.2   [64, 8192] 8.5 -> 5.0
+//            [512, 4096] 5.7 -> 4.5  [4096, 4096] 14.9 -> 13.0   [16384, 4096] 47.0 -> 45.8 (5.9 TB/s)
+//            [1024, 8192] with float32 weights 8.5 (9.4), [512 | 2048] 6.4 -> 5.9 | 16.0 -> 15.8
+//   float32  [64, 4096] 8.5 -> 3.6   [512, 4096] 11.4 -> 5.4   [4096, 4096] 31.7 -> 24.4  [16384, 4096] 136 -> 92
+//            [512, 2048] 4.3 -> 4.0
 template <typename T, typename WT, int NV, bool HAS_W>
 __global__ __launch_bounds__(256) void rmsnorm_row_block_kernel(const T* __restrict__ x, const WT* __restrict__ w,
                                                                 T* __restrict__ y, int64_t rows, int H, float eps) {
     constexpr int V = Elem<T>::kVec;
-    __shared__ float s_part[4];
-    const int nvec = H / V;
+    __shared__ uint4 s_row[NV * 256];
+    const int nvec = H / V, lane = lane_id();
     uint4 raw[NV], nxt[NV];
     float wreg[NV][V];
     auto fetch = [&](int64_t row, uint4(&to)[NV]) {
@@ -192,19 +196,19 @@ __global__ __launch_bounds__(256) void rmsnorm_row_block_kernel(const T* __restr
 #pragma unroll
         for (int i = 0; i < NV; ++i) raw[i] = nxt[i];
         if (row + gridDim.x < rows) fetch(row + gridDim.x, nxt);
+        __syncthreads();      // the row before this one has been added up
+#pragma unroll
+        for (int i = 0; i < NV; ++i) s_row[threadIdx.x + i * 256] = raw[i];
+        __syncthreads();
         float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
+        for (int i = 0; i < 4 * NV; ++i) {      // (vectors past the row are zero)
             float f[V];
-            Elem<T>::unpack(raw[i], f);
+            Elem<T>::unpack(s_row[lane + i * kWave], f);
 #pragma unroll
             for (int j = 0; j < V; ++j) ss += f[j] * f[j];
         }
         ss = wave_sum(ss);
-        __syncthreads();
-        if (lane_id() == 0) s_part[threadIdx.x >> 6] = ss;
-        __syncthreads();
-        ss = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
         const float r = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
