@@ -13,8 +13,10 @@
 //                of V, whose columns 64 jj + 4 (l % 16) + i belong to the output tile (jj, i).
 // The waves' partial results meet in LDS in wave order: nothing depends on timing.
 // Values are those of the materialised route: scale, causal fill with -1e4 (Src/Main_Scripts/core/model.py:813-817), the
-// additive mask of the keys (819-824), softmax.  A row whose visible scores all lie near or below the fill gives weight
-// to its future keys, as the fill does; the workgroup then walks all keys.
+// additive mask of the keys (819-824), softmax.  The fill is a score like any other: a row whose visible scores all lie near
+// or below it gives weight to its future keys, and so does a row before a key whose mask lifts the fill (it is added behind
+// it).  The workgroup then walks all keys; it skips future keys only where the largest of their scores, fill plus mask, is so far
+// below the row's maximum that its exponential is zero in float32.
 // Bounds: launches and the serial chain of a tile (32 MFMAs of 32 cycles per product) at short sequences, L1 traffic at long
 // ones (every tile is read in both layouts).  Materialised route -> this, microseconds, forward | backward:
 //   2 x 54, 4 heads of 128    88 ->    8 |   158 ->   21        1 x 1024, 32 heads of 128   287 ->  165 |   639 ->  712
@@ -30,9 +32,9 @@ namespace ats {
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-// Below this row maximum exp(-1e4 - max) is no longer zero in float32 (it is from 104 on).
-constexpr float kFillMatters = -9800.f;
 constexpr float kFill = -1e4f;
+// Whether a row of this maximum gives weight to keys whose largest score is `fill` (exp(-104) is zero in float32; not a number: yes).
+__device__ __forceinline__ bool gives_weight(float fill, float top) { return !(fill - top <= -200.f); }
 
 struct AttnF32Args {
     const float *q, *k, *v, *out, *dout;     // q [B,Hq,L,D], k, v [B,Hkv,Lk,D], out, dout [B,L,Hq*D]
@@ -103,10 +105,22 @@ __device__ __forceinline__ float score(float s, float scale, int key, int last_k
     return key < Lk ? t : -INFINITY;
 }
 
+// largest of kb[from .. Lk), in every thread of the wave whose workgroup shares the keys out (NaN as infinity)
+__device__ __forceinline__ float largest_bias(const float* kb, int from, int Lk) {
+    float m = -INFINITY;
+    for (int j = from + threadIdx.x; j < Lk; j += blockDim.x) {
+        const float b = kb[j];
+        m = b <= m ? m : b == b ? b : INFINITY;
+    }
+#pragma unroll
+    for (int s = 1; s < 64; s *= 2) m = fmaxf(m, __shfl_xor(m, s, 64));
+    return m;
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void attention_f32_fwd_kernel(AttnF32Args p) {
     constexpr int W = 4;
-    __shared__ float s_m[W][16], s_l[W][16];
+    __shared__ float s_m[W][16], s_l[W][16], s_b[W];
     __shared__ __align__(16) float s_o[W][16 * (D + 4)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
@@ -165,9 +179,14 @@ __global__ __launch_bounds__(256) void attention_f32_fwd_kernel(AttnF32Args p) {
         for (int w = 1; w < W; ++w) mx = fmaxf(mx, s_m[w][c]);
         return mx;
     };
+    if (kb && visible < all) {
+        const float b = largest_bias(kb, 16 * visible, p.Lk);
+        if (lane == 0) s_b[wave] = b;
+    }
     walk(0, visible);
     float top = exchange();
-    if (visible < all && __any(top < kFillMatters)) {      // the same rows in every wave, hence the same answer
+    const float fill = kb && visible < all ? kFill + fmaxf(fmaxf(s_b[0], s_b[1]), fmaxf(s_b[2], s_b[3])) : kFill;
+    if (visible < all && __any(gives_weight(fill, top))) {      // the same rows in every wave, hence the same answer
         __syncthreads();
         walk(visible, all);
         top = exchange();
@@ -203,7 +222,7 @@ __global__ __launch_bounds__(256) void attention_f32_fwd_kernel(AttnF32Args p) {
 template <int D>
 __global__ __launch_bounds__(256) void attention_f32_dq_kernel(AttnF32Args p) {
     constexpr int W = 4;
-    __shared__ float s_d[W][16];
+    __shared__ float s_d[W][16], s_b[W];
     __shared__ __align__(16) float s_o[W][16 * (D + 4)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
@@ -229,7 +248,14 @@ __global__ __launch_bounds__(256) void attention_f32_dq_kernel(AttnF32Args p) {
     const int all = (p.Lk + 15) / 16;
     const int past_last = q0 + 16 + p.Lk - p.L;
     int end = past_last < p.Lk ? (past_last + 15) / 16 : all;
-    if (__any(top < kFillMatters)) end = all;
+    float fill = kFill;
+    if (kb && end < all) {
+        const float bias = largest_bias(kb, 16 * end, p.Lk);
+        if (lane == 0) s_b[wave] = bias;
+        __syncthreads();
+        fill += fmaxf(fmaxf(s_b[0], s_b[1]), fmaxf(s_b[2], s_b[3]));
+    }
+    if (__any(gives_weight(fill, top))) end = all;
     auto weights = [&](int kt, f32x4v& w, f32x4v& dp) {
         const int j = 16 * kt + c < p.Lk ? 16 * kt + c : p.Lk - 1;
         f32x4v kf[D / 16], vf[D / 16];
@@ -307,13 +333,21 @@ __global__ __launch_bounds__(512) void attention_f32_dkv_kernel(AttnF32Args p) {
     f32x4v kf[D / 16], vf[D / 16];
     load_rows<D>(kf, p.k + ((int64_t)blockIdx.y * p.Lk + key) * D, g);
     load_rows<D>(vf, p.v + ((int64_t)blockIdx.y * p.Lk + key) * D, g);
+    float fill = kFill;                                          // largest score of these keys in the rows before them
+    if (kb) {
+        const float own = kb[key];
+        float bias = own == own ? own : INFINITY;
+#pragma unroll
+        for (int x = 1; x < 16; x *= 2) bias = fmaxf(bias, __shfl_xor(bias, x, 64));
+        fill += bias;
+    }
     // query tiles before `first` see none of these keys, unless a row gives weight to its future
     int first = k0 - off > 0 ? (k0 - off) / 16 : 0;
     const int tiles = (p.L + 15) / 16;
     first = first < tiles ? first : tiles;
     bool early = false;
     for (int h = 0; h < rep; ++h)
-        for (int i = threadIdx.x; i < first * 16; i += W * 64) early |= p.stats[((e0 + h) * p.L + i) * 2] < kFillMatters;
+        for (int i = threadIdx.x; i < first * 16; i += W * 64) early |= gives_weight(fill, p.stats[((e0 + h) * p.L + i) * 2]);
     if (__syncthreads_or(early)) first = 0;
     f32x4v dk[D / 64][4], dv[D / 64][4];
 #pragma unroll

@@ -81,3 +81,54 @@ def test_routes_that_stay_materialised(gpu):
     assert not ops.attention_f32_fused_supported(t, t, t, None, 0.1)
     assert not ops.attention_f32_fused_supported(t[..., :32].contiguous(), t, t, None, 0.0)
     assert not ops.attention_f32_fused_supported(t.transpose(1, 2), t, t, None, 0.0)
+
+
+@pytest.mark.parametrize("L,Lk,at,lift", [(100, 100, (0, 17, 50, 99), 1e4), (33, 70, (40, 69), 1.9e4), (20, 20, (16,), 9990.0),
+                                          (64, 64, (63,), 1e9), (300, 300, (299, 150), 9.93e3), (48, 48, (5, 47), float("inf"))])
+@pytest.mark.parametrize("masked", [False, True])
+def test_future_keys_that_their_bias_lifts_above_the_fill(gpu, L, Lk, at, lift, masked):
+    """The bias is added after the causal fill, so a future key whose bias outweighs the fill has weight in every row before it, in
+    whatever tile it lies; with `masked` the row's own keys lie lower still."""
+    print("case f32 attention lifted keys", L, Lk, at, lift, masked, flush=True)
+    from adaptivetrainingsystem_amd import ops
+    B, Hq, Hkv, D = 2, 4, 2, 64
+    g = torch.Generator().manual_seed(L + Lk)
+    q, dout = torch.randn(B, Hq, L, D, generator=g).to(gpu), torch.randn(B, L, Hq * D, generator=g).to(gpu)
+    k, v = (torch.randn(B, Hkv, Lk, D, generator=g).to(gpu) for _ in range(2))
+    bias = torch.zeros(B, Lk)
+    if masked:
+        bias[0, : Lk // 2] = -1e4
+        bias[1] = -3e3
+    for j in at:
+        bias[j % B, j] = lift
+    bias = bias.to(gpu)
+    scale = D ** -0.5
+    want, state = ops.attention_f32(q, k, v, scale, key_bias=bias, return_weights=True)
+    want_grads = ops.attention_f32_bwd(state, dout, B, Hq, Hkv, L, Lk, D, scale)
+    out, stats = ops.attention_f32_fused(q, k, v, scale, bias)
+    grads = ops.attention_f32_fused_bwd(q, k, v, out, stats, dout, scale, bias)
+    # scores near 1e4 .. 2e4 are known to 1e-3 .. 2e-3 in float32 on either route (one unit in the last place); where one key has all
+    # the weight, the gradients of q and k are zero up to the rounding of terms as large as dout (1.5e-6, as above)
+    for a, r in zip((out, *grads), (want, *want_grads)):
+        assert torch.equal(a.isnan(), r.isnan())
+        assert (a - r).nan_to_num().norm() <= 4e-3 * r.nan_to_num().norm() + 1.5e-6 * dout.norm()
+    assert torch.equal(ops.attention_f32(q, k, v, scale, key_bias=bias).nan_to_num(), out.nan_to_num())
+
+
+def test_a_mask_value_above_one_through_the_module(gpu):
+    """An attention mask holds (1 - m) * -1e4 as a bias: a value of 2 lifts its key by 1e4."""
+    from types import SimpleNamespace
+    from adaptivetrainingsystem_amd import ops
+    from adaptivetrainingsystem_amd.layers import GroupedQueryAttention
+    torch.manual_seed(2)
+    att = GroupedQueryAttention(SimpleNamespace(hidden_size=256, num_heads=4, num_kv_heads=2, seq_length=128)).to(gpu).eval()
+    x, mask = torch.randn(2, 80, 256, device=gpu), torch.ones(2, 80, device=gpu)
+    mask[:, 70] = 2.0
+    with torch.no_grad():
+        got = att(x, mask)
+        cos, sin = att.rope(80, x.device)
+        q, k, v = (ops.linear_nt(x.view(160, 256), p.weight).view(2, 80, -1, 64).transpose(1, 2) for p in (att.q_proj, att.k_proj, att.v_proj))
+        q, k = ops.rope(q, k, cos, sin)
+        a, _ = ops.attention_f32(q, k, v.contiguous(), 0.125, key_bias=(1.0 - mask) * -1e4, return_weights=True)
+        want = ops.linear_nt(a.view(160, 256), att.o_proj.weight).view_as(got)
+    assert (got - want).norm() <= 4e-3 * want.norm()
