@@ -1382,6 +1382,18 @@ def _pad_rows(t: torch.Tensor, rows: int) -> torch.Tensor:
     return out
 
 
+def _attention_f32_dims(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> Tuple[int, int, int, int, int, int]:
+    """(B, Hq, Hkv, L, Lk, D) of a float32 attention, on either of its routes; raises for tensors that do not fit together."""
+    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or q.dtype != torch.float32 or k.dtype != q.dtype or v.dtype != q.dtype:
+        raise AtsError("attention_f32: q, k, v must be 4-D float32 tensors [batch, heads, seq, head_dim]")
+    B, Hq, L, D = q.shape
+    Hkv, Lk = k.shape[1], k.shape[2]
+    if k.shape != (B, Hkv, Lk, D) or v.shape != (B, Hkv, Lk, D) or Hq % Hkv != 0 or Lk < L or D % 4 or B * Hq > 4096:
+        raise AtsError(f"attention_f32: shapes q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)} "
+                       "(head_dim a multiple of 4, at most 4096 (batch, head) pairs)")
+    return B, Hq, Hkv, L, Lk, D
+
+
 def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None,
                   key_bias: Optional[torch.Tensor] = None, pair_bias: Optional[torch.Tensor] = None,
                   dropout_p: float = 0.0, dropout_seed: int = 0, return_weights: bool = False):
@@ -1391,14 +1403,8 @@ def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Opti
     and multiplied with V by a second grouped product.  q [B,Hq,L,D], k, v [B,Hkv,Lk,D], D a multiple of 4;
     key_bias / pair_bias / dropout as in causal_attention.  Returns out [B, L, Hq*D]; with return_weights also
     the state the backward needs (padded weights before and after dropout)."""
+    B, Hq, Hkv, L, Lk, D = _attention_f32_dims(q, k, v)
     _need_gpu(q, k, v)
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or q.dtype != torch.float32 or k.dtype != q.dtype or v.dtype != q.dtype:
-        raise AtsError("attention_f32: q, k, v must be 4-D float32 tensors [batch, heads, seq, head_dim]")
-    B, Hq, L, D = q.shape
-    Hkv, Lk = k.shape[1], k.shape[2]
-    if k.shape != (B, Hkv, Lk, D) or v.shape != (B, Hkv, Lk, D) or Hq % Hkv != 0 or Lk < L or D % 4 or B * Hq > 4096:
-        raise AtsError(f"attention_f32: shapes q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)} "
-                       "(head_dim a multiple of 4, at most 4096 (batch, head) pairs)")
     key_bias = _key_bias(key_bias, B, Lk, q, "attention_f32")
     if not 0.0 <= dropout_p < 1.0:
         raise AtsError(f"attention_f32: dropout_p {dropout_p} must be in [0, 1)")
@@ -1440,42 +1446,44 @@ def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Opti
 def attention_f32_fused_supported(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pair_bias: Optional[torch.Tensor],
                                   dropout_p: float) -> bool:
     """Whether the kernels without materialised scores take this call (csrc/attention_f32_fused.hip)."""
-    return (pair_bias is None and dropout_p == 0.0 and q.shape[3] in (64, 128) and q.shape[2] > 0 and q.shape[0] > 0
+    return (pair_bias is None and dropout_p == 0.0 and q.shape[-1] in (64, 128) and q.numel() > 0
             and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (q, k, v)))
 
 
-def attention_f32_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float, key_bias: Optional[torch.Tensor],
-                        want_stats: bool = True) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+def attention_f32_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float],
+                        key_bias: Optional[torch.Tensor], want_stats: bool = True) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """attention_f32 in one launch: out [B, L, Hq*D] and, for the backward pass, the maximum and the reciprocal sum of
     every row [B*Hq, L, 2]."""
+    B, Hq, Hkv, L, Lk, D = _attention_f32_dims(q, k, v)
     _need_gpu(q, k, v)
-    B, Hq, L, D = q.shape
-    Hkv, Lk = k.shape[1], k.shape[2]
+    if not attention_f32_fused_supported(q, k, v, None, 0.0):
+        raise AtsError("attention_f32_fused: contiguous, 16-byte aligned rows of head_dim 64 or 128")
+    scale = float(D ** -0.5 if scale is None else scale)
     key_bias = _key_bias(key_bias, B, Lk, q, "attention_f32")
     out = torch.empty(B, L, Hq * D, dtype=torch.float32, device=q.device)
     stats = torch.empty(B * Hq, L, 2, dtype=torch.float32, device=q.device) if want_stats else None
     check(_lib.load().ats_attention_f32_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _ptr(stats), B, Hq, Hkv,
-                                            L, Lk, D, float(scale), _ptr(key_bias), _stream()), "ats_attention_f32_fwd")
+                                            L, Lk, D, scale, _ptr(key_bias), _stream()), "ats_attention_f32_fwd")
     return out, stats
 
 
 def attention_f32_fused_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, stats: torch.Tensor,
-                            dout: torch.Tensor, scale: float, key_bias: Optional[torch.Tensor]):
+                            dout: torch.Tensor, scale: Optional[float], key_bias: Optional[torch.Tensor]):
     """Gradients of attention_f32_fused: (dq, dk, dv) in two launches."""
+    B, Hq, Hkv, L, Lk, D = _attention_f32_dims(q, k, v)
+    if any(t.shape != shape or t.dtype != torch.float32 for t, shape in ((out, (B, L, Hq * D)), (dout, (B, L, Hq * D)),
+                                                                         (stats, (B * Hq, L, 2)))):
+        raise AtsError("attention_f32_fused_bwd: out and dout must be float32 [batch, seq, heads * head_dim], stats as handed out")
     _need_gpu(q, k, v, out, stats, dout)
-    B, Hq, L, D = q.shape
-    Hkv, Lk = k.shape[1], k.shape[2]
-    if dout.shape != out.shape or dout.dtype != torch.float32:
-        raise AtsError("attention_f32_fused_bwd: dout must be float32 of the output's shape")
-    dout = dout.contiguous()
-    if dout.data_ptr() % 16:
-        dout = dout.clone()
+    q, k, v, out, stats, dout = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+                                 for t in (q, k, v, out, stats, dout))
+    scale = float(D ** -0.5 if scale is None else scale)
     key_bias = _key_bias(key_bias, B, Lk, q, "attention_f32")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     delta = torch.empty(B * Hq * L, dtype=torch.float32, device=q.device)
     check(_lib.load().ats_attention_f32_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), stats.data_ptr(),
                                             dout.data_ptr(), delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B,
-                                            Hq, Hkv, L, Lk, D, float(scale), _ptr(key_bias), _stream()),
+                                            Hq, Hkv, L, Lk, D, scale, _ptr(key_bias), _stream()),
           "ats_attention_f32_bwd")
     return dq, dk, dv
 

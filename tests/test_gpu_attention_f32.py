@@ -132,3 +132,19 @@ def test_a_mask_value_above_one_through_the_module(gpu):
         a, _ = ops.attention_f32(q, k, v.contiguous(), 0.125, key_bias=(1.0 - mask) * -1e4, return_weights=True)
         want = ops.linear_nt(a.view(160, 256), att.o_proj.weight).view_as(got)
     assert (got - want).norm() <= 4e-3 * want.norm()
+
+
+def test_the_scale_may_be_left_to_the_head_dim_and_saved_tensors_may_come_back_elsewhere(gpu):
+    from adaptivetrainingsystem_amd.autograd import AttentionF32Function
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(2, h, 20, 64, generator=g).to(gpu).requires_grad_() for h in (4, 2, 2))
+    dout = torch.randn(2, 20, 256, generator=g).to(gpu)
+    want = torch.autograd.grad(AttentionF32Function.apply(q, k, v, 0.125), (q, k, v), dout)
+
+    def unpack(t):      # the same numbers behind another stride and alignment
+        room = torch.empty(t.numel() + 1, device=gpu)[1:]
+        return room.view(t.shape[::-1]).permute(*range(t.dim() - 1, -1, -1)).copy_(t)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        out = AttentionF32Function.apply(q, k, v, None)
+    for a, b in zip(torch.autograd.grad(out, (q, k, v), dout), want):
+        assert torch.equal(a, b)

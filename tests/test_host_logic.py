@@ -267,3 +267,28 @@ def test_slices_of_a_weight_gradient(rows, M, N, slices):
     """The choice at the measured sizes (the fastest or within 2 % of it)."""
     from adaptivetrainingsystem_amd import ops
     assert ops.wgrad_slices(M, N, rows) == slices
+
+
+# bfloat16, a smaller head_dim, fewer values than keys, fewer keys than queries, heads that do not divide, 3-D, more pairs than served
+@pytest.mark.parametrize("q,k,v,dtype", [((1, 4, 8, 64), (1, 2, 8, 64), (1, 2, 8, 64), torch.bfloat16), ((1, 4, 8, 64), (1, 2, 8, 32), (1, 2, 8, 32), None),
+                                         ((1, 4, 8, 64), (1, 2, 8, 64), (1, 2, 7, 64), None), ((1, 4, 8, 64), (1, 2, 7, 64), (1, 2, 7, 64), None),
+                                         ((1, 4, 8, 64), (1, 3, 8, 64), (1, 3, 8, 64), None), ((4, 8, 64), (4, 8, 64), (4, 8, 64), None),
+                                         ((2, 4, 8, 64), (1, 2, 8, 64), (1, 2, 8, 64), None), ((1, 4097, 1, 64), (1, 4097, 1, 64), (1, 4097, 1, 64), None)])
+def test_float32_attention_checks_its_operands_on_every_route(q, k, v, dtype):
+    from adaptivetrainingsystem_amd import autograd, ops
+    from adaptivetrainingsystem_amd._lib import AtsError
+    q, k, v = (torch.zeros(s, dtype=dtype or torch.float32) for s in (q, k, v))
+    out = torch.zeros(1)
+    for call in (lambda: ops.attention_f32(q, k, v), lambda: ops.attention_f32_fused(q, k, v, 0.125, None),
+                 lambda: autograd.AttentionF32Function.apply(q, k, v, 0.125), lambda: ops.attention_f32_fused_bwd(q, k, v, out, out, out, 0.125, None)):
+        with pytest.raises(AtsError, match="attention_f32: (shapes|q, k, v must be 4-D float32)"):
+            call()
+
+
+def test_float32_attention_gradient_checks_what_it_is_given():
+    from adaptivetrainingsystem_amd import ops
+    from adaptivetrainingsystem_amd._lib import AtsError
+    q, kv, out, stats = torch.zeros(1, 4, 8, 64), torch.zeros(1, 2, 8, 64), torch.zeros(1, 8, 256), torch.zeros(4, 8, 2)
+    for bad in ((out[:, :7], stats, out), (out, stats[:3], out), (out, stats, out[..., :64]), (out, stats, out.bfloat16())):
+        with pytest.raises(AtsError, match="as handed out"):
+            ops.attention_f32_fused_bwd(q, kv, kv, *bad, 0.125, None)
