@@ -285,13 +285,16 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> prompt_attention(const Tensor&
 
 }  // namespace
 
+// The interpreter lock is released through every call, as ctypes releases it: other threads run while a launch waits for a full
+// queue.  (check takes it again to raise.)
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("set_error", [](pybind11::object e) { g_error = e.release().ptr(); });
-    m.def("rmsnorm", &rmsnorm);
-    m.def("rope", &rope);
-    m.def("rope_append", &rope_append);
-    m.def("linear", &linear);
-    m.def("linear_rope_append", &linear_rope_append);
-    m.def("attention", &attention);
-    m.def("prompt_attention", &prompt_attention);
+    auto def = [&m](const char* name, auto function) { m.def(name, function, pybind11::call_guard<pybind11::gil_scoped_release>()); };
+    def("rmsnorm", &rmsnorm);
+    def("rope", &rope);
+    def("rope_append", &rope_append);
+    def("linear", &linear);
+    def("linear_rope_append", &linear_rope_append);
+    def("attention", &attention);
+    def("prompt_attention", &prompt_attention);
 }

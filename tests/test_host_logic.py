@@ -292,3 +292,38 @@ def test_float32_attention_gradient_checks_what_it_is_given():
     for bad in ((out[:, :7], stats, out), (out, stats[:3], out), (out, stats, out[..., :64]), (out, stats, out.bfloat16())):
         with pytest.raises(AtsError, match="as handed out"):
             ops.attention_f32_fused_bwd(q, kv, kv, *bad, 0.125, None)
+
+
+def test_native_calls_let_other_threads_run():
+    """With a switch interval of minutes another thread runs only where this one gives the interpreter lock up."""
+    import sys
+    import threading
+    import time
+    from adaptivetrainingsystem_amd import _lib
+    native, x = _lib.native(), torch.zeros(2, 3, 4, 8)
+    cache, table = torch.zeros(2, 3, 4, 8), torch.zeros(4, 8)
+    calls = {"rmsnorm": (x, None, 1e-6), "rope": (x, x, table, table, 0), "rope_append": (x, x, x, table, table, cache, cache, 0, 0),
+             "linear": (x, x, x, x, 8, 1), "linear_rope_append": (x, x, x, x, 2, table, table, cache, cache, 0, 1, 1),
+             "attention": (x, x, x, 1.0, True), "prompt_attention": (x, table, table, 2, 1, 8, 1.0, True)}
+    assert set(calls) == {n for n in dir(native) if not n.startswith("_")} - {"set_error"}
+    seen, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            seen[0] += 1
+            time.sleep(0)
+    before, thread = sys.getswitchinterval(), threading.Thread(target=other)
+    sys.setswitchinterval(300.0)
+    try:
+        thread.start()
+        for name, args in calls.items():
+            call, count = getattr(native, name), seen[0]
+            for _ in range(1000000):
+                assert call(*args) is None      # (not on the GPU: handed on to the general path)
+                if seen[0] > count + 3:
+                    break
+            assert seen[0] > count + 3, name
+    finally:
+        stop.set()
+        sys.setswitchinterval(before)
+        thread.join()
