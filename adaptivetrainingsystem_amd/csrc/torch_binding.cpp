@@ -4,12 +4,26 @@
 // A normalisation, a rotation or a projection of a decoding step runs 3-15 us on the card; its wrapper in Python, an
 // allocation and a foreign call with 8 to 30 arguments took 8-17 us, and a Python node in the backward pass 40 us more on the
 // engine's thread.  Every function here serves the ordinary form of its call and returns None for any other (types, strides,
-// devices, sizes of nothing, function transforms): the caller then takes the general path, which converts or raises.  The
-// kernels, their arguments and the results are those of that path.
+// devices, sizes of nothing, tensor subclasses, tracing, function transforms, forward-mode gradients): the caller then takes the
+// general path, which converts, records or raises.  The kernels, their arguments and the results are those of that path.
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
 #include "../../include/ats_gfx950.h"
+
+// An argument that is a torch.Tensor or a Parameter; of any other subclass nothing is taken over (an undefined tensor).
+struct Plain : at::Tensor {};
+namespace pybind11::detail {
+template <>
+struct type_caster<Plain> {
+    PYBIND11_TYPE_CASTER(Plain, const_name("torch.Tensor"));
+    bool load(handle src, bool) {
+        if (!THPVariable_Check(src.ptr())) return false;
+        if (THPVariable_CheckExact(src.ptr())) static_cast<at::Tensor&>(value) = THPVariable_Unpack(src.ptr());
+        return true;
+    }
+};
+}  // namespace pybind11::detail
 
 namespace {
 
@@ -34,11 +48,15 @@ ats_stream_t stream() { return reinterpret_cast<ats_stream_t>(c10::hip::getCurre
 bool served(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
 int tag(const Tensor& t) { return t.scalar_type() == at::kFloat ? ATS_F32 : ATS_BF16; }
 bool on_gpu(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided; }
-// function transforms (vmap, grad, ..) wrap their tensors; the general path has its own answer to them
+// Function transforms (vmap, grad, ..) wrap their tensors, dispatch modes and torch.jit.trace record what is called: the general path
+// has its own answer to them (a trace keeps a Python autograd function, of a node in here only its allocation).
 bool transformed() {
-    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
-           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python);
+    using c10::DispatchKey;
+    using c10::impl::tls_is_dispatch_key_included;
+    return tls_is_dispatch_key_included(DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+           tls_is_dispatch_key_included(DispatchKey::Python) || tls_is_dispatch_key_included(DispatchKey::Tracer);
 }
+bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(0).defined(); }
 bool wants_grad(const Tensor& a, const Tensor& b) {
     return at::GradMode::is_enabled() && (a.requires_grad() || (b.defined() && b.requires_grad()));
 }
@@ -80,10 +98,12 @@ struct RMSNormFunction : torch::autograd::Function<RMSNormFunction> {
     }
 };
 
-std::optional<Tensor> rmsnorm(const Tensor& x, const std::optional<Tensor>& weight, double eps) {
-    const Tensor w = weight.has_value() ? *weight : Tensor();
+std::optional<Tensor> rmsnorm(const Plain& input, const std::optional<Plain>& weight, double eps) {
+    const Tensor& x = input;      // (a node's inputs are found by their type)
+    const Tensor w = weight.has_value() ? static_cast<const Tensor&>(*weight) : Tensor();
     if (!on_gpu(x) || !served(x.scalar_type()) || x.dim() < 1 || x.numel() == 0 || !x.is_contiguous() || transformed()) return {};
-    if (w.defined() && (!on_gpu(w) || w.device() != x.device() || !served(w.scalar_type()) || w.numel() != x.size(-1) ||
+    if (has_tangent(x) || has_tangent(w)) return {};
+    if (weight.has_value() && (!on_gpu(w) || w.device() != x.device() || !served(w.scalar_type()) || w.numel() != x.size(-1) ||
                         !w.is_contiguous()))
         return {};
     if (wants_grad(x, w)) return RMSNormFunction::apply(x, w, eps);
@@ -149,8 +169,11 @@ bool heads_match(const Tensor& q, const Tensor& k) {
     return k.scalar_type() == q.scalar_type() && k.size(0) == q.size(0) && k.size(2) == q.size(2) && k.size(3) == q.size(3);
 }
 
-std::optional<std::tuple<Tensor, Tensor>> rope(const Tensor& q, const Tensor& k, const Tensor& cos, const Tensor& sin, int64_t offset) {
+std::optional<std::tuple<Tensor, Tensor>> rope(const Plain& q_in, const Plain& k_in, const Plain& cos_in, const Plain& sin_in,
+                                                   int64_t offset) {
+    const Tensor &q = q_in, &k = k_in, &cos = cos_in, &sin = sin_in;
     if (!heads_ok(q) || !heads_ok(k) || !heads_match(q, k) || !tables_ok(cos, sin) || transformed()) return {};
+    if (has_tangent(q) || has_tangent(k)) return {};
     if (wants_grad(q, k)) {
         const auto r = RoPEFunction::apply(q, k, cos, sin, offset);
         return std::make_tuple(r[0], r[1]);
@@ -162,8 +185,8 @@ std::optional<std::tuple<Tensor, Tensor>> rope(const Tensor& q, const Tensor& k,
 
 // ------------------------------------------------------------------ the launches of an attention sub-layer, inference
 // (their callers have decided that no gradient is wanted)
-std::optional<Tensor> rope_append(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cos, const Tensor& sin,
-                                  const Tensor& k_cache, const Tensor& v_cache, int64_t cache_pos, int64_t offset) {
+std::optional<Tensor> rope_append(const Plain& q, const Plain& k, const Plain& v, const Plain& cos, const Plain& sin,
+                                  const Plain& k_cache, const Plain& v_cache, int64_t cache_pos, int64_t offset) {
     if (!heads_ok(q) || !heads_ok(k) || !heads_ok(v) || !heads_match(q, k) || v.sizes() != k.sizes() ||
         v.scalar_type() != q.scalar_type() || !tables_ok(cos, sin) || !heads_ok(k_cache) || !heads_ok(v_cache) ||
         k_cache.scalar_type() != q.scalar_type() || v_cache.scalar_type() != q.scalar_type() || v_cache.sizes() != k_cache.sizes() ||
@@ -183,7 +206,7 @@ std::optional<Tensor> rope_append(const Tensor& q, const Tensor& k, const Tensor
 }
 
 // x [T, K] against one [N, K] matrix whose address is table[0]; splits as the caller's rule gives them
-std::optional<Tensor> linear(const Tensor& x, const Tensor& table, const Tensor& start, const Tensor& count, int64_t N, int64_t splits) {
+std::optional<Tensor> linear(const Plain& x, const Tensor& table, const Tensor& start, const Tensor& count, int64_t N, int64_t splits) {
     if (!on_gpu(x) || !served(x.scalar_type()) || x.dim() != 2 || !x.is_contiguous() || x.numel() == 0 || transformed()) return {};
     const int64_t T = x.size(0), K = x.size(1);
     const void* const* b = static_cast<const void* const*>(table.data_ptr());
@@ -204,8 +227,8 @@ std::optional<Tensor> linear(const Tensor& x, const Tensor& table, const Tensor&
 }
 
 // linear of stacked q, k, v weights with splits > 1, its sum fused with rope_append: x [B * L, K] -> rotated q [B, Hq, L, D]
-std::optional<Tensor> linear_rope_append(const Tensor& x, const Tensor& table, const Tensor& start, const Tensor& count, int64_t splits,
-                                         const Tensor& cos, const Tensor& sin, const Tensor& k_cache, const Tensor& v_cache,
+std::optional<Tensor> linear_rope_append(const Plain& x, const Tensor& table, const Tensor& start, const Tensor& count, int64_t splits,
+                                         const Plain& cos, const Plain& sin, const Plain& k_cache, const Plain& v_cache,
                                          int64_t cache_pos, int64_t Hq, int64_t L) {
     auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
     if (!on_gpu(x) || !served(x.scalar_type()) || x.dim() != 2 || !x.is_contiguous() || x.numel() == 0 || !tables_ok(cos, sin) ||
@@ -233,7 +256,7 @@ std::optional<Tensor> linear_rope_append(const Tensor& x, const Tensor& table, c
 }
 
 // causal attention without masks, dropout or log-sum-exp
-std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool split_keys) {
+std::optional<Tensor> attention(const Plain& q, const Plain& k, const Plain& v, double scale, bool split_keys) {
     if (!heads_ok(q) || !heads_ok(k) || !heads_ok(v) || q.scalar_type() != at::kBFloat16 || k.scalar_type() != q.scalar_type() ||
         v.scalar_type() != q.scalar_type() || v.sizes() != k.sizes() || k.size(0) != q.size(0) || k.size(3) != q.size(3) ||
         q.size(1) % k.size(1) != 0 || k.size(2) < q.size(2) || !q.is_contiguous() || transformed())
@@ -256,7 +279,7 @@ std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& 
 
 // causal attention of a prompt on its stacked projections qkv [B * L, (Hq + 2 Hkv) * D]: keys rotated (with the values beside them:
 // the prompt's cache), queries rotated as the attention loads them -> out, k, v
-std::optional<std::tuple<Tensor, Tensor, Tensor>> prompt_attention(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t B,
+std::optional<std::tuple<Tensor, Tensor, Tensor>> prompt_attention(const Plain& qkv, const Plain& cos, const Plain& sin, int64_t B,
                                                                    int64_t Hkv, int64_t D, double scale, bool keep_values) {
     auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
     if (!on_gpu(qkv) || qkv.scalar_type() != at::kBFloat16 || !qkv.is_contiguous() || !tables_ok(cos, sin) || cos.stride(0) % 4 ||

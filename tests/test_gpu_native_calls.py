@@ -187,3 +187,35 @@ def test_errors_and_transforms_are_those_of_the_general_path(gpu, general):
         assert kinds[0] == kinds[1]
     with torch.inference_mode():
         _same(norm(x), general(lambda: norm(x)))
+
+
+class _Marked(torch.Tensor):
+    pass
+
+
+@pytest.mark.filterwarnings("ignore")      # (of the tracer, about Python values)
+def test_traces_subclasses_and_tangents_take_the_general_path(gpu, general):
+    import torch.autograd.forward_ad as forward
+    from adaptivetrainingsystem_amd import RMSNorm, RotaryEmbedding, apply_rotary_pos_emb
+    g = torch.Generator().manual_seed(6)
+    norm, (cos, sin) = RMSNorm(64).to(gpu), RotaryEmbedding(64, 16)(8, gpu)
+    x, other = (torch.randn(1, 2, 8, 64, generator=g).to(gpu) for _ in range(2))
+    rotate = lambda t: apply_rotary_pos_emb(t, t, cos, sin)
+    for fn in (norm, rotate):
+        # a trace made with gradients keeps the autograd function, and with it what it computes
+        traced = torch.jit.trace(fn, (x.clone().requires_grad_(),), check_trace=False)
+        _same(traced(other), fn(other))
+        for grad in (False, True):
+            kinds = lambda: [type(t) for t in (lambda r: r if isinstance(r, tuple) else (r,))(fn(x.as_subclass(_Marked).requires_grad_(grad)))]
+            assert kinds() == general(kinds)
+
+        def tangent():
+            with forward.dual_level(), pytest.raises(Exception) as e:
+                fn(forward.make_dual(x.clone().requires_grad_(), torch.ones_like(x)))
+            return e.type
+        assert tangent() == general(tangent)
+    with torch.no_grad():
+        assert isinstance(norm(x.as_subclass(_Marked)), _Marked)
+    norm.weight = torch.nn.Parameter(norm.weight.detach().as_subclass(_Marked) * 3.0)
+    assert type(norm.weight) is not torch.nn.Parameter
+    _same(norm(x).as_subclass(torch.Tensor), general(lambda: norm(x).as_subclass(torch.Tensor)))
