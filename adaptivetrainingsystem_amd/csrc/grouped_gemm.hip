@@ -1266,8 +1266,9 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 #pragma unroll
         for (int j = 0; j < TN; ++j) fb_tr[j] = (lds_u8_t)smem + base0 + ((j ^ t4) * 32);
     }
-    const int b_slab = BKM ? (int)(p.ldb * 128) : 128;   // bytes from one slab of the weight operand to the next
-    const int a_slab = AKM ? (int)(p.lda * 128) : 128;
+    // bytes from one slab of an operand to the next (unsigned: the advance along K runs up to 4 GiB)
+    const unsigned b_slab = BKM ? (unsigned)(p.ldb * 128) : 128u;
+    const unsigned a_slab = AKM ? (unsigned)(p.lda * 128) : 128u;
     constexpr int RB2 = BKM ? 4 : 2;   // read instructions of two weight fragments
     constexpr int RA = AKM ? 2 : 1;    // read instructions of an activation fragment
     u32x4_t fa[2][4], fb[2][TN];
@@ -1275,19 +1276,19 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 // AKM: the advance along K is part of the lane offset, which the descriptor's end is checked against (the scalar offset is
 // not); otherwise it is the scalar offset.
 #define D16_LOAD(rsrc_, dst_, off_, adv_)                                                              \
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_, (lds_ptr_t)(dst_), 16, (off_) + (AKM ? (unsigned)(adv_) : 0u), \
-                                             AKM ? 0 : (adv_), 0, 0)
-#define D16_ISSUE_A1(kt_, aoff_, j_) D16_LOAD(rsrc_a, dma_a + (aoff_) + (j_) * NW * 1024, ao[j_], (kt_) * a_slab)
-#define D16_ISSUE_B1(kt_, boff_, j_) D16_LOAD(rsrc_b, dma_b + (boff_) + (j_) * NW * 1024, bo[j_], (kt_) * b_slab)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_, (lds_ptr_t)(dst_), 16, (off_) + (AKM ? (adv_) : 0u), \
+                                             AKM ? 0 : (int)(adv_), 0, 0)
+#define D16_ISSUE_A1(kt_, aoff_, j_) D16_LOAD(rsrc_a, dma_a + (aoff_) + (j_) * NW * 1024, ao[j_], (unsigned)(kt_) * a_slab)
+#define D16_ISSUE_B1(kt_, boff_, j_) D16_LOAD(rsrc_b, dma_b + (boff_) + (j_) * NW * 1024, bo[j_], (unsigned)(kt_) * b_slab)
 #define D16_ISSUE_A(kt_, aoff_)                                                                        \
     {                                                                                                  \
-        const int adv = (kt_) * a_slab;                                                                \
+        const unsigned adv = (unsigned)(kt_) * a_slab;                                                  \
         _Pragma("unroll") for (int j = 0; j < NIA; ++j)                                                \
             D16_LOAD(rsrc_a, dma_a + (aoff_) + j * NW * 1024, ao[j], adv);                             \
     }
 #define D16_ISSUE_B(kt_, boff_)                                                                        \
     {                                                                                                  \
-        const int adv = (kt_) * b_slab;                                                                \
+        const unsigned adv = (unsigned)(kt_) * b_slab;                                                  \
         _Pragma("unroll") for (int j = 0; j < NIB; ++j)                                                \
             D16_LOAD(rsrc_b, dma_b + (boff_) + j * NW * 1024, bo[j], adv);                             \
     }

@@ -41,3 +41,22 @@ def test_operands_that_keep_the_transposed_route(gpu):
     assert ok(t, t) and ok(t[:, 8:32], t)
     assert not ok(t.float(), t.float()) and not ok(t[:, :60], t) and not ok(t[:, 4:36], t) and not ok(t.t(), t.t())
     assert not ok(t[:0], t[:0])
+
+
+@pytest.mark.parametrize("T,pitch", [(300, 5_600_000), (3000, 600_000), (100, 12_000_000)])
+def test_operands_of_two_to_four_gib(gpu, T, pitch):
+    """Rows so far apart that the advance along K passes 2^31 bytes: the bits of contiguous copies."""
+    print("case wgrad tn extent", T, pitch, flush=True)
+    from adaptivetrainingsystem_amd import ops
+    M, N = 72, 264
+    g = torch.Generator().manual_seed(T)
+    dy, x = (torch.randn(T, n, generator=g).to(gpu, torch.bfloat16) for n in (M, N))
+    want = ops.wgrad_linear(dy, x)
+    for far in (0, 1):
+        pair = [dy, x]
+        wide = torch.empty((T - 1) * pitch + N, dtype=torch.bfloat16, device=gpu).as_strided((T, pair[far].shape[1]), (pitch, 1))
+        wide.copy_(pair[far])
+        assert 2 ** 31 < (T + 63) // 64 * 64 * pitch * 2 < 2 ** 32
+        pair[far] = wide
+        assert ops.wgrad_linear_supported(*pair)
+        assert torch.equal(ops.wgrad_linear(*pair), want)
