@@ -1334,6 +1334,8 @@ def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, B:
                      keep_values: bool):
     """rope and causal_attention of the stacked projections qkv [B * L, (Hq + 2 Hkv) * D]: (out [B, L, Hq * D], rotated k, v),
     v contiguous with keep_values and a view of qkv without; None for operands that the launches do not read as they are."""
+    if qkv.dim() != 2 or B <= 0 or Hkv <= 0 or D <= 0 or qkv.shape[0] % B or qkv.shape[1] % D or qkv.shape[1] <= 2 * Hkv * D:
+        raise AtsError(f"prompt_attention: qkv {tuple(qkv.shape)} is not [{B} * positions, (heads + 2 * {Hkv}) * {D}]")
     return _lib.native().prompt_attention(qkv, cos, sin, B, Hkv, D, scale, keep_values)
 
 
@@ -1588,6 +1590,11 @@ def linear_rope_append(x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor,
                        v_cache: torch.Tensor, cache_pos: int, seq: int) -> Optional[torch.Tensor]:
     """linear_nt(x [batch * seq, K], weight [(Hq + 2 Hkv) * D, K]) and rope_append of its columns: where the product runs in
     slices of K one launch adds them up, rotates and appends (the same bits).  None where it does not."""
+    if (x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1] or k_cache.dim() != 4 or v_cache.shape != k_cache.shape
+            or x.shape[0] != k_cache.shape[0] * seq or weight.shape[0] % k_cache.shape[3]
+            or weight.shape[0] <= 2 * k_cache.shape[1] * k_cache.shape[3]):
+        raise AtsError(f"linear_rope_append: x {tuple(x.shape)}, weight {tuple(weight.shape)}, {seq} positions, caches "
+                       f"{tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
     T, K = x.shape
     N, D = weight.shape[0], k_cache.shape[3]
     splits = _linear_slices(T, N, K, x.dtype)

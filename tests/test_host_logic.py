@@ -327,3 +327,20 @@ def test_native_calls_let_other_threads_run():
         stop.set()
         sys.setswitchinterval(before)
         thread.join()
+
+
+def test_joined_attention_launches_check_their_shapes():
+    from adaptivetrainingsystem_amd import ops
+    from adaptivetrainingsystem_amd._lib import AtsError
+    x, w, table, cache = torch.zeros(6, 4096), torch.zeros(512, 4096), torch.zeros(8, 64), torch.zeros(2, 2, 9, 64)
+    good = {"x": x, "weight": w, "cos": table, "sin": table, "k_cache": cache, "v_cache": cache, "cache_pos": 0, "seq": 3}
+    assert ops.linear_rope_append(**good) is None       # (not on the GPU)
+    for bad in ({"x": torch.zeros(6, 4104)}, {"x": x[0]}, {"x": x[:5]}, {"seq": 2}, {"weight": w[:500]}, {"weight": w[:256]},
+                {"weight": w[:, :4088]}, {"v_cache": cache[:, :1]}, {"k_cache": cache[0], "v_cache": cache[0]}):
+        with pytest.raises(AtsError, match="linear_rope_append: x"):
+            ops.linear_rope_append(**{**good, **bad})
+    qkv = torch.zeros(6, 512, dtype=torch.bfloat16)
+    assert ops.prompt_attention(qkv, table, table, 2, 2, 64, 0.125, True) is None
+    for args in ((qkv, 4, 2, 64), (qkv, 0, 2, 64), (qkv, 2, 4, 64), (qkv, 2, 2, 96), (qkv[0], 2, 2, 64), (qkv, 2, 0, 64)):
+        with pytest.raises(AtsError, match="prompt_attention: qkv"):
+            ops.prompt_attention(args[0], table, table, *args[1:], 0.125, True)
