@@ -1174,10 +1174,10 @@ def grouped_gemm_nn_sliced(b_ptrs: torch.Tensor, ldb: int, row_start: torch.Tens
                            max_rows: int, N: int, K: int, a: torch.Tensor, k_splits: int) -> torch.Tensor:
     """grouped_gemm_nn for groups of up to 256 rows on average: the product [n_rows_out, N], or with more than one slice of
     K the float32 partial results [k_splits, n_rows_out, N]."""
-    _need_gpu(a, b_ptrs, row_start, row_count)
     a = _rows_2d(a, "grouped_gemm_nn_sliced")
-    if a.shape[0] < max_rows or n_rows_out < max_rows:
-        raise AtsError("grouped_gemm_nn_sliced: fewer rows than max_rows")
+    if a.shape[0] < max_rows or n_rows_out < max_rows or a.shape[1] < K:
+        raise AtsError("grouped_gemm_nn_sliced: fewer rows than max_rows, or than K columns")
+    _need_gpu(a, b_ptrs, row_start, row_count)
     E = b_ptrs.numel()
     shape, dtype = ((n_rows_out, N), a.dtype) if k_splits == 1 else ((k_splits, n_rows_out, N), torch.float32)
     out = torch.empty(shape, dtype=dtype, device=b_ptrs.device)
@@ -1219,11 +1219,11 @@ def wgrad_f32(a: torch.Tensor, b: torch.Tensor, k_start: Optional[torch.Tensor] 
               b_rows: Optional[torch.Tensor] = None, b_row_div: int = 1) -> torch.Tensor:
     """a^T @ b for rows as they lie, a [R, M], b [R, N]; per group [E, M, N] over the k_count[e] rows from k_start[e] where
     these are given, with b's row r taken from b_rows[r] // b_row_div if a gather table is given."""
-    _need_gpu(a, b, k_start, k_count, b_rows)
     if not wgrad_f32_supported(a, b, 1 if k_count is None else k_count.numel()):
         raise AtsError("wgrad_f32: float32 rows of 16-byte multiples, of sizes that the small tiles serve")
-    if b_rows is None and k_count is None and a.shape[0] != b.shape[0]:
-        raise AtsError("wgrad_f32: a and b must have the same number of rows")
+    if (a.shape[0] != b.shape[0] if b_rows is None else b_rows.dtype != torch.int32 or b_rows.numel() < a.shape[0] or b_row_div < 1):
+        raise AtsError("wgrad_f32: a and b must have the same number of rows, or an int32 row of b for every row of a")
+    _need_gpu(a, b, k_start, k_count, b_rows)
     (R, M), N = a.shape, b.shape[1]
     E = 1 if k_count is None else k_count.numel()
     out = torch.empty((M, N) if k_count is None else (E, M, N), dtype=torch.float32, device=a.device)

@@ -344,3 +344,16 @@ def test_joined_attention_launches_check_their_shapes():
     for args in ((qkv, 4, 2, 64), (qkv, 0, 2, 64), (qkv, 2, 4, 64), (qkv, 2, 2, 96), (qkv[0], 2, 2, 64), (qkv, 2, 0, 64)):
         with pytest.raises(AtsError, match="prompt_attention: qkv"):
             ops.prompt_attention(args[0], table, table, *args[1:], 0.125, True)
+
+
+def test_products_of_operands_as_they_lie_check_their_rows():
+    from adaptivetrainingsystem_amd import ops
+    from adaptivetrainingsystem_amd._lib import AtsError
+    a, b, two = torch.zeros(64, 512), torch.zeros(64, 512), torch.zeros(2, dtype=torch.int32)
+    rows = torch.zeros(64, dtype=torch.int32)
+    for bad in ({"b": b[:60]}, {"b": b[:60], "k_start": two, "k_count": two}, {"b_rows": rows[:60]}, {"b_rows": rows.long()},
+                {"b_rows": rows, "b_row_div": 0}):
+        with pytest.raises(AtsError, match="wgrad_f32: a and b must have the same number of rows, or"):
+            ops.wgrad_f32(**{"a": a, "b": b, **bad})
+    with pytest.raises(AtsError, match="than K columns"):
+        ops.grouped_gemm_nn_sliced(two, 512, two, two, 64, 64, 512, 1024, a.bfloat16(), 2)
