@@ -447,8 +447,9 @@ extern "C" int ats_rope_sum_append(const float* parts, int n_parts, int64_t part
                 "%s: n_parts=%d B=%d Hq=%d Hkv=%d L=%d D=%d", name, n_parts, B, Hq, Hkv, L, D);
     if (B == 0 || L == 0) return ATS_OK;
     const int64_t heads = (int64_t)Hq + 2 * (int64_t)Hkv, total = (int64_t)B * L * heads * (D / 8);
-    ATS_REQUIRE(total < INT_MAX && part_stride % 4 == 0 && part_stride >= (int64_t)B * L * heads * D, ATS_ERR_INVALID_ARG,
-                "%s: part_stride=%lld for %lld x %d columns", name, (long long)part_stride, (long long)B * L * heads, D);
+    ATS_REQUIRE(total <= INT_MAX - 255 && part_stride % 4 == 0 && part_stride >= (int64_t)B * L * heads * D, ATS_ERR_INVALID_ARG,
+                "%s: part_stride=%lld for %lld x %d columns (thread numbers are 32 bits wide)", name, (long long)part_stride,
+                (long long)B * L * heads, D);
     ATS_REQUIRE(L <= table_len && table_stride >= D / 2, ATS_ERR_INVALID_ARG, "%s: %d positions, table of %d (stride %d)", name, L,
                 table_len, table_stride);
     ATS_REQUIRE(cache_pos >= 0 && cache_pos + L <= cache_capacity && cache_sl >= D, ATS_ERR_INVALID_ARG,
