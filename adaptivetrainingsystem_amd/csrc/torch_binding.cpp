@@ -200,8 +200,8 @@ std::optional<Tensor> rope_append(const Plain& q, const Plain& k, const Plain& v
                               static_cast<const float*>(cos.data_ptr()), static_cast<const float*>(sin.data_ptr()),
                               (int)cos.stride(0), (int)cos.size(0), (int)B, (int)Hq, (int)k.size(1), (int)L, (int)D, (int)offset,
                               q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1),
-                              v.stride(2), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), (int)cache_pos,
-                              (int)k_cache.size(2), tag(q), stream()), "ats_rope_fwd_append");
+                              v.stride(2), k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), cache_pos, k_cache.size(2),
+                              tag(q), stream()), "ats_rope_fwd_append");
     return qo;
 }
 

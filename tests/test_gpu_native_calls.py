@@ -219,3 +219,15 @@ def test_traces_subclasses_and_tangents_take_the_general_path(gpu, general):
     norm.weight = torch.nn.Parameter(norm.weight.detach().as_subclass(_Marked) * 3.0)
     assert type(norm.weight) is not torch.nn.Parameter
     _same(norm(x).as_subclass(torch.Tensor), general(lambda: norm(x).as_subclass(torch.Tensor)))
+
+
+def test_positions_past_32_bits_are_refused(gpu):
+    from adaptivetrainingsystem_amd import ops
+    from adaptivetrainingsystem_amd._lib import AtsError
+    q = torch.zeros(1, 2, 1, 64, device=gpu)
+    cos, sin = ops.rope_table(4, 64, 10000.0, None, half=True)
+    caches = [torch.full((1, 2, 8, 64), 7.0, device=gpu) for _ in range(2)]
+    for pos in (1 << 32, (1 << 32) + 3, -(1 << 32)):
+        with pytest.raises(AtsError, match="do not fit a cache"):
+            ops.rope_append(q, q, q, cos, sin, *caches, pos, 0)
+    assert all((c == 7.0).all() for c in caches)
