@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("counts,M,N", [([0, 1, 64, 65], 4104, 2056), ([200, 448, 0, 449, 31, 127], 2600, 2184), ([33] * 64, 264, 1416)])
 def test_short_k_weight_gradient(gpu, counts, M, N):
     print("case short K", counts[:6], M, N, flush=True)
-    from adaptivetrainingsystem_amd import ops
+    from adaptivetrainingsystem_amd import _lib, ops
     E, rows = len(counts), sum(counts)
     g = torch.Generator().manual_seed(rows)
     cnt = torch.tensor(counts, dtype=torch.int32, device=gpu)
@@ -27,6 +27,11 @@ def test_short_k_weight_gradient(gpu, counts, M, N):
     off = 0
     for e, c in enumerate(counts):
         ref = a[off:off + c].double().T @ b[off:off + c].double()
+        if c:      # the bits of the 256 x 256 tile, on the group's rows alone
+            one, (first, height) = torch.empty_like(out[e]), ops._single_group(M, gpu)
+            assert _lib.load().ats_wgrad_tn(a[off:].data_ptr(), M, b[off:].data_ptr(), N, one.data_ptr(), c, M, N, 1, first.data_ptr(),
+                                            height.data_ptr(), _lib.ATS_BF16, _lib.ATS_BF16, torch.cuda.current_stream().cuda_stream) == 0
+            assert torch.equal(out[e], one)
         off += c
         # float32 sums of exact products, one rounding to bfloat16
         bound = 2.0 ** -8 * ref.abs() + 4e-7 * max(c, 1) * a.abs().max().double() * b.abs().max().double()
