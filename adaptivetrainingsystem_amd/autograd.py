@@ -148,8 +148,9 @@ class AttentionF32Function(Function):
 
 class LinearFunction(Function):
     """y = x @ weight^T for x [T, K], weight [N, K] (a bias-free nn.Linear) through the grouped GEMM kernels
-    with one group: dgrad reads the weight as it is where the K-major kernel applies (bfloat16, more than 192
-    rows) and multiplies by a transposed copy otherwise, wgrad reads both operands as they are (bfloat16) or transposed."""
+    with one group: dgrad reads the weight as it is where a K-major kernel applies (bfloat16 of more than 192 rows, float32 where
+    that is the faster way) and multiplies by a transposed copy otherwise, wgrad likewise reads both operands as they are (bfloat16
+    of 16-byte aligned rows, float32 where that is the faster way) or transposed."""
 
     @staticmethod
     def forward(ctx, x, weight):
@@ -322,9 +323,10 @@ def _ffn_forward(x, wgu, wd, offsets, kept, rows, row_src, k, want_wgrad=False):
 def _ffn_backward(dy, x, wgu, wd, gu, h, offsets, kept, rows, row_src, k, need_x, need_w, hT=None, wplan=None):
     """Gradients of _ffn_forward: dx_rows [rows, H] (or None; float32 [slices, rows, H], to be added, where the product cut
     K), dWgu [E, 2I, H], dWd [E, H, I] (or None).
-    dgrad reads the weights as the forward holds them (float32 and sizes off its grid: per-step transposed copies); wgrad multiplies the transposed,
-    zero-padded activations of each expert (K = its padded row count).  h may be None when hT, its transposed
-    copy from the forward kernel, is given; the fused bfloat16 dgrad kernel likewise hands back dgu and its
+    dgrad reads the weights as the forward holds them, or per-step transposed copies where that is the faster way or the only
+    one (sizes off the kernels' grid).  wgrad of float32 rows reads them as they lie where that is the faster way; otherwise it
+    multiplies the transposed, zero-padded activations of each expert (K = its padded row count).  h may be None when hT, its
+    transposed copy from the forward kernel, is given; the fused bfloat16 dgrad kernel likewise hands back dgu and its
     transposed copy, so only dy and the gathered x go through a transposing pass."""
     E = len(wd)
     H, I = x.shape[1], wd[0].shape[1]

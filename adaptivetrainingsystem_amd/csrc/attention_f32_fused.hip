@@ -16,12 +16,15 @@
 // additive mask of the keys (819-824), softmax.  The fill is a score like any other: a row whose visible scores all lie near
 // or below it gives weight to its future keys, and so does a row before a key whose mask lifts the fill (it is added behind
 // it).  The workgroup then walks all keys; it skips future keys only where the largest of their scores, fill plus mask, is so far
-// below the row's maximum that its exponential is zero in float32.
+// below the row's maximum that its exponential is zero in float32.  (Infinities and NaN in the values of skipped keys, as in the
+// bfloat16 kernels, do not reach the row; the materialised product multiplied them by zero, to NaN.)
 // Bounds: launches and the serial chain of a tile (32 MFMAs of 32 cycles per product) at short sequences, L1 traffic at long
 // ones (every tile is read in both layouts).  Materialised route -> this, microseconds, forward | backward:
 //   2 x 54, 4 heads of 128    88 ->    8 |   158 ->   21        1 x 1024, 32 heads of 128   287 ->  165 |   639 ->  712
 //   2 x 256, 4 heads of 128   57 ->   12 |   133 ->   51        1 x 2048, 16 heads of  64   480 ->  156 |  1177 ->  622
 //   4 x 512, 4 heads of 128   77 ->   31 |   135 ->  112        1 x 4096, 32 heads of 128  6571 -> 1697 | 16260 -> 6697
+// (The backward of 1 x 1024 alone is the slower one.  Its materialised form needs the weights that only the materialised forward
+// keeps, so one route takes both passes: 926 -> 877 together.)
 // Errors against float64 (output, dq, dk, dv), 8 heads x 32: 1.1e-7, 1.9e-7, 2.1e-7, 1.5e-7 -> 1.2e-7, 1.8e-7, 1.8e-7,
 // 1.3e-7; 16 heads x 512: 3.4e-7, 4.2e-7, 6.1e-7, 5.9e-7 -> 1.7e-7, 2.2e-7, 2.9e-7, 2.7e-7.
 #include <math.h>

@@ -214,13 +214,14 @@ class GroupedQueryAttention(nn.Module):
     """Causal grouped-query attention with the reference's constructor fields, parameter names
     (q_proj / k_proj / v_proj / o_proj, no bias) and forward(x [B, L, hidden]) -> [B, L, hidden]
     (MS/core/model.py:561-731).  Projections run through the grouped GEMM kernels (one group), RoPE and the
-    attention itself through their HIP kernels; the score matrix is never materialised.  Built: gradients of
+    attention itself through their HIP kernels; the score matrix is not materialised (but see float32).  Built: gradients of
     every input and parameter, past_key_value / use_cache (model.py:700-708; the cache grows in place),
     attention_mask [batch, keys] or [batch, 1, queries, keys] (model.py:819-824), attention dropout in training
     mode (config.dropout > 0, model.py:622-623, 831-833: the mask is a hash of a per-call 62-bit seed drawn
     from torch's CPU generator, so torch.manual_seed reproduces it and a checkpointed recomputation, which
-    replays that generator's state, draws the same mask again), float32 activations (the scores are then
-    materialised between two float32 grouped products, as the reference's _standard_attention does)."""
+    replays that generator's state, draws the same mask again), float32 activations (with a per-pair mask, dropout or a
+    head_dim other than 64 and 128 the scores are then materialised between two float32 grouped products, as the
+    reference's _standard_attention does)."""
 
     def __init__(self, config):
         super().__init__()
@@ -345,7 +346,7 @@ class GroupedQueryAttention(nn.Module):
         if prompt is not None:
             a = prompt[0]
         elif x.dtype == torch.float32:
-            # the reference's own route for float32 (scores materialised, model.py:807-839), on the float32 kernels
+            # the values of the reference's own route for float32 (model.py:807-839), on the float32 kernels
             if grad:
                 a = ag.AttentionF32Function.apply(q.contiguous(), k.contiguous(), v.contiguous(), self.scale, key_bias,
                                                   pair_bias, drop_p, drop_seed)

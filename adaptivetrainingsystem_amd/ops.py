@@ -1399,10 +1399,10 @@ def _attention_f32_dims(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> Tu
 def attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None,
                   key_bias: Optional[torch.Tensor] = None, pair_bias: Optional[torch.Tensor] = None,
                   dropout_p: float = 0.0, dropout_seed: int = 0, return_weights: bool = False):
-    """Causal grouped-query attention on float32 tensors the way the reference's _standard_attention runs it
-    (MS/core/model.py:807-839): the scores of every (batch, head) are materialised by a grouped product
-    (float32 MFMA kernels), softmaxed in place (ats_attention_softmax_f32: scale, causal fill, masks, dropout)
-    and multiplied with V by a second grouped product.  q [B,Hq,L,D], k, v [B,Hkv,Lk,D], D a multiple of 4;
+    """Causal grouped-query attention on float32 tensors with the values of the reference's _standard_attention
+    (MS/core/model.py:807-839).  Where attention_f32_fused_supported takes the call it is one launch; otherwise the scores of
+    every (batch, head) are materialised by a grouped product (float32 MFMA kernels), softmaxed in place
+    (ats_attention_softmax_f32: scale, causal fill, masks, dropout) and multiplied with V by a second grouped product.  q [B,Hq,L,D], k, v [B,Hkv,Lk,D], D a multiple of 4;
     key_bias / pair_bias / dropout as in causal_attention.  Returns out [B, L, Hq*D]; with return_weights also
     the state the backward needs (padded weights before and after dropout)."""
     B, Hq, Hkv, L, Lk, D = _attention_f32_dims(q, k, v)
