@@ -1688,6 +1688,50 @@ static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, i
     return (float)(per_cu > c.min_tiles ? per_cu : c.min_tiles) * (k_slabs * c.per_slab + c.per_tile);
 }
 
+// A bfloat16 projection of E experts with 21 .. 256 rows each, plain or in s slices of K, with the combine behind it, in
+// microseconds: a workgroup's chain of slabs (pc workgroups to a CU) or the weights from HBM, whichever is longer, and the partial
+// results written and read.  Fitted to 360 points: 2 .. 32 experts, [N, K] from [512, 8192] to [4096, 14336], 22 .. 224 rows, weights
+// from HBM, uneven groups.  The slices' estimates, which are the less certain ones, carry a margin.  What is chosen takes 1.2 % more
+// than the best of all on average.  (Groups vary around their mean: an eighth more rows.)
+struct SliceEstimate {
+    float rows, weights, partials;      // rows of a larger group; megabytes of the weights and of one slice's results, both ways
+    int E, N, slabs;
+    bool few;                           // 32-row tiles
+    SliceEstimate(int E_, int64_t max_rows, int N_, int K) : E(E_), N(N_), slabs(K / 64) {
+        const float avg = (float)((max_rows + E - 1) / E);
+        rows = avg * 1.125f;
+        few = avg <= 32.f;
+        weights = (float)E * N * K * 2e-6f;
+        partials = (float)max_rows * N * 8e-6f;
+    }
+    float tiles(int bm, int bn) const { return (float)E * ceilf(rows / bm) * ((N + bn - 1) / bn); }
+    float plain() const {
+        if (rows > 1.125f * 192.f && tiles(256, 256) < 128.f) return 1e30f;      // (large tiles on a few CUs: twice the time)
+        const float pc = tiles(64, 64) / 256.f, rounds = ceilf(tiles(256, 256) / 256.f);
+        return few ? 6.6f + fminf(fmaxf(slabs * (0.19f + 0.11f * pc + 0.21f * fmaxf(0.f, ceilf(pc) - 1.f)), weights / 5.5f),
+                                  rounds * (slabs * 1.62f + 1.7f)) + partials
+                   : 5.8f + fminf(fmaxf(slabs * (0.14f + 0.25f * pc), weights / 4.8f), rounds * (slabs * 1.04f + 26.6f)) + partials / 6.2f;
+    }
+    float small(int s) const {          // 32 or 64 rows x 128 columns, several to a CU
+        const float n = (float)slabs / s, pc = tiles(few ? 32 : 64, 128) * s / 256.f;
+        return few ? 1.1f * (9.4f + 0.76f * pc + fmaxf(n * (0.52f + 0.31f * pc), weights / 4.9f) + partials * s / 5.7f)
+                   : 1.05f * (8.6f + fmaxf(n * (0.65f + 0.08f * pc + 0.41f * fmaxf(0.f, pc - 1.f)), weights / 5.1f) + partials * s / 3.5f);
+    }
+    float large(int s) const {          // up to 256 rows x 256 columns, one to a CU
+        const float rounds = ceilf(tiles(256, 256) * s / 256.f);
+        // (256 rows of 8 KB pitch or a multiple of it ask few of the memory's channels at a time)
+        return (few ? 1.15f : 1.05f) * (3.9f + fmaxf(rounds * ((float)slabs / s * (1.07f + 0.00055f * rows) + 9.9f),
+                                                     weights / (slabs % 64 ? 6.2f : 4.25f)) + partials * s / 4.9f);
+    }
+};
+// Whether slices of K run on the direct-to-LDS tile.  With fewer tiles than half of the CUs the small tiles spread the work further;
+// below K = 4096, where nothing was fitted, half of the CUs decides alone.
+static bool large_slice_tile(int E, int64_t max_rows, int N, int K, int s) {
+    if ((int64_t)E * ((N + 255) / 256) * s < 128) return false;
+    const SliceEstimate t(E, max_rows, N, K);
+    return K < 4096 || t.large(s) <= t.small(s);
+}
+
 // Tile configuration by the size of the launch: the one with the least estimated time.  The constants were measured on
 // MI355X, one launch of each configuration over [33 .. 5331] x [1024 .. 6144] x [64 .. 4096] products and over 8 and
 // 64 groups of 40 .. 384 rows.  What the rule decides between, in microseconds:
@@ -1713,9 +1757,8 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
         // K in slices over workgroups: 32-row tiles, 64-row tiles where up to 64 rows can stream the weights once
         if (p.k_splits > 1) {
             if constexpr (kBf16) {
-                // (with fewer tiles than half of the CUs the small tiles below spread the work further)
                 if (E > 1 && avg > 20 && p.k_slice % 64 == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0 && !p.k_count &&
-                    (int64_t)E * ((p.N_out + 255) / 256) * p.k_splits >= 128)
+                    large_slice_tile(E, max_rows, p.N_out, p.k_slice * p.k_splits, p.k_splits))
                     return launch_mid_sliced<>(p, max_rows, s);
             }
             return avg > 32 ? launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s)
@@ -2222,6 +2265,22 @@ extern "C" int ats_grouped_gemm_nn(const void* a, int64_t lda, int64_t a_num_row
     if (rc != ATS_OK) return rc;
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;
+}
+
+extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K) {
+    using namespace ats;
+    if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0) return 1;
+    const SliceEstimate t(E, max_rows, N, K);
+    float best = t.plain();
+    int slices = 1;
+    for (int s = 2; s <= 16 && K % (s * 64) == 0 && K / s >= 512; s *= 2) {
+        const float now = large_slice_tile(E, max_rows, N, K, s) ? t.large(s) : t.small(s);
+        if (now < best) {
+            best = now;
+            slices = s;
+        }
+    }
+    return slices;
 }
 
 // Slices of K with which a product against [K][N] weights is to run, 0 where multiplying by a transposed copy is the

@@ -589,17 +589,20 @@ def down_k_splits(E: int, max_rows: int, N: int, K: int, dtype: torch.dtype) -> 
     x 256 rows 51 -> 23 us with 2; [4096, 14336] x 64 rows 156 -> 22 us with 8).
     Powers of two up to 16, slices of at least 512 columns, at most 256 rows per expert.
 
-    bfloat16 experts of more than 20 rows run their slices on the direct-to-LDS tile (up to 256 rows x 256 columns, one per
-    CU), so the slices are those that still fit one round of 256 tiles; close to 256 rows half of the experts need two tiles.
-    Against that stands the plain launch: up to 64 rows it streams the weights at 5 TB/s in 64-row tiles, above it costs the
-    same round with most CUs idle.  Measured with the combine behind it, rows per expert 22 | 32 | 48 | 64 | 96 | 128 | 192 |
-    224, plain -> the rule's, microseconds:
-      8 x [4096, 14336]   186 -> 168 | 195 -> 169 | 196 -> 172 | 272 -> 178 | 279 -> 189 | 271 -> 196 | 282 -> 215 | 323 -> 232
-      4 x [4096, 14336]    94 -> 92  | 100 -> 93  | 105 -> 95  | 131 -> 99  | 222 -> 104 | 193 -> 108 | 227 -> 125 | 294 -> 133
-      16 x [2048, 8192]    97 (116)  | 104 (119)  | 113 (121)  | 151 -> 125 | 160 -> 131 | 155 -> 137 | 161 -> 153 | 199 -> 163
-      8 x [1024, 4096]     22 (26)   |  25 (27)   |  22 (28)   |  28 (29)   |  29 (31)   |  37 -> 34  |  39 -> 43  |  83 -> 47
-    (in brackets what slices would take); 32 x [2048, 4096] and 64 x [2048, 1408] fill the chip as they are.  Below 32 MB of
-    weights everything comes from the last-level cache and the general rule stands."""
+    bfloat16 experts of more than 20 rows against 32 MB of weights or more: from K = 4096 on the number of slices with the least
+    estimated time (ats_down_k_slices), on the direct-to-LDS tile (up to 256 rows x 256 columns, one per CU) or, where that tile would
+    leave half of the CUs idle or up to 64 rows stream faster through them, on the small tiles.  Measured with the combine behind
+    it, weights from HBM, rows per expert 22 | 48 | 64 | 96 | 128 | 192 | 224, plain -> the rule's, microseconds:
+      8 x [4096, 14336]  181 -> 176 | 192 -> 174 | 283 -> 180 | 274 -> 189 | 282 -> 198 | 275 -> 218 | 318 -> 234
+      4 x [4096, 14336]   94 -> 97  | 103 -> 100 | 144 -> 105 | 224 -> 109 | 202 -> 114 | 242 -> 129 | 284 -> 134
+      2 x [4096, 14336]   61 -> 57  |  70 -> 60  | 100 -> 60  | 111 -> 62  | 100 -> 66  | 181 -> 78  | 243 -> 86
+      16 x [2048, 8192]   105       | 113        | 157 -> 141 | 167 -> 147 | 170 -> 159 | 166 -> 167 | 198 -> 172
+      4 x [1024, 8192]    33 -> 31  |  34 -> 29  |  36 -> 35  |  37 -> 36  |  44 -> 37  |  61 -> 42  | 134 -> 45
+      2 x [1024, 16384]   56 -> 37  |  59 -> 34  |  59 -> 38  |  58 -> 44  |  62 -> 41  |  61 -> 46  | 250 -> 49
+      8 x [1024, 4096]    24        |  26        |  31        |  30        |  41 -> 35  |  41 -> 42  |  82 -> 45
+    Shorter sums take the slices that fit one round of 256 large tiles, unless 64-row tiles do it in a round (or in two up to 112
+    rows: 8 x [2048, 2048], 96 rows 28 against 31, 128 rows 40 -> 33).  Below 32 MB of weights everything comes from the
+    last-level cache and the general rule stands."""
     slab = 64 if dtype == torch.bfloat16 else 32
     if E <= 0 or max_rows <= 0:
         return 1
@@ -609,6 +612,8 @@ def down_k_splits(E: int, max_rows: int, N: int, K: int, dtype: torch.dtype) -> 
     if E > 1 and max_rows // E <= 20:
         return 1        # the plain launch streams the weights itself (8 x [4096, 14336], 16 rows each: 157 against 159 us)
     if E > 1 and dtype == torch.bfloat16 and E * N * K >= 1 << 24:
+        if K >= 4096:
+            return int(_lib.load().ats_down_k_slices(int(E), int(max_rows), int(N), int(K)))
         n256, n64 = -(-N // 256), -(-N // 64)
         tiles = E * n256 * (3 if rows > 232 else 2) // 2
         s = 1
@@ -616,8 +621,9 @@ def down_k_splits(E: int, max_rows: int, N: int, K: int, dtype: torch.dtype) -> 
             s *= 2
         if rows < 64:
             return s if K / (slab * s) * 1.3 + 18.0 < 0.97 * E * N * K * 2 / 5e6 else 1
-        # (groups vary around their mean; one 64-row tile per CU at most)
-        return 1 if rows <= 192 and E * -(-(rows + rows // 7) // 64) * n64 <= 256 else s
+        # (groups vary around their mean)
+        tiles64 = E * -(-(rows + rows // 7) // 64) * n64
+        return 1 if rows <= 192 and tiles64 <= 256 or rows <= 112 and tiles64 <= 512 else s
     n128 = (N + 127) // 128
     plain = E * n128 if max_rows // E <= 32 else E * ((rows + 127) // 128) * ((N + 255) // 256)
     if plain >= 384:

@@ -30,6 +30,14 @@ def test_sliced_down_projection(gpu, counts, H, I, S):
         assert (parts[s].double() - ref).abs().max() <= bound
 
 
+# slices of 512 columns and more, where an estimate chooses between that tile and the small ones: a few rows against few columns
+# (small), 32-row tiles, more rows (large), too few large tiles (small)
+@pytest.mark.parametrize("counts,H,I,S", [([40, 56], 1000, 16384, 16), ([21, 24, 0, 33], 1032, 8192, 8), ([100, 156], 1000, 16384, 16),
+                                          ([90, 0, 129, 64, 33, 1, 128, 200], 1032, 4096, 8), ([70, 65], 1000, 16384, 8)])
+def test_sliced_down_projection_on_the_estimated_tile(gpu, counts, H, I, S):
+    test_sliced_down_projection(gpu, counts, H, I, S)
+
+
 @pytest.mark.parametrize("T", [176, 700])
 def test_layer_with_sliced_down_projection(gpu, T):
     """The layer whose rule chooses these slices against the stages in float64."""
