@@ -281,7 +281,16 @@ static int launch_rmsnorm(const void* x, const void* w, void* y, int64_t rows, i
     const int64_t most = per_lane > 8 ? INT64_MAX : per_lane < 2 ? 0 : V == 4 ? 512 : per_lane <= 4 ? 4096
                          : HAS_W && sizeof(WT) == 4 ? 1024 : INT64_MAX;
     if (rows <= most) {
-        const unsigned grid = (unsigned)(rows < kRmsRowBlocks ? rows : kRmsRowBlocks);
+        // Float32 weights of a long bfloat16 row are twice its bytes: from 1024 rows on a workgroup that loads them takes two rows or
+        // more (at most four workgroups to a CU).  Wave per row | a row per workgroup | this, microseconds: [1024, 7168] 7.0 | 8.2 |
+        // 7.3, [1024, 8192] 7.8 | 8.9 | 7.9 (below 6144 columns one row is the better: [1024, 5120] 5.7 | 5.8 | 6.0), [1536, 8192]
+        // 12.4 | 13.2 | 11.7, [2048, 5120] 10.5 | 11.4 | 10.8, [2048, 8192] 14.8 | 15.9 | 15.0, [4096, 8192] 28.1 | 27.6 | 26.2,
+        // [8192, 7168] 45.1 | 45.0 | 43.2, [16384, 8192] 93.4 | 95.9 | 94.6
+        int64_t each = 1;
+        if (V == 8 && HAS_W && sizeof(WT) == 4 && per_lane > 8 && rows >= (per_lane >= 12 ? 1024 : 1025))
+            each = rows <= 2048 ? 2 : (rows + 1023) / 1024;
+        const int64_t groups = (rows + each - 1) / each;
+        const unsigned grid = (unsigned)(groups < kRmsRowBlocks ? groups : kRmsRowBlocks);
 #define ATS_RMS_ROW(NV)                                                                                               \
     hipLaunchKernelGGL((rmsnorm_row_block_kernel<T, WT, NV, HAS_W>), dim3(grid), dim3(256), 0, s, xp, wp, yp, rows, H, eps)
         if (per_lane <= 4) ATS_RMS_ROW(1);

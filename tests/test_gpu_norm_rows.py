@@ -52,3 +52,12 @@ def test_squares_are_added_in_the_order_of_one_wave(ops, gpu, H, rows):  # noqa:
     want = x.double() / (2.0 ** 24 / H + 1e-6) ** 0.5
     # division, root, reciprocal and product: a unit of 2^-23 at most each and half of one
     assert ((y - want).abs() <= want * 2.5 * 2.0 ** -23).all()
+
+
+# float32 weights: workgroups of one row below 1024 rows (1025 of shorter ones), of two and more from there, of as many as 1024 of them need
+@pytest.mark.parametrize("H,many", [(8192, 1024), (5640, 1023), (4104, 1025), (4104, 2049), (5120, 3073)])
+def test_rows_that_share_their_weights(ops, gpu, H, many):  # noqa: F811
+    print("case norm shared weights", H, many, flush=True)
+    x = (torch.randn(many, H, generator=gen(H)) * 1.3).bfloat16().to(gpu)
+    w = (1 + 0.1 * torch.randn(H, generator=gen(H + 1))).to(gpu)
+    assert torch.equal(ops.rmsnorm(x, w), torch.cat([ops.rmsnorm(part, w) for part in x.split(500)]))
