@@ -20,16 +20,16 @@
 // bfloat16 kernels, do not reach the row; the materialised product multiplied them by zero, to NaN.)
 // Bounds: launches and the serial chain of a tile (32 MFMAs of 32 cycles per product) at short sequences, L1 traffic at long
 // ones (every tile is read in both layouts).  Materialised route -> this, microseconds, forward | backward:
-//   2 x 54, 4 heads of 128    88 ->    8 |   158 ->   21        1 x 1024, 32 heads of 128   287 ->  165 |   639 ->  712
-//   2 x 256, 4 heads of 128   57 ->   12 |   133 ->   51        1 x 2048, 16 heads of  64   480 ->  156 |  1177 ->  622
-//   4 x 512, 4 heads of 128   77 ->   31 |   135 ->  112        1 x 4096, 32 heads of 128  6571 -> 1697 | 16260 -> 6697
-// (The backward of 1 x 1024 alone is the slower one.  Its materialised form needs the weights that only the materialised forward
-// keeps, so one route takes both passes: 926 -> 877 together.)
+//   2 x 54, 4 heads of 128    88 ->    7 |   158 ->   19        1 x 1024, 32 heads of 128   287 ->  127 |   639 ->  458
+//   2 x 256, 4 heads of 128   57 ->   12 |   133 ->   39        1 x 2048, 16 heads of  64   480 ->  123 |  1177 ->  435
+//   4 x 512, 4 heads of 128   77 ->   32 |   135 ->   92        1 x 4096, 32 heads of 128  6571 -> 1460 | 16260 -> 6104
+//   4 x 512, 32 heads of 128 284 ->  153 |   650 ->  562
 // Errors against float64 (output, dq, dk, dv), 8 heads x 32: 1.1e-7, 1.9e-7, 2.1e-7, 1.5e-7 -> 1.2e-7, 1.8e-7, 1.8e-7,
 // 1.3e-7; 16 heads x 512: 3.4e-7, 4.2e-7, 6.1e-7, 5.9e-7 -> 1.7e-7, 2.2e-7, 2.9e-7, 2.7e-7.
 #include <math.h>
 
 #include "ats_common.hpp"
+#include "tile_schedule.hpp"
 
 namespace ats {
 
@@ -120,6 +120,19 @@ __device__ __forceinline__ float largest_bias(const float* kb, int from, int Lk)
     return m;
 }
 
+// The tiles of a head on one XCD (consecutive workgroups go to different ones), whose L2 then holds the keys and values of the two or
+// three heads that it works on instead of all that run, where the heads divide by the XCDs; same bits.  4 x 512, 32 heads of 128:
+// 213 -> 153 us forward, 855 -> 562 backward.
+__device__ __forceinline__ void tile_and_head(int& tile, int& head) {
+    tile = blockIdx.x;
+    head = blockIdx.y;
+    if (gridDim.y % kNumXcd == 0) {
+        const unsigned id = blockIdx.y * gridDim.x + blockIdx.x, within = id / kNumXcd;
+        tile = (int)(within % gridDim.x);
+        head = (int)(within / gridDim.x * kNumXcd + id % kNumXcd);
+    }
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void attention_f32_fwd_kernel(AttnF32Args p) {
     constexpr int W = 4;
@@ -127,8 +140,10 @@ __global__ __launch_bounds__(256) void attention_f32_fwd_kernel(AttnF32Args p) {
     __shared__ __align__(16) float s_o[W][16 * (D + 4)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
-    const int e = blockIdx.y, b = e / p.Hq, h = e - b * p.Hq;
-    const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * 16;      // the longest rows first
+    int tile, e;
+    tile_and_head(tile, e);
+    const int b = e / p.Hq, h = e - b * p.Hq;
+    const int q0 = ((int)gridDim.x - 1 - tile) * 16;      // the longest rows first
     const int q = q0 + c < p.L ? q0 + c : p.L - 1;
     const int last_key = q + p.Lk - p.L;
     const int64_t kvh = (int64_t)b * p.Hkv + h / (p.Hq / p.Hkv);
@@ -229,8 +244,10 @@ __global__ __launch_bounds__(256) void attention_f32_dq_kernel(AttnF32Args p) {
     __shared__ __align__(16) float s_o[W][16 * (D + 4)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
-    const int e = blockIdx.y, b = e / p.Hq, h = e - b * p.Hq;
-    const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * 16;
+    int tile, e;
+    tile_and_head(tile, e);
+    const int b = e / p.Hq, h = e - b * p.Hq;
+    const int q0 = ((int)gridDim.x - 1 - tile) * 16;
     const int q = q0 + c < p.L ? q0 + c : p.L - 1;
     const int last_key = q + p.Lk - p.L;
     const int64_t kvh = (int64_t)b * p.Hkv + h / (p.Hq / p.Hkv);
@@ -327,15 +344,17 @@ __global__ __launch_bounds__(512) void attention_f32_dkv_kernel(AttnF32Args p) {
     __shared__ __align__(16) float s_o[W / 2][16 * (D + 4)];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
-    const int b = blockIdx.y / p.Hkv, hk = blockIdx.y - b * p.Hkv;
-    const int k0 = (int)blockIdx.x * 16;                         // the first keys have the most rows
+    int tile, kvh;
+    tile_and_head(tile, kvh);
+    const int b = kvh / p.Hkv, hk = kvh - b * p.Hkv;
+    const int k0 = tile * 16;                                    // the first keys have the most rows
     const int key = k0 + c < p.Lk ? k0 + c : p.Lk - 1;
     const int rep = p.Hq / p.Hkv, off = p.Lk - p.L;
     const float* kb = p.key_bias ? p.key_bias + (int64_t)b * p.Lk : nullptr;
     const int64_t e0 = (int64_t)b * p.Hq + hk * rep;             // first query head
     f32x4v kf[D / 16], vf[D / 16];
-    load_rows<D>(kf, p.k + ((int64_t)blockIdx.y * p.Lk + key) * D, g);
-    load_rows<D>(vf, p.v + ((int64_t)blockIdx.y * p.Lk + key) * D, g);
+    load_rows<D>(kf, p.k + ((int64_t)kvh * p.Lk + key) * D, g);
+    load_rows<D>(vf, p.v + ((int64_t)kvh * p.Lk + key) * D, g);
     float fill = kFill;                                          // largest score of these keys in the rows before them
     if (kb) {
         const float own = kb[key];
@@ -410,7 +429,7 @@ __global__ __launch_bounds__(512) void attention_f32_dkv_kernel(AttnF32Args p) {
 #pragma unroll
             for (int jj = 0; jj < D / 64; ++jj) {
                 const int at = r * (D + 4) + 64 * jj + 4 * part;
-                *reinterpret_cast<f32x4v*>(out + ((int64_t)blockIdx.y * p.Lk + k0 + r) * D + 64 * jj + 4 * part) =
+                *reinterpret_cast<f32x4v*>(out + ((int64_t)kvh * p.Lk + k0 + r) * D + 64 * jj + 4 * part) =
                     (ldv(s_o[0] + at) + ldv(s_o[1] + at)) + (ldv(s_o[2] + at) + ldv(s_o[3] + at));
             }
         }

@@ -148,3 +148,24 @@ def test_the_scale_may_be_left_to_the_head_dim_and_saved_tensors_may_come_back_e
         out = AttentionF32Function.apply(q, k, v, None)
     for a, b in zip(torch.autograd.grad(out, (q, k, v), dout), want):
         assert torch.equal(a, b)
+
+
+# heads that divide by the XCDs (their tiles keep to one) and heads that do not, odd numbers of tiles
+@pytest.mark.parametrize("B,Hq,Hkv,L,Lk,D", [(1, 8, 8, 40, 40, 64), (2, 12, 4, 100, 133, 64), (3, 16, 8, 17, 300, 128), (1, 24, 8, 257, 257, 128), (1, 9, 3, 65, 65, 64)])
+def test_a_head_has_the_same_bits_alone(gpu, B, Hq, Hkv, L, Lk, D):
+    from adaptivetrainingsystem_amd import ops
+    print("case f32 heads", B, Hq, Hkv, L, Lk, D, flush=True)
+    g = torch.Generator().manual_seed(L + Hq)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(gpu) for h, n in ((Hq, L), (Hkv, Lk), (Hkv, Lk)))
+    dout, rep = torch.randn(B, L, Hq * D, generator=g).to(gpu), Hq // Hkv
+    out, stats = ops.attention_f32_fused(q, k, v, None, None)
+    grads = ops.attention_f32_fused_bwd(q, k, v, out, stats, dout, None, None)
+    for b in range(B):
+        for h in range(Hkv):
+            heads, cols = slice(h * rep, (h + 1) * rep), slice(h * rep * D, (h + 1) * rep * D)
+            one = [t[b:b + 1, s].contiguous() for t, s in ((q, heads), (k, slice(h, h + 1)), (v, slice(h, h + 1)))]
+            o, st = ops.attention_f32_fused(*one, None, None)
+            assert torch.equal(o, out[b:b + 1, :, cols])
+            got = ops.attention_f32_fused_bwd(*one, o, st, dout[b:b + 1, :, cols].contiguous(), None, None)
+            for t, whole, s in zip(got, grads, (heads, slice(h, h + 1), slice(h, h + 1))):
+                assert torch.equal(t, whole[b:b + 1, s])
