@@ -226,7 +226,9 @@ __global__ __launch_bounds__(256) void route_bwd_kernel(const float* __restrict_
 }
 
 // Up to 8 experts (kept in registers): the kernel above reads and writes its gradients through memory once per term, a chain
-// of some twenty trips (512 tokens, 8 experts: 13.3 -> 7.6 us).  The same sums in the same order.
+// of some twenty trips (512 tokens, 8 experts: 13.3 -> 7.6 us).  The same sums in the same order.  N, the experts that have
+// registers: work for absent ones shows (512 tokens, top 1, 2 experts 3.1 us above, 4.1 with N = 8, 2.0 with N = 2; 4 experts 3.9,
+// 4.2, 2.4).
 template <int N>
 __global__ __launch_bounds__(64) void route_bwd_few_kernel(const float* __restrict__ z_route, const float* __restrict__ z_aux,
                                                            const int32_t* __restrict__ idx, const float* __restrict__ w,
@@ -644,11 +646,13 @@ extern "C" int ats_route_bwd(const float* logits_route, const float* logits_aux,
     if (T == 0) return ATS_OK;
     ATS_REQUIRE(logits_route && idx && w && dw && dlogits && (!usage || logits_aux), ATS_ERR_INVALID_ARG,
                 "ats_route_bwd: null pointer");
-    if (E <= 8)
-        hipLaunchKernelGGL(route_bwd_few_kernel<8>, dim3((unsigned)((T + 63) / 64)), dim3(64), 0, as_stream(stream),
+    if (E <= 8) {
+        auto kern = E <= 1 ? route_bwd_few_kernel<1> : E <= 2 ? route_bwd_few_kernel<2> : E <= 4 ? route_bwd_few_kernel<4>
+                                                                                                : route_bwd_few_kernel<8>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((T + 63) / 64)), dim3(64), 0, as_stream(stream),
                            logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, 1.0f / temperature, mode,
                            dlogits, T, E, k);
-    else
+    } else
         hipLaunchKernelGGL(route_bwd_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, as_stream(stream),
                            logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, 1.0f / temperature, mode,
                            dlogits, T, E, k);

@@ -28,6 +28,13 @@ def test_route_gradient_few_experts(gpu, T, E, k, mode):
     assert (out.cpu().double() - z.grad).abs().max() <= 4e-6 * (dw.abs().max().item() / tau + 1)
 
 
+# both ends of what each instance holds
+@pytest.mark.parametrize("T,E,k", [(65, 1, 1), (129, 2, 2), (64, 3, 1), (200, 3, 3), (63, 4, 2), (65, 4, 4), (64, 5, 5)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_route_gradient_of_each_instance(gpu, T, E, k, mode):
+    test_route_gradient_few_experts(gpu, T, E, k, mode)
+
+
 @pytest.mark.parametrize("T,E,H,dtype", [(256, 8, 512, torch.float32), (257, 8, 4096, torch.bfloat16), (9, 3, 72, torch.float32),
                                          (1000, 64, 2048, torch.bfloat16), (5000, 8, 264, torch.bfloat16)])
 def test_router_gradients_small_chunks(gpu, T, E, H, dtype):
