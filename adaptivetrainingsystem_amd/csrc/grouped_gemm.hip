@@ -1688,50 +1688,6 @@ static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, i
     return (float)(per_cu > c.min_tiles ? per_cu : c.min_tiles) * (k_slabs * c.per_slab + c.per_tile);
 }
 
-// A bfloat16 projection of E experts with 21 .. 256 rows each, plain or in s slices of K, with the combine behind it, in
-// microseconds: a workgroup's chain of slabs (pc workgroups to a CU) or the weights from HBM, whichever is longer, and the partial
-// results written and read.  Fitted to 360 points: 2 .. 32 experts, [N, K] from [512, 8192] to [4096, 14336], 22 .. 224 rows, weights
-// from HBM, uneven groups.  The slices' estimates, which are the less certain ones, carry a margin.  What is chosen takes 1.2 % more
-// than the best of all on average.  (Groups vary around their mean: an eighth more rows.)
-struct SliceEstimate {
-    float rows, weights, partials;      // rows of a larger group; megabytes of the weights and of one slice's results, both ways
-    int E, N, slabs;
-    bool few;                           // 32-row tiles
-    SliceEstimate(int E_, int64_t max_rows, int N_, int K) : E(E_), N(N_), slabs(K / 64) {
-        const float avg = (float)((max_rows + E - 1) / E);
-        rows = avg * 1.125f;
-        few = avg <= 32.f;
-        weights = (float)E * N * K * 2e-6f;
-        partials = (float)max_rows * N * 8e-6f;
-    }
-    float tiles(int bm, int bn) const { return (float)E * ceilf(rows / bm) * ((N + bn - 1) / bn); }
-    float plain() const {
-        if (rows > 1.125f * 192.f && tiles(256, 256) < 128.f) return 1e30f;      // (large tiles on a few CUs: twice the time)
-        const float pc = tiles(64, 64) / 256.f, rounds = ceilf(tiles(256, 256) / 256.f);
-        return few ? 6.6f + fminf(fmaxf(slabs * (0.19f + 0.11f * pc + 0.21f * fmaxf(0.f, ceilf(pc) - 1.f)), weights / 5.5f),
-                                  rounds * (slabs * 1.62f + 1.7f)) + partials
-                   : 5.8f + fminf(fmaxf(slabs * (0.14f + 0.25f * pc), weights / 4.8f), rounds * (slabs * 1.04f + 26.6f)) + partials / 6.2f;
-    }
-    float small(int s) const {          // 32 or 64 rows x 128 columns, several to a CU
-        const float n = (float)slabs / s, pc = tiles(few ? 32 : 64, 128) * s / 256.f;
-        return few ? 1.1f * (9.4f + 0.76f * pc + fmaxf(n * (0.52f + 0.31f * pc), weights / 4.9f) + partials * s / 5.7f)
-                   : 1.05f * (8.6f + fmaxf(n * (0.65f + 0.08f * pc + 0.41f * fmaxf(0.f, pc - 1.f)), weights / 5.1f) + partials * s / 3.5f);
-    }
-    float large(int s) const {          // up to 256 rows x 256 columns, one to a CU
-        const float rounds = ceilf(tiles(256, 256) * s / 256.f);
-        // (256 rows of 8 KB pitch or a multiple of it ask few of the memory's channels at a time)
-        return (few ? 1.15f : 1.05f) * (3.9f + fmaxf(rounds * ((float)slabs / s * (1.07f + 0.00055f * rows) + 9.9f),
-                                                     weights / (slabs % 64 ? 6.2f : 4.25f)) + partials * s / 4.9f);
-    }
-};
-// Whether slices of K run on the direct-to-LDS tile.  With fewer tiles than half of the CUs the small tiles spread the work further;
-// below K = 4096, where nothing was fitted, half of the CUs decides alone.
-static bool large_slice_tile(int E, int64_t max_rows, int N, int K, int s) {
-    if ((int64_t)E * ((N + 255) / 256) * s < 128) return false;
-    const SliceEstimate t(E, max_rows, N, K);
-    return K < 4096 || t.large(s) <= t.small(s);
-}
-
 // Tile configuration by the size of the launch: the one with the least estimated time.  The constants were measured on
 // MI355X, one launch of each configuration over [33 .. 5331] x [1024 .. 6144] x [64 .. 4096] products and over 8 and
 // 64 groups of 40 .. 384 rows.  What the rule decides between, in microseconds:
@@ -1747,6 +1703,119 @@ static bool large_slice_tile(int E, int64_t max_rows, int N, int K, int s) {
 // than 192 rows always run on the 16 x 16 x 32 kernel and float32 groups of more than 256 rows are not sliced along K,
 // because the fused training launches and the K-major products, which start at those sizes, accumulate in that order
 // (their results equal those of the separate launches bit for bit).
+enum class GroupTile { kSmall32, kSmall64, kSeq, kMid, kBig };      // kSeq: 64 rows, all of K in a wave
+template <bool kBf16, bool SWIGLU>
+static GroupTile pick_group_tile(int64_t max_rows, int E, int N, int nk) {
+    const int64_t avg = max_rows / E;
+    // (columns: output columns per tile, half of the weight rows with the SwiGLU epilogue)
+    constexpr TileCost kSmall32 = kBf16 ? TileCost{32, 32, SWIGLU ? 0.165f : 0.093f, 1.f, SWIGLU ? 1 : 2}
+                                        : TileCost{32, 32, SWIGLU ? 0.40f : 0.18f, 1.5f, 1};
+    constexpr TileCost kSmall64 = kBf16 ? TileCost{64, SWIGLU ? 32 : 64, 0.245f, 1.5f, 1}
+                                        : TileCost{64, SWIGLU ? 32 : 64, 0.58f, 3.f, 1};
+    constexpr TileCost kMid = kBf16 ? TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 0.58f : 1.05f, 5.f, 1}
+                                    : TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 2.0f : 3.65f, 5.f, 1};
+    const float mid = tile_time(kMid, max_rows, E, N, nk, true);
+    // (the 16 x 16 x 32 kernel computes only the 16-row fragments that a tile has; up to 192 rows its loads bound a slab)
+    const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? (avg <= 192 ? 1.3f : 1.45f) : 7.3f, 7.f, 1},
+                                max_rows, E, N, nk, true);
+    const float least_large = mid < big ? mid : big;
+    // (two full rounds of 256-row tiles: nothing is idle, and groups of unequal size fit them better; 8 experts with 20-45
+    // rows each, gate/up [28672, 4096]: 343 us against 372 in 32-row tiles)
+    const int64_t big_tiles = (int64_t)E * ((avg + 255) / 256) * ((N + (SWIGLU ? 127 : 255)) / (SWIGLU ? 128 : 256));
+    if (big_tiles < 512) {
+        if (avg <= (kBf16 ? 192 : 256)) {
+            const float small32 = tile_time(kSmall32, max_rows, E, N, nk);
+            // (a long K streams the weights from HBM: 8 groups x 128 rows, [4096, 14336]: 328 us against 258 in 128-row tiles)
+            TileCost c64 = kSmall64;
+            if (kBf16 && nk >= 128) c64.per_slab = 0.3f;
+            const float small64 = tile_time(c64, max_rows, E, N, nk);
+            if (small32 < least_large && small32 <= small64) return GroupTile::kSmall32;
+            if (small64 < least_large) return GroupTile::kSmall64;
+        } else if constexpr (!kBf16) {
+            constexpr TileCost kSeq = TileCost{64, 64, SWIGLU ? 1.4f : 0.74f, 3.f, 1};
+            if (tile_time(kSeq, max_rows, E, N, nk) < least_large) return GroupTile::kSeq;
+        }
+    }
+    return mid < big && !(kBf16 && avg > 192) ? GroupTile::kMid : GroupTile::kBig;
+}
+
+// up to 32 rows per expert against a long K, for callers that do not cut K (8 experts x 32 rows, [4096, 14336], with
+// the combine behind it: 178 us, 21 rows 165; two slices of K over workgroups 165 and 163; the launch in 256-row tiles
+// 264)
+static bool streams_long_k(int64_t avg, int pieces, int N) { return avg <= 32 && pieces >= 64 && N >= 32; }
+
+// A bfloat16 projection of E experts with 21 .. 256 rows each and 32 MB of weights or more, plain or in s slices of K, with the
+// combine behind it, in microseconds: a workgroup's chain of slabs and the weights from HBM, which overlap in part (hence the
+// root of the squares), the start, and the partial results written and read.  What the chain depends on is how the workgroups
+// fill the chip: two of the 64-row tiles share a CU, a third is a second round; the 256-column tiles come in supertiles of 32
+// that belong to one XCD each, so that ten tiles of a row band leave some XCDs a second round and others idle.  Fitted to 8071
+// points, 2 .. 64 experts, 512 .. 8192 columns, K from 1024 to 16384, uneven groups, weights from HBM: within 7 % (256 columns)
+// to 11 % (slices on the small tiles) of the times, root mean square.
+struct SliceEstimate {
+    int E, N, K;
+    int64_t max_rows;
+    float avg, slabs, weights, partials;      // megabytes of the weights and of one slice's results, written and read
+    SliceEstimate(int E_, int64_t max_rows_, int N_, int K_) : E(E_), N(N_), K(K_), max_rows(max_rows_) {
+        avg = (float)max_rows / E;
+        slabs = K / 64.f;
+        weights = (float)E * N * K * 2e-6f;
+        partials = (float)max_rows * N * 8e-6f;
+    }
+    // Tiles of bm rows per group, on average over groups whose sizes vary by their square root.
+    float row_tiles(float bm) const {
+        const float t = ceilf(avg / bm), w = 1.7f / sqrtf(avg);
+        return t + 1.f / (1.f + expf(w * (t * bm - avg))) - (t > 1.f ? 1.f / (1.f + expf(w * (avg - (t - 1.f) * bm))) : 0.f);
+    }
+    static float join(float a, float b) { return sqrtf(a * a + b * b); }
+    // bm rows x 256 columns, one to a CU; pitch: rows of 8 KB or a multiple of it ask few of the memory's channels at a time
+    struct Tall { float bm, slab, slab_row, tile, rate, start, parts, pitch; };
+    float tall(const Tall& c, int s) const {
+        const int n_tiles = (N + 255) / 256;
+        int sm, sn;
+        pick_supertile(n_tiles, &sm, &sn);
+        const float m = s * roundf(E * row_tiles(c.bm)), super = ceilf(m / sm) * ((n_tiles + sn - 1) / sn);
+        const float rounds = fmaxf(1.f, ceilf(ceilf(super / kNumXcd) * (m * n_tiles / (super * kSuperBlocks)) - 0.02f));
+        const float chain = rounds * (slabs / s * (c.slab + c.slab_row * fminf(avg, c.bm)) + c.tile);
+        const float load = weights / c.rate * sqrtf(sqrtf(kNumXcd / fminf(super, kNumXcd))) * (K % 4096 == 0 ? 1.f + c.pitch : 1.f);
+        return c.start + join(chain, load) + partials * s / c.parts;
+    }
+    float large(int s) const { return tall(Tall{256.f, 0.75f, 0.0016f, 7.7f, 6.5f, 5.1f, 5.7f, 0.11f}, s); }
+    // 32 or 64 rows x 128 columns, slices of K over workgroups; a row band is launched as whole supertiles of 32 columns' tiles, and
+    // the workgroups without a tile cost a microsecond per round
+    float small(int s) const {
+        const bool few = max_rows / E <= 32;
+        const float n = slabs / s, bands = E * s * row_tiles(few ? 32.f : 64.f), n_tiles = (N + 127) / 128;
+        const float tiles = bands * n_tiles / 256.f, pc = fmaxf(1.f, tiles);
+        const float empty = bands * (float)((N + 4095) / 4096) * 32.f / 256.f - tiles;
+        if (few) return 7.6f + n * (0.476f + 0.207f * pc + (pc > 3.1f ? 0.381f : 0.f)) + 0.476f * pc + 0.913f * empty + weights / 11.2f;
+        const float chain = n * (0.325f + 0.377f * pc + (pc > 2.12f ? 0.367f : 0.f)) + 0.077f * pc + 1.02f * empty;
+        return 8.6f + powf(powf(chain, 1.36f) + powf(weights / 9.7f, 1.36f), 1.f / 1.36f) + partials * s / 13.5f;
+    }
+    float plain() const {
+        if (streams_long_k(max_rows / E, K * 2 / 256, N)) return 8.65f + join(slabs * 0.172f, weights / 5.3f);
+        switch (pick_group_tile<true, false>(max_rows, E, N, (K + 63) / 64)) {
+            case GroupTile::kSmall32: return 8.06f + join(slabs * 0.164f, weights * (1.f + 0.497f * (row_tiles(32.f) - 1.f)) / 5.24f);
+            case GroupTile::kSmall64: {
+                const float r = row_tiles(64.f), pc = E * r * ((N + 63) / 64) / 256.f;
+                return 8.63f + join(slabs * (0.271f + (pc > 2.12f ? 0.318f : 0.f)), weights * (1.f + 0.396f * (r - 1.f)) / 5.28f) + partials / 4.65f;
+            }
+            case GroupTile::kMid: return tall(Tall{128.f, 0.897f, 0.f, 2.5f, 6.83f, 2.f, 4.7f, 0.108f}, 1);
+            default: return tall(Tall{256.f, 0.656f, 0.0018f, 8.f, 5.8f, 2.6f, 8.5f, 0.064f}, 1);
+        }
+    }
+    // What the plain launch and the slices on the small tiles have to exceed before the large one is taken: the estimates are off by a
+    // few microseconds and, where groups come close to a second row tile, by more.
+    float large_with_margin(int s) const { return large(s) * (avg <= 64.f ? 1.f : avg <= 208.f ? 1.03f : 1.06f) + 2.f; }
+};
+// Whether slices of K run on the direct-to-LDS tile.  Slices of less than 512 columns, which no rule asks for and nothing was fitted
+// to: with tiles for half of the CUs.  Less than 32 MB of weights come from the last-level cache: never.
+static bool large_slice_tile(int E, int64_t max_rows, int N, int K, int s) {
+    if (K / s < 512) return (int64_t)E * ((N + 255) / 256) * s >= 128;
+    if ((int64_t)E * N * K < (1 << 24)) return false;
+    const SliceEstimate t(E, max_rows, N, K);
+    return t.large_with_margin(s) < t.small(s);
+}
+
 template <typename T, typename TO, bool SWIGLU>
 static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s) {
     constexpr bool kBf16 = std::is_same<T, bf16_t>::value;
@@ -1798,43 +1867,15 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
         }
     }
     if constexpr (!SWIGLU) {
-        // up to 32 rows per expert against a long K, for callers that do not cut K (8 experts x 32 rows, [4096, 14336], with
-        // the combine behind it: 178 us, 21 rows 165; two slices of K over workgroups 165 and 163; the launch in 256-row tiles
-        // 264)
-        if (avg <= 32 && pieces >= 64 && p.N_out >= 32 && !p.k_count) return launch_stream<T, TO, 2, 4, 4, SWIGLU>(p, max_rows, s);
+        if (streams_long_k(avg, pieces, p.N_out) && !p.k_count) return launch_stream<T, TO, 2, 4, 4, SWIGLU>(p, max_rows, s);
     }
-    // (columns: output columns per tile, half of the weight rows with the SwiGLU epilogue)
-    constexpr TileCost kSmall32 = kBf16 ? TileCost{32, 32, SWIGLU ? 0.165f : 0.093f, 1.f, SWIGLU ? 1 : 2}
-                                        : TileCost{32, 32, SWIGLU ? 0.40f : 0.18f, 1.5f, 1};
-    constexpr TileCost kSmall64 = kBf16 ? TileCost{64, SWIGLU ? 32 : 64, 0.245f, 1.5f, 1}
-                                        : TileCost{64, SWIGLU ? 32 : 64, 0.58f, 3.f, 1};
-    constexpr TileCost kMid = kBf16 ? TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 0.58f : 1.05f, 5.f, 1}
-                                    : TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 2.0f : 3.65f, 5.f, 1};
-    const float mid = tile_time(kMid, max_rows, E, p.N_out, nk, true);
-    // (the 16 x 16 x 32 kernel computes only the 16-row fragments that a tile has; up to 192 rows its loads bound a slab)
-    const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? (avg <= 192 ? 1.3f : 1.45f) : 7.3f, 7.f, 1},
-                                max_rows, E, p.N_out, nk, true);
-    const float least_large = mid < big ? mid : big;
-    // (two full rounds of 256-row tiles: nothing is idle, and groups of unequal size fit them better; 8 experts with 20-45
-    // rows each, gate/up [28672, 4096]: 343 us against 372 in 32-row tiles)
-    const int64_t big_tiles = (int64_t)E * ((avg + 255) / 256) * ((p.N_out + (SWIGLU ? 127 : 255)) / (SWIGLU ? 128 : 256));
-    if (big_tiles < 512) {
-        if (avg <= (kBf16 ? 192 : 256)) {
-            const float small32 = tile_time(kSmall32, max_rows, E, p.N_out, nk);
-            // (a long K streams the weights from HBM: 8 groups x 128 rows, [4096, 14336]: 328 us against 258 in 128-row tiles)
-            TileCost c64 = kSmall64;
-            if (kBf16 && nk >= 128) c64.per_slab = 0.3f;
-            const float small64 = tile_time(c64, max_rows, E, p.N_out, nk);
-            if (small32 < least_large && small32 <= small64)
-                return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
-            if (small64 < least_large) return launch_small<T, TO, 2, 2, 4, 1, SWIGLU>(p, max_rows, s);
-        } else if constexpr (!kBf16) {
-            constexpr TileCost kSeq = TileCost{64, 64, SWIGLU ? 1.4f : 0.74f, 3.f, 1};
-            if (tile_time(kSeq, max_rows, E, p.N_out, nk) < least_large)
-                return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 1, 2, SWIGLU>(p, max_rows, s);
-        }
+    const GroupTile tile = pick_group_tile<kBf16, SWIGLU>(max_rows, E, p.N_out, nk);
+    if (tile == GroupTile::kSmall32) return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
+    if (tile == GroupTile::kSmall64) return launch_small<T, TO, 2, 2, 4, 1, SWIGLU>(p, max_rows, s);
+    if constexpr (!kBf16) {
+        if (tile == GroupTile::kSeq) return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 1, 2, SWIGLU>(p, max_rows, s);
     }
-    if (mid < big && !(kBf16 && avg > 192)) {
+    if (tile == GroupTile::kMid) {
         if constexpr (SWIGLU) return launch_cfg<T, TO, 128, 128, 2, 2, 4, 8, SWIGLU>(p, max_rows, s);
         else return launch_cfg<T, TO, 128, 256, 2, 4, 4, 8, SWIGLU>(p, max_rows, s);
     }
@@ -2267,16 +2308,20 @@ extern "C" int ats_grouped_gemm_nn(const void* a, int64_t lda, int64_t a_num_row
     return ATS_OK;
 }
 
-extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K) {
+// small: the slices that fill the chip with the small tiles (1: none are needed)
+extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K, int small) {
     using namespace ats;
-    if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0) return 1;
+    if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || small < 1) return 1;
     const SliceEstimate t(E, max_rows, N, K);
     float best = t.plain();
     int slices = 1;
+    if (small > 1 && t.small(small) <= best) {
+        best = t.small(small);
+        slices = small;
+    }
     for (int s = 2; s <= 16 && K % (s * 64) == 0 && K / s >= 512; s *= 2) {
-        const float now = large_slice_tile(E, max_rows, N, K, s) ? t.large(s) : t.small(s);
-        if (now < best) {
-            best = now;
+        if (t.large_with_margin(s) < best && large_slice_tile(E, max_rows, N, K, s)) {
+            best = t.large_with_margin(s);
             slices = s;
         }
     }

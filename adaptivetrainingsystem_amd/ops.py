@@ -589,20 +589,21 @@ def down_k_splits(E: int, max_rows: int, N: int, K: int, dtype: torch.dtype) -> 
     x 256 rows 51 -> 23 us with 2; [4096, 14336] x 64 rows 156 -> 22 us with 8).
     Powers of two up to 16, slices of at least 512 columns, at most 256 rows per expert.
 
-    bfloat16 experts of more than 20 rows against 32 MB of weights or more: from K = 4096 on the number of slices with the least
-    estimated time (ats_down_k_slices), on the direct-to-LDS tile (up to 256 rows x 256 columns, one per CU) or, where that tile would
-    leave half of the CUs idle or up to 64 rows stream faster through them, on the small tiles.  Measured with the combine behind
-    it, weights from HBM, rows per expert 22 | 48 | 64 | 96 | 128 | 192 | 224, plain -> the rule's, microseconds:
-      8 x [4096, 14336]  181 -> 176 | 192 -> 174 | 283 -> 180 | 274 -> 189 | 282 -> 198 | 275 -> 218 | 318 -> 234
-      4 x [4096, 14336]   94 -> 97  | 103 -> 100 | 144 -> 105 | 224 -> 109 | 202 -> 114 | 242 -> 129 | 284 -> 134
-      2 x [4096, 14336]   61 -> 57  |  70 -> 60  | 100 -> 60  | 111 -> 62  | 100 -> 66  | 181 -> 78  | 243 -> 86
-      16 x [2048, 8192]   105       | 113        | 157 -> 141 | 167 -> 147 | 170 -> 159 | 166 -> 167 | 198 -> 172
-      4 x [1024, 8192]    33 -> 31  |  34 -> 29  |  36 -> 35  |  37 -> 36  |  44 -> 37  |  61 -> 42  | 134 -> 45
-      2 x [1024, 16384]   56 -> 37  |  59 -> 34  |  59 -> 38  |  58 -> 44  |  62 -> 41  |  61 -> 46  | 250 -> 49
-      8 x [1024, 4096]    24        |  26        |  31        |  30        |  41 -> 35  |  41 -> 42  |  82 -> 45
-    Shorter sums take the slices that fit one round of 256 large tiles, unless 64-row tiles do it in a round (or in two up to 112
-    rows: 8 x [2048, 2048], 96 rows 28 against 31, 128 rows 40 -> 33).  Below 32 MB of weights everything comes from the
-    last-level cache and the general rule stands."""
+    bfloat16 experts of more than 20 rows against 32 MB of weights or more: those slices or the plain launch, or slices on the
+    direct-to-LDS tile (up to 256 rows x 256 columns, one per CU), whichever is estimated to take the least time
+    (ats_down_k_slices).  Measured with the combine behind it, weights from HBM, rows per expert 22 | 32 | 48 | 64 | 96 | 128 | 192 |
+    224, without that tile and the estimate -> with them, microseconds:
+      8 x [4096, 14336]  164 -> 173 | 197 -> 175 | 194 -> 177 | 261 -> 181 | 265 -> 185 | 269 -> 192 | 253 -> 216 | 324 -> 224
+      4 x [4096, 14336]   91        | 111 ->  92 | 100 ->  94 | 143 ->  98 | 213 -> 103 | 187 -> 108 | 245 -> 125 | 308 -> 135
+      2 x [4096, 14336]   51        |  54        |  55        |  56        |  87 ->  58 |  88 ->  59 | 135 ->  83 | 239 ->  74
+      16 x [2048, 8192]  136 ->  98 | 132 -> 107 | 116        | 153 -> 142 | 167 -> 147 | 158 -> 152 | 167        | 198 -> 173
+      16 x [2048, 5632]   79 ->  73 |  88 ->  75 |  79        | 112 ->  81 | 111 ->  88 | 142 ->  93 | 111 -> 106 | 139 -> 164
+      4 x [1024, 8192]    33        |  36 ->  33 |  29        |  33 ->  35 |  38 ->  36 |  41 ->  37 |  54 ->  47 |  61 ->  49
+      2 x [1024, 16384]   34        |  35        |  32        |  33        |  39        |  42 ->  46 |  46 ->  51 |  60 ->  55
+      8 x [1024, 4096]    26        |  32 ->  26 |  26        |  32 ->  30 |  36 ->  30 |  38 ->  40 |  47 ->  41 |  83 ->  50
+      64 x [2048, 1408] stays as it was, plain
+    5599 random points, K from 1024 to 16384: 10 % less time on average (K from 4096: 14 %), 4 % of them more than 4 % slower.
+    Below 32 MB of weights everything comes from the last-level cache and the first rule stands."""
     slab = 64 if dtype == torch.bfloat16 else 32
     if E <= 0 or max_rows <= 0:
         return 1
@@ -611,29 +612,17 @@ def down_k_splits(E: int, max_rows: int, N: int, K: int, dtype: torch.dtype) -> 
         return 1
     if E > 1 and max_rows // E <= 20:
         return 1        # the plain launch streams the weights itself (8 x [4096, 14336], 16 rows each: 157 against 159 us)
-    if E > 1 and dtype == torch.bfloat16 and E * N * K >= 1 << 24:
-        if K >= 4096:
-            return int(_lib.load().ats_down_k_slices(int(E), int(max_rows), int(N), int(K)))
-        n256, n64 = -(-N // 256), -(-N // 64)
-        tiles = E * n256 * (3 if rows > 232 else 2) // 2
-        s = 1
-        while s < 16 and 2 * s * tiles <= 256 and K % (2 * s * slab) == 0 and K // (2 * s) >= 512:
-            s *= 2
-        if rows < 64:
-            return s if K / (slab * s) * 1.3 + 18.0 < 0.97 * E * N * K * 2 / 5e6 else 1
-        # (groups vary around their mean)
-        tiles64 = E * -(-(rows + rows // 7) // 64) * n64
-        return 1 if rows <= 192 and tiles64 <= 256 or rows <= 112 and tiles64 <= 512 else s
     n128 = (N + 127) // 128
     plain = E * n128 if max_rows // E <= 32 else E * ((rows + 127) // 128) * ((N + 255) // 256)
-    if plain >= 384:
-        return 1
-    # 32-row tiles (three workgroups per CU) up to 32 rows, 64-row tiles (two per CU) above
-    groups = E * (1 if rows <= 32 else (rows + 63) // 64) * n128
-    enough = 384 if rows <= 32 else 256
     s = 1
-    while s < 16 and groups * s < enough and K % (2 * s * slab) == 0 and K // (2 * s) >= 512:
-        s *= 2
+    if plain < 384:
+        # 32-row tiles (three workgroups per CU) up to 32 rows, 64-row tiles (two per CU) above
+        groups = E * (1 if rows <= 32 else (rows + 63) // 64) * n128
+        enough = 384 if rows <= 32 else 256
+        while s < 16 and groups * s < enough and K % (2 * s * slab) == 0 and K // (2 * s) >= 512:
+            s *= 2
+    if E > 1 and dtype == torch.bfloat16 and E * N * K >= 1 << 24:
+        return int(_lib.load().ats_down_k_slices(int(E), int(max_rows), int(N), int(K), s))
     return s
 
 

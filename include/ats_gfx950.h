@@ -250,9 +250,10 @@ int ats_grouped_gateup_swiglu_save(const void* a, int64_t a_num_rows, const int3
 int ats_grouped_down_splitk(const void* h, const void* const* w_d, float* parts, const int32_t* row_start,
                             const int32_t* row_count, int E, int64_t max_rows, int64_t part_rows, int H,
                             int I, int k_splits, int dtype, ats_stream_t stream);
-/* The number of slices with which a bfloat16 down projection of more than one expert with 21 .. 256 rows on average and I >= 4096
- * is estimated to take the least time, ats_combine_partials included; 1: ats_grouped_down. */
-int ats_down_k_slices(int E, int64_t max_rows, int H, int I);
+/* The number of slices with which a bfloat16 down projection of more than one expert with 21 .. 256 rows on average and 32 MB of
+ * weights or more is estimated to take the least time, ats_combine_partials included; 1: ats_grouped_down.  small: the slices with
+ * which 32 or 64-row tiles fill the chip. */
+int ats_down_k_slices(int E, int64_t max_rows, int H, int I, int small);
 /* out[i] = sum_s parts[s*part_stride + i], i < n, added in slice order in float32 and rounded once
  * to out_dtype (n and part_stride multiples of 4). */
 int ats_sum_partials(const float* parts, int n_parts, int64_t part_stride, void* out, int64_t n,

@@ -30,15 +30,17 @@ def test_sliced_down_projection(gpu, counts, H, I, S):
         assert (parts[s].double() - ref).abs().max() <= bound
 
 
-# slices of 512 columns and more, where an estimate chooses between that tile and the small ones: a few rows against few columns
-# (small), 32-row tiles, more rows (large), too few large tiles (small)
+# slices of 512 columns and more, where an estimate chooses between that tile and the small ones: a few rows (small, 32-row tiles,
+# small), more rows of few (large) and of more groups (large)
 @pytest.mark.parametrize("counts,H,I,S", [([40, 56], 1000, 16384, 16), ([21, 24, 0, 33], 1032, 8192, 8), ([100, 156], 1000, 16384, 16),
-                                          ([90, 0, 129, 64, 33, 1, 128, 200], 1032, 4096, 8), ([70, 65], 1000, 16384, 8)])
+                                          ([90, 0, 129, 64, 33, 1, 128, 200], 1032, 4096, 8), ([70, 65], 1000, 16384, 8),
+                                          ([230, 100, 140, 170], 1032, 8192, 8)])
 def test_sliced_down_projection_on_the_estimated_tile(gpu, counts, H, I, S):
     test_sliced_down_projection(gpu, counts, H, I, S)
 
 
-@pytest.mark.parametrize("T", [176, 700])
+# 44, 175 and 224 rows per expert; up to 192 the plain launch is the faster one (192 rows 25 us, in four slices 35; 224 rows 48 and 38)
+@pytest.mark.parametrize("T", [176, 700, 896])
 def test_layer_with_sliced_down_projection(gpu, T):
     """The layer whose rule chooses these slices against the stages in float64."""
     print("case layer sliced", T, flush=True)
@@ -49,7 +51,7 @@ def test_layer_with_sliced_down_projection(gpu, T):
     w = W.make_moe_workload("c1_cpu_reference", device="cpu", overrides=ov)
     wg = W.make_moe_workload("c1_cpu_reference", device=gpu, overrides=ov)
     layer = W.build_layer(wg, "none")
-    assert ops.down_k_splits(8, 2 * T, 1024, 2048, torch.bfloat16) == (1 if T == 176 else 4)
+    assert ops.down_k_splits(8, 2 * T, 1024, 2048, torch.bfloat16) == (4 if T == 896 else 1)
     with torch.no_grad():
         out, _ = layer(wg.x)
     ref = O.moe_forward_nocap(w.x.float(), w.gate.float(), [t.float() for t in w.gate_up], [t.float() for t in w.down], k=2,

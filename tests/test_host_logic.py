@@ -269,10 +269,11 @@ def test_slices_of_a_weight_gradient(rows, M, N, slices):
     assert ops.wgrad_slices(M, N, rows) == slices
 
 
-@pytest.mark.parametrize("E,rows,N,K,slices", [(2, 22, 1024, 16384, 16), (2, 48, 1024, 16384, 16), (2, 128, 1024, 16384, 16), (4, 48, 1024, 8192, 8),
-                                               (4, 192, 1024, 8192, 8), (2, 64, 4096, 14336, 8), (2, 192, 4096, 14336, 8), (8, 22, 4096, 14336, 2),
+@pytest.mark.parametrize("E,rows,N,K,slices", [(2, 22, 1024, 16384, 16), (2, 48, 1024, 16384, 16), (4, 48, 1024, 8192, 8),
+                                               (2, 64, 4096, 14336, 8), (2, 192, 4096, 14336, 8), (4, 96, 4096, 14336, 4), (8, 22, 4096, 14336, 2),
                                                (8, 96, 4096, 14336, 2), (16, 22, 2048, 8192, 1), (16, 48, 2048, 8192, 1), (16, 96, 2048, 8192, 2),
-                                               (8, 48, 1024, 4096, 1), (8, 128, 1024, 4096, 8), (8, 96, 2048, 2048, 1), (8, 128, 2048, 2048, 4)])
+                                               (16, 48, 2048, 5632, 2), (16, 128, 2048, 5632, 2), (8, 48, 1024, 4096, 4), (8, 96, 1024, 4096, 1),
+                                               (8, 96, 2048, 2048, 1), (8, 128, 2048, 2048, 4), (8, 192, 1024, 2048, 1), (64, 128, 2048, 1408, 1)])
 def test_slices_of_a_down_projection(E, rows, N, K, slices):
     """The choice at measured sizes: the fastest, or within 10 % of it."""
     from adaptivetrainingsystem_amd import ops
