@@ -1678,10 +1678,10 @@ struct TileCost {
     float per_slab, per_tile;
     int min_tiles;
 };
-// spread: groups vary around their mean, so those of a mean just below a multiple of the tile height need one tile more (64
-// experts of 108 rows on average, 81-140: gate/up 182 us in 128-row tiles, 161 in 256-row ones; of 94 rows 167 both).
-static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs, bool spread = false) {
-    const int64_t rows = spread && E > 1 ? max_rows + max_rows / 5 : max_rows;
+// spread: groups vary around their mean, so those of a mean just below a multiple of the tile height need one tile more; counted as
+// rows / spread more of them.
+static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs, int spread = 0) {
+    const int64_t rows = spread && E > 1 ? max_rows + max_rows / spread : max_rows;
     const int64_t avg = (rows + E - 1) / E;
     const int64_t tiles = (int64_t)E * ((avg + c.rows - 1) / c.rows) * ((n_cols + c.cols - 1) / c.cols);
     const int64_t per_cu = (tiles + 255) / 256;
@@ -1714,10 +1714,15 @@ static GroupTile pick_group_tile(int64_t max_rows, int E, int N, int nk) {
                                         : TileCost{64, SWIGLU ? 32 : 64, 0.58f, 3.f, 1};
     constexpr TileCost kMid = kBf16 ? TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 0.58f : 1.05f, 5.f, 1}
                                     : TileCost{128, SWIGLU ? 64 : 256, SWIGLU ? 2.0f : 3.65f, 5.f, 1};
-    const float mid = tile_time(kMid, max_rows, E, N, nk, true);
+    // A fifth where many groups make it likely that one of them is that much larger (64 experts of 108 rows on average, 81-140: gate/up
+    // 182 us in 128-row tiles, 161 in 256-row ones; of 94 rows 167 both), a tenth for a few (4 experts of 110 rows, [16384, 2048]: 67.5
+    // us, with a fifth 74) and in float32, whose tiles of 128 rows lose less than the taller ones (2 x 226 rows, [8192, 1024]: 66 us, with a
+    // fifth 88; 32 x 225 rows, [1536, 1024]: 188, 241; 4 x 331 rows, [16384, 2048]: 734, 944).
+    const int spread = kBf16 && E >= 8 ? 5 : 10;
+    const float mid = tile_time(kMid, max_rows, E, N, nk, spread);
     // (the 16 x 16 x 32 kernel computes only the 16-row fragments that a tile has; up to 192 rows its loads bound a slab)
     const float big = tile_time(TileCost{256, SWIGLU ? 128 : 256, kBf16 ? (avg <= 192 ? 1.3f : 1.45f) : 7.3f, 7.f, 1},
-                                max_rows, E, N, nk, true);
+                                max_rows, E, N, nk, spread);
     const float least_large = mid < big ? mid : big;
     // (two full rounds of 256-row tiles: nothing is idle, and groups of unequal size fit them better; 8 experts with 20-45
     // rows each, gate/up [28672, 4096]: 343 us against 372 in 32-row tiles)
