@@ -2001,6 +2001,19 @@ static int launch_kmajor(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
     return ATS_OK;
 }
 
+// Supertiles that the busiest XCD takes, one after another: the time of a tile for each, however few tiles they hold, since tiles
+// at the same place of a supertile run on the same CU (32 rows x 4096 columns are 16 supertiles of 8 x 4 tiles with one row of
+// tiles each: twice the time of 2048 columns).
+static int64_t xcd_rounds(int64_t m_tiles, int n_tiles) {
+    int sm, sn;
+    pick_supertile(n_tiles, &sm, &sn);
+    return ((m_tiles + sm - 1) / sm * ((n_tiles + sn - 1) / sn) + kNumXcd - 1) / kNumXcd;
+}
+static float rounds_time(const TileCost& c, int64_t max_rows, int E, int n_cols, int k_slabs) {
+    const int64_t avg = (max_rows + E - 1) / E;
+    return xcd_rounds(E * ((avg + c.rows - 1) / c.rows), (n_cols + c.cols - 1) / c.cols) * (k_slabs * c.per_slab + c.per_tile);
+}
+
 // Float32 products against K-major operands on the small tiles, in microseconds, and what a transposing pass costs.  The
 // tiles' constants are those of launch_grouped, a tenth more per slab for the 4-byte fragment reads (and less per tile for
 // short sums, of which several share a CU).  Copies and their product -> operands as they lie:
@@ -2412,7 +2425,18 @@ extern "C" int ats_grouped_gemm_nn_sliced(const void* a, int64_t lda, const void
 extern "C" int ats_grouped_gemm_nn_f32_supported(int E, int64_t max_rows, int N, int K) {
     using namespace ats;
     if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || N % 4 != 0 || K % 4 != 0) return 0;
-    return small_kmajor_time(max_rows, E, N, K) <= transposed_time(max_rows, E, N, K, (int64_t)E * N * K, 1) ? 1 : 0;
+    // The weights as they lie against their copies (4.6 TB/s, a launch and its host work: 11 us) and the product of these, for a few
+    // rows the stream of weights.  3992 points, 1 .. 64 groups: half the time of the copies, 50 of them more than 4 % slower.  1 x 13 rows x [1408, 8192]: as they lie 90 us, copies 47; 5 rows x [1408, 6144] 69, 37; 8
+    // rows x [2560, 8192] 92, 61; 8 rows x [2048, 2048] 16, 28.
+    const int nk = (K + 31) / 32;
+    const float t32 = rounds_time(TileCost{32, 32, 0.20f, 3.f, 1}, max_rows, E, N, nk);
+    const float t64 = rounds_time(TileCost{64, 64, 0.64f, 2.5f, 1}, max_rows, E, N, nk);
+    float copied = rounds_time(TileCost{256, 256, 7.3f, 25.f, 1}, max_rows, E, N, nk);
+    for (const TileCost& c : {TileCost{128, 256, 3.65f, 5.f, 1}, TileCost{64, 64, 0.58f, 3.f, 1}, TileCost{32, 32, 0.18f, 1.5f, 1}})
+        copied = fminf(copied, rounds_time(c, max_rows, E, N, nk));
+    const float weights = (float)E * N * K * 4e-6f;
+    if (max_rows / E <= (E == 1 ? 32 : 20)) copied = fminf(copied, 3.f + fmaxf(K * 0.0024f, weights / 4.5f));
+    return 0.95f * fminf(t32, t64) <= copied + weights * 2.f / 4.6f + 11.f ? 1 : 0;
 }
 extern "C" int ats_grouped_gemm_nn_f32(const float* a, int64_t lda, const void* const* b_ptrs, int64_t ldb, float* out, int64_t ldo,
                                        const int32_t* row_start, const int32_t* row_count, int E, int64_t max_rows, int N, int K,

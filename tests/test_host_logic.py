@@ -280,6 +280,16 @@ def test_slices_of_a_down_projection(E, rows, N, K, slices):
     assert ops.down_k_splits(E, E * rows, N, K, torch.bfloat16) == slices
 
 
+# a few rows against a long K: the stream of a copy's weights is the faster one; short sums, more rows and groups of them: not
+@pytest.mark.parametrize("E,rows,N,K,direct", [(1, 13, 1408, 8192, False), (1, 5, 1408, 6144, False), (1, 8, 256, 8192, False), (1, 4, 2560, 8192, False),
+                                               (2, 11, 1408, 8192, False), (1, 8, 2048, 2048, True), (1, 13, 1408, 256, True), (1, 512, 512, 1024, True),
+                                               (8, 1024, 512, 2816, True), (8, 2000, 1408, 512, True), (1, 4096, 4096, 4096, False)])
+def test_float32_data_gradient_reads_weights_as_they_lie(E, rows, N, K, direct):
+    """The choice at measured sizes: the faster way."""
+    from adaptivetrainingsystem_amd import ops
+    assert ops.grouped_gemm_nn_f32_supported(E, rows, N, K) == direct
+
+
 # bfloat16, a smaller head_dim, fewer values than keys, fewer keys than queries, heads that do not divide, 3-D, more pairs than served
 @pytest.mark.parametrize("q,k,v,dtype", [((1, 4, 8, 64), (1, 2, 8, 64), (1, 2, 8, 64), torch.bfloat16), ((1, 4, 8, 64), (1, 2, 8, 32), (1, 2, 8, 32), None),
                                          ((1, 4, 8, 64), (1, 2, 8, 64), (1, 2, 7, 64), None), ((1, 4, 8, 64), (1, 2, 7, 64), (1, 2, 7, 64), None),
