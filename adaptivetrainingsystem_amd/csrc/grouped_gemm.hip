@@ -2739,14 +2739,12 @@ extern "C" int ats_linear_nt(const void* x, const void* const* w, void* out, con
     if (dtype == ATS_F32 && T > 256 && T <= 0x7fffffff && N > 0 && K > 0 && N % 4 == 0 && K % 4 == 0 && x && w && out && row_start &&
         row_count && aligned16(x) && aligned16(out)) {
         const int nk = (K + 31) / 32;
-        const int64_t tiles = ((T + 63) / 64) * ((N + 63) / 64);
-        const float t64 = (float)(tiles <= 256 ? 1 : (tiles + 511) / 512 * 2) * (nk * 0.58f + 3.f);
-        const float t32 = tile_time(TileCost{32, 32, 0.18f, 1.5f, 1}, T, 1, N, nk);
-        float others = tile_time(TileCost{64, 64, 0.74f, 3.f, 1}, T, 1, N, nk);
-        for (const TileCost& c : {TileCost{128, 256, 3.65f, 5.f, 1}, TileCost{256, 256, 7.3f, 7.f, 1}}) {
-            const float t = tile_time(c, T, 1, N, nk);
-            if (t < others) others = t;
-        }
+        const int64_t rounds = xcd_rounds((T + 63) / 64, (N + 63) / 64);
+        const float t64 = (float)(rounds <= 1 ? 1 : (rounds + 1) / 2 * 2) * (nk * 0.58f + 3.f);
+        const float t32 = rounds_time(TileCost{32, 32, 0.18f, 1.5f, 1}, T, 1, N, nk);
+        float others = rounds_time(TileCost{64, 64, 0.74f, 3.f, 1}, T, 1, N, nk);
+        for (const TileCost& c : {TileCost{128, 256, 3.65f, 5.f, 1}, TileCost{256, 256, 7.3f, 7.f, 1}})
+            others = fminf(others, rounds_time(c, T, 1, N, nk));
         if (t32 < others || t64 < others) {
             GroupedArgs p{};
             p.a = x;

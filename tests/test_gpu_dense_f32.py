@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,N,K", [(256, 512, 512), (257, 512, 512), (300, 36, 68), (511, 1024, 516), (700, 1000, 1000), (1500, 2048, 2048),
-                                   (2001, 512, 1408), (4100, 516, 512), (257, 4, 8)])
+                                   (2001, 512, 1408), (4100, 516, 512), (257, 4, 8), (276, 6144, 512), (390, 11008, 256)])
 def test_linear(gpu, T, N, K):
     print("case dense f32", T, N, K, flush=True)
     from adaptivetrainingsystem_amd import ops
