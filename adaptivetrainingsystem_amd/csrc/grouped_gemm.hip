@@ -1545,10 +1545,25 @@ constexpr size_t dma_lds_bytes(int BM, int BN) { return (size_t)(3 * BM + 2 * BN
 // Rows per group on average below which the 16 x 16 x 32 kernel runs in its MIDROWS form (measured there).
 constexpr int64_t kMidRowsMaxAvg = 768;
 static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1) < kMidRowsMaxAvg; }
+// Tiles of the busiest CU.  Supertile S runs on XCD S % 8; the last band of rows and the last one of columns hold fewer than 32 tiles
+// (18 x 43 tiles of 256 rows: 33 supertiles, five for XCD 0, of which one has eight tiles and the others leave it four rounds).
+static int64_t busiest_cu(int64_t m_tiles, int n_tiles, int sm, int sn) {
+    const int64_t bands = (m_tiles + sm - 1) / sm, super = bands * ((n_tiles + sn - 1) / sn);
+    if (super > 256) return (super + kNumXcd - 1) / kNumXcd;
+    int64_t tiles[kNumXcd] = {}, most = 0;
+    for (int64_t i = 0; i < super; ++i) {
+        const int64_t rows = m_tiles - i % bands * sm, cols = n_tiles - i / bands * sn;
+        tiles[i % kNumXcd] += (rows < sm ? rows : sm) * (cols < sn ? cols : sn);
+    }
+    for (int64_t t : tiles) most = t > most ? t : most;
+    return (most + kSuperBlocks - 1) / kSuperBlocks;
+}
+
 // Tile height of a bfloat16 launch with one group (its row count is exact), 0 for the full 256 rows.  An XCD takes whole
 // supertiles of 32 tiles and its 32 CUs hold one tile each, so a launch lasts as many rounds as there are supertiles per XCD,
-// and lower tiles pay where they turn a round that is mostly empty into work for all CUs.  Microseconds per 64-element slab
-// by height as measured (a round of K = 4096: 256 rows 94, 224: 84, 192: 76, 160: 60, 128: 54; odd multiples of 16 between).
+// and lower tiles pay where they turn a round that is mostly empty into work for all CUs (4524 x [11008, 2048]: 240 rows in four
+// rounds 185 us, 144 rows, thought to take six as 256 rows five, 215).  Microseconds per 64-element slab by height: medians over 415
+// launches.
 // Rows x [N, K], 256-row tiles -> heights in steps of 32 -> in steps of 16: 5331 x [4096, 4096] 188 -> 143 -> 134 us, x
 // [6144, 4096] 248 -> 207 -> 200, 4200 x [4096, 4096] 123 -> 116, 10000 x [6144, 4096] 369 -> 346, 5331 x [3072, 2048] 67 -> 62,
 // 3000 x [4096, 4096] 95 -> 76 -> 74, 1500 x [4096, 4096] 78 -> 58 -> 56, 1000 x [6144, 4096] 93 -> 57 -> 56; 2048 x [6144, 4096]
@@ -1557,13 +1572,12 @@ static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1
 static int dense_tile_rows(int64_t rows, int n_tiles, int k_slabs, int sm, int sn) {
     float best = 0.f;
     int best_rows = 0;
-    constexpr float kPerSlab[] = {0.75f, 0.80f, 0.86f, 0.97f, 1.08f, 1.14f, 1.20f, 1.28f, 1.36f};     // 128, 144, .. 256 rows
+    constexpr float kPerSlab[] = {0.75f, 0.86f, 0.94f, 1.00f, 1.07f, 1.15f, 1.23f, 1.28f, 1.35f};     // 128, 144, .. 256 rows
     for (int h = 256; h >= 128; h -= 16) {
         const int64_t m_tiles = (rows + h - 1) / h;
         const int64_t height = ((rows + m_tiles - 1) / m_tiles + 15) / 16 * 16;     // tiles of a group have one height
         const float per_slab = kPerSlab[height > 128 ? (height - 128) / 16 : 0];
-        const int64_t rounds = ((m_tiles + sm - 1) / sm * ((n_tiles + sn - 1) / sn) + kNumXcd - 1) / kNumXcd;
-        const float t = (float)rounds * (k_slabs * per_slab + 7.f);
+        const float t = (float)busiest_cu(m_tiles, n_tiles, sm, sn) * (k_slabs * per_slab + 7.f);
         if (h == 256 || t < 0.97f * best) {
             best = t;
             best_rows = h == 256 ? 0 : h;
