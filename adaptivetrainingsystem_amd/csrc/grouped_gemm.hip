@@ -1562,7 +1562,7 @@ static int64_t busiest_cu(int64_t m_tiles, int n_tiles, int sm, int sn) {
 // Tile height of a bfloat16 launch with one group (its row count is exact), 0 for the full 256 rows.  An XCD takes whole
 // supertiles of 32 tiles and its 32 CUs hold one tile each, so a launch lasts as many rounds as there are supertiles per XCD,
 // and lower tiles pay where they turn a round that is mostly empty into work for all CUs (4524 x [11008, 2048]: 240 rows in four
-// rounds 185 us, 144 rows, thought to take six as 256 rows five, 215).  Microseconds per 64-element slab by height: medians over 415
+// rounds 174 us, 144 rows in six 215).  Microseconds per 64-element slab by height: medians over 415
 // launches.
 // Rows x [N, K], 256-row tiles -> heights in steps of 32 -> in steps of 16: 5331 x [4096, 4096] 188 -> 143 -> 134 us, x
 // [6144, 4096] 248 -> 207 -> 200, 4200 x [4096, 4096] 123 -> 116, 10000 x [6144, 4096] 369 -> 346, 5331 x [3072, 2048] 67 -> 62,
@@ -2745,7 +2745,8 @@ extern "C" int ats_grouped_gemm_nt(const void* a, const void* const* a_ptrs, int
 // any number of rows (up to 256 launch_grouped does so itself).  Two of the 64-row workgroups share a CU: an odd third costs as
 // much as a fourth.  [N, K] x rows, all of K in a wave -> slices, microseconds (half the error: four chains instead of one):
 //   [1024, 512] x 512 18 -> 10, x 1000 18 -> 15, x 2000 28 -> 27; [512, 1408] x 512 40 -> 13, x 2000 40 -> 33;
-//   [2048, 2048] x 257 58 -> 42, x 700 91 -> 76, x 1500 140 (147), x 2000 193 -> 160; x 4096 240 in 256-row tiles
+//   [2048, 2048] x 257 58 -> 42, x 700 91 -> 76, x 1500 140 (147), x 2000 193 -> 160; x 4096 240 in 256-row tiles;
+//   [6144, 512] x 276, three rounds of 64-row tiles on the XCDs with full bands: 41 -> 29 in 32-row ones (64-row slices 47)
 extern "C" int ats_linear_nt(const void* x, const void* const* w, void* out, const int32_t* row_start, const int32_t* row_count,
                              int64_t T, int N, int K, int dtype, ats_stream_t stream) {
     using namespace ats;
