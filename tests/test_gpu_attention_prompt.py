@@ -26,6 +26,19 @@ def test_prompt_attention(gpu, B, L, Hq, Hkv, D, keep_values):
     assert ops.prompt_attention(qkv.float(), cos, sin, B, Hkv, D, 0.1, keep_values) is None
 
 
+# on both sides of the size from which a prompt without a cache has its queries rotated in the attention too (6 M of them)
+@pytest.mark.parametrize("B,L", [(2, 241), (1, 6143), (1, 6144), (3, 2049)])
+def test_prompt_without_a_cache(gpu, B, L):
+    print("case prompt without cache", B, L, flush=True)
+    from adaptivetrainingsystem_amd import GroupedQueryAttention
+    from adaptivetrainingsystem_amd.workloads import LayerConfig
+    torch.manual_seed(L)
+    att = GroupedQueryAttention(LayerConfig(1024, 4096, 1, 1, num_heads=8, num_kv_heads=2, seq_length=8192)).to(gpu, torch.bfloat16).eval()
+    x = torch.randn(B, L, 1024, generator=torch.Generator().manual_seed(L)).to(gpu, torch.bfloat16)
+    with torch.no_grad():
+        assert torch.equal(att(x), att(x, use_cache=True)[0])
+
+
 def test_prompt_attention_refusals(gpu):
     from adaptivetrainingsystem_amd import _lib
     lib = _lib.load()
