@@ -24,10 +24,12 @@
 // kernel of its own, attention_decode.hpp.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "ats_common.hpp"
 #include "attention_extra.hpp"
+#include "attention_parts.hpp"
 
 namespace ats {
 
@@ -827,9 +829,9 @@ __device__ __forceinline__ void attention_q_tile_pipe(const bf16_t* __restrict__
     }
 }
 
-// Each workgroup takes a long query tile and its mirror-image short one, so every workgroup of a launch
-// does the same work: the hardware hands workgroups to XCDs and shader engines strictly in turn and waits
-// for the next target to have room, so workgroups of uneven length leave whole shader engines idle.
+// Every workgroup of a launch does about the same work: the hardware hands workgroups to XCDs and shader engines strictly
+// in turn and waits for the next target to have room, so workgroups of uneven length leave whole shader engines
+// idle.  A workgroup takes a long query tile and its mirror-image short one, or the tiles that AttnParts gives it.
 // Consecutive ids go to different XCDs; the blocks of one (batch, kv head) are kept on one XCD so that
 // its K and V stay in that XCD's L2.  Two waves per SIMD (register budget 256): one wave's softmax runs
 // in the shadow of the other's MFMAs.
@@ -839,13 +841,13 @@ __global__ __launch_bounds__(NT, 512 / NT) void attention_fwd_kernel(const bf16_
                                                             const bf16_t* __restrict__ v, int64_t v_sb, int v_sl, int64_t v_sh,
                                                             const float* __restrict__ key_bias, bf16_t* __restrict__ out,
                                                             float* __restrict__ lse, int Hq, int Hkv, int L, int Lk,
-                                                            float scale_log2, int B, int pack, RopeQ rope) {
+                                                            float scale_log2, int B, int pack, RopeQ rope, AttnParts parts) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kAttBM = att_rows_per_block(NT);
     const int heads_per_group = pack ? 1 : Hq / Hkv;     // packed: the group's heads share the rows of a tile
     const int n_qt = (L * (pack ? Hq / Hkv : 1) + kAttBM - 1) / kAttBM;
-    const int n_pairs = (n_qt + 1) / 2;
-    const int per_group = n_pairs * heads_per_group;     // workgroups sharing one K/V
+    const int n_parts = parts.count ? parts.count : (n_qt + 1) / 2;
+    const int per_group = n_parts * heads_per_group;     // workgroups sharing one K/V
     const int n_groups = B * Hkv;
     int group, within;
     if (n_groups % 8 == 0) {
@@ -857,14 +859,22 @@ __global__ __launch_bounds__(NT, 512 / NT) void attention_fwd_kernel(const bf16_
         within = blockIdx.x % per_group;
     }
     const int b = group / Hkv;
-    const int head = pack ? group % Hkv : (group % Hkv) * heads_per_group + within / n_pairs;
-    const int pair = within % n_pairs;
-    const int qt_long = n_qt - 1 - pair;
+    const int head = pack ? group % Hkv : (group % Hkv) * heads_per_group + within / n_parts;
+    const int part = within % n_parts;
+    uint32_t todo = parts.count ? parts.tiles[part] : 0;
+    int qt = parts.count ? 31 - __clz(todo) : n_qt - 1 - part;
 #pragma unroll 1
-    for (int half = 0; half < 2; ++half) {
-        if (half && pair == qt_long) break;   // an odd tile count leaves the middle tile on its own
+    while (true) {
         attention_q_tile_pipe<D, BIAS, NT, ROPE>(q, k, k_sb, k_sh, v, v_sb, v_sl, v_sh, key_bias, out, lse, Hq, Hkv, L, Lk,
-                                                 scale_log2, half ? pair : qt_long, head, b, pack != 0, rope, smem);
+                                                 scale_log2, qt, head, b, pack != 0, rope, smem);
+        if (parts.count) {
+            todo &= ~(1u << qt);
+            if (!todo) break;
+            qt = 31 - __clz(todo);
+        } else {
+            if (qt == part) break;      // the short tile, or the middle one of an odd number
+            qt = part;
+        }
     }
 }
 
@@ -1060,8 +1070,14 @@ static int launch_attention_fwd(const char* name, const void* q, const void* k, 
     const int nt = L >= 4096 ? 512 : 256;
     const int kAttBM = att_rows_per_block(nt);
     const int pack = (L < kAttBM && Hq > Hkv) ? 1 : 0;
-    const int64_t n_blocks = pack ? (int64_t)((((int64_t)L * (Hq / Hkv) + kAttBM - 1) / kAttBM + 1) / 2) * Hkv * B
-                                  : (int64_t)(((L + kAttBM - 1) / kAttBM + 1) / 2) * Hq * B;
+    const int rp = pack ? Hq / Hkv : 1;
+    const int64_t n_rows = (int64_t)L * rp, n_qt = (n_rows + kAttBM - 1) / kAttBM;
+    const int64_t heads = (int64_t)B * (pack ? Hkv : Hq);
+    const bool by_xcd = (int64_t)B * Hkv % 8 == 0;
+    const AttnParts parts = attn_parts((int)n_qt, by_xcd ? heads / 8 : heads, by_xcd ? 32 : 256, nt == 256, [&](int t) {
+        return (int)((std::min((int64_t)(t + 1) * kAttBM, n_rows) - 1) / rp + Lk - L) / kAttBN + 1;
+    });
+    const int64_t n_blocks = (parts.count ? parts.count : (n_qt + 1) / 2) * heads;
     ATS_REQUIRE(n_blocks <= 0x7fffffff, ATS_ERR_UNSUPPORTED, "%s: %lld workgroups", name, (long long)n_blocks);
     const dim3 grid((unsigned)n_blocks);
     static LdsReservation reserved_lds[12];      // one per kernel instance
@@ -1074,7 +1090,7 @@ static int launch_attention_fwd(const char* name, const void* q, const void* k, 
         hipLaunchKernelGGL(kernel, grid, dim3(nt), smem, s, static_cast<const bf16_t*>(q),
                            static_cast<const bf16_t*>(k), k_sb, k_sh, static_cast<const bf16_t*>(v), v_sb, (int)v_sl, v_sh,
                            key_bias,
-                           static_cast<bf16_t*>(out), lse, Hq, Hkv, L, Lk, scale_log2, B, pack, rope ? *rope : RopeQ{});
+                           static_cast<bf16_t*>(out), lse, Hq, Hkv, L, Lk, scale_log2, B, pack, rope ? *rope : RopeQ{}, parts);
         return ATS_OK;
     };
     // K tile, V tile (two stages each, rows unpadded) and, with a bias, two stages of one float per key

@@ -19,10 +19,12 @@
 // its 16-byte chunks swizzled so that both access patterns stay free of bank conflicts (SwzTile below).
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "ats_common.hpp"
 #include "attention_extra.hpp"
+#include "attention_parts.hpp"
 
 namespace ats {
 
@@ -387,18 +389,18 @@ __device__ __forceinline__ void attention_bwd_dq_tile(const bf16_t* __restrict__
     }
 }
 
-// A workgroup takes a long query tile and its mirror-image short one (equal work per workgroup: the
-// hardware hands workgroups out strictly in turn), and the workgroups of one (batch, kv head) share an XCD.
+// A workgroup takes a long query tile and its mirror-image short one, or the tiles that AttnParts gives it (equal work per
+// workgroup: the hardware hands workgroups out strictly in turn), and the workgroups of one (batch, kv head) share an XCD.
 template <int D, bool BIAS, bool EXTRA = false>
 __global__ __launch_bounds__(256, 2) void attention_bwd_dq_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     const bf16_t* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta,
     const float* __restrict__ key_bias, bf16_t* __restrict__ dq, int Hq, int Hkv, int L, int Lk, float scale, int B,
-    AttnExtra ex, const bf16_t* __restrict__ out_rows, float* __restrict__ delta_w) {
+    AttnExtra ex, const bf16_t* __restrict__ out_rows, float* __restrict__ delta_w, AttnParts parts) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int n_qt = (L + kBwdRows - 1) / kBwdRows;
-    const int n_pairs = (n_qt + 1) / 2;
-    const int per_group = n_pairs * (Hq / Hkv);
+    const int n_parts = parts.count ? parts.count : (n_qt + 1) / 2;
+    const int per_group = n_parts * (Hq / Hkv);
     const int n_groups = B * Hkv;
     int group, within;
     if (n_groups % 8 == 0) {
@@ -410,14 +412,22 @@ __global__ __launch_bounds__(256, 2) void attention_bwd_dq_kernel(
         within = blockIdx.x % per_group;
     }
     const int b = group / Hkv;
-    const int hq = (group % Hkv) * (Hq / Hkv) + within / n_pairs;
-    const int pair = within % n_pairs;
-    const int qt_long = n_qt - 1 - pair;
+    const int hq = (group % Hkv) * (Hq / Hkv) + within / n_parts;
+    const int part = within % n_parts;
+    uint32_t todo = parts.count ? parts.tiles[part] : 0;
+    int qt = parts.count ? 31 - __clz(todo) : n_qt - 1 - part;
 #pragma unroll 1
-    for (int half = 0; half < 2; ++half) {
-        if (half && pair == qt_long) break;
+    while (true) {
         attention_bwd_dq_tile<D, BIAS, EXTRA>(q, k, v, dout, lse, delta, key_bias, dq, Hq, Hkv, L, Lk, scale,
-                                              half ? pair : qt_long, hq, b, smem, &ex, out_rows, delta_w);
+                                              qt, hq, b, smem, &ex, out_rows, delta_w);
+        if (parts.count) {
+            todo &= ~(1u << qt);
+            if (!todo) break;
+            qt = 31 - __clz(todo);
+        } else {
+            if (qt == part) break;
+            qt = part;
+        }
     }
 }
 
@@ -828,7 +838,11 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
     ATS_REQUIRE((int64_t)Lk * D * 2 < 0x7fffffffLL && (int64_t)L * Hq * D * 2 < 0x7fffffffLL, ATS_ERR_UNSUPPORTED,
                 "ats_attention_bwd: L=%d Lk=%d (one head's K or V, and one batch entry's dO, must stay under 2 GiB)", L, Lk);
     const int n_qt = (L + kBwdRows - 1) / kBwdRows, n_kt = (Lk + kBwdRows - 1) / kBwdRows;
-    const int64_t dq_blocks = (int64_t)((n_qt + 1) / 2) * Hq * B;
+    const bool by_xcd = (int64_t)B * Hkv % 8 == 0;
+    const AttnParts parts = attn_parts(n_qt, by_xcd ? (int64_t)B * Hq / 8 : (int64_t)B * Hq, by_xcd ? 32 : 256, true, [&](int t) {
+        return (std::min((t + 1) * kBwdRows, L) - 1 + Lk - L) / kDqBN + 1;
+    });
+    const int64_t dq_blocks = (int64_t)(parts.count ? parts.count : (n_qt + 1) / 2) * Hq * B;
     const int64_t dkv_blocks = (int64_t)((n_kt + 1) / 2) * Hkv * B;
     ATS_REQUIRE(dq_blocks <= 0x7fffffff && dkv_blocks <= 0x7fffffff, ATS_ERR_UNSUPPORTED, "ats_attention_bwd: grid");
     const bf16_t* q_ = static_cast<const bf16_t*>(q);
@@ -862,7 +876,7 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
             ATS_REQUIRE(e == hipSuccess, ATS_ERR_LAUNCH, "ats_attention_bwd_ex: cannot reserve %d bytes of LDS: %s", smem_dkv,
                         hipGetErrorString(e));
             hipLaunchKernelGGL((attention_bwd_dq_kernel<128, false, true>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s,
-                               q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws);
+                               q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<128, true>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_,
                                k_, v_, do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv,
                                L, Lk, scale, ex);
@@ -870,11 +884,11 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
             if (key_bias)
                 hipLaunchKernelGGL((attention_bwd_dq_kernel<128, true>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s,
                                    q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B,
-                                   ex, out_, delta_ws);
+                                   ex, out_, delta_ws, parts);
             else
                 hipLaunchKernelGGL((attention_bwd_dq_kernel<128, false>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s,
                                    q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B,
-                                   ex, out_, delta_ws);
+                                   ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<128>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_, k_,
                                v_, do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv, L,
                                Lk, scale, ex);
@@ -884,17 +898,17 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
         constexpr int smem_dkv = 4 * kDkvBQ * 64 * 2 + 4 * kDkvBQ * 4 + kBwdRows * (64 * 2 + 16);
         if (extras) {
             hipLaunchKernelGGL((attention_bwd_dq_kernel<64, false, true>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s,
-                               q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws);
+                               q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<64, true>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_,
                                k_, v_, do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv,
                                L, Lk, scale, ex);
         } else {
             if (key_bias)
                 hipLaunchKernelGGL((attention_bwd_dq_kernel<64, true>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s, q_,
-                                   k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws);
+                                   k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             else
                 hipLaunchKernelGGL((attention_bwd_dq_kernel<64, false>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s, q_,
-                                   k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws);
+                                   k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<64>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_, k_, v_,
                                do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv, L, Lk,
                                scale, ex);

@@ -1,0 +1,68 @@
+// Which query tiles of a head a workgroup of the causal attention kernels takes.
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace ats {
+
+constexpr int kAttnMaxTiles = 32, kAttnMaxParts = 16;
+
+// count workgroups per head; bit t of tiles[p]: part p takes tile t.  count == 0: part p takes tile n - 1 - p and tile p.
+struct AttnParts {
+    int count;
+    uint32_t tiles[kAttnMaxParts];
+};
+
+// A part's work is counted in key tiles, kTileStart more for each query tile (its first loads, its epilogue: 1.0 us a key tile and
+// 4-6 of them measured).  The parts of a launch run one or two at a time on a compute unit, two of them 1.5 times as long as one by
+// itself (1.95 against 1.08 us a key tile were they all long; the shorter ones leave their partner alone).  Pairs are even, but
+// as many as the tiles make: 96 heads of 14 tiles are 84 pairs of 30 key tiles on an XCD's 32 units, three on some and two on others.
+// Five parts of 42 (28 + 14, 26 + 16, 24 + 18, 22 + 20, the rest) are two on nearly every unit: 3 x 1777 positions, 32 heads of 128,
+// 120 -> 103 us (with the queries' rotation 145 -> 129; the layer 505 -> 500, its products run a little slower behind it: board
+// power), 1 x 4737 of 32 heads of 64 185 -> 130 (the layer 314 -> 254).  70 random shapes of 1-8 sequences of 129-8192 positions: the forward takes
+// 6.6 % less time on average than in pairs (0.67 .. 1.0 of it, single calls to 1.03), dQ with dK and dV behind it 2.8 %.  A twentieth
+// is what the estimate has to promise; more than 32 tiles of a head keep to pairs, whose number is then large.
+//
+// work(t): key tiles that query tile t sees (not falling with t); n_heads heads share `cus` compute units, each of which runs
+// `two` or one workgroup at a time.
+template <typename F>
+inline AttnParts attn_parts(int n_tiles, int64_t n_heads, int cus, bool two, F work) {
+    constexpr int kTileStart = 6;
+    AttnParts best{};
+    if (n_tiles < 2 || n_tiles > kAttnMaxTiles) return best;
+    int w[kAttnMaxTiles], total = 0;
+    for (int t = 0; t < n_tiles; ++t) total += w[t] = work(t) + kTileStart;
+    auto cost = [&](int parts, int64_t most) {
+        const int64_t per_cu = (n_heads * parts + cus - 1) / cus;
+        return most * (two ? 3 * (per_cu / 2) + 2 * (per_cu % 2) : 2 * per_cu);
+    };
+    int most = n_tiles % 2 ? w[n_tiles / 2] : 0;
+    for (int p = 0; p < n_tiles / 2; ++p) most = std::max(most, w[p] + w[n_tiles - 1 - p]);
+    int64_t least = cost((n_tiles + 1) / 2, most) * 19 / 20;
+    for (int parts = std::min(n_tiles, kAttnMaxParts); parts >= 1; --parts) {
+        // first fit, the longest tile first, into the least room that holds all tiles
+        for (int room = std::max(w[n_tiles - 1], (total + parts - 1) / parts); cost(parts, room) < least; ++room) {
+            AttnParts a{};
+            a.count = parts;
+            int left[kAttnMaxParts], t = n_tiles - 1;
+            for (int p = 0; p < parts; ++p) left[p] = room;
+            for (; t >= 0; --t) {
+                int p = 0;
+                while (p < parts && left[p] < w[t]) ++p;
+                if (p == parts) break;
+                left[p] -= w[t];
+                a.tiles[p] |= 1u << t;
+            }
+            if (t >= 0) continue;
+            if (a.tiles[parts - 1]) {      // (fewer parts hold them as well: a later turn)
+                least = cost(parts, room);
+                best = a;
+            }
+            break;
+        }
+    }
+    return best;
+}
+
+}  // namespace ats

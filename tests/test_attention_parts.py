@@ -1,0 +1,80 @@
+"""The query tiles that a workgroup of the causal attention kernels takes (csrc/attention_parts.hpp): every tile once, on the host,
+and results that do not depend on how a launch is cut."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = """
+#include "attention_parts.hpp"
+extern "C" int parts(int n, long heads, int cus, int two, int per_tile, int off, unsigned* tiles) {
+    const ats::AttnParts p = ats::attn_parts(n, heads, cus, two, [&](int t) { return (t + 1) * per_tile + off; });
+    for (int i = 0; i < p.count; ++i) tiles[i] = p.tiles[i];
+    return p.count;
+}
+"""
+
+
+def test_every_tile_belongs_to_one_part(tmp_path):
+    src, lib = tmp_path / "parts.cpp", tmp_path / "parts.so"
+    src.write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I" + os.path.join(ROOT, "adaptivetrainingsystem_amd", "csrc"),
+                    str(src), "-o", str(lib)], check=True)
+    f = ctypes.CDLL(str(lib)).parts
+    f.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_uint)]
+    seen = set()
+    for n in list(range(1, 34)) + [64]:
+        for heads in (1, 4, 12, 16, 20, 32, 33, 96, 256, 100000):
+            for cus, two, per_tile, off in ((32, 1, 2, 0), (256, 1, 2, 0), (32, 0, 4, 0), (256, 1, 2, 40), (32, 1, 0, 3)):
+                tiles = (ctypes.c_uint * 16)()
+                count = f(n, heads, cus, two, per_tile, off, tiles)
+                seen.add(count)
+                assert 0 <= count <= min(n, 16) and (count == 0 or 2 <= n <= 32)
+                if count:
+                    assert all(tiles[i] for i in range(count))
+                    assert sum(bin(tiles[i]).count("1") for i in range(count)) == n
+                    assert sum(tiles[i] for i in range(count)) == (1 << n) - 1
+    assert {0, 1, 2, 3, 5} <= seen
+
+
+# tiles of 128 rows in 2, 3, 5, 7, 14 and 32 (33: pairs again), of 256 rows in 17; cached keys; packed heads of a short chunk
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hq,Hkv,L,Lk,D", [(5, 32, 8, 225, 225, 128), (5, 32, 8, 372, 372, 64), (3, 12, 4, 640, 640, 128),
+                                             (3, 32, 8, 897, 1100, 128), (3, 32, 8, 1777, 1777, 128), (1, 8, 8, 4090, 4090, 64),
+                                             (1, 8, 2, 4200, 4200, 64), (7, 16, 8, 100, 900, 128)])
+def test_results_do_not_depend_on_the_parts(gpu, B, Hq, Hkv, L, Lk, D):
+    from adaptivetrainingsystem_amd import ops
+    print("case", B, Hq, Hkv, L, Lk, D, flush=True)
+    g = torch.Generator(device=gpu).manual_seed(11)
+    q, k, v, do = (torch.randn(*s, generator=g, device=gpu).bfloat16()
+                   for s in ((B, Hq, L, D), (B, Hkv, Lk, D), (B, Hkv, Lk, D), (B, L, Hq * D)))
+    out, lse = ops.causal_attention(q, k, v, return_lse=True)
+    dq, dk, dv = ops.causal_attention_bwd(q, k, v, out, lse, do)
+    # one sequence by itself, with one kv head's queries, is cut otherwise: the same rows, the same bits
+    rep = Hq // Hkv
+    for b, h in {(0, 0), (B - 1, Hkv - 1)}:
+        hq = slice(h * rep, (h + 1) * rep)
+        q1, k1, v1 = q[b:b + 1, hq].contiguous(), k[b:b + 1, h:h + 1].contiguous(), v[b:b + 1, h:h + 1].contiguous()
+        o1, l1 = ops.causal_attention(q1, k1, v1, return_lse=True)
+        cols = slice(h * rep * D, (h + 1) * rep * D)
+        if L * rep >= 128 * rep:     # (fewer rows against many keys: ranges of keys, whose sums have another order)
+            assert torch.equal(o1[0], out[b, :, cols]) and torch.equal(l1[0], lse[b, hq])
+        d1 = ops.causal_attention_bwd(q1, k1, v1, out[b:b + 1, :, cols].contiguous(), lse[b:b + 1, hq].contiguous(), do[b:b + 1, :, cols].contiguous())
+        assert torch.equal(d1[0][0], dq[b, hq])
+        # against float32 of the same values (bfloat16 bar of the attention tests: 2e-2 of the largest value, gradients 3e-2)
+        s = torch.einsum("hld,kd->hlk", q1[0].float(), k1[0, 0].float()) * D ** -0.5
+        s = s.masked_fill(torch.ones(L, Lk, dtype=torch.bool, device=gpu).triu(Lk - L + 1), float("-inf"))
+        p = s.softmax(-1)
+        ref = torch.matmul(p, v1[0, 0].float())
+        got = out[b, :, cols].view(L, rep, D).transpose(0, 1).float()
+        assert (got - ref).abs().max() <= 2e-2 * ref.abs().max()
+        do1 = do[b, :, cols].view(L, rep, D).transpose(0, 1).float()
+        dp = torch.matmul(do1, v1[0, 0].float().t())
+        ds = p * (dp - (do1 * ref).sum(-1, keepdim=True)) * D ** -0.5
+        for have, want in ((dq[b, hq].float(), torch.matmul(ds, k1[0, 0].float())),
+                           (dk[b, h].float(), torch.matmul(ds.transpose(1, 2), q1[0].float()).sum(0)),
+                           (dv[b, h].float(), torch.matmul(p.transpose(1, 2), do1).sum(0))):
+            assert (have - want).abs().max() <= 3e-2 * want.abs().max()
