@@ -141,6 +141,9 @@ _SIGNATURES = {
                              [c_float, c_void_p]),
     "ats_attention_bwd_out": (c_int, [c_void_p] * 9 + [c_int64, c_int64, c_float, c_uint64] + [c_void_p] * 3 + [c_int] * 6 +
                               [c_float, c_void_p]),
+    "ats_attention_bwd_out_ws": (c_int, [c_void_p] * 9 + [c_int64, c_int64, c_float, c_uint64] + [c_void_p] * 3 + [c_int] * 6 +
+                              [c_float, c_void_p, c_size_t, c_void_p]),
+    "ats_attention_bwd_workspace": (c_size_t, [c_int] * 6),
     "ats_attention_f32_fwd": (c_int, [c_void_p] * 5 + [c_int] * 6 + [c_float, c_void_p, c_void_p]),
     "ats_attention_f32_bwd": (c_int, [c_void_p] * 10 + [c_int] * 6 + [c_float, c_void_p, c_void_p]),
     "ats_attention_softmax_f32": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p,

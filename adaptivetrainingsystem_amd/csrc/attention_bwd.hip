@@ -445,8 +445,8 @@ __device__ __forceinline__ void attention_bwd_dkv_tile(const bf16_t* __restrict_
                                                        const float* __restrict__ lse, const float* __restrict__ delta,
                                                        const float* __restrict__ key_bias, bf16_t* __restrict__ dk,
                                                        bf16_t* __restrict__ dv, int Hq, int Hkv, int L, int Lk, float scale,
-                                                       int kt_idx, int hkv, int b, unsigned char* smem,
-                                                       const AttnExtra* ex = nullptr) {
+                                                       int kt_idx, int hkv, int b, unsigned char* smem, const AttnExtra* ex,
+                                                       int range, int ranges, int n_groups, float* __restrict__ part_out) {
     using SW = SwzTile<D>;
     constexpr int KS = D / 16;
     constexpr int DB = D / 32;
@@ -571,19 +571,27 @@ __device__ __forceinline__ void attention_bwd_dkv_tile(const bf16_t* __restrict_
     const int key_wave_last = key_wave_first + 31;
     // first query that sees any key of the block: q + off >= key_block_first
     const int q_first = max(key_block_first - off, 0) / kDkvBQ * kDkvBQ;
-    const int n_steps = rep * ((L - q_first + kDkvBQ - 1) / kDkvBQ);
+    int hh = 0, q0 = q_first, n_steps;
+    {   // this range of the tile's steps (an empty one of a short tile writes zeros; its first loads are those of step 0)
+        const int per_head = (L - q_first + kDkvBQ - 1) / kDkvBQ, all = rep * per_head;
+        const int first = (int)((int64_t)all * range / ranges);
+        n_steps = (int)((int64_t)all * (range + 1) / ranges) - first;
+        if (n_steps > 0) {
+            hh = first / per_head;
+            q0 = q_first + (first - hh * per_head) * kDkvBQ;
+        }
+    }
 
-    DKV_LOAD(0, q_first, 0)
+    DKV_LOAD(hh, q0, 0)
     {
         float l0 = 0.f, d0 = 0.f;
-        DKV_ROW_SCALARS(0, q_first, l0, d0)
-        DKV_STORE_SCALARS(q_first, 0, l0, d0)
+        DKV_ROW_SCALARS(hh, q0, l0, d0)
+        DKV_STORE_SCALARS(q0, 0, l0, d0)
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    DKV_CLEAR_TAIL(q_first, 0)
+    DKV_CLEAR_TAIL(q0, 0)
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    int hh = 0, q0 = q_first;
     for (int i = 0; i < n_steps; ++i) {
         const int par = i & 1;
         const blds_u8_t st = sm + par * STAGE;     // this step's stage; the other one receives step i+1
@@ -733,6 +741,23 @@ __device__ __forceinline__ void attention_bwd_dkv_tile(const bf16_t* __restrict_
 #undef DKV_STORE_SCALARS
 #undef DKV_PREFETCH
 
+    if (part_out) {     // [range][dK, dV][row of all heads][D] float32
+        if (key_row < Lk) {
+            const int64_t rows = n_groups * (int64_t)Lk;
+            float* const krow = part_out + ((int64_t)range * 2 * rows + (int64_t)(b * Hkv + hkv) * Lk + key_row) * D;
+            float* const vrow = krow + rows * D;
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    *reinterpret_cast<float4*>(krow + d * 32 + r * 8 + g * 4) =
+                        make_float4(acc_dk[d][r * 4 + 0], acc_dk[d][r * 4 + 1], acc_dk[d][r * 4 + 2], acc_dk[d][r * 4 + 3]);
+                    *reinterpret_cast<float4*>(vrow + d * 32 + r * 8 + g * 4) =
+                        make_float4(acc_dv[d][r * 4 + 0], acc_dv[d][r * 4 + 1], acc_dv[d][r * 4 + 2], acc_dv[d][r * 4 + 3]);
+                }
+        }
+        return;
+    }
     if (key_row < Lk) {
         bf16_t* krow = dk + ((int64_t)(b * Hkv + hkv) * Lk + key_row) * D;
         bf16_t* vrow = dv + ((int64_t)(b * Hkv + hkv) * Lk + key_row) * D;
@@ -751,40 +776,110 @@ __device__ __forceinline__ void attention_bwd_dkv_tile(const bf16_t* __restrict_
     }
 }
 
-// Early key tiles are seen by more queries than late ones: a workgroup takes tile j and tile n-1-j.
+// Early key tiles are seen by more queries than late ones: a workgroup takes tile j and tile n-1-j, or what AttnParts deals it (its
+// tile t is key tile n-1-t).  There is a workgroup per key tile and kv head only, too few for the chip where few sequences are trained:
+// then the steps of a tile (queries of all heads of the group) are cut into `ranges`, each a workgroup's, whose float32 sums
+// attention_dkv_sum_kernel adds in order.
 template <int D, bool EXTRA = false>
 __global__ __launch_bounds__(256, 2) void attention_bwd_dkv_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     const bf16_t* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta,
     const float* __restrict__ key_bias, bf16_t* __restrict__ dk, bf16_t* __restrict__ dv, int Hq, int Hkv, int L, int Lk,
-    float scale, AttnExtra ex) {
+    float scale, AttnExtra ex, int n_groups, int ranges, float* __restrict__ part_out, AttnParts parts) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int n_kt = (Lk + kBwdRows - 1) / kBwdRows;
-    const int n_pairs = (n_kt + 1) / 2;
+    const int n_parts = parts.count ? parts.count : (n_kt + 1) / 2;
+    const int per_group = n_parts * ranges;
     // consecutive ids go to different XCDs: keep the workgroups of one (batch, kv head), which read the
     // same queries, on one XCD
-    const int n_groups = (int)gridDim.x / n_pairs;
-    int group, pair;
+    int group, within;
     if (n_groups % 8 == 0) {
         const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-        group = (idx / n_pairs) * 8 + xcd;
-        pair = idx % n_pairs;
+        group = (idx / per_group) * 8 + xcd;
+        within = idx % per_group;
     } else {
-        group = blockIdx.x / n_pairs;
-        pair = blockIdx.x % n_pairs;
+        group = blockIdx.x / per_group;
+        within = blockIdx.x % per_group;
     }
     const int hkv = group % Hkv;
     const int b = group / Hkv;
-    const int kt_far = n_kt - 1 - pair;
+    const int range = within / n_parts, part = within % n_parts;
+    uint32_t todo = parts.count ? parts.tiles[part] : 0;
+    int kt = parts.count ? n_kt - 32 + __clz(todo) : part;
 #pragma unroll 1
-    for (int half = 0; half < 2; ++half) {
-        if (half && pair == kt_far) break;
-        attention_bwd_dkv_tile<D, EXTRA>(q, k, v, dout, lse, delta, key_bias, dk, dv, Hq, Hkv, L, Lk, scale,
-                                         half ? kt_far : pair, hkv, b, smem, &ex);
+    while (true) {
+        attention_bwd_dkv_tile<D, EXTRA>(q, k, v, dout, lse, delta, key_bias, dk, dv, Hq, Hkv, L, Lk, scale, kt, hkv, b, smem, &ex,
+                                         range, ranges, n_groups, part_out);
+        if (parts.count) {
+            todo &= ~(1u << (n_kt - 1 - kt));
+            if (!todo) break;
+            kt = n_kt - 32 + __clz(todo);
+        } else {
+            if (kt == n_kt - 1 - part) break;
+            kt = n_kt - 1 - part;
+        }
     }
 }
 
+// dk, dv [rows, D] = sums of the ranges' parts, in their order.  HBM: 8 * ranges + 4 bytes per pair of elements.
+__global__ __launch_bounds__(256) void attention_dkv_sum_kernel(const float* __restrict__ part, bf16_t* __restrict__ dk,
+                                                                bf16_t* __restrict__ dv, int64_t elems, int ranges) {
+    const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (at >= 2 * elems) return;
+    float4 lo = *reinterpret_cast<const float4*>(part + at), hi = *reinterpret_cast<const float4*>(part + at + 4);
+    for (int r = 1; r < ranges; ++r) {
+        const float4 a = *reinterpret_cast<const float4*>(part + 2 * r * elems + at);
+        const float4 c = *reinterpret_cast<const float4*>(part + 2 * r * elems + at + 4);
+        lo.x += a.x, lo.y += a.y, lo.z += a.z, lo.w += a.w;
+        hi.x += c.x, hi.y += c.y, hi.z += c.z, hi.w += c.w;
+    }
+    bu32x4_t w;
+    w.x = pack_bf16x2(lo.x, lo.y);
+    w.y = pack_bf16x2(lo.z, lo.w);
+    w.z = pack_bf16x2(hi.x, hi.y);
+    w.w = pack_bf16x2(hi.z, hi.w);
+    *reinterpret_cast<bu32x4_t*>(at < elems ? dk + at : dv + (at - elems)) = w;
+}
+
+struct DkvPlan {
+    int ranges;
+    AttnParts parts;
+};
+
+// Ranges of a key tile's steps and the tiles of a workgroup, by the least estimated time: attn_parts of the steps (0.58 us alone on a
+// unit, 0.49 at head_dim 64), and the traffic of the sums.  Fitted to the whole backward of 60 random shapes of 1-8 sequences of 65-7511
+// positions (best of all numbers of ranges 0.2 % better on average, 5 % at most): 1 x 1777, 32 heads of 128 on 8: 349 -> 155 us,
+// 3 x 1777 434 -> 361, 1 x 4328 of 8 heads 847 -> 284, 8 x 2048 (the chip is full) one range as before.
+static DkvPlan dkv_plan(int B, int Hq, int Hkv, int L, int Lk, int D, bool workspace) {
+    const int n_kt = (Lk + kBwdRows - 1) / kBwdRows, rep = Hq / Hkv, off = Lk - L, steps = (L + kDkvBQ - 1) / kDkvBQ;
+    const int64_t groups = (int64_t)B * Hkv;
+    const bool by_xcd = groups % 8 == 0;
+    const double by_range = (double)groups * Lk * D * 16 / 7.6e6;      // a range's sums written and read
+    DkvPlan best{};
+    double least = 0;
+    for (const int ranges : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        int64_t quarters = 0;
+        const AttnParts parts = attn_parts(n_kt, (by_xcd ? groups / 8 : groups) * ranges, by_xcd ? 32 : 256, true, [&](int t) {
+            const int first = std::max((n_kt - 1 - t) * kBwdRows - off, 0) / kDkvBQ;
+            return (rep * (steps - first) + ranges - 1) / ranges;
+        }, &quarters);
+        const double us = quarters * (D == 128 ? 0.29 : 0.245) + (ranges > 1 ? ranges * by_range + (D == 128 ? 2 : 6) : 0);
+        if (ranges == 1 || us < least) {
+            least = ranges == 1 ? us * 0.95 - 1 : us;
+            best = {ranges, parts};
+        }
+        if (!workspace) break;
+    }
+    return best;
+}
+
 }  // namespace ats
+
+extern "C" size_t ats_attention_bwd_workspace(int B, int Hq, int Hkv, int L, int Lk, int D) {
+    if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || L <= 0 || Lk < L || (D != 64 && D != 128)) return 0;
+    const int ranges = ats::dkv_plan(B, Hq, Hkv, L, Lk, D, true).ranges;
+    return ranges > 1 ? (size_t)ranges * 2 * B * Hkv * Lk * D * sizeof(float) : 0;
+}
 
 extern "C" int ats_attention_delta(const void* out, const void* dout, float* delta, int B, int Hq, int L, int D,
                                    ats_stream_t stream) {
@@ -821,7 +916,7 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
                                 const float* lse, const float* delta, float* delta_ws, const float* key_bias,
                                 const float* bias_qk, int64_t bias_sb, int64_t bias_sh, float dropout_p,
                                 uint64_t dropout_seed, void* dq, void* dk, void* dv, int B, int Hq, int Hkv, int L, int Lk,
-                                int D, float scale, ats_stream_t stream) {
+                                int D, float scale, void* workspace, size_t workspace_bytes, ats_stream_t stream) {
     using namespace ats;
     ATS_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && L >= 0 && Lk >= L && scale > 0.f, ATS_ERR_INVALID_ARG,
                 "ats_attention_bwd: B=%d Hq=%d Hkv=%d L=%d Lk=%d scale=%g", B, Hq, Hkv, L, Lk, scale);
@@ -843,7 +938,12 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
         return (std::min((t + 1) * kBwdRows, L) - 1 + Lk - L) / kDqBN + 1;
     });
     const int64_t dq_blocks = (int64_t)(parts.count ? parts.count : (n_qt + 1) / 2) * Hq * B;
-    const int64_t dkv_blocks = (int64_t)((n_kt + 1) / 2) * Hkv * B;
+    const int n_groups = B * Hkv;
+    DkvPlan plan = dkv_plan(B, Hq, Hkv, L, Lk, D, workspace != nullptr);
+    if (plan.ranges > 1 && ((size_t)plan.ranges * 2 * n_groups * Lk * D * sizeof(float) > workspace_bytes || !aligned16(workspace)))
+        plan = dkv_plan(B, Hq, Hkv, L, Lk, D, false);
+    float* const part_out = plan.ranges > 1 ? static_cast<float*>(workspace) : nullptr;
+    const int64_t dkv_blocks = (int64_t)(plan.parts.count ? plan.parts.count : (n_kt + 1) / 2) * plan.ranges * Hkv * B;
     ATS_REQUIRE(dq_blocks <= 0x7fffffff && dkv_blocks <= 0x7fffffff, ATS_ERR_UNSUPPORTED, "ats_attention_bwd: grid");
     const bf16_t* q_ = static_cast<const bf16_t*>(q);
     const bf16_t* k_ = static_cast<const bf16_t*>(k);
@@ -879,7 +979,7 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
                                q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<128, true>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_,
                                k_, v_, do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv,
-                               L, Lk, scale, ex);
+                               L, Lk, scale, ex, n_groups, plan.ranges, part_out, plan.parts);
         } else {
             if (key_bias)
                 hipLaunchKernelGGL((attention_bwd_dq_kernel<128, true>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s,
@@ -891,7 +991,7 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
                                    ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<128>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_, k_,
                                v_, do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv, L,
-                               Lk, scale, ex);
+                               Lk, scale, ex, n_groups, plan.ranges, part_out, plan.parts);
         }
     } else {
         constexpr int smem_dq = 4 * kDqBN * 64 * 2 + 2 * kDqBN * 4;
@@ -901,7 +1001,7 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
                                q_, k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<64, true>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_,
                                k_, v_, do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv,
-                               L, Lk, scale, ex);
+                               L, Lk, scale, ex, n_groups, plan.ranges, part_out, plan.parts);
         } else {
             if (key_bias)
                 hipLaunchKernelGGL((attention_bwd_dq_kernel<64, true>), dim3((unsigned)dq_blocks), dim3(256), smem_dq, s, q_,
@@ -911,10 +1011,16 @@ static int attention_bwd_launch(const void* q, const void* k, const void* v, con
                                    k_, v_, do_, lse, delta, key_bias, static_cast<bf16_t*>(dq), Hq, Hkv, L, Lk, scale, B, ex, out_, delta_ws, parts);
             hipLaunchKernelGGL((attention_bwd_dkv_kernel<64>), dim3((unsigned)dkv_blocks), dim3(256), smem_dkv, s, q_, k_, v_,
                                do_, lse, delta_kv, key_bias, static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), Hq, Hkv, L, Lk,
-                               scale, ex);
+                               scale, ex, n_groups, plan.ranges, part_out, plan.parts);
         }
     }
     ATS_CHECK_LAUNCH("ats_attention_bwd");
+    if (part_out) {
+        const int64_t elems = (int64_t)n_groups * Lk * D;
+        hipLaunchKernelGGL(attention_dkv_sum_kernel, dim3((unsigned)((2 * elems / 8 + 255) / 256)), dim3(256), 0, s, part_out,
+                           static_cast<bf16_t*>(dk), static_cast<bf16_t*>(dv), elems, plan.ranges);
+        ATS_CHECK_LAUNCH("ats_attention_bwd(sum)");
+    }
     return ATS_OK;
 }
 
@@ -923,7 +1029,17 @@ extern "C" int ats_attention_bwd_ex(const void* q, const void* k, const void* v,
                                     int64_t bias_sh, float dropout_p, uint64_t dropout_seed, void* dq, void* dk, void* dv, int B, int Hq,
                                     int Hkv, int L, int Lk, int D, float scale, ats_stream_t stream) {
     return attention_bwd_launch(q, k, v, nullptr, dout, lse, delta, nullptr, key_bias, bias_qk, bias_sb, bias_sh, dropout_p,
-                                dropout_seed, dq, dk, dv, B, Hq, Hkv, L, Lk, D, scale, stream);
+                                dropout_seed, dq, dk, dv, B, Hq, Hkv, L, Lk, D, scale, nullptr, 0, stream);
+}
+
+extern "C" int ats_attention_bwd_out_ws(const void* q, const void* k, const void* v, const void* out, const void* dout,
+                                     const float* lse, float* delta_ws, const float* key_bias, const float* bias_qk,
+                                     int64_t bias_sb, int64_t bias_sh, float dropout_p, uint64_t dropout_seed, void* dq,
+                                     void* dk, void* dv, int B, int Hq, int Hkv, int L, int Lk, int D, float scale,
+                                        void* workspace, size_t workspace_bytes, ats_stream_t stream) {
+    ATS_REQUIRE(out != nullptr || B == 0 || L == 0, ATS_ERR_INVALID_ARG, "ats_attention_bwd_out_ws: null pointer");
+    return attention_bwd_launch(q, k, v, out, dout, lse, nullptr, delta_ws, key_bias, bias_qk, bias_sb, bias_sh, dropout_p,
+                                dropout_seed, dq, dk, dv, B, Hq, Hkv, L, Lk, D, scale, workspace, workspace_bytes, stream);
 }
 
 extern "C" int ats_attention_bwd_out(const void* q, const void* k, const void* v, const void* out, const void* dout,
@@ -933,5 +1049,5 @@ extern "C" int ats_attention_bwd_out(const void* q, const void* k, const void* v
                                      ats_stream_t stream) {
     ATS_REQUIRE(out != nullptr || B == 0 || L == 0, ATS_ERR_INVALID_ARG, "ats_attention_bwd_out: null pointer");
     return attention_bwd_launch(q, k, v, out, dout, lse, nullptr, delta_ws, key_bias, bias_qk, bias_sb, bias_sh, dropout_p,
-                                dropout_seed, dq, dk, dv, B, Hq, Hkv, L, Lk, D, scale, stream);
+                                dropout_seed, dq, dk, dv, B, Hq, Hkv, L, Lk, D, scale, nullptr, 0, stream);
 }

@@ -15,8 +15,8 @@ struct AttnParts {
 };
 
 // A part's work is counted in key tiles, kTileStart more for each query tile (its first loads, its epilogue: 1.0 us a key tile and
-// 4-6 of them measured).  The parts of a launch run one or two at a time on a compute unit, two of them 1.5 times as long as one by
-// itself (1.95 against 1.08 us a key tile were they all long; the shorter ones leave their partner alone).  Pairs are even, but
+// 4-6 of them measured).  The parts of a launch run one or two at a time on a compute unit, two of them 1.25 times as long as one by
+// itself (1.95 against 1.08 us a key tile were they in step all the way; the factor that chose best among 2.5 .. 4 quarters a pair).  Pairs are even, but
 // as many as the tiles make: 96 heads of 14 tiles are 84 pairs of 30 key tiles on an XCD's 32 units, three on some and two on others.
 // Five parts of 42 (28 + 14, 26 + 16, 24 + 18, 22 + 20, the rest) are two on nearly every unit: 3 x 1777 positions, 32 heads of 128,
 // 120 -> 103 us (with the queries' rotation 145 -> 129; the layer 505 -> 500, its products run a little slower behind it: board
@@ -25,21 +25,22 @@ struct AttnParts {
 // is what the estimate has to promise; more than 32 tiles of a head keep to pairs, whose number is then large.
 //
 // work(t): key tiles that query tile t sees (not falling with t); n_heads heads share `cus` compute units, each of which runs
-// `two` or one workgroup at a time.
+// `two` or one workgroup at a time.  *estimate: time of the fullest compute unit in quarters of a lone workgroup's key tile.
 template <typename F>
-inline AttnParts attn_parts(int n_tiles, int64_t n_heads, int cus, bool two, F work) {
+inline AttnParts attn_parts(int n_tiles, int64_t n_heads, int cus, bool two, F work, int64_t* estimate = nullptr) {
     constexpr int kTileStart = 6;
     AttnParts best{};
-    if (n_tiles < 2 || n_tiles > kAttnMaxTiles) return best;
-    int w[kAttnMaxTiles], total = 0;
-    for (int t = 0; t < n_tiles; ++t) total += w[t] = work(t) + kTileStart;
     auto cost = [&](int parts, int64_t most) {
         const int64_t per_cu = (n_heads * parts + cus - 1) / cus;
-        return most * (two ? 3 * (per_cu / 2) + 2 * (per_cu % 2) : 2 * per_cu);
+        return most * (two ? 5 * (per_cu / 2) + 4 * (per_cu % 2) : 4 * per_cu);
     };
-    int most = n_tiles % 2 ? w[n_tiles / 2] : 0;
-    for (int p = 0; p < n_tiles / 2; ++p) most = std::max(most, w[p] + w[n_tiles - 1 - p]);
+    int most = n_tiles % 2 ? work(n_tiles / 2) + kTileStart : 0;
+    for (int p = 0; p < n_tiles / 2; ++p) most = std::max(most, work(p) + work(n_tiles - 1 - p) + 2 * kTileStart);
+    if (estimate) *estimate = cost((n_tiles + 1) / 2, most);
+    if (n_tiles < 2 || n_tiles > kAttnMaxTiles) return best;
     int64_t least = cost((n_tiles + 1) / 2, most) * 19 / 20;
+    int w[kAttnMaxTiles], total = 0;
+    for (int t = 0; t < n_tiles; ++t) total += w[t] = work(t) + kTileStart;
     for (int parts = std::min(n_tiles, kAttnMaxParts); parts >= 1; --parts) {
         // first fit, the longest tile first, into the least room that holds all tiles
         for (int room = std::max(w[n_tiles - 1], (total + parts - 1) / parts); cost(parts, room) < least; ++room) {
@@ -58,6 +59,7 @@ inline AttnParts attn_parts(int n_tiles, int64_t n_heads, int cus, bool two, F w
             if (a.tiles[parts - 1]) {      // (fewer parts hold them as well: a later turn)
                 least = cost(parts, room);
                 best = a;
+                if (estimate) *estimate = least;
             }
             break;
         }

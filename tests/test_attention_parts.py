@@ -40,6 +40,30 @@ def test_every_tile_belongs_to_one_part(tmp_path):
     assert {0, 1, 2, 3, 5} <= seen
 
 
+# keys of a tile whose queries are cut into ranges, some of them empty (the last tile sees 2 queries, 1 of 4 heads' steps each)
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hq,Hkv,L,Lk,D", [(1, 4, 1, 130, 130, 128), (1, 8, 1, 33, 33, 64), (1, 4, 4, 1500, 1500, 64), (1, 8, 2, 700, 900, 64), (2, 32, 2, 2, 300, 128)])
+@pytest.mark.parametrize("dropout", [0.0, 0.2])
+def test_ranges_of_queries_add_up(gpu, B, Hq, Hkv, L, Lk, D, dropout):
+    from adaptivetrainingsystem_amd import _lib, ops
+    print("case", B, Hq, Hkv, L, Lk, D, dropout, flush=True)
+    lib = _lib.load()
+    g = torch.Generator(device=gpu).manual_seed(5)
+    q, k, v, do = (torch.randn(*s, generator=g, device=gpu).bfloat16()
+                   for s in ((B, Hq, L, D), (B, Hkv, Lk, D), (B, Hkv, Lk, D), (B, L, Hq * D)))
+    out, lse = ops.causal_attention(q, k, v, return_lse=True, dropout_p=dropout, dropout_seed=3)
+    assert lib.ats_attention_bwd_workspace(B, Hq, Hkv, L, Lk, D) > 0
+    dq, dk, dv = ops.causal_attention_bwd(q, k, v, out, lse, do, dropout_p=dropout, dropout_seed=3)
+    q1, k1, v1, delta = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), torch.empty_like(lse)
+    assert lib.ats_attention_bwd_out(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), do.data_ptr(), lse.data_ptr(),
+                                     delta.data_ptr(), None, None, 0, 0, dropout, 3, q1.data_ptr(), k1.data_ptr(), v1.data_ptr(), B, Hq,
+                                     Hkv, L, Lk, D, D ** -0.5, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(dq, q1)
+    # the same float32 sums in another order, then one rounding to bfloat16 (8 bits: neighbours lie up to 2^-7 of their value apart)
+    for a, b in ((dk, k1), (dv, v1)):
+        assert ((a.float() - b.float()).abs() <= 2 ** -7 * b.float().abs() + 1e-5 * b.float().abs().max()).all()
+
+
 # tiles of 128 rows in 2, 3, 5, 7, 14 and 32 (33: pairs again), of 256 rows in 17; cached keys; packed heads of a short chunk
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,L,Lk,D", [(5, 32, 8, 225, 225, 128), (5, 32, 8, 372, 372, 64), (3, 12, 4, 640, 640, 128),
