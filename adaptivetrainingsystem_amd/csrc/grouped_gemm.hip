@@ -1869,7 +1869,18 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     //   128 tokens (32 rows per expert), gate/up: 430 against 343 with 256-row tiles, hence the bound.
     const int pieces = (int)(((int64_t)p.K * (int)sizeof(T) + 255) / 256);
     if (avg <= (E == 1 ? 32 : 20) && p.N_out >= 32 && !p.k_count) {
-        if constexpr (SWIGLU) return launch_stream<T, TO, 2, 2, 4, SWIGLU>(p, max_rows, s);
+        // (tiles of 16 activation rows for few rows per group: half of the registers for them; gate/up [2816, 2048] x 64, 24 tokens
+        // with the down projection 179 -> 175 us, [28672, 4096] x 8, 1 token 129.5 -> 126.5.  A group beyond 16 rows reads its weights
+        // twice: 8 experts with 16 rows each 457 -> 555 us, hence the bound well below them.)
+        auto panels = [&](auto np, auto kw) {
+            constexpr int NP = decltype(np)::value, KW = decltype(kw)::value;
+            return avg <= 4 ? launch_stream<T, TO, NP, 1, KW, SWIGLU>(p, max_rows, s) : launch_stream<T, TO, NP, 2, KW, SWIGLU>(p, max_rows, s);
+        };
+        typedef std::integral_constant<int, 1> One;
+        typedef std::integral_constant<int, 2> Two;
+        typedef std::integral_constant<int, 4> Four;
+        typedef std::integral_constant<int, 8> Eight;
+        if constexpr (SWIGLU) return panels(Two{}, Four{});
         else {
             // Eight waves split K where there are at least four pieces for each (a panel of 16 rows then reads 2 KB of
             // every row per step): [4096, 4096] x 16 rows 10.3 us against 11.7 with four waves and 14.5 with four waves
@@ -1878,11 +1889,11 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
             // 3 tokens: 23 against 37 us).
             const int64_t groups = max_rows < E ? max_rows : E;
             if (pieces >= 32 && (pieces >= 64 || groups * p.N_out <= 16 * 1024)) {
-                if (E == 1 || avg <= 8) return launch_stream<T, TO, 1, 2, 8, SWIGLU>(p, max_rows, s);
-                return launch_stream<T, TO, 2, 2, 8, SWIGLU>(p, max_rows, s);
+                if (E == 1 || avg <= 8) return panels(One{}, Eight{});
+                return panels(Two{}, Eight{});
             }
-            if (groups * p.N_out < 32 * 256) return launch_stream<T, TO, 1, 2, 4, SWIGLU>(p, max_rows, s);
-            return launch_stream<T, TO, 2, 2, 4, SWIGLU>(p, max_rows, s);
+            if (groups * p.N_out < 32 * 256) return panels(One{}, Four{});
+            return panels(Two{}, Four{});
         }
     }
     if constexpr (!SWIGLU) {

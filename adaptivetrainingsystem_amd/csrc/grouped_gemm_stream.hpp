@@ -43,6 +43,52 @@ struct StreamTile {
     static constexpr int kLds = KW * (kStage > kRows * kRedPitch * 4 ? kStage : kRows * kRedPitch * 4);
 };
 
+// Block -> (group, m-tile, n-tile).  The panels of all groups form one list (a group's n-tiles in turn, its m-tiles innermost), dealt to
+// the XCDs (block % 8) in whole rounds of `chunk` panels each, what is left (chunk 0: everything) in eight equal pieces, so that no XCD
+// has more than its share: in supertiles of 32, the order of the wide tiles, 17 experts of 64 panels are 34 supertiles, five on some XCDs
+// and four on others.  One piece per XCD is the fastest for many small groups, an XCD then reads a few weights at a time: 64 experts
+// [2816, 2048] + [2048, 1408], whole layer, 24 tokens 183.5 us in supertiles, 181 in chunks, 179 in pieces; 128 experts of 768, 60 tokens
+// 309 -> 281 -> 279.  Eight large experts, one to an XCD, would be slower than in chunks (64 tokens 457 against 469), and sixteen with
+// skewed routing (41 tokens of 16 x [11264, 2048] 113 -> 109 in chunks, 118 in pieces): pieces from 32 experts on.
+__device__ __forceinline__ bool decode_panel_wave(unsigned block, const int32_t* __restrict__ row_count, int E, int BM, int n_tiles,
+                                                  unsigned chunk, TileCoord* out) {
+    const int lane = threadIdx.x & 63;
+    int t0 = 0, p0 = 0;
+    unsigned total = 0;
+    for (int g0 = 0; g0 < E; g0 += 64) {
+        int t, p;
+        tile_scan64(row_count, E, E, g0, BM, 1, false, lane, &t, &p);
+        if (g0 == 0) t0 = t, p0 = p;
+        total += (unsigned)__builtin_amdgcn_readlane(p, 63);
+    }
+    const unsigned all = total * (unsigned)n_tiles, xcd = block % kNumXcd, li = block / kNumXcd;
+    const unsigned whole = chunk ? all / (kNumXcd * chunk) * chunk : 0;      // an XCD's panels in whole rounds
+    if (li < whole) block = (li / chunk * kNumXcd + xcd) * chunk + li % chunk;
+    else {
+        const unsigned rest = all - kNumXcd * whole, per = (rest + kNumXcd - 1) / kNumXcd, at = xcd * per + li - whole;
+        if (li - whole >= per || at >= rest) return false;
+        block = kNumXcd * whole + at;
+    }
+    const int pos = (int)(block / (unsigned)n_tiles);      // in the list of all groups' m-tiles
+    int base = 0;
+    for (int g0 = 0; g0 < E; g0 += 64) {
+        int t = t0, p = p0;
+        if (g0 > 0) tile_scan64(row_count, E, E, g0, BM, 1, false, lane, &t, &p);
+        const unsigned long long hit = __ballot(base + p > pos);
+        if (hit) {
+            const int first = __ffsll((long long)hit) - 1;
+            const unsigned tiles = (unsigned)__builtin_amdgcn_readlane(t, first);
+            const unsigned at = block - (unsigned)(base + __builtin_amdgcn_readlane(p, first) - (int)tiles) * (unsigned)n_tiles;
+            out->e = g0 + first;
+            out->nt = (int)(at / tiles);
+            out->mt = (int)(at % tiles);
+            return true;
+        }
+        base += __builtin_amdgcn_readlane(p, 63);
+    }
+    return false;
+}
+
 template <typename T, typename TO, int NP, int MT, int KW, bool SWIGLU>
 __global__ __launch_bounds__(KW * 64, KW == 4 && MT <= 2 ? 3 : 2) void grouped_gemm_stream_kernel(GroupedArgs p) {
     typedef StreamTile<NP, MT, KW> Tile;
@@ -56,7 +102,7 @@ __global__ __launch_bounds__(KW * 64, KW == 4 && MT <= 2 ? 3 : 2) void grouped_g
     extern __shared__ __align__(16) unsigned char smem[];
 
     TileCoord tc;
-    if (!decode_tile_wave(blockIdx.x, p.row_count, p.E, Tile::kRows, p.n_tiles, p.sm, p.sn, false, &tc)) return;
+    if (!decode_panel_wave(blockIdx.x, p.row_count, p.E, Tile::kRows, p.n_tiles, (unsigned)p.sm, &tc)) return;
     const int count = p.row_count[tc.e];
     const int row0 = p.row_start[tc.e];
     const int K = p.K;
@@ -204,8 +250,7 @@ static int launch_stream(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
     constexpr int kCols = SWIGLU ? Tile::kWRows / 2 : Tile::kWRows;
     GroupedArgs p = p0;
     p.n_tiles = (p.N_out + kCols - 1) / kCols;
-    p.sm = 1;
-    p.sn = 32;
+    p.sm = p.E >= 32 ? 0 : 32;      // panels of a chunk
     auto kern = grouped_gemm_stream_kernel<T, TO, NP, MT, KW, SWIGLU>;
     if (Tile::kLds > 64 * 1024) {
         static LdsReservation reserved;
@@ -215,7 +260,8 @@ static int launch_stream(const GroupedArgs& p0, int64_t max_rows, hipStream_t s)
             return ATS_ERR_LAUNCH;
         }
     }
-    const int64_t blocks = grid_blocks(max_rows, p.E, Tile::kRows, p.n_tiles, p.sm, p.sn, false);
+    // a tile has at least one row; a multiple of 8, so that every XCD has room for an eighth
+    const int64_t blocks = (std::min(max_rows, max_rows / Tile::kRows + p.E) * p.n_tiles + kNumXcd - 1) / kNumXcd * kNumXcd;
     if (blocks > 0x7fffffffLL) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;

@@ -98,3 +98,24 @@ def test_native_layer_call_equals_the_stages(A, gpu, T, k, mode, onto, I):  # no
         assert torch.equal(plan[name], ref[name].view(plan[name].shape)), name
     n = int(ref["kept"].sum())
     assert torch.equal(plan["row_src"][:n], ref["row_src"][:n])
+
+
+# panels dealt to the XCDs in one piece each (32 groups and more) or in chunks; more than 64 groups; tiles of 16 rows (up to 4 rows per
+# group on average) with groups that need several
+@pytest.mark.parametrize("counts,N,K", [([1] * 31, 40, 136), ([1] * 32, 40, 136), ([40] + [0] * 29 + [1] * 5, 72, 520), ([17, 16, 0, 1] + [0] * 6, 1032, 264),
+                                        ([2, 0, 1] * 24, 264, 136), ([0] * 129 + [33], 72, 264), ([3, 0, 19] * 45, 40, 136)])
+def test_stream_panels_of_many_groups(ops, gpu, counts, N, K):  # noqa: F811
+    print("case stream panels", len(counts), sum(counts), N, K, flush=True)
+    g = gen(313)
+    E, n = len(counts), sum(counts)
+    w = [(torch.randn(N, K, generator=g) * 0.1).bfloat16().to(gpu) for _ in range(E)]
+    count = torch.tensor(counts, dtype=torch.int32)
+    start = (torch.cumsum(count, 0) - count).to(torch.int32).to(gpu)
+    a = torch.randn(n, K, generator=g).bfloat16().to(gpu)
+    # (n + 5 rows at most: the launch may have more blocks than panels)
+    out = ops.grouped_gemm_nt(ops.weight_pointer_table(w), K, N, start, count.to(gpu), n + 5, n + 5, N, K, a=a, out_dtype=torch.float32)
+    off = 0
+    for e, c in enumerate(counts):
+        if c:
+            assert rel_err(out[off:off + c], a[off:off + c].cpu().double() @ w[e].cpu().double().T) <= F32_TOL
+        off += c
