@@ -441,7 +441,8 @@ class MoEFunction(Function):
     """The whole MoE FFN layer on [T, H] tokens.  apply(x, gate_weight, cfg, *expert_weights) with
     expert_weights = E gate/up matrices [2I, H] followed by E down matrices [H, I]; cfg is a dict:
     top_k, temperature, variant, capacity (C, or T for no dropping), load_balancing_weight,
-    noise_std (0 in eval), logit_bias (tensor or None), stats (dict filled with the plan).
+    noise_std (0 in eval), logit_bias (tensor or None), stats (dict filled with the plan), counts (device counters of
+    ops.routing_counts, or None).
     Returns (out [T, H], aux scalar)."""
 
     @staticmethod
@@ -461,12 +462,12 @@ class MoEFunction(Function):
         if cfg.get("noise_std", 0.0) > 0:
             logits_route = logits + torch.randn_like(logits) * cfg["noise_std"]
         route = ops.route_topk(logits_route, k, cfg["temperature"], cfg["variant"], cfg["load_balancing_weight"])
-        usage = route["hist"].float() / (T * k + 1e-9)
         if logits_route is logits:
             aux = route["aux"][0]
         else:   # importance from the noise-free logits (model.py:1190-1192)
             aux = ops.aux_loss_clean_logits(logits, route["hist"], k, cfg["variant"], cfg["load_balancing_weight"])
         plan = ops.dispatch_plan(route["indices"], E, C)
+        usage = ops.routing_counts(route["hist"], plan["kept"], T * k, cfg.get("counts"))
         rows = min(T * k, E * C)
         hT = wplan = None
         if rows > 0:
@@ -514,12 +515,9 @@ class MoEFunction(Function):
             dx_rows, dwgu, dwd = _ffn_backward(dy, x, ctx.wgu, ctx.wd, gu, h, offsets, kept, rows, row_src, k, need_x,
                                                need_w, hT=hT, wplan=wplan)
             if need_x:
-                ones = torch.ones(T, k, dtype=torch.float32, device=dev)
-                if dx_rows.dim() == 3 and k <= 8:
-                    dx = ops.combine_partials(dx_rows, row_of, ones, T, k, dtype)
-                else:
-                    dx_rows = ops.sum_partials(dx_rows, dtype) if dx_rows.dim() == 3 else dx_rows
-                    dx = ops.combine(dx_rows, row_of, ones, T, k, out_dtype=dtype)
+                if dx_rows.dim() == 3 and k > 8:
+                    dx_rows = ops.sum_partials(dx_rows, dtype)
+                dx = ops.gather_sum(dx_rows, row_of, T, k, dtype)
         else:
             dw = torch.zeros(T, k, dtype=torch.float32, device=dev)
             dx = torch.zeros(T, H, dtype=dtype, device=dev) if need_x else None
@@ -529,20 +527,19 @@ class MoEFunction(Function):
 
         # routing rule + load-balancing loss -> router logits -> x and the gate weight
         lbw = ctx.cfg["load_balancing_weight"]
-        scale_dev = (daux.detach().float() * (aux < 1.0).float()).reshape(1).contiguous()
         dz = ops.route_bwd(logits_route, idx, w, dw, ctx.cfg["temperature"], ctx.cfg["variant"], logits_aux=logits,
-                           usage=usage, aux_scale=E * lbw / T, aux_scale_dev=scale_dev)
+                           usage=usage, aux_scale=E * lbw / T, aux_scale_dev=daux.detach().float(), aux_value=aux)
         dx_out, dwg = ops.router_bwd(dz, x, wg, base=dx if need_x else None, out=dx if need_x else None,
                                      need_dx=need_x, need_dw=need_wg)
 
         gate_dtype, wdtypes = ctx.param_dtypes
         grads_w = [None] * ctx.n_weights
         if need_w:
-            for e in range(E):
+            for e, (g, d) in enumerate(zip(dwgu, dwd)):
                 if ctx.needs_input_grad[3 + e]:
-                    grads_w[e] = dwgu[e].to(wdtypes[e])
+                    grads_w[e] = g.to(wdtypes[e])
                 if ctx.needs_input_grad[3 + E + e]:
-                    grads_w[E + e] = dwd[e].to(wdtypes[E + e])
+                    grads_w[E + e] = d.to(wdtypes[E + e])
         return (dx_out if need_x else None, dwg.to(gate_dtype) if need_wg else None, None, *grads_w)
 
 

@@ -169,14 +169,15 @@ __global__ __launch_bounds__(256) void fill_f32_kernel(float* __restrict__ p, in
 //   dz[i_j] = w_j * (dw_j - sum_m dw_m w_m) / tau
 // Load-balancing loss (model.py:1244-1263) with q = softmax(z_aux), usage constant:
 //   dz_aux[e] += aux_scale * q_e * (usage_e - sum_e' usage_e' q_e'),  aux_scale = dL/daux * E * weight / T
-// (aux_scale = host factor times an optional device scalar, so dL/daux needs no host read-back)
+// (aux_scale = host factor times an optional device scalar, so dL/daux needs no host read-back; times 0 where the optional
+// aux_value, the loss itself, reached its clamp at 1)
 // One thread per token (E is small).
 __global__ __launch_bounds__(256) void route_bwd_kernel(const float* __restrict__ z_route,
                                                         const float* __restrict__ z_aux,
                                                         const int32_t* __restrict__ idx, const float* __restrict__ w,
                                                         const float* __restrict__ dw, const float* __restrict__ usage,
                                                         float aux_scale, const float* __restrict__ aux_scale_dev,
-                                                        float inv_tau, int mode,
+                                                        const float* __restrict__ aux_value, float inv_tau, int mode,
                                                         float* __restrict__ dz, int64_t T, int E, int k) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= T) return;
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(256) void route_bwd_kernel(const float* __restrict_
         for (int e = 0; e < E; ++e) out[e] = 0.f;
         for (int j = 0; j < k; ++j) out[it[j]] += wt[j] * (dwt[j] - dot) * inv_tau;
     }
-    if (aux_scale_dev) aux_scale *= aux_scale_dev[0];
+    if (aux_scale_dev) aux_scale *= aux_value ? aux_scale_dev[0] * (aux_value[0] < 1.f ? 1.f : 0.f) : aux_scale_dev[0];
     if (usage && aux_scale != 0.f) {
         const float* za = z_aux + t * E;
         float mx = -INFINITY;
@@ -225,6 +226,19 @@ __global__ __launch_bounds__(256) void route_bwd_kernel(const float* __restrict_
     }
 }
 
+// usage[e] = hist[e] * inv; with counts, hist is added to counts[0 .. E) and the dropped assignments to counts[E].  Integer atomics: passes
+// of one layer may run on several streams.
+__global__ __launch_bounds__(256) void routing_counts_kernel(const int32_t* __restrict__ hist, const int32_t* __restrict__ kept, int E,
+                                                             float inv, float* __restrict__ usage, unsigned long long* __restrict__ counts) {
+    for (int e = threadIdx.x; e < E; e += 256) {
+        const int h = hist[e];
+        usage[e] = (float)h * inv;
+        if (!counts) continue;
+        atomicAdd(&counts[e], (unsigned long long)h);
+        if (h != kept[e]) atomicAdd(&counts[E], (unsigned long long)(h - kept[e]));
+    }
+}
+
 // Up to 8 experts (kept in registers): the kernel above reads and writes its gradients through memory once per term, a chain
 // of some twenty trips (512 tokens, 8 experts: 13.3 -> 7.6 us).  The same sums in the same order.  N, the experts that have
 // registers: work for absent ones shows (512 tokens, top 1, 2 experts 3.1 us above, 4.1 with N = 8, 2.0 with N = 2; 4 experts 3.9,
@@ -234,13 +248,13 @@ __global__ __launch_bounds__(64) void route_bwd_few_kernel(const float* __restri
                                                            const int32_t* __restrict__ idx, const float* __restrict__ w,
                                                            const float* __restrict__ dw, const float* __restrict__ usage,
                                                            float aux_scale, const float* __restrict__ aux_scale_dev,
-                                                           float inv_tau, int mode, float* __restrict__ dz, int64_t T, int E,
+                                                           const float* __restrict__ aux_value, float inv_tau, int mode, float* __restrict__ dz, int64_t T, int E,
                                                            int k) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= T) return;
     float z[N], za[N], us[N], out[N], wt[N], g[N];
     int it[N];
-    if (aux_scale_dev) aux_scale *= aux_scale_dev[0];
+    if (aux_scale_dev) aux_scale *= aux_value ? aux_scale_dev[0] * (aux_value[0] < 1.f ? 1.f : 0.f) : aux_scale_dev[0];
     const bool aux = usage && aux_scale != 0.f;
 #pragma unroll
     for (int e = 0; e < N; ++e) {
@@ -639,6 +653,14 @@ extern "C" int ats_route_bwd(const float* logits_route, const float* logits_aux,
                              const float* dw, const float* usage, float aux_scale, const float* aux_scale_dev,
                              float temperature, int mode, float* dlogits, int64_t T, int E, int k,
                              ats_stream_t stream) {
+    return ats_route_bwd_clamped(logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, nullptr, temperature, mode,
+                                 dlogits, T, E, k, stream);
+}
+
+extern "C" int ats_route_bwd_clamped(const float* logits_route, const float* logits_aux, const int32_t* idx, const float* w,
+                                     const float* dw, const float* usage, float aux_scale, const float* aux_scale_dev,
+                                     const float* aux_value, float temperature, int mode, float* dlogits, int64_t T, int E, int k,
+                                     ats_stream_t stream) {
     using namespace ats;
     ATS_REQUIRE(T >= 0 && E > 0 && k > 0 && k <= E && temperature > 0.f && (mode == 0 || mode == 1),
                 ATS_ERR_INVALID_ARG, "ats_route_bwd: T=%lld E=%d k=%d temperature=%g mode=%d", (long long)T, E, k,
@@ -650,13 +672,25 @@ extern "C" int ats_route_bwd(const float* logits_route, const float* logits_aux,
         auto kern = E <= 1 ? route_bwd_few_kernel<1> : E <= 2 ? route_bwd_few_kernel<2> : E <= 4 ? route_bwd_few_kernel<4>
                                                                                                 : route_bwd_few_kernel<8>;
         hipLaunchKernelGGL(kern, dim3((unsigned)((T + 63) / 64)), dim3(64), 0, as_stream(stream),
-                           logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, 1.0f / temperature, mode,
+                           logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, aux_value, 1.0f / temperature, mode,
                            dlogits, T, E, k);
     } else
         hipLaunchKernelGGL(route_bwd_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, as_stream(stream),
-                           logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, 1.0f / temperature, mode,
+                           logits_route, logits_aux, idx, w, dw, usage, aux_scale, aux_scale_dev, aux_value, 1.0f / temperature, mode,
                            dlogits, T, E, k);
     ATS_CHECK_LAUNCH("ats_route_bwd");
+    return ATS_OK;
+}
+
+extern "C" int ats_routing_counts(const int32_t* hist, const int32_t* kept, int E, int64_t assignments, float* usage, int64_t* counts,
+                                  ats_stream_t stream) {
+    using namespace ats;
+    ATS_REQUIRE(E > 0 && hist && usage && (!counts || kept), ATS_ERR_INVALID_ARG, "ats_routing_counts: E=%d, or a null pointer", E);
+    // (the reciprocal of the float32 divisor, as torch divides by a number)
+    const float inv = 1.0f / (float)((double)assignments + 1e-9);
+    hipLaunchKernelGGL(routing_counts_kernel, dim3(1), dim3(256), 0, as_stream(stream), hist, kept, E, inv, usage,
+                       reinterpret_cast<unsigned long long*>(counts));
+    ATS_CHECK_LAUNCH("ats_routing_counts");
     return ATS_OK;
 }
 

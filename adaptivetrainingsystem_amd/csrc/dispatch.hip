@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const TY* __restrict__ y, 
         float my_w = 0.f;
         if (lane < k) {
             my_row = row_of[t * k + lane];
-            my_w = w[t * k + lane];
+            my_w = w ? w[t * k + lane] : 1.f;      // (null: ats_gather_sum)
         }
         // position of this lane's row among the kept rows of the token
         int my_rank = 0;
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const TY* __restrict__
         float my_w = 0.f;
         if (lane < k) {
             my_row = row_of[t * k + lane];
-            my_w = w[t * k + lane];
+            my_w = w ? w[t * k + lane] : 1.f;      // (null: ats_gather_sum)
         }
         // the source lanes below are the same for the whole wave: scalar reads, no shuffles through LDS
         int my_rank = 0;
@@ -529,17 +529,16 @@ extern "C" int ats_sum_partials(const float* parts, int n_parts, int64_t part_st
     return ATS_OK;
 }
 
-extern "C" int ats_combine_partials(const float* parts, int n_parts, int64_t part_stride, const int32_t* row_of,
-                                    const float* w, const void* residual, void* out, int64_t T, int k, int H,
-                                    int out_dtype, ats_stream_t stream) {
+static int combine_partials(const char* name, const float* parts, int n_parts, int64_t part_stride, const int32_t* row_of,
+                            const float* w, const void* residual, void* out, int64_t T, int k, int H, int out_dtype,
+                            ats_stream_t stream) {
     using namespace ats;
-    const char* name = "ats_combine_partials";
     ATS_REQUIRE(T >= 0 && k > 0 && k <= 8 && H > 0 && H % 8 == 0 && n_parts >= 1 && part_stride % 4 == 0,
                 ATS_ERR_INVALID_ARG, "%s: T=%lld k=%d (<= 8) H=%d (multiple of 8) n_parts=%d part_stride=%lld", name,
                 (long long)T, k, H, n_parts, (long long)part_stride);
     ATS_REQUIRE(out_dtype == ATS_F32 || out_dtype == ATS_BF16, ATS_ERR_UNSUPPORTED, "%s: dtype tag %d", name, out_dtype);
     if (T == 0) return ATS_OK;
-    ATS_REQUIRE(parts && row_of && w && out && aligned16(parts) && aligned16(out) && (!residual || aligned16(residual)),
+    ATS_REQUIRE(parts && row_of && out && aligned16(parts) && aligned16(out) && (!residual || aligned16(residual)),
                 ATS_ERR_INVALID_ARG, "%s: null or misaligned pointer", name);
     const int cols = combine_cols_per_wave(T, H);
     int64_t blocks = (T * ((H + cols - 1) / cols) + 3) / 4;
@@ -561,6 +560,19 @@ extern "C" int ats_combine_partials(const float* parts, int n_parts, int64_t par
 #undef ATS_COMBINE_PARTS
     ATS_CHECK_LAUNCH(name);
     return ATS_OK;
+}
+
+extern "C" int ats_combine_partials(const float* parts, int n_parts, int64_t part_stride, const int32_t* row_of,
+                                    const float* w, const void* residual, void* out, int64_t T, int k, int H,
+                                    int out_dtype, ats_stream_t stream) {
+    ATS_REQUIRE(w || T == 0, ATS_ERR_INVALID_ARG, "ats_combine_partials: null or misaligned pointer");
+    return combine_partials("ats_combine_partials", parts, n_parts, part_stride, row_of, w, residual, out, T, k, H, out_dtype, stream);
+}
+
+extern "C" int ats_gather_sum_partials(const float* parts, int n_parts, int64_t part_stride, const int32_t* row_of, void* out, int64_t T,
+                                       int k, int H, int out_dtype, ats_stream_t stream) {
+    return combine_partials("ats_gather_sum_partials", parts, n_parts, part_stride, row_of, nullptr, nullptr, out, T, k, H, out_dtype,
+                            stream);
 }
 
 extern "C" size_t ats_dispatch_plan_workspace(int64_t T, int k, int E) {
@@ -776,15 +788,15 @@ extern "C" int ats_combine_scatter_add(const void* y, const int32_t* row_of, con
     return ATS_OK;
 }
 
-extern "C" int ats_combine(const void* y, const int32_t* row_of, const float* w, const void* residual, void* out,
-                           int64_t T, int k, int H, int y_dtype, int out_dtype, ats_stream_t stream) {
+static int combine_rows(const char* name, const void* y, const int32_t* row_of, const float* w, const void* residual, void* out,
+                        int64_t T, int k, int H, int y_dtype, int out_dtype, ats_stream_t stream) {
     using namespace ats;
-    ATS_REQUIRE(T >= 0 && k > 0 && k <= 64 && H > 0, ATS_ERR_INVALID_ARG, "ats_combine: T=%lld k=%d H=%d",
+    ATS_REQUIRE(T >= 0 && k > 0 && k <= 64 && H > 0, ATS_ERR_INVALID_ARG, "%s: T=%lld k=%d H=%d", name,
                 (long long)T, k, H);
     ATS_REQUIRE((y_dtype == ATS_F32 || y_dtype == ATS_BF16) && (out_dtype == ATS_F32 || out_dtype == ATS_BF16),
-                ATS_ERR_UNSUPPORTED, "ats_combine: dtype tags %d/%d", y_dtype, out_dtype);
+                ATS_ERR_UNSUPPORTED, "%s: dtype tags %d/%d", name, y_dtype, out_dtype);
     if (T == 0) return ATS_OK;
-    ATS_REQUIRE(y && row_of && w && out, ATS_ERR_INVALID_ARG, "ats_combine: null pointer");
+    ATS_REQUIRE(y && row_of && out, ATS_ERR_INVALID_ARG, "%s: null pointer", name);
     hipStream_t s = as_stream(stream);
     if (y_dtype == ATS_F32 && out_dtype == ATS_F32) launch_combine<float, float>(y, row_of, w, residual, out, T, k, H, s);
     else if (y_dtype == ATS_BF16 && out_dtype == ATS_BF16)
@@ -793,6 +805,17 @@ extern "C" int ats_combine(const void* y, const int32_t* row_of, const float* w,
         launch_combine<float, bf16_t>(y, row_of, w, residual, out, T, k, H, s);
     else
         launch_combine<bf16_t, float>(y, row_of, w, residual, out, T, k, H, s);
-    ATS_CHECK_LAUNCH("ats_combine");
+    ATS_CHECK_LAUNCH(name);
     return ATS_OK;
+}
+
+extern "C" int ats_combine(const void* y, const int32_t* row_of, const float* w, const void* residual, void* out,
+                           int64_t T, int k, int H, int y_dtype, int out_dtype, ats_stream_t stream) {
+    ATS_REQUIRE(w || T == 0, ATS_ERR_INVALID_ARG, "ats_combine: null pointer");
+    return combine_rows("ats_combine", y, row_of, w, residual, out, T, k, H, y_dtype, out_dtype, stream);
+}
+
+extern "C" int ats_gather_sum(const void* y, const int32_t* row_of, void* out, int64_t T, int k, int H, int y_dtype, int out_dtype,
+                              ats_stream_t stream) {
+    return combine_rows("ats_gather_sum", y, row_of, nullptr, nullptr, out, T, k, H, y_dtype, out_dtype, stream);
 }

@@ -235,6 +235,21 @@ def route_topk(logits: torch.Tensor, k: int, temperature: float = 1.0, variant: 
     return {"indices": idx, "weights": w, "hist": hist, "prob_colsum": colsum, "aux": aux}
 
 
+def routing_counts(hist: torch.Tensor, kept: torch.Tensor, assignments: int, counts: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """float32 [E] share of the assignments that each expert was chosen for; with counts (int64 [E + 1]) hist is added to its
+    first E and the number of dropped assignments to its last element."""
+    _need_gpu(hist, kept, counts)
+    E = hist.numel()
+    if hist.dtype != torch.int32 or kept.dtype != torch.int32 or kept.numel() != E:
+        raise AtsError("routing_counts: hist and kept must be int32 of one size")
+    if counts is not None and (counts.dtype != torch.int64 or counts.numel() != E + 1 or not counts.is_contiguous()):
+        raise AtsError("routing_counts: counts must be contiguous int64 [experts + 1]")
+    usage = torch.empty(E, dtype=torch.float32, device=hist.device)
+    check(_lib.load().ats_routing_counts(hist.contiguous().data_ptr(), kept.contiguous().data_ptr(), E, int(assignments),
+                                         usage.data_ptr(), _ptr(counts), _stream()), "ats_routing_counts")
+    return usage
+
+
 def aux_loss_clean_logits(clean_logits: torch.Tensor, hist: torch.Tensor, k: int, variant: int,
                           load_balancing_weight: float) -> torch.Tensor:
     """Load-balancing loss when routing ran on noisy logits: usage from the routed histogram, importance from
@@ -655,6 +670,27 @@ def sum_partials(parts: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
 
 
 # --------------------------------------------------------------------------- combine
+def gather_sum(y: torch.Tensor, row_of: torch.Tensor, num_tokens: int, k: int, out_dtype: torch.dtype) -> torch.Tensor:
+    """combine with every weight 1: y [rows, H], or float32 partial results [slices, rows, H] as in combine_partials
+    (k <= 8, H % 8 == 0)."""
+    _need_gpu(y, row_of)
+    if row_of.dtype != torch.int32 or row_of.numel() != num_tokens * k or y.dim() not in (2, 3):
+        raise AtsError("gather_sum: y [rows, H] or [slices, rows, H], row_of int32 with tokens*k entries")
+    if y.dim() == 3 and (y.dtype != torch.float32 or not y.is_contiguous()):
+        raise AtsError("gather_sum: partial results must be a contiguous float32 [slices, rows, H] tensor")
+    H = y.shape[-1]
+    out = torch.empty(num_tokens, H, dtype=out_dtype, device=y.device)
+    row_of = row_of.contiguous()
+    if y.dim() == 3:
+        check(_lib.load().ats_gather_sum_partials(y.data_ptr(), y.shape[0], y.shape[1] * H, row_of.data_ptr(), out.data_ptr(), num_tokens,
+                                                  int(k), H, _tag(out), _stream()), "ats_gather_sum_partials")
+    else:
+        y = y.contiguous()
+        check(_lib.load().ats_gather_sum(y.data_ptr(), row_of.data_ptr(), out.data_ptr(), num_tokens, int(k), H, _tag(y), _tag(out),
+                                         _stream()), "ats_gather_sum")
+    return out
+
+
 def combine(y: torch.Tensor, row_of: torch.Tensor, weights: torch.Tensor, num_tokens: int, k: int,
             out_dtype: Optional[torch.dtype] = None, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y [rows, H] (any leading shape); row_of int32 [T*k]; weights f32 [T,k] -> out [T,H]."""
@@ -1000,10 +1036,13 @@ def combine_bwd(dout: torch.Tensor, y: torch.Tensor, token_map: torch.Tensor, w:
 def route_bwd(logits_route: torch.Tensor, idx: torch.Tensor, w: torch.Tensor, dw: torch.Tensor,
               temperature: float = 1.0, mode: int = ROUTE_SOFTMAX_TOPK, logits_aux: Optional[torch.Tensor] = None,
               usage: Optional[torch.Tensor] = None, aux_scale: float = 0.0,
-              aux_scale_dev: Optional[torch.Tensor] = None) -> torch.Tensor:
+              aux_scale_dev: Optional[torch.Tensor] = None, aux_value: Optional[torch.Tensor] = None) -> torch.Tensor:
     """dlogits [T,E] float32 of the routing rule (and of the load-balancing loss when usage is given;
-    its factor is aux_scale times the optional float32 device scalar aux_scale_dev)."""
-    _need_gpu(logits_route, idx, w, dw, logits_aux, usage, aux_scale_dev)
+    its factor is aux_scale times the optional float32 device scalar aux_scale_dev, which counts as 0 unless the optional
+    float32 device scalar aux_value is below 1)."""
+    _need_gpu(logits_route, idx, w, dw, logits_aux, usage, aux_scale_dev, aux_value)
+    if aux_value is not None and (aux_value.dtype != torch.float32 or aux_value.numel() != 1):
+        raise AtsError("route_bwd: aux_value must be a float32 scalar tensor")
     if aux_scale_dev is not None and (aux_scale_dev.dtype != torch.float32 or aux_scale_dev.numel() != 1):
         raise AtsError("route_bwd: aux_scale_dev must be a float32 scalar tensor")
     T, E = logits_route.shape
@@ -1016,10 +1055,10 @@ def route_bwd(logits_route: torch.Tensor, idx: torch.Tensor, w: torch.Tensor, dw
         usage = usage.contiguous().float()
         logits_aux = (logits_route if logits_aux is None else logits_aux).contiguous()
     out = torch.empty(T, E, dtype=torch.float32, device=logits_route.device)
-    check(_lib.load().ats_route_bwd(logits_route.data_ptr(), _ptr(logits_aux), idx.data_ptr(), w.data_ptr(),
-                                    dw.data_ptr(), _ptr(usage), float(aux_scale), _ptr(aux_scale_dev),
-                                    float(temperature), int(mode), out.data_ptr(), T, E, k, _stream()),
-          "ats_route_bwd")
+    check(_lib.load().ats_route_bwd_clamped(logits_route.data_ptr(), _ptr(logits_aux), idx.data_ptr(), w.data_ptr(),
+                                            dw.data_ptr(), _ptr(usage), float(aux_scale), _ptr(aux_scale_dev), _ptr(aux_value),
+                                            float(temperature), int(mode), out.data_ptr(), T, E, k, _stream()),
+          "ats_route_bwd_clamped")
     return out
 
 

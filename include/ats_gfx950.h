@@ -268,6 +268,9 @@ int ats_sum_partials(const float* parts, int n_parts, int64_t part_stride, void*
  * If residual != NULL, out[t,:] = residual[t,:] + that sum. */
 int ats_combine(const void* y, const int32_t* row_of, const float* w, const void* residual,
                 void* out, int64_t T, int k, int H, int y_dtype, int out_dtype, ats_stream_t stream);
+/* ats_combine with every weight 1 and no residual (the gradient of the gather of the experts' rows). */
+int ats_gather_sum(const void* y, const int32_t* row_of, void* out, int64_t T, int k, int H, int y_dtype, int out_dtype,
+                   ats_stream_t stream);
 /* ats_combine whose token-major result is added onto rows of a larger tensor instead of being stored:
  * out[out_rows[t], :] += round(sum_j w[t,j] * y[row_of[t*k+j], :]) for out_rows[t] >= 0 (distinct rows), the
  * sum rounded to out_dtype first as the stored result would be; the bits of ats_combine followed by
@@ -281,6 +284,9 @@ int ats_combine_scatter_add(const void* y, const int32_t* row_of, const float* w
 int ats_combine_partials(const float* parts, int n_parts, int64_t part_stride, const int32_t* row_of,
                          const float* w, const void* residual, void* out, int64_t T, int k, int H,
                          int out_dtype, ats_stream_t stream);
+/* The same with every weight 1 and no residual. */
+int ats_gather_sum_partials(const float* parts, int n_parts, int64_t part_stride, const int32_t* row_of, void* out, int64_t T,
+                            int k, int H, int out_dtype, ats_stream_t stream);
 
 /* ---- The whole layer, inference -------------------------------------------
  * ats_router_logits, ats_route_topk, ats_dispatch_plan, ats_grouped_gateup_swiglu, ats_grouped_down and
@@ -412,6 +418,15 @@ int ats_route_bwd(const float* logits_route, const float* logits_aux, const int3
                   const float* dw, const float* usage, float aux_scale, const float* aux_scale_dev,
                   float temperature, int mode, float* dlogits, int64_t T, int E, int k,
                   ats_stream_t stream);
+/* ats_route_bwd with the clamp of the loss (model.py:1263): aux_value (optional) is the loss of the forward, *aux_scale_dev counts as 0
+ * unless *aux_value < 1. */
+int ats_route_bwd_clamped(const float* logits_route, const float* logits_aux, const int32_t* idx, const float* w, const float* dw,
+                          const float* usage, float aux_scale, const float* aux_scale_dev, const float* aux_value, float temperature,
+                          int mode, float* dlogits, int64_t T, int E, int k, ats_stream_t stream);
+/* usage[e] = hist[e] / (assignments + 1e-9) in float32 (model.py:1244-1263); with counts [E + 1] (optional, needs kept) hist[e] is added
+ * to counts[e] and the assignments that were not kept to counts[E] (integer atomics). */
+int ats_routing_counts(const int32_t* hist, const int32_t* kept, int E, int64_t assignments, float* usage, int64_t* counts,
+                       ats_stream_t stream);
 /* Gradient of ats_router_logits: out[t,:] = base[t,:] + dlogits[t,:] . Wg (base NULL or == out),
  * dWg[e,:] = sum_t dlogits[t,e] * x[t,:] (float32, fixed order). */
 int ats_router_bwd_dx(const float* dlogits, const void* wg, const void* base, void* out, int64_t T, int E,
