@@ -1536,6 +1536,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
 }  // namespace ats
 
 #include "grouped_gemm_short.hpp"
+#include "grouped_gemm_band.hpp"
 
 namespace ats {
 
@@ -1559,7 +1560,7 @@ static int64_t busiest_cu(int64_t m_tiles, int n_tiles, int sm, int sn) {
     return (most + kSuperBlocks - 1) / kSuperBlocks;
 }
 
-// Tile height of a bfloat16 launch with one group (its row count is exact), 0 for the full 256 rows.  An XCD takes whole
+// Tile height of a bfloat16 launch with one group (its row count is exact) on the 256-row tile, 0 for the full 256 rows.  An XCD takes whole
 // supertiles of 32 tiles and its 32 CUs hold one tile each, so a launch lasts as many rounds as there are supertiles per XCD,
 // and lower tiles pay where they turn a round that is mostly empty into work for all CUs (4524 x [11008, 2048]: 240 rows in four
 // rounds 174 us, 144 rows in six 215).  Microseconds per 64-element slab by height: medians over 415
@@ -1569,7 +1570,7 @@ static int64_t busiest_cu(int64_t m_tiles, int n_tiles, int sm, int sn) {
 // 3000 x [4096, 4096] 95 -> 76 -> 74, 1500 x [4096, 4096] 78 -> 58 -> 56, 1000 x [6144, 4096] 93 -> 57 -> 56; 2048 x [6144, 4096]
 // stays (92; 128 rows 113).  Weights stored [K][N] take the same heights: 1000 x [4096, 4096] 90 -> 55, 300 x 55 -> 49, 5331 x
 // 176 -> 136, x [6144, 4096] 238 -> 202, 2048 x [2048, 2048] 50 -> 32.  Sums over K are in the same order.
-static int dense_tile_rows(int64_t rows, int n_tiles, int k_slabs, int sm, int sn) {
+static int dense_tile_rows(int64_t rows, int n_tiles, int k_slabs, int sm, int sn, float* time = nullptr) {
     float best = 0.f;
     int best_rows = 0;
     constexpr float kPerSlab[] = {0.75f, 0.86f, 0.94f, 1.00f, 1.07f, 1.15f, 1.23f, 1.28f, 1.35f};     // 128, 144, .. 256 rows
@@ -1583,6 +1584,7 @@ static int dense_tile_rows(int64_t rows, int n_tiles, int k_slabs, int sm, int s
             best_rows = h == 256 ? 0 : h;
         }
     }
+    if (time) *time = best;
     return best_rows;
 }
 
@@ -1835,12 +1837,64 @@ static bool large_slice_tile(int E, int64_t max_rows, int N, int K, int s) {
     return t.large_with_margin(s) < t.small(s);
 }
 
+// The band tiles (grouped_gemm_band.hpp) for E > 1 groups.  They lose where a group needs a second tile while the first ones fill no
+// more than one round of the chip (8 x [4096, 14336] in two slices, unequal groups of 72 rows 189 -> 230 us, of 56 rows 181 -> 164), and
+// among many workgroups where most groups do (64 x [2816, 2048], 96 rows each 176 -> 143, 128 rows 169 -> 180); with a few rows per
+// group the weight streams' narrower panels leave fewer CUs idle (16 x [2048, 5632], 16 rows in all 44 -> 52, 32 rows 60 -> 53; 64 x
+// [2048, 1408], 6 rows 11 -> 14, 18 rows 19 -> 16) and their gate/up launch is the faster one up to about twelve rows per group
+// (64 x [2816, 2048], 4 rows each 107 -> 111, 12 rows 114 -> 114, 16 rows 122 -> 115).
+static bool band_groups(int E, int64_t max_rows, int n_tiles, int slices, bool swiglu) {
+    const int64_t avg = max_rows / E;
+    if (avg > ((int64_t)E * n_tiles >= 512 ? 100 : 72)) return false;
+    if (swiglu) return avg >= 12 && (int64_t)E * n_tiles >= 256;
+    const float used = E * (1.f - expf(-(float)max_rows / E));      // groups that get rows, if these fall at random
+    return used * n_tiles * slices >= 200.f;
+}
+// One group of more than 32 rows x [N, K]: the band tiles' time in microseconds, plain or with s slices of K and their sum, by the
+// tiles' most rows h; 109 measured points of [2048 .. 6144] x [2048, 4096] within 8 % (root mean square), the choice between them costs
+// 2 % on average.  A CU takes one slab of a tile in slab1 alone and in slabn as one of several.
+static float band_time(int64_t rows, int N, int K, int s, int h) {
+    constexpr float slab1[] = {0.40f, 0.44f, 0.53f, 0.63f}, slabn[] = {0.30f, 0.36f, 0.42f, 0.49f};      // 32, 64, 96, 128 rows
+    const int64_t m_tiles = (rows + h - 1) / h;
+    const int f = (int)((rows + m_tiles - 1) / m_tiles + 31) / 32 - 1;
+    const float per_cu = (float)(m_tiles * ((N + kBandCols - 1) / kBandCols) * s) / 256.f;
+    const float slab = per_cu <= 1.f ? slab1[f] : slabn[f] * 0.5f * (per_cu + ceilf(per_cu));
+    const float chain = K / 64.f / s * slab, weights = (float)N * K * 2e-6f / 7.f;
+    return 5.f + sqrtf(chain * chain + weights * weights) + (s > 1 ? (float)rows * N * (8 * s - 4) / 4.5e6f + 3.f : 0.f);
+}
+static int band_height(int64_t rows, int N, int K, int s) {
+    return rows > 64 && band_time(rows, N, K, s, 128) < band_time(rows, N, K, s, 64) ? 128 : 64;
+}
+// The same rows on the other tiles: half a chip of 64 x 64 tiles with K split in the workgroup ([2048, 2048] x 128 rows 10.4 us, [4096,
+// 4096] 20.8; with more of them 38: [6144, 4096]) or the 256-column tiles (10 % off).
+static float other_dense_time(int64_t rows, int N, int K, bool small) {
+    float best;
+    int sm, sn;
+    const int n_tiles = (N + 255) / 256;
+    pick_supertile(n_tiles, &sm, &sn);
+    dense_tile_rows(rows, n_tiles, K / 64, sm, sn, &best);
+    if (small && (rows + 63) / 64 * ((N + 63) / 64) <= 128) best = fminf(best, 2.f + K / 64 * 0.28f);
+    return best;
+}
+static bool band_dense(int64_t rows, int N, int K) {
+    return rows > 32 && band_time(rows, N, K, 1, band_height(rows, N, K, 1)) < other_dense_time(rows, N, K, true);
+}
+
 template <typename T, typename TO, bool SWIGLU>
 static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s) {
     constexpr bool kBf16 = std::is_same<T, bf16_t>::value;
     constexpr int BK = 128 / (int)sizeof(T);
     const int E = p.E > 0 ? p.E : 1;
     const int64_t avg = max_rows / E;
+    // (the band tiles address their operands with 32-bit lane offsets; slices of small weights, which come from the last-level cache,
+    // keep the register-staged tiles)
+    const bool band_ok = kBf16 && !p.k_count && p.K % 64 == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0;
+    const int band_tiles = (p.N_out + (SWIGLU ? kBandCols / 2 : kBandCols) - 1) / (SWIGLU ? kBandCols / 2 : kBandCols);
+    if constexpr (kBf16 && !SWIGLU && std::is_same<TO, float>::value) {
+        if (p.k_splits > 1 && band_ok && p.k_slice % 64 == 0 &&
+            (E == 1 ? max_rows > 32 : (int64_t)E * p.N_out * p.K >= 1 << 24 && avg > 20 && band_groups(E, max_rows, band_tiles, p.k_splits, false)))
+            return launch_band<TO, false, true>(p, max_rows, E == 1 ? band_height(max_rows, p.N_out, p.K, p.k_splits) : kBandRows, s);
+    }
     if constexpr (!SWIGLU) {
         // K in slices over workgroups: 32-row tiles, 64-row tiles where up to 64 rows can stream the weights once
         if (p.k_splits > 1) {
@@ -1851,6 +1905,13 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
             }
             return avg > 32 ? launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s)
                             : launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+        }
+    }
+    if constexpr (kBf16) {
+        if (band_ok && E > 1 && band_groups(E, max_rows, band_tiles, 1, SWIGLU)) return launch_band<TO, SWIGLU, false>(p, max_rows, kBandRows, s);
+        if constexpr (!SWIGLU) {
+            if (band_ok && E == 1 && band_dense(max_rows, p.N_out, p.K))
+                return launch_band<TO, false, false>(p, max_rows, band_height(max_rows, p.N_out, p.K, 1), s);
         }
     }
     // (with a K per group, p.K is the bound on their sum)
@@ -2365,6 +2426,24 @@ extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K, int smal
     for (int s = 2; s <= 16 && K % (s * 64) == 0 && K / s >= 512; s *= 2) {
         if (t.large_with_margin(s) < best && large_slice_tile(E, max_rows, N, K, s)) {
             best = t.large_with_margin(s);
+            slices = s;
+        }
+    }
+    return slices;
+}
+
+// Slices of K of a bfloat16 linear layer (1: plain), by the estimated times.
+extern "C" int ats_linear_k_slices(int64_t rows, int N, int K) {
+    using namespace ats;
+    if (rows <= 32 || rows > 256 || N <= 0 || K <= 0 || K % 64 != 0) return 1;
+    // (against a long K slices on the band tiles are as fast as the small tiles: [4096, 4096] x 100 rows 19 and 20 us, 128 rows 22 and 21;
+    // and a rotation behind the product adds them up on its way)
+    float best = fminf(band_time(rows, N, K, 1, band_height(rows, N, K, 1)), other_dense_time(rows, N, K, K <= 2048));
+    int slices = 1;
+    for (int s = 2; s <= 8 && K % (s * 64) == 0 && K / s >= 256; s *= 2) {
+        const float t = band_time(rows, N, K, s, band_height(rows, N, K, s));
+        if (t < best) {
+            best = t;
             slices = s;
         }
     }

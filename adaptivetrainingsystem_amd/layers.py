@@ -466,7 +466,7 @@ class SwiGLUExpert(nn.Module):
         start = torch.zeros(1, dtype=torch.int32, device=x.device)
         count = torch.full((1,), n, dtype=torch.int32, device=x.device)
         h = ops.grouped_gateup_swiglu(x2, ops.weight_pointer_table([wgu]), start, count, n, n, H, I)
-        splits = ops.down_k_splits(1, n, H, I, x2.dtype) if H % 8 == 0 and n > 32 else 1
+        splits = ops.linear_k_splits(n, H, I, x2.dtype)
         if splits > 1:       # a few rows: slices of K keep every CU streaming the down weights
             y = ops.sum_partials(ops.grouped_down_splitk(h, ops.weight_pointer_table([wd]), start, count, n, H, I,
                                                          splits), x2.dtype)

@@ -8,6 +8,7 @@ GPU; there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from array import array
 from typing import Optional, Sequence, Tuple
@@ -1361,7 +1362,7 @@ def prompt_attention_supported(x: torch.Tensor, weight: torch.Tensor, B: int, L:
     in slices of K has its rotation in the sum of the slices."""
     return (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == x.dtype
             and bool(_lib.load().ats_attention_fwd_rope_supported(B, Hq, Hkv, L, L, D))
-            and _linear_slices(B * L, weight.shape[0], x.shape[1], x.dtype) == 1)
+            and linear_k_splits(B * L, weight.shape[0], x.shape[1], x.dtype) == 1)
 
 
 def prompt_attention(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, B: int, Hkv: int, D: int, scale: float,
@@ -1616,11 +1617,16 @@ def _single_group(T: int, device: torch.device):
     return pair
 
 
-def _linear_slices(T: int, N: int, K: int, dtype: torch.dtype) -> int:
-    # 33-256 rows against a long K: slices of K over workgroups.  Up to 32 rows the plain launch streams the weights itself
-    # ([4096, 4096] x 16 rows: 10.3 us against 14.2 with the slices and their sum), and a short K leaves its small tiles
-    # less to do than the sum costs ([2048, 2048] x 64 rows: 8.8 against 11.3).
-    return down_k_splits(1, T, N, K, dtype) if T > 32 and K * dtype.itemsize > 4096 and K % 8 == 0 and N % 8 == 0 else 1
+@functools.lru_cache(maxsize=4096)
+def linear_k_splits(T: int, N: int, K: int, dtype: torch.dtype) -> int:
+    """Slices of K for a product with one weight [N, K].  33-256 rows only: bfloat16 by the estimated times of every route,
+    float32 against a long K.  Up to 32 rows the plain launch streams the weights itself ([4096, 4096] x 16 rows: 10.3 us against
+    14.2 with the slices and their sum)."""
+    if not 32 < T <= 256 or K % 8 or N % 8:
+        return 1
+    if dtype == torch.bfloat16:
+        return _lib.load().ats_linear_k_slices(T, N, K)
+    return down_k_splits(1, T, N, K, dtype) if K * dtype.itemsize > 4096 else 1
 
 
 def linear_rope_append(x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor,
@@ -1634,7 +1640,7 @@ def linear_rope_append(x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor,
                        f"{tuple(k_cache.shape)} / {tuple(v_cache.shape)}")
     T, K = x.shape
     N, D = weight.shape[0], k_cache.shape[3]
-    splits = _linear_slices(T, N, K, x.dtype)
+    splits = linear_k_splits(T, N, K, x.dtype)
     if splits == 1 or not x.is_cuda or weight.dtype != x.dtype or not weight.is_contiguous():
         return None
     start, count = _single_group(T, x.device)
@@ -1654,7 +1660,7 @@ def linear_nt(x: torch.Tensor, weight: torch.Tensor, table: Optional[torch.Tenso
     if table is None:
         table = weight_pointer_table([weight])
     start, count = _single_group(T, x.device)
-    splits = _linear_slices(T, N, K, x.dtype)
+    splits = linear_k_splits(T, N, K, x.dtype)
     done = _lib.native().linear(x, table, start, count, N, splits)
     if done is not None:
         return done

@@ -254,6 +254,9 @@ int ats_grouped_down_splitk(const void* h, const void* const* w_d, float* parts,
  * weights or more is estimated to take the least time, ats_combine_partials included; 1: ats_grouped_down.  small: the slices with
  * which 32 or 64-row tiles fill the chip. */
 int ats_down_k_slices(int E, int64_t max_rows, int H, int I, int small);
+/* Slices of K with which ats_grouped_down_splitk and ats_sum_partials multiply `rows` rows by one bfloat16 [N, K] weight
+ * fastest; 1: ats_linear_nt does. */
+int ats_linear_k_slices(int64_t rows, int N, int K);
 /* out[i] = sum_s parts[s*part_stride + i], i < n, added in slice order in float32 and rounded once
  * to out_dtype (n and part_stride multiples of 4). */
 int ats_sum_partials(const float* parts, int n_parts, int64_t part_stride, void* out, int64_t n,

@@ -1,0 +1,114 @@
+"""Grouped products of groups with some dozens of rows, and of one group with up to a few hundred, on the band tiles (GPU).
+
+Bound: a result is a float32 sum of K products of bfloat16 operands, at most K * 2^-24 * sum |a||w| off (the SwiGLU epilogue's
+factor is below 1.1 |u| with unit-sized g), and rounded once to bfloat16 (2^-8 of its value); float32 results only have the first.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs an MI355X")
+    return torch.device("cuda")
+
+
+def _groups(counts, N, K, ldb, seed):
+    g = torch.Generator().manual_seed(seed)
+    w = [(torch.randn(N, ldb, generator=g) * 0.05).bfloat16() for _ in counts]
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    return g, w, off
+
+
+def _device(counts, off, gpu):
+    return torch.tensor(off[:-1], device=gpu), torch.tensor(counts, dtype=torch.int32, device=gpu)
+
+
+def _check(got, ref, mag, K, rounded=True):
+    bound = K * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if rounded else 0) + 1e-30
+    assert ((got.double().cpu() - ref).abs() <= bound).all()
+
+
+# heights of 32, 64, 96 and 128 rows and their edges, groups of two tiles, without rows; one, two and more slabs; a ragged N
+@pytest.mark.parametrize("counts,N,K", [([31, 32, 33, 0, 64, 65] * 7, 1000, 64), ([96, 97, 127, 1] * 10, 1032, 128), ([128, 129, 0, 2] * 16, 1032, 192),
+                                        ([1, 2, 0, 3] * 16, 1096, 448), ([40] * 63 + [400], 1024, 320)])
+@pytest.mark.parametrize("gather", [False, True])
+def test_groups(gpu, counts, N, K, gather):
+    from adaptivetrainingsystem_amd import ops
+    print("case band groups", len(counts), N, K, gather, flush=True)
+    ldb = K + 8
+    g, w, off = _groups(counts, N, K, ldb, N + K)
+    n = int(off[-1])
+    a = torch.randn(n, K + 16, generator=g).bfloat16()
+    idx = torch.randint(0, 2 * n, (n,), generator=g, dtype=torch.int32) if gather else None
+    start, count = _device(counts, off, gpu)
+    wd = [t.to(gpu) for t in w]
+    ptrs = torch.tensor([t.data_ptr() for t in wd], device=gpu)
+    got = ops.grouped_gemm_nt(ptrs, ldb, N, start, count, n, n, N, K, a=a.to(gpu)[:, :K], lda=K + 16, a_rows=None if idx is None else idx.to(gpu),
+                              a_row_div=2)
+    rows = a[:, :K].double() if idx is None else a[:, :K].double()[(idx // 2).long()]
+    for e in range(len(counts)):
+        s = slice(off[e], off[e + 1])
+        _check(got[s], rows[s] @ w[e][:, :K].double().T, rows[s].abs() @ w[e][:, :K].double().abs().T, K)
+
+
+@pytest.mark.parametrize("counts,I,K", [([31, 33, 64, 0, 65] * 4, 1000, 64), ([97, 128, 1, 96] * 4, 1032, 192), ([12, 129, 0, 20] * 8, 1096, 576)])
+def test_gate_up(gpu, counts, I, K):
+    from adaptivetrainingsystem_amd import ops
+    print("case band gate/up", len(counts), I, K, flush=True)
+    g, w, off = _groups(counts, 2 * I, K, K, I + K)
+    n = int(off[-1])
+    x = torch.randn(n // 2 + 1, K, generator=g).bfloat16()
+    idx = torch.randint(0, n, (n,), generator=g, dtype=torch.int32)
+    start, count = _device(counts, off, gpu)
+    wd = [t.to(gpu) for t in w]
+    got = ops.grouped_gateup_swiglu(x.to(gpu), torch.tensor([t.data_ptr() for t in wd], device=gpu), start, count, n, n, K, I, a_rows=idx.to(gpu), a_row_div=2)
+    rows = x.double()[(idx // 2).long()]
+    for e in range(len(counts)):
+        s = slice(off[e], off[e + 1])
+        gu, mag = rows[s] @ w[e].double().T, rows[s].abs() @ w[e].double().abs().T
+        gate, up = gu[:, :I], gu[:, I:]
+        ref = gate * torch.sigmoid(gate) * up
+        # (the exponential and the division of the sigmoid: 2^-20 of the value)
+        _check(got[s], ref, 1.1 * mag[:, :I] * up.abs() + gate.abs() * mag[:, I:] + 2.0 ** 4 / K * ref.abs(), K)
+
+
+@pytest.mark.parametrize("T,N,K", [(33, 1032, 512), (64, 4096, 1024), (65, 1032, 4096), (96, 2056, 2048), (97, 1032, 1024), (128, 3072, 2048), (129, 2056, 1024),
+                                   (200, 1032, 2048), (256, 4104, 1024), (257, 2048, 512), (300, 2056, 64), (640, 1032, 1024), (1000, 2048, 2048)])
+def test_one_group(gpu, T, N, K):
+    """A linear layer, plain or in slices of K by the rule; with slices every slice as well."""
+    from adaptivetrainingsystem_amd import ops
+    print("case band one group", T, N, K, ops.linear_k_splits(T, N, K, torch.bfloat16), flush=True)
+    g = torch.Generator().manual_seed(T + N)
+    x, w = torch.randn(T, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * 0.05).bfloat16()
+    ref, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    xd, wd = x.to(gpu), w.to(gpu)
+    _check(ops.linear_nt(xd, wd), ref, mag, K)
+    if T <= 256:
+        start, count = torch.zeros(1, dtype=torch.int32, device=gpu), torch.full((1,), T, dtype=torch.int32, device=gpu)
+        for s in (2, 4):
+            parts = ops.grouped_down_splitk(xd, ops.weight_pointer_table([wd]), start, count, T, N, K, s)
+            for i in range(s):
+                k = slice(i * K // s, (i + 1) * K // s)
+                _check(parts[i], x[:, k].double() @ w[:, k].double().T, x[:, k].double().abs() @ w[:, k].double().abs().T, K // s, rounded=False)
+
+
+@pytest.mark.parametrize("counts,H,I,S", [([40, 30, 33, 0, 96, 1, 70, 128] * 2, 2056, 1024, 2), ([25, 64, 65, 129], 4104, 2048, 4)])
+def test_slices_of_groups(gpu, counts, H, I, S):
+    from adaptivetrainingsystem_amd import ops
+    print("case band slices", len(counts), H, I, S, flush=True)
+    g, w, off = _groups(counts, H, I, I, H + I)
+    n = int(off[-1])
+    h = torch.randn(n, I, generator=g).bfloat16()
+    start, count = _device(counts, off, gpu)
+    wd = [t.to(gpu) for t in w]
+    parts = ops.grouped_down_splitk(h.to(gpu), torch.tensor([t.data_ptr() for t in wd], device=gpu), start, count, n, H, I, S)
+    for i in range(S):
+        k = slice(i * I // S, (i + 1) * I // S)
+        for e in range(len(counts)):
+            s = slice(off[e], off[e + 1])
+            _check(parts[i][s], h[s, k].double() @ w[e][:, k].double().T, h[s, k].double().abs() @ w[e][:, k].double().abs().T, I // S, rounded=False)
