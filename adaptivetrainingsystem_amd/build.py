@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(PKG_DIR, "csrc")
@@ -64,25 +65,31 @@ def build_library(verbose: bool = True, jobs: int = 6) -> str:
     os.makedirs(obj_dir, exist_ok=True)
     compile_flags = [f for f in HIPCC_FLAGS if f != "-shared"]
     procs, objs = [], []
+
+    def start(cmd):     # (output to a file: a compiler with much to say would wait for a reader of its pipe, and this waits for it)
+        log = tempfile.TemporaryFile("w+", errors="replace")
+        return subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT), log
+
     binding_obj = os.path.join(obj_dir, "torch_binding.o")
     binding_cmd, binding_link = _compile_binding(binding_obj)
-    procs.append(("torch_binding.cpp", subprocess.Popen(binding_cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+    procs.append(("torch_binding.cpp", *start(binding_cmd)))
     for src in sources():
         obj = os.path.join(obj_dir, os.path.basename(src)[:-4] + ".o")
         objs.append(obj)
         cmd = [hipcc, *compile_flags, "-c", src, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-        while sum(p.poll() is None for _, p in procs) >= jobs:
-            for _, p in procs:
+        procs.append((src, *start(cmd)))
+        while sum(p.poll() is None for _, p, _ in procs) >= jobs:
+            for _, p, _ in procs:
                 if p.poll() is None:
                     p.wait()
                     break
     failed = False
-    for src, p in procs:
-        out, _ = p.communicate()
-        out = "\n".join(l for l in out.splitlines() if "packed-fp32-ops" not in l)
+    for src, p, log in procs:
+        p.wait()
+        log.seek(0)
+        out = "\n".join(l for l in log.read().splitlines() if "packed-fp32-ops" not in l)
         if p.returncode != 0:
             failed = True
             print(f"FAILED: {src}\n{out}", file=sys.stderr)
