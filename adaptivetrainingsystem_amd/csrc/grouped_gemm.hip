@@ -84,6 +84,7 @@ struct GroupedArgs {
     const int32_t* b_rows;
 };
 
+constexpr int kNonTemporal = 2;  // cache policy of a buffer load
 constexpr int kRowPitch = 144;  // bytes per staged row: 128 data + 16 pad
 
 template <typename T>
@@ -1106,8 +1107,14 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // AKM: the other operand is stored [K][rows] as well (one group; p.b is the operand itself, p.K its exact number of rows): the
 // weight gradient of a linear layer from the gradients and activations as they lie, tokens along the rows, without
 // transposed copies.  The same slabs, swizzle and transposing reads; same bits as the product of transposed copies.
+//
+// ONCE: groups of one tile each, whose weights are read from HBM by nobody else: loaded non-temporally, and in the gate/up product the
+// eight XCDs are an eighth of K apart (its rows of 4 and 8 KB put a column of all of them into a few of the memory's channels; the down
+// projections' gain nothing).  Layers, microseconds: 8 experts top-2 of [28672, 4096], 550 tokens 594 -> 577, 700 655 -> 606, 900 693 ->
+// 656, their down projection in slices another 10; 64 experts top-6 of [2816, 2048], 1150 tokens 295 -> 287, 2200 331 -> 324.  Where
+// groups reach a second tile it costs what it gained: 1100 tokens of 8 experts 868 -> 873, 3000 of 64 448 -> 459, hence kOnceMaxAvgRows.
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
-          bool MIDROWS = false, bool SLICED = false, bool AKM = false>
+          bool MIDROWS = false, bool SLICED = false, bool AKM = false, bool ONCE = false>
 __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, unsigned char* smem,
                                                          const int32_t* __restrict__ row_count) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1275,22 +1282,23 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 
 // AKM: the advance along K is part of the lane offset, which the descriptor's end is checked against (the scalar offset is
 // not); otherwise it is the scalar offset.
-#define D16_LOAD(rsrc_, dst_, off_, adv_)                                                              \
+#define D16_LOAD(rsrc_, dst_, off_, adv_, policy_)                                                     \
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_, (lds_ptr_t)(dst_), 16, (off_) + (AKM ? (adv_) : 0u), \
-                                             AKM ? 0 : (int)(adv_), 0, 0)
-#define D16_ISSUE_A1(kt_, aoff_, j_) D16_LOAD(rsrc_a, dma_a + (aoff_) + (j_) * NW * 1024, ao[j_], (unsigned)(kt_) * a_slab)
-#define D16_ISSUE_B1(kt_, boff_, j_) D16_LOAD(rsrc_b, dma_b + (boff_) + (j_) * NW * 1024, bo[j_], (unsigned)(kt_) * b_slab)
+                                             AKM ? 0 : (int)(adv_), 0, policy_)
+#define D16_ISSUE_A1(kt_, aoff_, j_) D16_LOAD(rsrc_a, dma_a + (aoff_) + (j_) * NW * 1024, ao[j_], (unsigned)(kt_) * a_slab, 0)
+#define D16_ISSUE_B1(kt_, boff_, j_) \
+    D16_LOAD(rsrc_b, dma_b + (boff_) + (j_) * NW * 1024, bo[j_], (unsigned)(kt_) * b_slab, ONCE ? kNonTemporal : 0)
 #define D16_ISSUE_A(kt_, aoff_)                                                                        \
     {                                                                                                  \
         const unsigned adv = (unsigned)(kt_) * a_slab;                                                  \
         _Pragma("unroll") for (int j = 0; j < NIA; ++j)                                                \
-            D16_LOAD(rsrc_a, dma_a + (aoff_) + j * NW * 1024, ao[j], adv);                             \
+            D16_LOAD(rsrc_a, dma_a + (aoff_) + j * NW * 1024, ao[j], adv, 0);                          \
     }
 #define D16_ISSUE_B(kt_, boff_)                                                                        \
     {                                                                                                  \
         const unsigned adv = (unsigned)(kt_) * b_slab;                                                  \
         _Pragma("unroll") for (int j = 0; j < NIB; ++j)                                                \
-            D16_LOAD(rsrc_b, dma_b + (boff_) + j * NW * 1024, bo[j], adv);                             \
+            D16_LOAD(rsrc_b, dma_b + (boff_) + j * NW * 1024, bo[j], adv, ONCE ? kNonTemporal : 0);    \
     }
 #define D16_B_ROW(j_) (SWIGLU ? ((j_) < TN / 2 ? (j_) * 16 : HALF + ((j_) - TN / 2) * 16) : (j_) * 16)
 #define D16_READ_A(aoff_, ks_, f0_, nf_, buf_)                                                         \
@@ -1378,7 +1386,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
         const int ca_ = MIDROWS ? STG * A_STAGE : s_cur, na_ = MIDROWS ? (STG ^ 1) * A_STAGE : s_nxt; \
         const int cb_ = MIDROWS ? s_cur : STG * B_STAGE, nb_ = MIDROWS ? s_nxt : (STG ^ 1) * B_STAGE; \
         __builtin_amdgcn_s_setprio(0);                                                  \
-        const int ka_ = min((kt_) + 2, nk - 1);                                         \
+        const int kr_ = min((kt_) + 2, nk - 1) + k0, ka_ = kr_ < nk ? kr_ : kr_ - nk;   \
         if (N1) D16_READ_A(ca_, 0, N0, N1, 1);                                       \
         D16_ISSUE_FAR(0);                                                                 \
         if (N0) {                                                                       \
@@ -1441,15 +1449,18 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
         if (kt < nk) D16_ITER(kt, 0, N0, N1);                                           \
     }
 
-    D16_ISSUE_B(0, 0);
-    D16_ISSUE_B(min(1, nk - 1), B_STAGE);
+    // first two slabs
+    const int k0 = ONCE && SWIGLU ? (int)(blockIdx.x % kNumXcd) * nk / kNumXcd : 0;
+    const int k1 = k0 + 1 < nk ? k0 + 1 : nk > 1 ? 0 : k0;
+    D16_ISSUE_B(k0, 0);
+    D16_ISSUE_B(k1, B_STAGE);
 #pragma unroll
     for (int j = 0; j < NIA && !AKM; ++j) {
         const int64_t src = gather ? (int64_t)(a_idx[j] / p.a_row_div) : (int64_t)a_idx[j];
         ao[j] = (unsigned)(src * p.lda * ES + dchunk * 16);
     }
-    D16_ISSUE_A(0, 0);
-    D16_ISSUE_A(min(1, nk - 1), A_STAGE);
+    D16_ISSUE_A(k0, 0);
+    D16_ISSUE_A(k1, A_STAGE);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NIA) : "memory");
     int s_cur = 0, s_nxt = A_STAGE;
     // rows of the expert in this wave's share of the tile (wave-uniform)
@@ -1515,7 +1526,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
 }
 
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
-          bool MIDROWS = false, bool SLICED = false, bool AKM = false>
+          bool MIDROWS = false, bool SLICED = false, bool AKM = false, bool ONCE = false>
 __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) {
     // The body is a function of its own for one reason: a __restrict__ parameter that it reads through gives every
     // other memory access in it (the transposing LDS reads among them) "does not alias that parameter" metadata once
@@ -1524,7 +1535,7 @@ __global__ __launch_bounds__(512) void grouped_gemm_dma16_kernel(GroupedArgs p) 
     // the K-major variant is preceded by s_waitcnt vmcnt(0), i.e. waits for all of the slab loads just issued (the
     // plain 16-byte fragment reads carry type-based alias metadata and never had that wait): 27-37 % slower.
     extern __shared__ __align__(16) unsigned char smem_k[];
-    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS, SLICED, AKM>(p, smem_k, p.row_count);
+    grouped_gemm_dma16_body<TO, SM, SN, SWIGLU, SAVEGU, DSILU, BKM, MIDROWS, SLICED, AKM, ONCE>(p, smem_k, p.row_count);
 }
 
 #undef PL_STORE
@@ -1545,6 +1556,8 @@ constexpr size_t dma_lds_bytes(int BM, int BN) { return (size_t)(3 * BM + 2 * BN
 
 // Rows per group on average below which the 16 x 16 x 32 kernel runs in its MIDROWS form (measured there).
 constexpr int64_t kMidRowsMaxAvg = 768;
+// Rows per group on average up to which hardly any group exceeds a tile's 256 rows.
+constexpr int64_t kOnceMaxAvgRows = 224;
 static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1) < kMidRowsMaxAvg; }
 // Tiles of the busiest CU.  Supertile S runs on XCD S % 8; the last band of rows and the last one of columns hold fewer than 32 tiles
 // (18 x 43 tiles of 256 rows: 33 supertiles, five for XCD 0, of which one has eight tiles and the others leave it four rounds).
@@ -1618,12 +1631,20 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
         else if constexpr (DMA) return grouped_gemm_dma_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
         else return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, kSliced>;
     }();
+    auto kern_once = [] {      // one tile per group
+        if constexpr (DMA && SWIGLU && std::is_same<T, bf16_t>::value)
+            return grouped_gemm_dma16_kernel<TO, SM, SN, true, false, false, false, true, false, false, true>;
+        else if constexpr (DMA && std::is_same<T, bf16_t>::value) return grouped_gemm_dma16_kernel<TO, SM, SN, SWIGLU, false, false, false, true>;
+        else if constexpr (DMA) return grouped_gemm_dma_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU>;
+        else return grouped_gemm_pipelined_kernel<T, TO, BM, BN, WM, WN, SM, SN, SWIGLU, kWarm, kSliced>;
+    }();
     if (smem > 64 * 1024) {
         static LdsReservation reserved;      // one per tile configuration (this function is a template)
         hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern_general),
                                               reinterpret_cast<const void*>(kern_pipe),
                                               reinterpret_cast<const void*>(kern_dma),
-                                              reinterpret_cast<const void*>(kern_mid)}, (int)smem);
+                                              reinterpret_cast<const void*>(kern_mid),
+                                              reinterpret_cast<const void*>(kern_once)}, (int)smem);
         if (e != hipSuccess) {
             set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
             return ATS_ERR_LAUNCH;
@@ -1651,7 +1672,8 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;
     }
-    auto kern = dma_ok ? (p.tile_rows || mid_rows(max_rows, p.E) ? kern_mid : kern_dma) : (p.K % BK == 0) ? kern_pipe : kern_general;
+    const bool once = p.E > 1 && max_rows / p.E <= kOnceMaxAvgRows;
+    auto kern = dma_ok ? (once ? kern_once : p.tile_rows || mid_rows(max_rows, p.E) ? kern_mid : kern_dma) : (p.K % BK == 0) ? kern_pipe : kern_general;
     const size_t smem_launch = (!dma_ok && p.K % BK == 0) ? smem_staged : smem;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WM * WN * 64), smem_launch, s, p);
     return ATS_OK;
@@ -1666,9 +1688,11 @@ static int launch_mid_sliced(const GroupedArgs& p0, int64_t max_rows, hipStream_
     GroupedArgs p = p0;
     p.n_tiles = (p.N_out + 255) / 256;
     constexpr size_t smem = dma_lds_bytes(256, 256);
-    auto kern = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, BKM, true, true>;
+    auto kern_many = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, BKM, true, true>;
+    auto kern_once = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, BKM, true, true, false, !BKM>;
+    auto kern = max_rows / p.E <= kOnceMaxAvgRows ? kern_once : kern_many;
     static LdsReservation reserved;
-    hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern)}, (int)smem);
+    hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern_many), reinterpret_cast<const void*>(kern_once)}, (int)smem);
     if (e != hipSuccess) {
         set_error("grouped GEMM: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
         return ATS_ERR_LAUNCH;

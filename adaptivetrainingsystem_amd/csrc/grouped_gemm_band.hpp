@@ -29,7 +29,6 @@ namespace ats {
 
 constexpr int kBandRows = 128, kBandCols = 128;     // most activation rows and weight rows of a tile
 constexpr int kBandWStage = kBandCols * 128;        // bytes of a slab of weights: 64 elements of every row
-constexpr int kNonTemporal = 2;                     // cache policy of a buffer load
 constexpr int kBandLds = 80 * 1024;                 // two workgroups per CU
 
 // MT: 16-row fragments of activations.  once: weights to be loaded non-temporally.  k0: first slab.

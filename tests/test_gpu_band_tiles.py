@@ -56,7 +56,9 @@ def test_groups(gpu, counts, N, K, gather):
         _check(got[s], rows[s] @ w[e][:, :K].double().T, rows[s].abs() @ w[e][:, :K].double().abs().T, K)
 
 
-@pytest.mark.parametrize("counts,I,K", [([31, 33, 64, 0, 65] * 4, 1000, 64), ([97, 128, 1, 96] * 4, 1032, 192), ([12, 129, 0, 20] * 8, 1096, 576)])
+# (the last three on the 256-row tile whose XCDs begin an eighth of K apart: one slab, fewer and more than eight, a group of two tiles)
+@pytest.mark.parametrize("counts,I,K", [([31, 33, 64, 0, 65] * 4, 1000, 64), ([97, 128, 1, 96] * 4, 1032, 192), ([12, 129, 0, 20] * 8, 1096, 576),
+                                        ([200, 256, 0, 300], 264, 64), ([223, 224, 225, 200], 1032, 320), ([130, 255, 257, 1, 410], 520, 1216)])
 def test_gate_up(gpu, counts, I, K):
     from adaptivetrainingsystem_amd import ops
     print("case band gate/up", len(counts), I, K, flush=True)
