@@ -353,18 +353,28 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const TY* __restrict__
             rows[n] = __builtin_amdgcn_readlane(my_row, src);
             wts[n] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_w), src));
         }
-#pragma unroll 4
         for (int h0 = h_first + lane * V; h0 < h_end; h0 += kWave * V) {
             float acc[V];
 #pragma unroll
             for (int j = 0; j < V; ++j) acc[j] = 0.f;
-            float yv[MAXK][V];
+            TO* o = out + t_out * H + h0;
+            constexpr int OV = (int)sizeof(TO) / 2;      // 16-byte vectors of eight columns
+            uint4 old[OV], res[OV];
+            if (residual) {
 #pragma unroll
-            for (int n = 0; n < MAXK; ++n) {
-                if (n < n_kept) {
-                    const TY* yr = y + rows[n] * H + h0;
-                    if constexpr (PARTS) {
-                        static_assert(sizeof(TY) == 4, "partial results are float32");
+                for (int q = 0; q < OV; ++q) res[q] = reinterpret_cast<const uint4*>(residual + t * H + h0)[q];
+            }
+            if (out_rows) {
+#pragma unroll
+                for (int q = 0; q < OV; ++q) old[q] = reinterpret_cast<const uint4*>(o)[q];
+            }
+            if constexpr (PARTS) {
+                static_assert(sizeof(TY) == 4, "partial results are float32");
+                float yv[MAXK][V];
+#pragma unroll
+                for (int n = 0; n < MAXK; ++n) {
+                    if (n < n_kept) {
+                        const TY* yr = y + rows[n] * H + h0;
 #pragma unroll
                         for (int j = 0; j < V; ++j) yv[n][j] = 0.f;
                         for (int s2 = 0; s2 < n_parts; ++s2) {
@@ -378,44 +388,55 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const TY* __restrict__
 #pragma unroll
                             for (int j = 0; j < V; ++j) yv[n][j] = bf16_bits_to_float(float_to_bf16_bits(yv[n][j]));
                         }
-                    } else if constexpr (sizeof(TY) == 2) {
-                        Elem<TY>::unpack(*reinterpret_cast<const uint4*>(yr), yv[n]);
-                    } else {
-                        Elem<TY>::unpack(*reinterpret_cast<const uint4*>(yr), yv[n]);
-                        Elem<TY>::unpack(*reinterpret_cast<const uint4*>(yr + 4), yv[n] + 4);
                     }
                 }
-            }
 #pragma unroll
-            for (int n = 0; n < MAXK; ++n) {
-                if (n < n_kept) {
+                for (int n = 0; n < MAXK; ++n) {
+                    if (n < n_kept) {
 #pragma unroll
-                    for (int j = 0; j < V; ++j) acc[j] = ((acc[j]) + (((wts[n]) * (yv[n][j]))));
+                        for (int j = 0; j < V; ++j) acc[j] = ((acc[j]) + (((wts[n]) * (yv[n][j]))));
+                    }
+                }
+            } else if (n_kept > 0) {
+                // All rows are asked for before the first is used, without branches between the loads (behind each of those the
+                // compiler waits for its load and the trips to memory follow one another: 4096 tokens x 6 choices x 2048 columns
+                // 33.6 -> 25.6 us, 9000 64 -> 46, 16384 x 2 x 4096 54 -> 52); choices that were dropped ask for the first row once more, and their products are passed by.
+                constexpr int YV = (int)sizeof(TY) / 2;
+                uint4 raw[MAXK][YV];
+#pragma unroll
+                for (int n = 0; n < MAXK; ++n) {
+                    const uint4* yr = reinterpret_cast<const uint4*>(y + (n < n_kept ? rows[n] : rows[0]) * H + h0);
+#pragma unroll
+                    for (int q = 0; q < YV; ++q) raw[n][q] = yr[q];
+                }
+#pragma unroll
+                for (int n = 0; n < MAXK; ++n) {
+                    float yv[V];
+#pragma unroll
+                    for (int q = 0; q < YV; ++q) Elem<TY>::unpack(raw[n][q], yv + q * (V / YV));
+#pragma unroll
+                    for (int j = 0; j < V; ++j) {
+                        const float sum = ((acc[j]) + (((wts[n]) * (yv[j]))));
+                        acc[j] = n < n_kept ? sum : acc[j];
+                    }
                 }
             }
             if (residual) {
                 float rv[V];
-                const TO* rr = residual + t * H + h0;
-                if constexpr (sizeof(TO) == 2) {
-                    Elem<TO>::unpack(*reinterpret_cast<const uint4*>(rr), rv);
-                } else {
-                    Elem<TO>::unpack(*reinterpret_cast<const uint4*>(rr), rv);
-                    Elem<TO>::unpack(*reinterpret_cast<const uint4*>(rr + 4), rv + 4);
-                }
+#pragma unroll
+                for (int q = 0; q < OV; ++q) Elem<TO>::unpack(res[q], rv + q * (V / OV));
 #pragma unroll
                 for (int j = 0; j < V; ++j) acc[j] = ((rv[j]) + (acc[j]));
             }
-            TO* o = out + t_out * H + h0;
             if (out_rows) {
                 // the sum as the token-major result would hold it, then the addition a scatter-add performs
                 float ov[V];
+#pragma unroll
+                for (int q = 0; q < OV; ++q) Elem<TO>::unpack(old[q], ov + q * (V / OV));
                 if constexpr (sizeof(TO) == 2) {
-                    Elem<TO>::unpack(*reinterpret_cast<const uint4*>(o), ov);
 #pragma unroll
                     for (int j = 0; j < V; ++j) acc[j] = ((ov[j]) + (bf16_bits_to_float(float_to_bf16_bits(acc[j]))));
                 } else {
-                    Elem<TO>::unpack(*reinterpret_cast<const uint4*>(o), ov);
-                    Elem<TO>::unpack(*reinterpret_cast<const uint4*>(o + 4), ov + 4);
 #pragma unroll
                     for (int j = 0; j < V; ++j) acc[j] = ((ov[j]) + (acc[j]));
                 }
@@ -432,7 +453,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(const TY* __restrict__
 
 // Columns of a token that one wave combines: 1024-column pieces (two steps of 64 lanes x 8 columns) for many
 // tokens, 512-column pieces for few, so that a handful of tokens still fills the chip.  Whole rows per wave
-// were slower where a token has many choices (4096 tokens x 6 choices x 2048 columns: 39 -> 34 us), the same
+// were slower where a token has many choices (4096 tokens x 6 choices x 2048 columns, one load at a time: 39 -> 34 us), the same
 // elsewhere: every wave spends its first microseconds on the row and weight look-up, and shorter waves overlap
 // that with other waves' loads.
 static int combine_cols_per_wave(int64_t T, int H) {
@@ -456,6 +477,9 @@ static bool launch_combine(const void* y, const int32_t* row_of, const float* w,
                            op, T, k, H, cols, 1, (int64_t)0, out_rows);
     else if (vec && k <= 4)
         hipLaunchKernelGGL((combine_vec_kernel<TY, TO, 4>), dim3((unsigned)blocks), dim3(256), 0, s, yp, row_of, w, rp,
+                           op, T, k, H, cols, 1, (int64_t)0, out_rows);
+    else if (vec && k <= 6)
+        hipLaunchKernelGGL((combine_vec_kernel<TY, TO, 6>), dim3((unsigned)blocks), dim3(256), 0, s, yp, row_of, w, rp,
                            op, T, k, H, cols, 1, (int64_t)0, out_rows);
     else if (vec)
         hipLaunchKernelGGL((combine_vec_kernel<TY, TO, 8>), dim3((unsigned)blocks), dim3(256), 0, s, yp, row_of, w, rp,
