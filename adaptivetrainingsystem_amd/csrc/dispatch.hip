@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void plan_rank_kernel(const IdxT* __restrict__
     const int64_t stride = (int64_t)gridDim.x * 256;
     const int64_t ec = (int64_t)E * C;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ec; i += stride) {
-        const int e = (int)(i / C);
+        const int e = (int)((unsigned)i / (unsigned)C);      // (E * C is below 2^31)
         const int pos = (int)(i - (int64_t)e * C);
         if (pos >= kept[e]) token_map[i] = -1;
     }
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void plan_fused_kernel(const IdxT* __restrict_
     const int64_t stride = (int64_t)gridDim.x * 256;
     const int64_t ec = (int64_t)E * C;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ec; i += stride) {
-        const int e = (int)(i / C);
+        const int e = (int)((unsigned)i / (unsigned)C);      // (E * C is below 2^31)
         const int pos = (int)(i - (int64_t)e * C);
         if (pos >= s_kept[e]) token_map[i] = -1;
     }

@@ -120,31 +120,23 @@ __device__ void chunk_rank_and_write(const IdxT* idx, int64_t n, int k, int E, i
     __syncthreads();
     int* my_base = s_cnt + wave * E;
     const unsigned long long lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    // up to 64 experts: lane l keeps the running base of expert l in a register, so the loop below touches no LDS
-    const bool in_regs = E <= kWave;
-    int base_reg = (in_regs && lane < E) ? my_base[lane] : 0;
     for (int step = 0; step < PERWAVE / kWave; ++step) {
         const int64_t a = chunk_base + wave * PERWAVE + step * kWave + lane;
         bool bad = false;
         const int e = load_expert(idx, a, n, E, &bad);
         int rank = -1;
-        unsigned long long remaining = __ballot(e >= 0);
-        while (remaining) {
-            // the leader and its expert are the same in all lanes: scalar reads instead of shuffles
-            const int leader = __builtin_amdgcn_readfirstlane(__ffsll((long long)remaining) - 1);
-            const int le = __builtin_amdgcn_readlane(e, leader);
-            const unsigned long long same = __ballot(e == le);
-            const int n_same = __popcll(same);
-            if (in_regs) {
-                const int b = __builtin_amdgcn_readlane(base_reg, le);
-                if (e == le) rank = b + __popcll(same & lt_mask);
-                if (lane == le) base_reg += n_same;
-            } else {
-                if (e == le) rank = my_base[le] + __popcll(same & lt_mask);
-                // all lanes have read my_base[le]; the leader advances it for the next step
-                if (lane == leader) my_base[le] += n_same;
-            }
-            remaining &= ~same;
+        // the lanes of the same expert are those that agree with this one on every bit of its number (a turn of a loop per expert
+        // took 4 us more where a step's 64 assignments name 40 of 64 experts: whole plans of 3600 assignments 10.7 -> 6.8 us, of 24576
+        // 19.4 -> 14.9)
+        unsigned long long same = __ballot(e >= 0);
+        for (int b = 0; (E - 1) >> b; ++b) {
+            const unsigned long long ones = __ballot(e >= 0 && ((e >> b) & 1));
+            same &= ((e >> b) & 1) ? ones : ~ones;
+        }
+        if (e >= 0) {
+            rank = my_base[e] + __popcll(same & lt_mask);
+            asm volatile("" ::: "memory");        // every lane has read its base before a leader advances it
+            if ((same & lt_mask) == 0) my_base[e] += __popcll(same);
         }
         if (a < n) {
             if (e >= 0 && rank < C) {
