@@ -441,8 +441,7 @@ class MoEFunction(Function):
     """The whole MoE FFN layer on [T, H] tokens.  apply(x, gate_weight, cfg, *expert_weights) with
     expert_weights = E gate/up matrices [2I, H] followed by E down matrices [H, I]; cfg is a dict:
     top_k, temperature, variant, capacity (C, or T for no dropping), load_balancing_weight,
-    noise_std (0 in eval), logit_bias (tensor or None), stats (dict filled with the plan), counts (device counters of
-    ops.routing_counts, or None).
+    noise_std (0 in eval), logit_bias (tensor or None), stats (dict filled with the plan).
     Returns (out [T, H], aux scalar)."""
 
     @staticmethod
@@ -467,7 +466,7 @@ class MoEFunction(Function):
         else:   # importance from the noise-free logits (model.py:1190-1192)
             aux = ops.aux_loss_clean_logits(logits, route["hist"], k, cfg["variant"], cfg["load_balancing_weight"])
         plan = ops.dispatch_plan(route["indices"], E, C)
-        usage = ops.routing_counts(route["hist"], plan["kept"], T * k, cfg.get("counts"))
+        usage = ops.routing_counts(route["hist"], plan["kept"], T * k)
         rows = min(T * k, E * C)
         hT = wplan = None
         if rows > 0:

@@ -622,11 +622,11 @@ class MoEFFNLayer(nn.Module):
             cfg = {"top_k": k, "temperature": self.routing_temperature, "variant": ag.moe_variant(self.routing),
                    "capacity": C, "load_balancing_weight": self.load_balancing_weight,
                    "noise_std": self.noise_std if self.training else 0.0, "logit_bias": self.router_logit_bias,
-                   "stats": stats, "counts": self._counts_on(x.device) if self.training and x.is_cuda else None}
+                   "stats": stats}
             out, aux = ag.MoEFunction.apply(x_flat, self.gate.weight, cfg, *params[1:])
             self.last_plan = stats
-            if self.training:
-                self._routing_stats["total_routed"] += T
+            if self.training:       # (behind apply: the recomputation of a checkpointed block ends inside it)
+                self._update_routing_stats(stats, T)
             return out.view(B, L, H), aux
 
         tm = self.stage_timer

@@ -81,3 +81,44 @@ def test_layer_statistics_over_passes_streams_and_copies(gpu):
     layer.reset_routing_stats()
     layer(x)
     assert layer.get_routing_stats()["expert_usage_percentages"] == (layer.last_plan["hist"].cpu().float() / 100 * 100).tolist()
+
+
+def _config(**more):
+    from adaptivetrainingsystem_amd.workloads import LayerConfig
+    return LayerConfig(128, 128, 4, 2, 1.0, num_heads=2, num_kv_heads=1, seq_length=32, moe_capacity_mode="fcfs", routing_noise_std=0.0, **more)
+
+
+def test_a_checkpointed_pass_counts_once(gpu):
+    from adaptivetrainingsystem_amd.layers import TransformerBlock
+    torch.manual_seed(3)
+    config = _config()
+    config.gradient_checkpointing, config.use_moe = True, True
+    block = TransformerBlock(config, 0).to(gpu).train()
+    x = torch.randn(2, 25, 128, device=gpu, requires_grad=True)
+    for n in (1, 2):
+        out, aux = block(x)
+        (out.sum() + aux).backward()
+        stats, plan = block.ffn.get_routing_stats(), block.ffn.last_plan
+        assert stats["total_tokens_routed"] == n * 50
+        assert stats["dropped_tokens"] == n * int((plan["hist"] - plan["kept"]).sum()) > 0
+        assert stats["expert_usage_percentages"] == (n * plan["hist"].cpu().float() / (n * 50) * 100).tolist()
+
+
+def test_a_failed_pass_counts_nothing(gpu, monkeypatch):
+    from adaptivetrainingsystem_amd import ops as product_ops
+    from adaptivetrainingsystem_amd.layers import MoEFFNLayer
+    layer = MoEFFNLayer(_config()).to(gpu).train()
+    x = torch.randn(2, 25, 128, device=gpu)
+
+    def fails(*args, **kwargs):
+        raise RuntimeError("no combine")
+
+    with monkeypatch.context() as m:
+        m.setattr(product_ops, "combine", fails)
+        with pytest.raises(RuntimeError, match="no combine"):
+            layer(x)
+    assert layer.get_routing_stats() == {"error": "No routing statistics available"}
+    layer(x)
+    stats = layer.get_routing_stats()
+    assert stats["total_tokens_routed"] == 50
+    assert stats["expert_usage_percentages"] == (layer.last_plan["hist"].cpu().float() / 50 * 100).tolist()
