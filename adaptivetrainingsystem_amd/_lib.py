@@ -101,6 +101,7 @@ _SIGNATURES = {
     "ats_combine_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int,
                                 c_int, c_int, c_int, c_void_p]),
     "ats_routing_counts": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p]),
+    "ats_routing_totals": (c_int, [c_void_p, c_void_p, c_int, c_int64, c_void_p, c_void_p]),
     "ats_gather_sum": (c_int, [c_void_p] * 3 + [c_int64] + [c_int] * 4 + [c_void_p]),
     "ats_gather_sum_partials": (c_int, [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "ats_route_bwd_clamped": (c_int, [c_void_p] * 6 + [c_float, c_void_p, c_void_p, c_float, c_int, c_void_p, c_int64, c_int, c_int,

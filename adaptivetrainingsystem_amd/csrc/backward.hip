@@ -226,13 +226,15 @@ __global__ __launch_bounds__(256) void route_bwd_kernel(const float* __restrict_
     }
 }
 
-// usage[e] = hist[e] * inv; with counts, hist is added to counts[0 .. E) and the dropped assignments to counts[E].  Integer atomics: passes
-// of one layer may run on several streams.
+// usage[e] = hist[e] * inv; with counts, hist is added to counts[0 .. E), the dropped assignments to counts[E] and `tokens`, unless it is
+// 0, to counts[E + 1].  Integer atomics: passes of one layer may run on several streams.
 __global__ __launch_bounds__(256) void routing_counts_kernel(const int32_t* __restrict__ hist, const int32_t* __restrict__ kept, int E,
-                                                             float inv, float* __restrict__ usage, unsigned long long* __restrict__ counts) {
+                                                             float inv, float* __restrict__ usage, unsigned long long* __restrict__ counts,
+                                                             unsigned long long tokens) {
+    if (tokens && threadIdx.x == 0) atomicAdd(&counts[E + 1], tokens);
     for (int e = threadIdx.x; e < E; e += 256) {
         const int h = hist[e];
-        usage[e] = (float)h * inv;
+        if (usage) usage[e] = (float)h * inv;
         if (!counts) continue;
         atomicAdd(&counts[e], (unsigned long long)h);
         if (h != kept[e]) atomicAdd(&counts[E], (unsigned long long)(h - kept[e]));
@@ -689,8 +691,18 @@ extern "C" int ats_routing_counts(const int32_t* hist, const int32_t* kept, int 
     // (the reciprocal of the float32 divisor, as torch divides by a number)
     const float inv = 1.0f / (float)((double)assignments + 1e-9);
     hipLaunchKernelGGL(routing_counts_kernel, dim3(1), dim3(256), 0, as_stream(stream), hist, kept, E, inv, usage,
-                       reinterpret_cast<unsigned long long*>(counts));
+                       reinterpret_cast<unsigned long long*>(counts), 0ull);
     ATS_CHECK_LAUNCH("ats_routing_counts");
+    return ATS_OK;
+}
+
+extern "C" int ats_routing_totals(const int32_t* hist, const int32_t* kept, int E, int64_t tokens, int64_t* counts, ats_stream_t stream) {
+    using namespace ats;
+    ATS_REQUIRE(E > 0 && tokens >= 0 && hist && kept && counts, ATS_ERR_INVALID_ARG, "ats_routing_totals: E=%d tokens=%lld, or a null pointer",
+                E, (long long)tokens);
+    hipLaunchKernelGGL(routing_counts_kernel, dim3(1), dim3(256), 0, as_stream(stream), hist, kept, E, 0.f, (float*)nullptr,
+                       reinterpret_cast<unsigned long long*>(counts), (unsigned long long)tokens);
+    ATS_CHECK_LAUNCH("ats_routing_totals");
     return ATS_OK;
 }
 

@@ -29,6 +29,7 @@ Differences that are deliberate:
 from __future__ import annotations
 
 import math
+import threading
 from typing import Any, Dict, Optional, Tuple
 
 import torch
@@ -487,6 +488,63 @@ def _as_dtype(w: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
 
 
 # ============================================================================ MoE layer
+def _no_routing(num_experts: int) -> Dict[str, Any]:
+    return {"expert_usage": torch.zeros(num_experts, device="cpu"), "total_routed": 0, "dropped_tokens": 0}
+
+
+class _RoutingStatistics:
+    """Routing statistics of one layer: the host's dictionary, and per device what training passes have counted since it was last
+    read (int64: assignments of each expert, dropped ones, tokens).  One object serves a layer and its replicas on other devices.
+    Passes only add to the device's counters, all three in one launch behind the pass, so that a pass that is recorded in a graph
+    counts when it is replayed; reading them in the pass had the host wait for the device in the middle of every step (a float32
+    block of 2 x 256 tokens, forward and backward, 1280 us; so, and with seven launches less for the scalars of the routing, 1116)."""
+
+    def __init__(self, values: Dict[str, Any]):
+        self.values = values
+        self._counters: Dict[torch.device, list] = {}       # device -> [counters, what of them the host has read, their stream]
+        self._lock = threading.Lock()
+
+    def add(self, hist: torch.Tensor, kept: torch.Tensor, tokens: int) -> None:
+        E, device = hist.numel(), hist.device
+        with self._lock:
+            entry = self._counters.get(device)
+            if entry is None or entry[0].numel() != E + 2:      # (an expert was added or pruned)
+                self._read()
+                # copied from the host, which waits: zeros for every stream that a pass may run on
+                seen = torch.zeros(E + 2, dtype=torch.int64, device="cpu")
+                entry = self._counters[device] = [seen.to(device, copy=True), seen, ops._stream()]
+            counts = entry[0]
+            if ops._stream() != entry[2]:
+                counts.record_stream(torch.cuda.current_stream(device))
+            ops.routing_totals(hist, kept, tokens, counts)
+
+    def read(self) -> Dict[str, Any]:
+        with self._lock:
+            self._read()
+            return self.values
+
+    def replace(self, values: Dict[str, Any]) -> None:
+        with self._lock:
+            self._read()
+            self.values = values
+
+    def _read(self) -> None:
+        for device, entry in self._counters.items():
+            if device.type == "cuda":
+                torch.cuda.synchronize(device)          # every stream that a pass ran on
+            now = entry[0].to("cpu", copy=True)
+            new, entry[1] = now - entry[1], now
+            usage, E = self.values["expert_usage"], now.numel() - 2
+            if usage.numel() != E:                      # an expert was added or pruned since the last reading
+                grown = torch.zeros(E, device="cpu")
+                n = min(usage.numel(), E)
+                grown[:n] = usage[:n]
+                self.values["expert_usage"] = usage = grown
+            usage += new[:E].float()
+            self.values["dropped_tokens"] += int(new[E])
+            self.values["total_routed"] += int(new[E + 1])
+
+
 class MoEFFNLayer(nn.Module):
     """Mixture-of-experts FFN: gate Linear -> routing -> (capacity) dispatch -> SwiGLU experts ->
     weighted combine, plus the load-balancing auxiliary loss.  forward(x [B,L,H]) -> (out, aux).
@@ -523,8 +581,7 @@ class MoEFFNLayer(nn.Module):
         self.router_logit_bias: Optional[torch.Tensor] = None   # optional per-expert skew (benchmarks)
         self._gate_param_count = sum(p.numel() for p in self.gate.parameters())
         self._expert_param_count = self.experts[0]._param_count
-        self._routing_stats = {"expert_usage": torch.zeros(config.num_experts, device="cpu"), "total_routed": 0,
-                               "dropped_tokens": 0}
+        self._routing_store = _RoutingStatistics(_no_routing(config.num_experts))
         self._wcache_key = None
         self._wcache = None
         self._last_plan = None
@@ -578,10 +635,22 @@ class MoEFFNLayer(nn.Module):
         super().__setstate__(state)
         # modules pickled before the property existed hold the plan under its own name
         self.__dict__.setdefault("_last_plan", self.__dict__.pop("last_plan", None))
+        # the statistics are pickled as the plain dictionary that they are
+        self._routing_store = _RoutingStatistics(self.__dict__.pop("_routing_stats", None) or _no_routing(self.num_experts))
 
     def __getstate__(self):
-        self._read_routing_counts()
-        return {n: v for n, v in self.__dict__.items() if n not in ("_routing_counts", "_routing_seen", "_routing_stream")}
+        state = dict(self.__dict__)
+        state["_routing_stats"] = state.pop("_routing_store").read()
+        return state
+
+    @property
+    def _routing_stats(self) -> Dict[str, Any]:
+        """expert_usage (float32 on the host), total_routed and dropped_tokens of all training passes so far (waits for them)."""
+        return self._routing_store.read()
+
+    @_routing_stats.setter
+    def _routing_stats(self, values: Dict[str, Any]) -> None:
+        self._routing_store.replace(values)
 
     def forward(self, x: torch.Tensor, add_onto: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
                 ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -702,63 +771,25 @@ class MoEFFNLayer(nn.Module):
         return (k <= 8 and H % 8 == 0 and target.is_contiguous() and target.data_ptr() % 16 == 0
                 and rows_to.dtype == torch.int32 and rows_to.is_contiguous() and x.data_ptr() % 16 == 0)
 
-    # Assignments per expert and dropped ones, added up on the device by every training pass, and those of them that the host has
-    # read.  (Reading them in the pass had the host wait for the device in the middle of every step: a float32 block of 2 x 256
-    # tokens, forward and backward, 1280 us; so, and with seven launches less for the scalars of the routing, 1116.)
-    _routing_counts: Optional[torch.Tensor] = None
-    _routing_seen: Optional[torch.Tensor] = None
-
-    def _counts_on(self, device: torch.device) -> torch.Tensor:
-        counts = self._routing_counts
-        if counts is None or counts.numel() != self.num_experts + 1 or counts.device != device:
-            self._read_routing_counts()         # (an expert was added or pruned, or the layer moved)
-            # copied from the host, which waits: zeros for every stream that a pass may run on
-            counts = torch.zeros(self.num_experts + 1, dtype=torch.int64).to(device)
-            self._routing_seen, self._routing_counts = torch.zeros(self.num_experts + 1, dtype=torch.int64), counts
-            self._routing_stream = ops._stream()
-        if ops._stream() != self._routing_stream:
-            counts.record_stream(torch.cuda.current_stream(device))
-        return counts
-
-    def _read_routing_counts(self) -> None:
-        """Adds what the device has counted since the last reading to the statistics (waits for every stream)."""
-        counts = self._routing_counts
-        if counts is None:
-            return
-        torch.cuda.synchronize(counts.device)
-        now = counts.cpu()
-        new, self._routing_seen = now - self._routing_seen, now
-        usage, E = self._routing_stats["expert_usage"], now.numel() - 1
-        if usage.numel() != E:                  # an expert was added or pruned since the last reading
-            grown = torch.zeros(E, device="cpu")
-            n = min(usage.numel(), E)
-            grown[:n] = usage[:n]
-            self._routing_stats["expert_usage"] = usage = grown
-        usage += new[:E].float()
-        self._routing_stats["dropped_tokens"] += int(new[E])
-
     def _update_routing_stats(self, plan, total_tokens: int) -> None:
-        ops.routing_counts(plan["hist"], plan["kept"], max(1, total_tokens) * self.top_k, self._counts_on(plan["hist"].device))
-        self._routing_stats["total_routed"] += total_tokens
+        self._routing_store.add(plan["hist"], plan["kept"], total_tokens)
 
     def get_routing_stats(self) -> Dict[str, Any]:
-        self._read_routing_counts()
-        total = self._routing_stats["total_routed"]
+        values = self._routing_stats
+        total = values["total_routed"]
         if total == 0:
             return {"error": "No routing statistics available"}
-        usage = self._routing_stats["expert_usage"].clone()
+        usage = values["expert_usage"].clone()
         pct = (usage / total * 100).tolist()
         return {
             "expert_usage_percentages": pct, "total_tokens_routed": total,
-            "dropped_tokens": self._routing_stats["dropped_tokens"],
+            "dropped_tokens": values["dropped_tokens"],
             "usage_std": float(torch.std(usage / total)), "usage_min": min(pct), "usage_max": max(pct),
             "imbalance_ratio": max(pct) / max(min(pct), 0.1),
         }
 
     def reset_routing_stats(self) -> None:
-        self._read_routing_counts()
-        self._routing_stats = {"expert_usage": torch.zeros(self.num_experts, device="cpu"), "total_routed": 0,
-                               "dropped_tokens": 0}
+        self._routing_stats = _no_routing(self.num_experts)
 
 
 class CapacityMoEFFNLayer(MoEFFNLayer):

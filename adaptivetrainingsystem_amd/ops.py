@@ -251,6 +251,18 @@ def routing_counts(hist: torch.Tensor, kept: torch.Tensor, assignments: int, cou
     return usage
 
 
+def routing_totals(hist: torch.Tensor, kept: torch.Tensor, tokens: int, counts: torch.Tensor) -> None:
+    """Adds hist to the first E of counts (int64 [E + 2]), the number of dropped assignments to the next and tokens to the last."""
+    _need_gpu(hist, kept, counts)
+    E = hist.numel()
+    if hist.dtype != torch.int32 or kept.dtype != torch.int32 or kept.numel() != E:
+        raise AtsError("routing_totals: hist and kept must be int32 of one size")
+    if counts.dtype != torch.int64 or counts.numel() != E + 2 or not counts.is_contiguous():
+        raise AtsError("routing_totals: counts must be contiguous int64 [experts + 2]")
+    check(_lib.load().ats_routing_totals(hist.contiguous().data_ptr(), kept.contiguous().data_ptr(), E, int(tokens), counts.data_ptr(),
+                                         _stream()), "ats_routing_totals")
+
+
 def aux_loss_clean_logits(clean_logits: torch.Tensor, hist: torch.Tensor, k: int, variant: int,
                           load_balancing_weight: float) -> torch.Tensor:
     """Load-balancing loss when routing ran on noisy logits: usage from the routed histogram, importance from

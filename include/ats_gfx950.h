@@ -430,6 +430,8 @@ int ats_route_bwd_clamped(const float* logits_route, const float* logits_aux, co
  * to counts[e] and the assignments that were not kept to counts[E] (integer atomics). */
 int ats_routing_counts(const int32_t* hist, const int32_t* kept, int E, int64_t assignments, float* usage, int64_t* counts,
                        ats_stream_t stream);
+/* The same additions to counts [E + 2] alone, and `tokens` to counts[E + 1]. */
+int ats_routing_totals(const int32_t* hist, const int32_t* kept, int E, int64_t tokens, int64_t* counts, ats_stream_t stream);
 /* Gradient of ats_router_logits: out[t,:] = base[t,:] + dlogits[t,:] . Wg (base NULL or == out),
  * dWg[e,:] = sum_t dlogits[t,e] * x[t,:] (float32, fixed order). */
 int ats_router_bwd_dx(const float* dlogits, const void* wg, const void* base, void* out, int64_t T, int E,

@@ -24,6 +24,12 @@ def test_routing_counts(ops, gpu, E, n):  # noqa: F811
     assert torch.equal(ops.routing_counts(hist, kept, n), hist.float() / (n + 1e-9))
     with pytest.raises(ops.AtsError):
         ops.routing_counts(hist, kept, n, counts[:E])
+    totals = torch.full((E + 3,), 2 ** 40, dtype=torch.int64, device=gpu)
+    for i in range(2):
+        ops.routing_totals(hist, kept, n, totals[:E + 2])
+    assert torch.equal(totals[:E + 1] - 2 ** 40, counts - 2 ** 40) and (totals[E + 1:] - 2 ** 40).tolist() == [2 * n, 0]
+    with pytest.raises(ops.AtsError):
+        ops.routing_totals(hist, kept, n, totals)
 
 
 @pytest.mark.parametrize("T,k,H", [(5, 1, 8), (33, 2, 520), (7, 6, 64), (4, 3, 37), (3, 12, 40)])
@@ -122,3 +128,52 @@ def test_a_failed_pass_counts_nothing(gpu, monkeypatch):
     stats = layer.get_routing_stats()
     assert stats["total_tokens_routed"] == 50
     assert stats["expert_usage_percentages"] == (layer.last_plan["hist"].cpu().float() / 50 * 100).tolist()
+
+
+def test_the_dictionary_and_replicas_agree_with_the_passes(gpu):
+    from adaptivetrainingsystem_amd.layers import MoEFFNLayer
+    layer = MoEFFNLayer(_config()).to(gpu).train()
+    x = torch.randn(2, 25, 128, device=gpu)
+    replica = layer._replicate_for_data_parallel()      # its experts and gate are the layer's own modules
+    used, dropped = torch.zeros(4), 0
+    for n, one in enumerate((replica, layer, replica), 1):
+        one(x * n)
+        used += one.last_plan["hist"].cpu().float()
+        dropped += int((one.last_plan["hist"] - one.last_plan["kept"]).sum())
+        for reader in (layer, replica):
+            values = reader._routing_stats
+            assert torch.equal(values["expert_usage"], used) and values["dropped_tokens"] == dropped and values["total_routed"] == 50 * n
+    assert layer.get_routing_stats()["expert_usage_percentages"] == (used / 150 * 100).tolist()
+
+
+def test_a_recorded_pass_counts_when_it_is_replayed(gpu):
+    from adaptivetrainingsystem_amd.layers import MoEFFNLayer
+    torch.manual_seed(3)
+    layer = MoEFFNLayer(_config()).to(gpu).train()
+    x = torch.randn(2, 25, 128, device=gpu)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        layer(x)
+    torch.cuda.current_stream().wait_stream(side)
+    layer.reset_routing_stats()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, _ = layer(x)
+    plan = layer.last_plan
+    assert layer.get_routing_stats() == {"error": "No routing statistics available"}
+    used, dropped = torch.zeros(4), 0
+    for n in range(1, 4):
+        x.copy_(torch.randn(2, 25, 128, device=gpu))
+        graph.replay()
+        torch.cuda.synchronize()
+        used += plan["hist"].cpu().float()
+        dropped += int((plan["hist"] - plan["kept"]).sum())
+        stats = layer.get_routing_stats()
+        assert stats["total_tokens_routed"] == 50 * n and stats["dropped_tokens"] == dropped
+        assert stats["expert_usage_percentages"] == (used / (50 * n) * 100).tolist()
+        replayed = out.clone()
+        layer.eval()
+        with torch.enable_grad():
+            assert torch.equal(replayed, layer(x)[0])
+        layer.train()

@@ -389,3 +389,32 @@ def test_joined_rotation_refuses_more_threads_than_its_numbers_hold():
         rows = pieces // 3
         assert 2 ** 31 - 1 - 255 < 3 * rows < 2 ** 31 - 1
         assert call(rows) == -1, lib.ats_last_error_string()       # an argument that is not served, not a failed launch
+
+
+def test_routing_statistics_are_pickled_as_a_plain_dictionary():
+    import copy
+    import pickle
+    import adaptivetrainingsystem_amd as A
+    from adaptivetrainingsystem_amd.workloads import LayerConfig
+    layer = A.MoEFFNLayer(LayerConfig(32, 64, 4, 2))
+    store = layer._routing_store
+    counts = torch.tensor([3, 0, 1, 4, 2, 5])          # what a device would have counted: 4 experts, 2 dropped, 5 tokens
+    store._counters[torch.device("cpu")] = [counts, torch.tensor([1, 0, 1, 0, 2, 1]), 0]
+    assert layer._routing_stats["total_routed"] == 4 and layer._routing_stats["dropped_tokens"] == 0
+    assert layer.__getstate__()["_routing_stats"] is layer._routing_stats and "_routing_store" not in layer.__getstate__()
+    for twin in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
+        assert twin._routing_stats["expert_usage"].tolist() == [2, 0, 0, 4] and twin._routing_stats["total_routed"] == 4
+        twin._routing_stats["total_routed"] = 7
+        assert layer._routing_stats["total_routed"] == 4
+        twin.reset_routing_stats()
+        assert twin.get_routing_stats() == {"error": "No routing statistics available"}
+    counts += 1
+    assert layer._routing_stats["expert_usage"].tolist() == [3, 1, 1, 5] and layer._routing_stats["total_routed"] == 5
+    layer.num_experts = 5                              # an expert was added
+    store._counters[torch.device("cpu")] = [torch.ones(7, dtype=torch.int64), torch.zeros(7, dtype=torch.int64), 0]
+    assert layer._routing_stats["expert_usage"].tolist() == [4, 2, 2, 6, 1]
+    # a layer pickled when the dictionary was an attribute of its own
+    state = layer.__getstate__()
+    old = A.MoEFFNLayer.__new__(A.MoEFFNLayer)
+    old.__setstate__({**state, "_routing_stats": {"expert_usage": torch.ones(5), "total_routed": 3, "dropped_tokens": 1}})
+    assert old._routing_stats["total_routed"] == 3
