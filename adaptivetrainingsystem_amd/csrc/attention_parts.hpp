@@ -37,31 +37,48 @@ inline AttnParts attn_parts(int n_tiles, int64_t n_heads, int cus, bool two, F w
     int most = n_tiles % 2 ? work(n_tiles / 2) + kTileStart : 0;
     for (int p = 0; p < n_tiles / 2; ++p) most = std::max(most, work(p) + work(n_tiles - 1 - p) + 2 * kTileStart);
     if (estimate) *estimate = cost((n_tiles + 1) / 2, most);
-    if (n_tiles < 2 || n_tiles > kAttnMaxTiles) return best;
+    if (n_tiles < 2 || n_tiles > kAttnMaxTiles || n_heads < 1) return best;
     int64_t least = cost((n_tiles + 1) / 2, most) * 19 / 20;
     int w[kAttnMaxTiles], total = 0;
     for (int t = 0; t < n_tiles; ++t) total += w[t] = work(t) + kTileStart;
+    // first fit, the longest tile first: whether `parts` parts of that much room hold all tiles
+    auto fit = [&](int parts, int room, AttnParts* a) {
+        *a = AttnParts{};
+        a->count = parts;
+        int left[kAttnMaxParts];
+        for (int p = 0; p < parts; ++p) left[p] = room;
+        for (int t = n_tiles - 1; t >= 0; --t) {
+            int p = 0;
+            while (p < parts && left[p] < w[t]) ++p;
+            if (p == parts) return false;
+            left[p] -= w[t];
+            a->tiles[p] |= 1u << t;
+        }
+        return true;
+    };
     for (int parts = std::min(n_tiles, kAttnMaxParts); parts >= 1; --parts) {
-        // first fit, the longest tile first, into the least room that holds all tiles
-        for (int room = std::max(w[n_tiles - 1], (total + parts - 1) / parts); cost(parts, room) < least; ++room) {
-            AttnParts a{};
-            a.count = parts;
-            int left[kAttnMaxParts], t = n_tiles - 1;
-            for (int p = 0; p < parts; ++p) left[p] = room;
-            for (; t >= 0; --t) {
-                int p = 0;
-                while (p < parts && left[p] < w[t]) ++p;
-                if (p == parts) break;
-                left[p] -= w[t];
-                a.tiles[p] |= 1u << t;
+        // the least room between what a part needs at least and the most that promises anything, which lie a few key tiles apart where
+        // all keys are new (0.3-3 us a call); by halves where tiles are longer (with a million cached keys they are tens of thousands
+        // of key tiles, and trying each room took 6 ms of every call)
+        int lo = std::max(w[n_tiles - 1], (total + parts - 1) / parts);
+        int hi = (int)std::min<int64_t>((least - 1) / cost(parts, 1), total);
+        AttnParts a;
+        if (hi - lo < 64) {
+            while (lo <= hi && !fit(parts, lo, &a)) ++lo;
+            if (lo > hi) continue;
+        } else {
+            if (!fit(parts, hi, &a)) continue;
+            while (lo < hi) {
+                const int mid = lo + (hi - lo) / 2;
+                AttnParts b;
+                if (fit(parts, mid, &b)) hi = mid, a = b;
+                else lo = mid + 1;
             }
-            if (t >= 0) continue;
-            if (a.tiles[parts - 1]) {      // (fewer parts hold them as well: a later turn)
-                least = cost(parts, room);
-                best = a;
-                if (estimate) *estimate = least;
-            }
-            break;
+        }
+        if (a.tiles[parts - 1]) {      // (fewer parts hold them as well: a later turn)
+            least = cost(parts, lo);
+            best = a;
+            if (estimate) *estimate = least;
         }
     }
     return best;
