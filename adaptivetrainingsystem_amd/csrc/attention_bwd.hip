@@ -850,6 +850,11 @@ struct DkvPlan {
 // unit, 0.49 at head_dim 64), and the traffic of the sums.  Fitted to the whole backward of 60 random shapes of 1-8 sequences of 65-7511
 // positions (best of all numbers of ranges 0.2 % better on average, 5 % at most): 1 x 1777, 32 heads of 128 on 8: 349 -> 155 us,
 // 3 x 1777 434 -> 361, 1 x 4328 of 8 heads 847 -> 284, 8 x 2048 (the chip is full) one range as before.
+//
+// The sums take scratch memory by the length, which the time saved does not follow (1 x 50 000: 2.5 GB for 75.7 -> 68.5 ms; what it gains
+// is the last, mostly empty round of tiles): at most kDkvMaxScratch, which holds every number of ranges that is chosen up to 16 000
+// positions of 32 heads on 8 (4 x 4100 in three 2301 -> 2186 us with 403 MB, 1 x 12 000 in four 4519 -> 4114 with 393).
+constexpr double kDkvMaxScratch = 512e6;
 static DkvPlan dkv_plan(int B, int Hq, int Hkv, int L, int Lk, int D, bool workspace) {
     const int n_kt = (Lk + kBwdRows - 1) / kBwdRows, rep = Hq / Hkv, off = Lk - L, steps = (L + kDkvBQ - 1) / kDkvBQ;
     const int64_t groups = (int64_t)B * Hkv;
@@ -858,6 +863,7 @@ static DkvPlan dkv_plan(int B, int Hq, int Hkv, int L, int Lk, int D, bool works
     DkvPlan best{};
     double least = 0;
     for (const int ranges : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        if (ranges > 1 && (double)ranges * 2 * groups * Lk * D * sizeof(float) > kDkvMaxScratch) break;
         int64_t quarters = 0;
         const AttnParts parts = attn_parts(n_kt, (by_xcd ? groups / 8 : groups) * ranges, by_xcd ? 32 : 256, true, [&](int t) {
             const int first = std::max((n_kt - 1 - t) * kBwdRows - off, 0) / kDkvBQ;

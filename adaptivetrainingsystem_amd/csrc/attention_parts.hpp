@@ -21,7 +21,7 @@ struct AttnParts {
 // Five parts of 42 (28 + 14, 26 + 16, 24 + 18, 22 + 20, the rest) are two on nearly every unit: 3 x 1777 positions, 32 heads of 128,
 // 120 -> 103 us (with the queries' rotation 145 -> 129; the layer 505 -> 500, its products run a little slower behind it: board
 // power), 1 x 4737 of 32 heads of 64 185 -> 130 (the layer 314 -> 254).  70 random shapes of 1-8 sequences of 129-8192 positions: the forward takes
-// 6.6 % less time on average than in pairs (0.67 .. 1.0 of it, single calls to 1.03), dQ with dK and dV behind it 2.8 %.  A twentieth
+// 11 % less time on average than in pairs (0.76 .. 1.05 of it), the backward with its queries in one range 10 % (0.69 .. 1.03).  A twentieth
 // is what the estimate has to promise; more than 32 tiles of a head keep to pairs, whose number is then large.
 //
 // work(t): key tiles that query tile t sees (not falling with t); n_heads heads share `cus` compute units, each of which runs

@@ -1406,9 +1406,12 @@ def causal_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out:
     # delta = rowsum(dO * O) is formed inside the dQ kernel and handed to the dK/dV kernel through this buffer
     delta = torch.empty(B, Hq, L, dtype=torch.float32, device=q.device)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    # few key tiles: float32 sums of ranges of queries that run side by side
+    # few key tiles: float32 sums of ranges of queries that run side by side; without memory for them in one range
     ws_bytes = lib.ats_attention_bwd_workspace(B, Hq, Hkv, L, Lk, D)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    try:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    except torch.OutOfMemoryError:
+        ws = None
     check(lib.ats_attention_bwd_out_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dout.data_ptr(),
                                        lse.data_ptr(), delta.data_ptr(), _ptr(key_bias), _ptr(pair_bias), pair_sb, pair_sh,
                                        float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF, dq.data_ptr(), dk.data_ptr(),

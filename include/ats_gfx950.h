@@ -614,7 +614,7 @@ int ats_attention_bwd_out(const void* q, const void* k, const void* v, const voi
                           const float* lse, float* delta_ws, const float* key_bias, const float* bias_qk,
                           int64_t bias_sb, int64_t bias_sh, float dropout_p, uint64_t dropout_seed, void* dq, void* dk,
                           void* dv, int B, int Hq, int Hkv, int L, int Lk, int D, float scale, ats_stream_t stream);
-/* ats_attention_bwd_out with scratch of ats_attention_bwd_workspace bytes (0: none is of use; 16-byte aligned; less than that, or
+/* ats_attention_bwd_out with scratch of ats_attention_bwd_workspace bytes (at most 512 MB, 0: none is of use; 16-byte aligned; less than that, or
  * null, is ats_attention_bwd_out): where the key tiles are too few for the chip, dK and dV are summed by several workgroups a tile, in
  * float32, and the sums added in a fixed order. */
 size_t ats_attention_bwd_workspace(int B, int Hq, int Hkv, int L, int Lk, int D);

@@ -97,6 +97,41 @@ def test_every_tile_belongs_to_one_part(tmp_path):
     assert {0, 1, 2, 3, 5} <= seen
 
 
+def test_scratch_of_the_backward_is_bounded():
+    from adaptivetrainingsystem_amd import _lib
+    f = _lib.load().ats_attention_bwd_workspace
+    for B, Hq, Hkv in ((1, 32, 8), (4, 32, 8), (1, 8, 8), (1, 128, 1), (3, 16, 4), (8, 32, 32)):
+        for D in (64, 128):
+            for L in (1, 300, 1777, 4100, 6144, 12000, 50000, 84340, 100000, 1000000):
+                for Lk in (L, L + 5000):
+                    size = f(B, Hq, Hkv, L, Lk, D)
+                    assert size <= 512 * 10 ** 6 and size % (2 * B * Hkv * Lk * D * 4) == 0, (B, Hq, Hkv, L, Lk, D, size)
+    # 8, 3 and 4 ranges of one, three and four sequences' queries, as before
+    assert [f(B, 32, 8, L, L, 128) // (2 * B * 8 * L * 128 * 4) for B, L in ((1, 1777), (3, 1777), (8, 2048), (1, 12000))] == [8, 3, 0, 4]
+
+
+@pytest.mark.gpu
+def test_without_memory_for_the_scratch(gpu, monkeypatch):
+    from adaptivetrainingsystem_amd import ops
+    q, k, v, do = (torch.randn(*s, device=gpu).bfloat16() for s in ((1, 4, 300, 64), (1, 2, 300, 64), (1, 2, 300, 64), (1, 300, 256)))
+    out, lse = ops.causal_attention(q, k, v, return_lse=True)
+    want = ops.causal_attention_bwd(q, k, v, out, lse, do)
+    empty = torch.empty
+
+    def full(*shape, dtype=None, **more):
+        if dtype == torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*shape, dtype=dtype, **more)
+
+    monkeypatch.setattr(torch, "empty", full)
+    got = ops.causal_attention_bwd(q, k, v, out, lse, do)
+    monkeypatch.undo()
+    assert torch.equal(got[0], want[0])
+    # the same float32 sums in another order, then one rounding to bfloat16 (8 bits: neighbours lie up to 2^-7 of their value apart)
+    for a, b in zip(got[1:], want[1:]):
+        assert ((a.float() - b.float()).abs() <= 2 ** -7 * b.float().abs() + 1e-5 * b.float().abs().max()).all()
+
+
 # keys of a tile whose queries are cut into ranges, some of them empty (the last tile sees 2 queries, 1 of 4 heads' steps each)
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,L,Lk,D", [(1, 4, 1, 130, 130, 128), (1, 8, 1, 33, 33, 64), (1, 4, 4, 1500, 1500, 64), (1, 8, 2, 700, 900, 64), (2, 32, 2, 2, 300, 128)])
