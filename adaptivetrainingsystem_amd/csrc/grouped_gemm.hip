@@ -1108,11 +1108,14 @@ __global__ __launch_bounds__(WM* WN * 64) void grouped_gemm_dma_kernel(GroupedAr
 // weight gradient of a linear layer from the gradients and activations as they lie, tokens along the rows, without
 // transposed copies.  The same slabs, swizzle and transposing reads; same bits as the product of transposed copies.
 //
-// ONCE: groups of one tile each, whose weights are read from HBM by nobody else: loaded non-temporally, and in the gate/up product the
-// eight XCDs are an eighth of K apart (its rows of 4 and 8 KB put a column of all of them into a few of the memory's channels; the down
-// projections' gain nothing).  Layers, microseconds: 8 experts top-2 of [28672, 4096], 550 tokens 594 -> 577, 700 655 -> 606, 900 693 ->
-// 656, their down projection in slices another 10; 64 experts top-6 of [2816, 2048], 1150 tokens 295 -> 287, 2200 331 -> 324.  Where
-// groups reach a second tile it costs what it gained: 1100 tokens of 8 experts 868 -> 873, 3000 of 64 448 -> 459, hence kOnceMaxAvgRows.
+// ONCE: groups of one tile each, whose weights are read from HBM by nobody else: loaded non-temporally, and in the gate/up product eight
+// supertiles in turn begin K an eighth of it apart and come round (its rows of 4 and 8 KB put a column of all of them into a few of the
+// memory's channels; the down projections' gain nothing).  Where every group has its tile these are the eight XCDs, each in step by
+// itself; the start follows from expert and columns alone, so that the order of a row's sums does not depend on the other groups.
+// Layers, microseconds, as the instance for every group -> non-temporal -> out of step: 8 experts top-2 of [28672, 4096], 550 tokens
+// 610 -> 572 -> 559, 700 642 -> 597 -> 586, 890 690 -> 640 -> 633; 64 experts top-6 of [2816, 2048], 1500 tokens 309 -> 297 -> 291, 2200
+// 338 -> 319 -> 313.  Where groups reach a second tile it costs what it gained: 1100 tokens of 8 experts 868 -> 873, 3000 of 64 448 ->
+// 459, hence kOnceMaxAvgRows.
 template <typename TO, int SM, int SN, bool SWIGLU, bool SAVEGU = false, bool DSILU = false, bool BKM = false,
           bool MIDROWS = false, bool SLICED = false, bool AKM = false, bool ONCE = false>
 __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, unsigned char* smem,
@@ -1450,7 +1453,7 @@ __device__ __forceinline__ void grouped_gemm_dma16_body(const GroupedArgs& p, un
     }
 
     // first two slabs
-    const int k0 = ONCE && SWIGLU ? (int)(blockIdx.x % kNumXcd) * nk / kNumXcd : 0;
+    const int k0 = ONCE && SWIGLU ? (tc.e / p.sm * ((p.n_tiles + p.sn - 1) / p.sn) + tc.nt / p.sn) % kNumXcd * nk / kNumXcd : 0;
     const int k1 = k0 + 1 < nk ? k0 + 1 : nk > 1 ? 0 : k0;
     D16_ISSUE_B(k0, 0);
     D16_ISSUE_B(k1, B_STAGE);
@@ -1742,7 +1745,8 @@ static float tile_time(const TileCost& c, int64_t max_rows, int E, int n_cols, i
 // Two bounds on the choice keep results independent of the route that a training step takes: bfloat16 groups of more
 // than 192 rows always run on the 16 x 16 x 32 kernel and float32 groups of more than 256 rows are not sliced along K,
 // because the fused training launches and the K-major products, which start at those sizes, accumulate in that order
-// (their results equal those of the separate launches bit for bit).
+// (their results equal those of the separate launches bit for bit).  The gate/up product with its activation, which training does not
+// run (it rounds the pre-activations that it keeps), is outside of that: up to kOnceMaxAvgRows it begins K elsewhere.
 enum class GroupTile { kSmall32, kSmall64, kSeq, kMid, kBig };      // kSeq: 64 rows, all of K in a wave
 template <bool kBf16, bool SWIGLU>
 static GroupTile pick_group_tile(int64_t max_rows, int E, int N, int nk) {

@@ -56,7 +56,7 @@ def test_groups(gpu, counts, N, K, gather):
         _check(got[s], rows[s] @ w[e][:, :K].double().T, rows[s].abs() @ w[e][:, :K].double().abs().T, K)
 
 
-# (the last three on the 256-row tile whose XCDs begin an eighth of K apart: one slab, fewer and more than eight, a group of two tiles)
+# (the last three on the 256-row tile whose supertiles begin K an eighth apart: one slab, fewer and more than eight, a group of two tiles)
 @pytest.mark.parametrize("counts,I,K", [([31, 33, 64, 0, 65] * 4, 1000, 64), ([97, 128, 1, 96] * 4, 1032, 192), ([12, 129, 0, 20] * 8, 1096, 576),
                                         ([200, 256, 0, 300], 264, 64), ([223, 224, 225, 200], 1032, 320), ([130, 255, 257, 1, 410], 520, 1216)])
 def test_gate_up(gpu, counts, I, K):
@@ -77,6 +77,25 @@ def test_gate_up(gpu, counts, I, K):
         ref = gate * torch.sigmoid(gate) * up
         # (the exponential and the division of the sigmoid: 2^-20 of the value)
         _check(got[s], ref, 1.1 * mag[:, :I] * up.abs() + gate.abs() * mag[:, I:] + 2.0 ** 4 / K * ref.abs(), K)
+
+
+@pytest.mark.parametrize("rows,I,K", [(60, 1048, 1024), (200, 1048, 1024)])
+def test_gate_up_sums_do_not_depend_on_other_groups(gpu, rows, I, K):
+    """Band tiles and 256-row tiles that begin K out of step: an expert's rows have the same bits whatever the others get."""
+    from adaptivetrainingsystem_amd import ops
+    E = 24
+    g = torch.Generator().manual_seed(9)
+    w = [(torch.randn(2 * I, K, generator=g) * 0.05).bfloat16().to(gpu) for _ in range(E)]
+    x = torch.randn(E * rows, K, generator=g).bfloat16().to(gpu)
+    ptrs = ops.weight_pointer_table(w)
+    start = (torch.arange(E, dtype=torch.int32) * rows).to(gpu)
+    out = []
+    for none in ([], list(range(8)), [1, 9, 10, 11, 20]):
+        count = torch.tensor([0 if e in none else rows for e in range(E)], dtype=torch.int32, device=gpu)
+        out.append((none, ops.grouped_gateup_swiglu(x, ptrs, start, count, E * rows, E * rows, K, I).view(E, rows, I)))
+    for none, one in out[1:]:
+        for e in range(E):
+            assert e in none or torch.equal(one[e], out[0][1][e]), e
 
 
 @pytest.mark.parametrize("T,N,K", [(33, 1032, 512), (64, 4096, 1024), (65, 1032, 4096), (96, 2056, 2048), (97, 1032, 1024), (128, 3072, 2048), (129, 2056, 1024),
