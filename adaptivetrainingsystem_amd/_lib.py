@@ -73,6 +73,7 @@ _SIGNATURES = {
     "ats_wgrad_tn": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_void_p,
                              c_int, c_int, c_void_p]),
     "ats_down_k_slices": (c_int, [c_int, c_int64, c_int, c_int, c_int]),
+    "ats_grouped_gemm_route": (c_int, [c_int, c_int64, c_int, c_int, c_int, c_int, c_int]),
     "ats_linear_k_slices": (c_int, [c_int64, c_int, c_int]),
     "ats_grouped_gemm_nn_slices": (c_int, [c_int, c_int64, c_int, c_int, c_int64, c_int]),
     "ats_grouped_gemm_nn_sliced": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,

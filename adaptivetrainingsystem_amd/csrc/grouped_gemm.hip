@@ -1908,8 +1908,15 @@ static bool band_dense(int64_t rows, int N, int K) {
     return rows > 32 && band_time(rows, N, K, 1, band_height(rows, N, K, 1)) < other_dense_time(rows, N, K, true);
 }
 
+// The kernel of a launch.  Streams: panels of np * 16 weight rows, tiles of mt * 16 activation rows, kw waves along K.
+enum class Route { kSlices32, kSlices64, kSlices256, kBandSlices, kBand, kShort, kStream, kSmall32, kSmall64, kSeq, kMid, kBig };
+struct GroupedRoute {
+    Route kernel;
+    int np, mt, kw;
+};
+
 template <typename T, typename TO, bool SWIGLU>
-static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s) {
+static GroupedRoute grouped_route(const GroupedArgs& p, int64_t max_rows) {
     constexpr bool kBf16 = std::is_same<T, bf16_t>::value;
     constexpr int BK = 128 / (int)sizeof(T);
     const int E = p.E > 0 ? p.E : 1;
@@ -1921,7 +1928,7 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     if constexpr (kBf16 && !SWIGLU && std::is_same<TO, float>::value) {
         if (p.k_splits > 1 && band_ok && p.k_slice % 64 == 0 &&
             (E == 1 ? max_rows > 32 : (int64_t)E * p.N_out * p.K >= 1 << 24 && avg > 20 && band_groups(E, max_rows, band_tiles, p.k_splits, false)))
-            return launch_band<TO, false, true>(p, max_rows, E == 1 ? band_height(max_rows, p.N_out, p.K, p.k_splits) : kBandRows, s);
+            return {Route::kBandSlices};
     }
     if constexpr (!SWIGLU) {
         // K in slices over workgroups: 32-row tiles, 64-row tiles where up to 64 rows can stream the weights once
@@ -1929,17 +1936,15 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
             if constexpr (kBf16) {
                 if (E > 1 && avg > 20 && p.k_slice % 64 == 0 && p.a_extent_bytes != 0 && p.b_extent_bytes != 0 && !p.k_count &&
                     large_slice_tile(E, max_rows, p.N_out, p.k_slice * p.k_splits, p.k_splits))
-                    return launch_mid_sliced<>(p, max_rows, s);
+                    return {Route::kSlices256};
             }
-            return avg > 32 ? launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s)
-                            : launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+            return {avg > 32 ? Route::kSlices64 : Route::kSlices32};
         }
     }
     if constexpr (kBf16) {
-        if (band_ok && E > 1 && band_groups(E, max_rows, band_tiles, 1, SWIGLU)) return launch_band<TO, SWIGLU, false>(p, max_rows, kBandRows, s);
+        if (band_ok && E > 1 && band_groups(E, max_rows, band_tiles, 1, SWIGLU)) return {Route::kBand};
         if constexpr (!SWIGLU) {
-            if (band_ok && E == 1 && band_dense(max_rows, p.N_out, p.K))
-                return launch_band<TO, false, false>(p, max_rows, band_height(max_rows, p.N_out, p.K, 1), s);
+            if (band_ok && E == 1 && band_dense(max_rows, p.N_out, p.K)) return {Route::kBand};
         }
     }
     // (with a K per group, p.K is the bound on their sum)
@@ -1947,7 +1952,7 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
     if constexpr (kBf16 && !SWIGLU && std::is_same<TO, bf16_t>::value) {
         // weight gradients over up to 512 padded rows per group that are large enough to fill the chip four deep
         if (p.k_count && !p.a_rows && nk <= 8 && (int64_t)E * ((avg + kShortBM - 1) / kShortBM) * ((p.N_out + kShortBN - 1) / kShortBN) >= 2048)
-            return launch_short(p, max_rows, s);
+            return {Route::kShort};
     }
     // Few rows per group: a stream of weights (E == 1: the row count is exact; several groups vary around their mean, and
     // a group beyond 32 rows reads its weights twice).  Measured, microseconds, weights from HBM, against the register-
@@ -1961,15 +1966,8 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
         // (tiles of 16 activation rows for few rows per group: half of the registers for them; gate/up [2816, 2048] x 64, 24 tokens
         // with the down projection 179 -> 175 us, [28672, 4096] x 8, 1 token 129.5 -> 126.5.  A group beyond 16 rows reads its weights
         // twice: 8 experts with 16 rows each 457 -> 555 us, hence the bound well below them.)
-        auto panels = [&](auto np, auto kw) {
-            constexpr int NP = decltype(np)::value, KW = decltype(kw)::value;
-            return avg <= 4 ? launch_stream<T, TO, NP, 1, KW, SWIGLU>(p, max_rows, s) : launch_stream<T, TO, NP, 2, KW, SWIGLU>(p, max_rows, s);
-        };
-        typedef std::integral_constant<int, 1> One;
-        typedef std::integral_constant<int, 2> Two;
-        typedef std::integral_constant<int, 4> Four;
-        typedef std::integral_constant<int, 8> Eight;
-        if constexpr (SWIGLU) return panels(Two{}, Four{});
+        const int mt = avg <= 4 ? 1 : 2;
+        if constexpr (SWIGLU) return {Route::kStream, 2, mt, 4};
         else {
             // Eight waves split K where there are at least four pieces for each (a panel of 16 rows then reads 2 KB of
             // every row per step): [4096, 4096] x 16 rows 10.3 us against 11.7 with four waves and 14.5 with four waves
@@ -1977,26 +1975,71 @@ static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s)
             // (8 experts x 16 rows, [4096, 14336]: 157 against 167).  A short K keeps four waves (64 experts, [2048, 1408],
             // 3 tokens: 23 against 37 us).
             const int64_t groups = max_rows < E ? max_rows : E;
-            if (pieces >= 32 && (pieces >= 64 || groups * p.N_out <= 16 * 1024)) {
-                if (E == 1 || avg <= 8) return panels(One{}, Eight{});
-                return panels(Two{}, Eight{});
-            }
-            if (groups * p.N_out < 32 * 256) return panels(One{}, Four{});
-            return panels(Two{}, Four{});
+            if (pieces >= 32 && (pieces >= 64 || groups * p.N_out <= 16 * 1024)) return {Route::kStream, E == 1 || avg <= 8 ? 1 : 2, mt, 8};
+            return {Route::kStream, groups * p.N_out < 32 * 256 ? 1 : 2, mt, 4};
         }
     }
     if constexpr (!SWIGLU) {
-        if (streams_long_k(avg, pieces, p.N_out) && !p.k_count) return launch_stream<T, TO, 2, 4, 4, SWIGLU>(p, max_rows, s);
+        if (streams_long_k(avg, pieces, p.N_out) && !p.k_count) return {Route::kStream, 2, 4, 4};
     }
-    const GroupTile tile = pick_group_tile<kBf16, SWIGLU>(max_rows, E, p.N_out, nk);
-    if (tile == GroupTile::kSmall32) return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
-    if (tile == GroupTile::kSmall64) return launch_small<T, TO, 2, 2, 4, 1, SWIGLU>(p, max_rows, s);
-    if constexpr (!kBf16) {
-        if (tile == GroupTile::kSeq) return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 1, 2, SWIGLU>(p, max_rows, s);
+    switch (pick_group_tile<kBf16, SWIGLU>(max_rows, E, p.N_out, nk)) {
+        case GroupTile::kSmall32: return {Route::kSmall32};
+        case GroupTile::kSmall64: return {Route::kSmall64};
+        case GroupTile::kSeq: return {Route::kSeq};
+        case GroupTile::kMid: return {Route::kMid};
+        default: return {Route::kBig};
     }
-    if (tile == GroupTile::kMid) {
-        if constexpr (SWIGLU) return launch_cfg<T, TO, 128, 128, 2, 2, 4, 8, SWIGLU>(p, max_rows, s);
-        else return launch_cfg<T, TO, 128, 256, 2, 4, 4, 8, SWIGLU>(p, max_rows, s);
+}
+
+template <typename T, typename TO, bool SWIGLU>
+static int launch_grouped(const GroupedArgs& p, int64_t max_rows, hipStream_t s) {
+    constexpr bool kBf16 = std::is_same<T, bf16_t>::value, kF32Out = std::is_same<TO, float>::value;
+    const GroupedRoute r = grouped_route<T, TO, SWIGLU>(p, max_rows);
+    switch (r.kernel) {
+        case Route::kBandSlices:
+            if constexpr (kBf16 && !SWIGLU && kF32Out)
+                return launch_band<TO, false, true>(p, max_rows, p.E <= 1 ? band_height(max_rows, p.N_out, p.K, p.k_splits) : kBandRows, s);
+            break;
+        case Route::kSlices256:
+            if constexpr (kBf16 && !SWIGLU) return launch_mid_sliced<>(p, max_rows, s);
+            break;
+        case Route::kSlices64:
+            if constexpr (!SWIGLU) return launch_cfg<T, TO, 64, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+            break;
+        case Route::kSlices32:
+            if constexpr (!SWIGLU) return launch_cfg<T, TO, 32, 128, 1, 4, 1, 32, SWIGLU>(p, max_rows, s);
+            break;
+        case Route::kBand:
+            if constexpr (kBf16) return launch_band<TO, SWIGLU, false>(p, max_rows, p.E <= 1 ? band_height(max_rows, p.N_out, p.K, 1) : kBandRows, s);
+            break;
+        case Route::kShort:
+            if constexpr (kBf16 && !SWIGLU && !kF32Out) return launch_short(p, max_rows, s);
+            break;
+        case Route::kStream: {
+            auto panels = [&](auto np, auto kw) {
+                constexpr int NP = decltype(np)::value, KW = decltype(kw)::value;
+                return r.mt == 1 ? launch_stream<T, TO, NP, 1, KW, SWIGLU>(p, max_rows, s) : launch_stream<T, TO, NP, 2, KW, SWIGLU>(p, max_rows, s);
+            };
+            typedef std::integral_constant<int, 1> One;
+            typedef std::integral_constant<int, 2> Two;
+            typedef std::integral_constant<int, 4> Four;
+            typedef std::integral_constant<int, 8> Eight;
+            if constexpr (SWIGLU) return panels(Two{}, Four{});
+            else {
+                if (r.mt == 4) return launch_stream<T, TO, 2, 4, 4, SWIGLU>(p, max_rows, s);
+                if (r.kw == 8) return r.np == 1 ? panels(One{}, Eight{}) : panels(Two{}, Eight{});
+                return r.np == 1 ? panels(One{}, Four{}) : panels(Two{}, Four{});
+            }
+        }
+        case Route::kSmall32: return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 4, 1, SWIGLU>(p, max_rows, s);
+        case Route::kSmall64: return launch_small<T, TO, 2, 2, 4, 1, SWIGLU>(p, max_rows, s);
+        case Route::kSeq:
+            if constexpr (!kBf16) return launch_small<T, TO, 1, SWIGLU ? 2 : 1, 1, 2, SWIGLU>(p, max_rows, s);
+            break;
+        case Route::kMid:
+            if constexpr (SWIGLU) return launch_cfg<T, TO, 128, 128, 2, 2, 4, 8, SWIGLU>(p, max_rows, s);
+            else return launch_cfg<T, TO, 128, 256, 2, 4, 4, 8, SWIGLU>(p, max_rows, s);
+        case Route::kBig: break;
     }
     // 256 x 256 tile, 8 waves (2 per SIMD: one wave's LDS / memory waits are covered by the other's MFMAs), 128
     // accumulator registers per lane.
@@ -2216,6 +2259,29 @@ static int check_common(const char* name, const void* a, const void* const* w, c
 }
 
 }  // namespace ats
+
+extern "C" int ats_grouped_gemm_route(int E, int64_t max_rows, int N, int K, int k_splits, int swiglu, int out_dtype) {
+    using namespace ats;
+    if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || k_splits < 1 || K % k_splits != 0 || (swiglu && k_splits > 1)) return -1;
+    GroupedArgs p{};
+    p.E = E;
+    p.N_out = N;
+    p.K = K;
+    p.k_splits = k_splits;
+    p.k_slice = K / k_splits;
+    p.a_extent_bytes = p.b_extent_bytes = 0xffffffffu;
+    const Route r = (swiglu ? grouped_route<bf16_t, bf16_t, true>(p, max_rows) : out_dtype == ATS_F32 ? grouped_route<bf16_t, float, false>(p, max_rows)
+                                                                                                 : grouped_route<bf16_t, bf16_t, false>(p, max_rows)).kernel;
+    switch (r) {
+        case Route::kBand:
+        case Route::kBandSlices: return ATS_ROUTE_BAND;
+        case Route::kStream: return ATS_ROUTE_STREAM;
+        case Route::kBig: return swiglu && K % 64 == 0 && E > 1 && max_rows / E <= kOnceMaxAvgRows ? ATS_ROUTE_256_ONCE : ATS_ROUTE_256;
+        case Route::kSlices256: return max_rows / E <= kOnceMaxAvgRows ? ATS_ROUTE_256_ONCE : ATS_ROUTE_256;
+        case Route::kMid: return ATS_ROUTE_128;
+        default: return ATS_ROUTE_SMALL;
+    }
+}
 
 extern "C" int ats_grouped_gateup_swiglu_save_supported(int64_t a_num_rows, int E, int64_t max_rows, int H, int I,
                                                         int dtype) {

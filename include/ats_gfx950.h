@@ -254,6 +254,17 @@ int ats_grouped_down_splitk(const void* h, const void* const* w_d, float* parts,
  * weights or more is estimated to take the least time, ats_combine_partials included; 1: ats_grouped_down.  small: the slices with
  * which 32 or 64-row tiles fill the chip. */
 int ats_down_k_slices(int E, int64_t max_rows, int H, int I, int small);
+/* The kernel that a bfloat16 product of up to max_rows rows with E [N, K] weights runs on (ats_grouped_gemm_nt; k_splits > 1:
+ * ats_grouped_down_splitk; swiglu: ats_grouped_gateup_swiglu with N = I), operands below 4 GiB; -1 for arguments that none takes. */
+enum {
+    ATS_ROUTE_STREAM = 0,   /* streams of weights */
+    ATS_ROUTE_SMALL,        /* register-staged tiles of up to 64 rows */
+    ATS_ROUTE_BAND,         /* 128 x 128 tiles, weights straight to LDS */
+    ATS_ROUTE_128,          /* 128-row tiles */
+    ATS_ROUTE_256,          /* 256-row tiles */
+    ATS_ROUTE_256_ONCE      /* 256-row tiles, weights past the caches */
+};
+int ats_grouped_gemm_route(int E, int64_t max_rows, int N, int K, int k_splits, int swiglu, int out_dtype);
 /* Slices of K with which ats_grouped_down_splitk and ats_sum_partials multiply `rows` rows by one bfloat16 [N, K] weight
  * fastest; 1: ats_linear_nt does. */
 int ats_linear_k_slices(int64_t rows, int N, int K);
