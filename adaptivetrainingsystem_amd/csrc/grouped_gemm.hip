@@ -1890,33 +1890,46 @@ static bool band_groups(int E, int64_t max_rows, int n_tiles, int slices, bool s
     return used * n_tiles * slices >= 200.f;
 }
 // One group of more than 32 rows x [N, K]: the band tiles' time in microseconds, plain or with s slices of K and their sum, by the
-// tiles' most rows h; 109 measured points of [2048 .. 6144] x [2048, 4096] within 8 % (root mean square), the choice between them costs
-// 2 % on average.  A CU takes one slab of a tile in slab1 alone and in slabn as one of several.
+// tiles' most rows h.  A CU takes one slab of a tile in slab1 alone and in slabn as one of several.  Fitted to 1900 launches of 33 .. 1000
+// rows x [512 .. 32000, 512 .. 14336], weights from HBM, within 6 % (root mean square; 22 % at most).
 static float band_time(int64_t rows, int N, int K, int s, int h) {
-    constexpr float slab1[] = {0.40f, 0.44f, 0.53f, 0.63f}, slabn[] = {0.30f, 0.36f, 0.42f, 0.49f};      // 32, 64, 96, 128 rows
+    constexpr float slab1[] = {0.44f, 0.55f, 0.67f}, slabn[] = {0.44f, 0.48f, 0.54f};      // up to 64, 96, 128 rows
     const int64_t m_tiles = (rows + h - 1) / h;
-    const int f = (int)((rows + m_tiles - 1) / m_tiles + 31) / 32 - 1;
+    const int f = std::max((int)((rows + m_tiles - 1) / m_tiles + 31) / 32 - 2, 0);
     const float per_cu = (float)(m_tiles * ((N + kBandCols - 1) / kBandCols) * s) / 256.f;
     const float slab = per_cu <= 1.f ? slab1[f] : slabn[f] * 0.5f * (per_cu + ceilf(per_cu));
-    const float chain = K / 64.f / s * slab, weights = (float)N * K * 2e-6f / 7.f;
-    return 5.f + sqrtf(chain * chain + weights * weights) + (s > 1 ? (float)rows * N * (8 * s - 4) / 4.5e6f + 3.f : 0.f);
+    const float chain = K / 64.f / s * slab, weights = (float)N * K * 2e-6f / (per_cu <= 1.f ? 5.6f : 6.1f);
+    return 3.6f + sqrtf(chain * chain + weights * weights) + (s > 1 ? (float)rows * N * (8 * s - 4) / 4.75e6f + 2.7f : 0.f);
 }
 static int band_height(int64_t rows, int N, int K, int s) {
     return rows > 64 && band_time(rows, N, K, s, 128) < band_time(rows, N, K, s, 64) ? 128 : 64;
 }
-// The same rows on the other tiles: half a chip of 64 x 64 tiles with K split in the workgroup ([2048, 2048] x 128 rows 10.4 us, [4096,
-// 4096] 20.8; with more of them 38: [6144, 4096]) or the 256-column tiles (10 % off).
-static float other_dense_time(int64_t rows, int N, int K, bool small) {
+// The same rows on the tile that pick_group_tile takes for them: up to 192 rows the register-staged ones, two workgroups of which share a
+// CU (the launches above, within 9 %), beyond that the 256-column tile.  What the choice between the two and the slices costs over those
+// launches is 0.8 % on average, 18 % at most (with the constants of 109 points of [2048 .. 6144] x [2048, 4096], and small tiles also
+// beyond 192 rows, where none run: 5.6 %, 140 %).  Microseconds, band tiles <- other: 200 rows x [512, 512] 6.9 <- 10.5, [1024, 1024] 10.3 <- 15.0,
+// 512 x [1024, 4096] 32 <- 56, 100 x [32000, 4096] 67 <- 91; other <- band tiles: 160 x [3072, 1024] 9.0 <- 10.6, 64 x [2048, 2048] 9.5 <- 17.
+static float other_dense_time(int64_t rows, int N, int K) {
+    const float slabs = K / 64.f, weights = (float)N * K * 2e-6f;
+    switch (pick_group_tile<true, false>(rows, 1, N, (K + 63) / 64)) {
+        case GroupTile::kSmall32: {
+            const float half = (float)((rows + 31) / 32 * ((N + 31) / 32)) / 512.f;
+            const float chain = slabs * (0.166f + 0.068f * fminf(half, 1.f)) * ceilf(half);
+            return 3.9f + powf(powf(chain, 3.2f) + powf(weights / 2.41f, 3.2f), 1.f / 3.2f);
+        }
+        case GroupTile::kSmall64: return 4.4f + slabs * 0.318f * ceilf((float)((rows + 63) / 64 * ((N + 63) / 64)) / 512.f) + weights / 6.2f;
+        case GroupTile::kMid: return 4.f + weights / 3.f;
+        default: break;
+    }
     float best;
     int sm, sn;
     const int n_tiles = (N + 255) / 256;
     pick_supertile(n_tiles, &sm, &sn);
     dense_tile_rows(rows, n_tiles, K / 64, sm, sn, &best);
-    if (small && (rows + 63) / 64 * ((N + 63) / 64) <= 128) best = fminf(best, 2.f + K / 64 * 0.28f);
-    return best;
+    return 1.1f * best;      // (the heights are held against each other there, not against other kernels: 300 x [12288, 4096] 62 us for 55)
 }
 static bool band_dense(int64_t rows, int N, int K) {
-    return rows > 32 && band_time(rows, N, K, 1, band_height(rows, N, K, 1)) < other_dense_time(rows, N, K, true);
+    return rows > 32 && band_time(rows, N, K, 1, band_height(rows, N, K, 1)) < other_dense_time(rows, N, K);
 }
 
 // The kernel of a launch.  Streams: panels of np * 16 weight rows, tiles of mt * 16 activation rows, kw waves along K.
@@ -2543,7 +2556,11 @@ extern "C" int ats_linear_k_slices(int64_t rows, int N, int K) {
     if (rows <= 32 || rows > 256 || N <= 0 || K <= 0 || K % 64 != 0) return 1;
     // (against a long K slices on the band tiles are as fast as the small tiles: [4096, 4096] x 100 rows 19 and 20 us, 128 rows 22 and 21;
     // and a rotation behind the product adds them up on its way)
-    float best = fminf(band_time(rows, N, K, 1, band_height(rows, N, K, 1)), other_dense_time(rows, N, K, K <= 2048));
+    float best = band_time(rows, N, K, 1, band_height(rows, N, K, 1));
+    if (K <= 2048 || rows > 192) best = fminf(best, other_dense_time(rows, N, K));
+    // (below that the second launch is what a caller waits for: [2048, 2048] x 40 rows 8.9 plain, 10.1 in slices behind other launches,
+    // 10.9 and 9.8 each by itself)
+    if (best < 13.f) return 1;
     int slices = 1;
     for (int s = 2; s <= 8 && K % (s * 64) == 0 && K / s >= 256; s *= 2) {
         const float t = band_time(rows, N, K, s, band_height(rows, N, K, s));

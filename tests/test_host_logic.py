@@ -431,3 +431,16 @@ def test_weights_go_past_the_caches_only_where_they_are_larger():
         for avg in (200, 224):
             assert route(E, E * avg, N, K, slices, swiglu, _lib.ATS_F32 if slices > 1 else _lib.ATS_BF16) == want, (E, N, K, avg)
         assert route(E, E * 225, N, K, slices, swiglu, _lib.ATS_F32 if slices > 1 else _lib.ATS_BF16) == rows256
+
+
+@pytest.mark.parametrize("rows,N,K,slices,route", [
+    (200, 512, 512, 1, "band"), (512, 512, 512, 1, "band"), (400, 1024, 1024, 1, "band"), (300, 1000, 1536, 1, "band"), (512, 1024, 4096, 1, "band"),
+    (100, 32000, 4096, 1, "band"), (200, 1536, 512, 1, "band"), (300, 12288, 4096, 1, "band"), (160, 3072, 1024, 1, "small"), (64, 2048, 2048, 1, "small"),
+    (100, 1024, 1024, 1, "small"), (128, 2048, 1408, 1, "small"), (200, 1024, 1024, 1, "band"), (200, 1000, 1536, 4, None), (256, 2048, 1408, 2, None), (200, 2048, 2048, 4, None),
+    (256, 2048, 2048, 4, None), (64, 6144, 4096, 4, None), (64, 4096, 4096, 8, None), (100, 4096, 14336, 8, None), (64, 3072, 2048, 1, "small")])
+def test_route_of_one_weight(rows, N, K, slices, route):
+    """The fastest of every route measured alone, or within 10 % of it (band tiles, slices of K, other tiles; weights from HBM)."""
+    from adaptivetrainingsystem_amd import _lib, ops
+    assert ops.linear_k_splits(rows, N, K, torch.bfloat16) == slices
+    if route:
+        assert _lib.load().ats_grouped_gemm_route(1, rows, N, K, 1, 0, _lib.ATS_BF16) == {"small": 1, "band": 2, "256": 4}[route]
