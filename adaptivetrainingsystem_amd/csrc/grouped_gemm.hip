@@ -1564,14 +1564,14 @@ constexpr int64_t kOnceMaxAvgRows = 224;
 // The ONCE instance.  Only the mean of the groups is known here.  With sizes that fall as rank^-1.5 the larger ones take two or three tiles
 // and load their weights non-temporally in each, and it still gains where the weights are large: 110 .. 222 rows on average, gate/up 8 x
 // [28672, 4096] 0.96 .. 1.00 of the time, 64 x [2816, 2048] 0.94 .. 0.97, 12 x [8192, 3072] 1.00 .. 1.03, sliced down 8 x [4096, 14336]
-// 0.91 .. 0.95, 16 x [2048, 5632] 0.95 .. 0.98 (equal chances: 0.90 .. 0.98, 0.80 .. 0.94, 0.93 .. 0.97, 0.86 .. 0.95, 0.84 .. 0.94).  Less than
-// a last-level cache of weights (256 MB) gains nothing and loses where the sizes differ: sliced 8 x [1024, 2816] 31.3 -> 35.1 us, equal
-// chances 41.3 -> 41.5; gate/up 8 x [5632, 1024] 45.0 -> 46.4, equal 31.0 -> 30.5.  (A choice per group inside the kernel, as the band
-// tiles make it, costs more than it saves: with both bodies, or with a branch at the loads, registers spill and skewed groups take 1.1 .. 1.9
-// times as long.)
-static bool once_weights(int64_t max_rows, int E, int64_t weight_rows, int K) {
-    return E > 1 && max_rows / E <= kOnceMaxAvgRows && E * weight_rows * K >= (int64_t)1 << 27;
-}
+// 0.91 .. 0.95, 16 x [2048, 5632] 0.95 .. 0.98 (equal chances: 0.90 .. 0.98, 0.80 .. 0.94, 0.93 .. 0.97, 0.86 .. 0.95, 0.84 .. 0.94).  Sliced
+// products of less than a last-level cache of weights (256 MB) gain nothing and lose where the sizes differ: 8 x [1024, 2816] 31.3 -> 35.1
+// us, equal chances 41.3 -> 41.5.  Small gate/up products by themselves are even (8 x [5632, 1024] 31.0 -> 30.5, 45.0 -> 46.4), but leave the
+// cache to the down projection behind them: the layer 82 -> 76 us, 98 -> 95.  (A choice per group inside the kernel, as the band tiles make
+// it, costs more than it saves: with both bodies, or with a branch at the loads, registers spill and skewed groups take 1.1 .. 1.9 times as
+// long.)
+static bool once_weights(int64_t max_rows, int E) { return E > 1 && max_rows / E <= kOnceMaxAvgRows; }
+static bool once_slices(int64_t max_rows, int E, int N, int K) { return once_weights(max_rows, E) && (int64_t)E * N * K >= (int64_t)1 << 27; }
 static bool mid_rows(int64_t max_rows, int E) { return max_rows / (E > 0 ? E : 1) < kMidRowsMaxAvg; }
 // Tiles of the busiest CU.  Supertile S runs on XCD S % 8; the last band of rows and the last one of columns hold fewer than 32 tiles
 // (18 x 43 tiles of 256 rows: 33 supertiles, five for XCD 0, of which one has eight tiles and the others leave it four rounds).
@@ -1686,7 +1686,7 @@ static int launch_cfg(const GroupedArgs& p0, int64_t max_rows, hipStream_t s) {
         set_error("grouped GEMM: grid of %lld blocks", (long long)blocks);
         return ATS_ERR_UNSUPPORTED;
     }
-    const bool once = once_weights(max_rows, p.E, SWIGLU ? 2 * (int64_t)p.N_out : p.N_out, p.K);
+    const bool once = once_weights(max_rows, p.E);
     auto kern = dma_ok ? (once ? kern_once : p.tile_rows || mid_rows(max_rows, p.E) ? kern_mid : kern_dma) : (p.K % BK == 0) ? kern_pipe : kern_general;
     const size_t smem_launch = (!dma_ok && p.K % BK == 0) ? smem_staged : smem;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WM * WN * 64), smem_launch, s, p);
@@ -1704,7 +1704,7 @@ static int launch_mid_sliced(const GroupedArgs& p0, int64_t max_rows, hipStream_
     constexpr size_t smem = dma_lds_bytes(256, 256);
     auto kern_many = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, BKM, true, true>;
     auto kern_once = grouped_gemm_dma16_kernel<float, 4, 8, false, false, false, BKM, true, true, false, !BKM>;
-    auto kern = once_weights(max_rows, p.E, p.N_out, p.K) ? kern_once : kern_many;
+    auto kern = once_slices(max_rows, p.E, p.N_out, p.K) ? kern_once : kern_many;
     static LdsReservation reserved;
     hipError_t e = reserve_lds(reserved, {reinterpret_cast<const void*>(kern_many), reinterpret_cast<const void*>(kern_once)}, (int)smem);
     if (e != hipSuccess) {
@@ -2300,8 +2300,8 @@ extern "C" int ats_grouped_gemm_route(int E, int64_t max_rows, int N, int K, int
         case Route::kBand:
         case Route::kBandSlices: return ATS_ROUTE_BAND;
         case Route::kStream: return ATS_ROUTE_STREAM;
-        case Route::kBig: return swiglu && K % 64 == 0 && once_weights(max_rows, E, 2 * (int64_t)N, K) ? ATS_ROUTE_256_ONCE : ATS_ROUTE_256;
-        case Route::kSlices256: return once_weights(max_rows, E, N, K) ? ATS_ROUTE_256_ONCE : ATS_ROUTE_256;
+        case Route::kBig: return swiglu && K % 64 == 0 && once_weights(max_rows, E) ? ATS_ROUTE_256_ONCE : ATS_ROUTE_256;
+        case Route::kSlices256: return once_slices(max_rows, E, N, K) ? ATS_ROUTE_256_ONCE : ATS_ROUTE_256;
         case Route::kMid: return ATS_ROUTE_128;
         default: return ATS_ROUTE_SMALL;
     }
