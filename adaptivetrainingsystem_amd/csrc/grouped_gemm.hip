@@ -1851,6 +1851,21 @@ struct SliceEstimate {
         const float chain = n * (0.325f + 0.377f * pc + (pc > 2.12f ? 0.367f : 0.f)) + 0.077f * pc + 1.02f * empty;
         return 8.6f + powf(powf(chain, 1.36f) + powf(weights / 9.7f, 1.36f), 1.f / 1.36f) + partials * s / 13.5f;
     }
+    // The band tiles, where band_groups takes them: one tile to a CU or several, whose slabs then follow one another.  Fitted to 791 points
+    // of groups with equal chances, 2 .. 64 experts of 21 .. 100 rows on average, [768 .. 5120, 1408 .. 14336] weights, within 5 % (18 % at
+    // most).  Where plain tiles just fill the CUs once, sizes that differ more give some of them a second one: with sizes that fall as
+    // rank^-1.5, 8 x [4096, 14336] of 50 rows take 226 us plain and 193 in two slices, with equal chances 154 and 164.  Hence 11 % on such
+    // launches: what is chosen is 1.4 % slower than the fastest of every route with equal chances and 3.5 % with such sizes (by the
+    // estimates of the tiles that ran there before 6 and 7 %, without the 11 % 0.8 and 6).
+    float band(int s) const {
+        const float used = E * (1.f - expf(-avg)) * (1.f + 1.f / (1.f + expf(1.7f / sqrtf(avg) * (128.f - avg))));
+        const float pc = used * ((N + kBandCols - 1) / kBandCols) * s / 256.f;
+        const bool alone = pc <= 1.02f;
+        const float slab = alone ? 0.481f + 0.0022f * avg : (0.431f + 0.0021f * avg) * (0.07f * pc + 0.93f * ceilf(pc - 0.02f));
+        const float chain = slabs / s * slab, load = weights / (alone ? 6.9f : 6.24f);
+        const float time = 8.3f + powf(powf(chain, 5.f) + powf(load, 5.f), 0.2f) + (s > 1 ? 2.6f + partials * s / 5.43f : partials / 6.46f);
+        return s == 1 && alone && pc > 0.8f ? 1.11f * time : time;
+    }
     float plain() const {
         if (streams_long_k(max_rows / E, K * 2 / 256, N)) return 8.65f + join(slabs * 0.172f, weights / 5.3f);
         switch (pick_group_tile<true, false>(max_rows, E, N, (K + 63) / 64)) {
@@ -2535,15 +2550,22 @@ extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K, int smal
     using namespace ats;
     if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || small < 1) return 1;
     const SliceEstimate t(E, max_rows, N, K);
-    float best = t.plain();
+    auto band = [&](int s) {
+        return E > 1 && max_rows / E > 20 && K % (s * 64) == 0 && band_groups(E, max_rows, (N + kBandCols - 1) / kBandCols, s, false);
+    };
+    float best = band(1) ? t.band(1) : t.plain();
     int slices = 1;
-    if (small > 1 && t.small(small) <= best) {
+    if (small > 1 && !band(small) && t.small(small) <= best) {
         best = t.small(small);
         slices = small;
     }
     for (int s = 2; s <= 16 && K % (s * 64) == 0 && K / s >= 512; s *= 2) {
-        if (t.large_with_margin(s) < best && large_slice_tile(E, max_rows, N, K, s)) {
-            best = t.large_with_margin(s);
+        const bool on_band = band(s);
+        if (!on_band && !large_slice_tile(E, max_rows, N, K, s)) continue;
+        // (0.7: against another fit than its own; 8 x [1024, 2048], 44 rows 16.6 us plain, 17.3 in four slices)
+        const float time = on_band ? t.band(s) + (band(1) ? 0.f : 0.7f) : t.large_with_margin(s);
+        if (time < best) {
+            best = time;
             slices = s;
         }
     }

@@ -617,20 +617,21 @@ def down_k_splits(E: int, max_rows: int, N: int, K: int, dtype: torch.dtype) -> 
     x 256 rows 51 -> 23 us with 2; [4096, 14336] x 64 rows 156 -> 22 us with 8).
     Powers of two up to 16, slices of at least 512 columns, at most 256 rows per expert.
 
-    bfloat16 experts of more than 20 rows against 32 MB of weights or more: those slices or the plain launch, or slices on the
-    direct-to-LDS tile (up to 256 rows x 256 columns, one per CU), whichever is estimated to take the least time
-    (ats_down_k_slices).  Measured with the combine behind it, weights from HBM, rows per expert 22 | 32 | 48 | 64 | 96 | 128 | 192 |
-    224, without that tile and the estimate -> with them, microseconds:
-      8 x [4096, 14336]  164 -> 173 | 197 -> 175 | 194 -> 177 | 261 -> 181 | 265 -> 185 | 269 -> 192 | 253 -> 216 | 324 -> 224
-      4 x [4096, 14336]   91        | 111 ->  92 | 100 ->  94 | 143 ->  98 | 213 -> 103 | 187 -> 108 | 245 -> 125 | 308 -> 135
-      2 x [4096, 14336]   51        |  54        |  55        |  56        |  87 ->  58 |  88 ->  59 | 135 ->  83 | 239 ->  74
-      16 x [2048, 8192]  136 ->  98 | 132 -> 107 | 116        | 153 -> 142 | 167 -> 147 | 158 -> 152 | 167        | 198 -> 173
-      16 x [2048, 5632]   79 ->  73 |  88 ->  75 |  79        | 112 ->  81 | 111 ->  88 | 142 ->  93 | 111 -> 106 | 139 -> 164
-      4 x [1024, 8192]    33        |  36 ->  33 |  29        |  33 ->  35 |  38 ->  36 |  41 ->  37 |  54 ->  47 |  61 ->  49
-      2 x [1024, 16384]   34        |  35        |  32        |  33        |  39        |  42 ->  46 |  46 ->  51 |  60 ->  55
-      8 x [1024, 4096]    26        |  32 ->  26 |  26        |  32 ->  30 |  36 ->  30 |  38 ->  40 |  47 ->  41 |  83 ->  50
-      64 x [2048, 1408] stays as it was, plain
-    5599 random points, K from 1024 to 16384: 10 % less time on average (K from 4096: 14 %), 4 % of them more than 4 % slower.
+    bfloat16 experts of more than 20 rows against 32 MB of weights or more: those slices or the plain launch, slices on the band tiles
+    (up to 72 rows on average, 100 with many experts) or on the direct-to-LDS tile (up to 256 rows x 256 columns, one per CU), whichever
+    is estimated to take the least time (ats_down_k_slices).  Measured with the combine behind it, weights from HBM, rows per expert
+    24 | 32 | 48 | 64 | 72 | 96 | 128 | 192 | 224, plain -> in the slices that are chosen, microseconds:
+      8 x [4096, 14336]  160 -> 159 | 161 -> 164 | 164 | 173 -> 170 | 179 -> 172 | 267 -> 169 | 262 -> 169 | 264 -> 191 | 331 -> 222
+      4 x [4096, 14336]  97 -> 90 | 104 -> 90 | 97 -> 85 | 126 -> 90 | 184 -> 92 | 227 -> 94 | 191 -> 102 | 239 -> 141 | 279 -> 178
+      2 x [4096, 14336]  60 -> 47 | 67 -> 48 | 72 -> 50 | 99 -> 53 | 106 -> 53 | 116 -> 64
+      16 x [2048, 8192]  102 -> 105 | 101 -> 102 | 107 -> 106 | 109 -> 111 | 110 -> 112 | 168 -> 142 | 162 -> 133 | 162 -> 141 | 198 -> 156
+      16 x [2048, 5632]  66 -> 68 | 69 -> 71 | 73 -> 76 | 75 -> 78 | 77 -> 83 | 121 -> 81 | 147 -> 83 | 117 -> 110 | 143 -> 115
+      8 x [2048, 5632]   43 -> 39 | 49 -> 39 | 46 -> 40 | 64 -> 43 | 64 -> 44 | 64 -> 52 | 88 -> 53 | 100 -> 72 | 132 -> 76
+      4 x [1024, 8192]   32 -> 23 | 37 -> 24 | 35 -> 26 | 37 -> 27 | 38 -> 27 | 38 -> 36 | 44 -> 38 | 61 -> 47 | 135 -> 44
+      8 x [1024, 4096]   24 -> 21 | 25 -> 21 | 25 -> 23 | 31 -> 23 | 31 -> 25 | 31 | 40 | 43 | 85 -> 50
+      64 x [2048, 1408]  plain everywhere
+    (all with equal chances for every expert; slices that gain nothing with these gain a fifth where sizes fall as rank^-1.5).  385
+    points, 2-64 experts of 21-100 rows: 1.4 % slower than the fastest of all routes on average.
     Below 32 MB of weights everything comes from the last-level cache and the first rule stands."""
     slab = 64 if dtype == torch.bfloat16 else 32
     if E <= 0 or max_rows <= 0:
