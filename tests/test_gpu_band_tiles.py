@@ -137,6 +137,19 @@ def test_one_group(gpu, T, N, K, route):
                 _check(parts[i], x[:, k].double() @ w[:, k].double().T, x[:, k].double().abs() @ w[:, k].double().abs().T, K // s, rounded=False)
 
 
+# one float32 chain of K is 4.7e-7, 7.6e-7 and 4.0e-7 off here (standard normal operands), four of them 2.2e-7, 3.7e-7 and 1.9e-7
+@pytest.mark.parametrize("E,rows,N,K,most", [(16, 48, 2048, 5632, 3.2e-7), (8, 32, 4096, 14336, 5.3e-7), (1, 150, 6144, 4096, 2.8e-7)])
+def test_float32_results_keep_four_chains(gpu, E, rows, N, K, most):
+    from adaptivetrainingsystem_amd import ops
+    g = torch.Generator(device=gpu).manual_seed(E)
+    w = [torch.randn(N, K, generator=g, device=gpu).bfloat16() for _ in range(E)]
+    x = torch.randn(E * rows, K, generator=g, device=gpu).bfloat16()
+    start, count = (torch.arange(E, dtype=torch.int32) * rows).to(gpu), torch.full((E,), rows, dtype=torch.int32, device=gpu)
+    got = ops.grouped_gemm_nt(ops.weight_pointer_table(w), K, N, start, count, E * rows, E * rows, N, K, a=x, out_dtype=torch.float32)
+    ref = torch.cat([x[e * rows:(e + 1) * rows].double() @ w[e].double().T for e in range(E)])
+    assert (got.double() - ref).norm() <= most * ref.norm()
+
+
 @pytest.mark.parametrize("counts,H,I,S", [([40, 30, 33, 0, 96, 1, 70, 128] * 2, 2056, 1024, 2), ([25, 64, 65, 129], 4104, 2048, 4)])
 def test_slices_of_groups(gpu, counts, H, I, S):
     from adaptivetrainingsystem_amd import ops
