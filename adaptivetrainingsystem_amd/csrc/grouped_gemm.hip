@@ -1829,17 +1829,27 @@ struct SliceEstimate {
     static float join(float a, float b) { return sqrtf(a * a + b * b); }
     // bm rows x 256 columns, one to a CU; pitch: rows of 8 KB or a multiple of it ask few of the memory's channels at a time
     struct Tall { float bm, slab, slab_row, tile, rate, start, parts, pitch; };
-    float tall(const Tall& c, int s) const {
+    float tall(const Tall& c, int s, float* rounds_out = nullptr) const {
         const int n_tiles = (N + 255) / 256;
         int sm, sn;
         pick_supertile(n_tiles, &sm, &sn);
         const float m = s * roundf(E * row_tiles(c.bm)), super = ceilf(m / sm) * ((n_tiles + sn - 1) / sn);
         const float rounds = fmaxf(1.f, ceilf(ceilf(super / kNumXcd) * (m * n_tiles / (super * kSuperBlocks)) - 0.02f));
+        if (rounds_out) *rounds_out = rounds;
         const float chain = rounds * (slabs / s * (c.slab + c.slab_row * fminf(avg, c.bm)) + c.tile);
         const float load = weights / c.rate * sqrtf(sqrtf(kNumXcd / fminf(super, kNumXcd))) * (K % 4096 == 0 ? 1.f + c.pitch : 1.f);
         return c.start + join(chain, load) + partials * s / c.parts;
     }
-    float large(int s) const { return tall(Tall{256.f, 0.75f, 0.0016f, 7.7f, 6.5f, 5.1f, 5.7f, 0.11f}, s); }
+    float large(int s, float* rounds = nullptr) const { return tall(Tall{256.f, 0.75f, 0.0016f, 7.7f, 6.5f, 5.1f, 5.7f, 0.11f}, s, rounds); }
+    // Slices on it against the band tiles.  Fitted before the ONCE instance, which takes 4 .. 14 % less where one round of tiles fills the
+    // chip and rows are no multiple of 8 KB: 8 x [4096, 14336] of 48 .. 72 rows in two slices 158-161 us, on the band tiles 164-172.  Where sizes
+    // fall as rank^-1.5 its taller tiles hold the largest group (two fifths of all rows) up to 600 rows in all: 166-176 for 182-193.
+    bool large_beats_band(int s) const {
+        float rounds;
+        const float time = large(s, &rounds) + 2.f;
+        return s > 1 && avg <= 72.f && max_rows <= 600 && once_slices(max_rows, E, N, K) && K / s >= 512 && rounds == 1.f && K % 4096 != 0 &&
+               0.93f * time < fminf(small(s), band(s));
+    }
     // 32 or 64 rows x 128 columns, slices of K over workgroups; a row band is launched as whole supertiles of 32 columns' tiles, and
     // the workgroups without a tile cost a microsecond per round
     float small(int s) const {
@@ -1888,7 +1898,7 @@ static bool large_slice_tile(int E, int64_t max_rows, int N, int K, int s) {
     if (K / s < 512) return (int64_t)E * ((N + 255) / 256) * s >= 128;
     if ((int64_t)E * N * K < (1 << 24)) return false;
     const SliceEstimate t(E, max_rows, N, K);
-    return t.large_with_margin(s) < t.small(s);
+    return t.large_with_margin(s) < t.small(s) || t.large_beats_band(s);
 }
 
 // The band tiles (grouped_gemm_band.hpp) for E > 1 groups.  They lose where a group needs a second tile while the first ones fill no
@@ -1966,7 +1976,8 @@ static GroupedRoute grouped_route(const GroupedArgs& p, int64_t max_rows) {
     const int band_tiles = (p.N_out + (SWIGLU ? kBandCols / 2 : kBandCols) - 1) / (SWIGLU ? kBandCols / 2 : kBandCols);
     if constexpr (kBf16 && !SWIGLU && std::is_same<TO, float>::value) {
         if (p.k_splits > 1 && band_ok && p.k_slice % 64 == 0 &&
-            (E == 1 ? max_rows > 32 : (int64_t)E * p.N_out * p.K >= 1 << 24 && avg > 20 && band_groups(E, max_rows, band_tiles, p.k_splits, false)))
+            (E == 1 ? max_rows > 32 : ((int64_t)E * p.N_out * p.K >= 1 << 24 && avg > 20 && band_groups(E, max_rows, band_tiles, p.k_splits, false) &&
+                                      !SliceEstimate(E, max_rows, p.N_out, p.K).large_beats_band(p.k_splits))))
             return {Route::kBandSlices};
     }
     if constexpr (!SWIGLU) {
@@ -2555,7 +2566,8 @@ extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K, int smal
     if (E <= 0 || max_rows <= 0 || N <= 0 || K <= 0 || small < 1) return 1;
     const SliceEstimate t(E, max_rows, N, K);
     auto band = [&](int s) {
-        return E > 1 && max_rows / E > 20 && K % (s * 64) == 0 && band_groups(E, max_rows, (N + kBandCols - 1) / kBandCols, s, false);
+        return E > 1 && max_rows / E > 20 && K % (s * 64) == 0 && band_groups(E, max_rows, (N + kBandCols - 1) / kBandCols, s, false) &&
+               !t.large_beats_band(s);
     };
     float best = band(1) ? t.band(1) : t.plain();
     int slices = 1;
@@ -2567,7 +2579,7 @@ extern "C" int ats_down_k_slices(int E, int64_t max_rows, int N, int K, int smal
         const bool on_band = band(s);
         if (!on_band && !large_slice_tile(E, max_rows, N, K, s)) continue;
         // (0.7: against another fit than its own; 8 x [1024, 2048], 44 rows 16.6 us plain, 17.3 in four slices)
-        const float time = on_band ? t.band(s) + (band(1) ? 0.f : 0.7f) : t.large_with_margin(s);
+        const float time = on_band ? t.band(s) + (band(1) ? 0.f : 0.7f) : t.large_beats_band(s) ? 0.93f * (t.large(s) + 2.f) : t.large_with_margin(s);
         if (time < best) {
             best = time;
             slices = s;

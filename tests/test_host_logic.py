@@ -447,3 +447,12 @@ def test_route_of_one_weight(rows, N, K, slices, route):
     assert ops.linear_k_splits(rows, N, K, torch.bfloat16) == slices
     if route:
         assert _lib.load().ats_grouped_gemm_route(1, rows, N, K, 1, 0, _lib.ATS_BF16) == {"small": 1, "band": 2, "256": 4}[route]
+
+
+@pytest.mark.parametrize("E,rows,N,K,slices,route", [(8, 32, 4096, 14336, 2, 2), (8, 48, 4096, 14336, 2, 5), (8, 72, 4096, 14336, 2, 5), (16, 64, 2048, 5632, 2, 2),
+                                                     (12, 64, 2048, 5632, 4, 2), (4, 64, 4096, 14336, 2, 2), (8, 48, 2048, 5632, 2, 2)])
+def test_tiles_of_a_sliced_down_projection(E, rows, N, K, slices, route):
+    """Band tiles (2) or 256-row tiles (5) for the slices that the rule chooses, as measured with equal and with unequal groups."""
+    from adaptivetrainingsystem_amd import _lib, ops
+    assert ops.down_k_splits(E, E * rows, N, K, torch.bfloat16) == slices
+    assert _lib.load().ats_grouped_gemm_route(E, E * rows, N, K, slices, 0, _lib.ATS_F32) == route
