@@ -1915,7 +1915,7 @@ static bool band_groups(int E, int64_t max_rows, int n_tiles, int slices, bool s
     return used * n_tiles * slices >= 200.f;
 }
 // One group of more than 32 rows x [N, K]: the band tiles' time in microseconds, plain or with s slices of K and their sum, by the
-// tiles' most rows h.  A CU takes one slab of a tile in slab1 alone and in slabn as one of several.  Fitted to 1900 launches of 33 .. 1000
+// tiles' most rows h.  A CU takes one slab of a tile in slab1 alone and in slabn as one of several.  Fitted to 1500 launches of 33 .. 1000
 // rows x [512 .. 32000, 512 .. 14336], weights from HBM, within 6 % (root mean square; 22 % at most).
 static float band_time(int64_t rows, int N, int K, int s, int h) {
     constexpr float slab1[] = {0.44f, 0.55f, 0.67f}, slabn[] = {0.44f, 0.48f, 0.54f};      // up to 64, 96, 128 rows
@@ -1931,7 +1931,7 @@ static int band_height(int64_t rows, int N, int K, int s) {
 }
 // The same rows on the tile that pick_group_tile takes for them: up to 192 rows the register-staged ones, two workgroups of which share a
 // CU (the launches above, within 9 %), beyond that the 256-column tile.  What the choice between the two and the slices costs over those
-// launches is 0.8 % on average, 18 % at most (with the constants of 109 points of [2048 .. 6144] x [2048, 4096], and small tiles also
+// launches is 0.9 % on average, 18 % at most (with the constants of 109 points of [2048 .. 6144] x [2048, 4096], and small tiles also
 // beyond 192 rows, where none run: 5.6 %, 140 %).  Microseconds, band tiles <- other: 200 rows x [512, 512] 6.9 <- 10.5, [1024, 1024] 10.3 <- 15.0,
 // 512 x [1024, 4096] 32 <- 56, 100 x [32000, 4096] 67 <- 91; other <- band tiles: 160 x [3072, 1024] 9.0 <- 10.6, 64 x [2048, 2048] 9.5 <- 17.
 static float other_dense_time(int64_t rows, int N, int K) {
